@@ -84,6 +84,16 @@ def test_error_codes_without_gpu(rt):
     assert L.vpx_nce_task(C.byref(t), None) == rt.ERROR_INVALID_NULL_HANDLE
 
 
+@pytest.mark.parametrize("value", ["1,1,0", "0,1,1", "1,0,1", "1,1,9", "2,2,-1", "4,4,2", "2,4,4", "3,1,1", "65536,1,1"])
+def test_a_tile_that_no_kernel_has_is_refused(rt, value):
+    """(no waves, or a tile of no channels or positions, ended the process at the next layer)"""
+    with pytest.raises(rt.VpxError) as e:
+        rt.set_tuning("VPX_NCE_DIRECT", value)
+    assert e.value.code == rt.ERROR_INVALID_ARGUMENT and value in e.value.text
+    for good in ("1,1,8", "2,2,4", "2,1,3", "2,4,1", "4,4,1", "off", None):
+        rt.set_tuning("VPX_NCE_DIRECT", good)
+
+
 def test_half_conversion_matches_oracle(rt, orc):
     L = rt.lib()
     rng = np.random.default_rng(11)
