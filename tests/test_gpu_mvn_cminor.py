@@ -94,3 +94,17 @@ def test_in_a_graph(rt, dev):
         graph.replay()
         torch.cuda.synchronize()
         assert close(y, want(x))
+
+
+def test_more_workgroups_than_a_launch_holds(rt, dev):
+    """65535 images of 128 blocks of 64 channels would be 2^32 lanes in one launch: the three-launch path has them."""
+    import torch
+    shape = (65535, 2, 1, 8192)
+    g = torch.Generator(device="cuda").manual_seed(1)
+    x = torch.randint(-2048, 2048, shape, dtype=torch.int16, device=dev, generator=g).half()
+    y = torch.full(shape, 7.0, dtype=torch.float16, device=dev)
+    rt.mvn(x, y, False, True, 1e-5, "NHWC")
+    for n in (0, 1, 32767, 65533, 65534):
+        assert close(y[n:n + 1], want(x[n:n + 1]))
+    # two values differ from their mean by the same amount: 0 or plus and minus one
+    assert bool((y[:, 0].abs() <= 1.001).all()) and torch.equal(y[:, 0], -y[:, 1])

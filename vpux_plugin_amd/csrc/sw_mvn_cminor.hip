@@ -478,6 +478,9 @@ int launch_mvn_cminor_resident(const void* in, void* out, int64_t N, int64_t S, 
     // In place, a workgroup that has to read its partners' values again could find results there: those launches take
     // the kernels that finish all reads first.  (A workgroup alone with its channels reads everything before it writes.)
     if (best.parts > 1 && in == out) return VPX_RESULT_SUCCESS;
+    // A launch holds fewer than 2^32 lanes; small images of many channels ask for more from N * nb = 2^23 on.
+    const uint64_t blocks = ((uint64_t)best.units + 7) / 8 * best.nb * 8;
+    if (blocks * kT >= (1ull << 32)) return VPX_RESULT_SUCCESS;
     void* sync = nullptr;
     if (best.parts > 1) {
         rc = get_sync_area(s, &sync);
@@ -485,7 +488,7 @@ int launch_mvn_cminor_resident(const void* in, void* out, int64_t N, int64_t S, 
         sync = (char*)sync + kSyncCminor;
     }
     const unsigned long long spin = mode == 2 ? 0ull : 50000ull;  // 0.5 ms of the 100 MHz counter
-    const dim3 grid((best.units + 7) / 8 * best.nb * 8);
+    const dim3 grid((unsigned)blocks);
 #define VPX_CMINOR_AS(V, FORM) \
     hipLaunchKernelGGL((mvn_cminor_resident<V, FORM>), grid, dim3(kT), 0, s, (const half_t*)in, (half_t*)out, best, (unsigned*)sync, nv, eps, spin)
 #define VPX_CMINOR(V)                         \
