@@ -36,6 +36,20 @@ def test_large(rt, dev, shape):
     check(rt, dev, shape, 1)
 
 
+def test_more_slabs_than_a_launch_holds(rt, dev):
+    """2^24 workgroups of four waves are 2^32 lanes."""
+    import torch
+    shape = (1 << 24, 17, 3)
+    g = torch.Generator(device="cuda").manual_seed(2)
+    x = torch.randint(-9, 10, shape, dtype=torch.int8, device=dev, generator=g).half()
+    y = torch.empty_like(x)
+    rt.softmax(x, y, 1)
+    for part in (slice(0, 1000), slice(1 << 23, (1 << 23) + 1000), slice((1 << 24) - 1000, None)):
+        want = torch.softmax(x[part].float(), 1)
+        assert bool(((y[part].float() - want).abs() <= 2e-3 * want + 2.0 ** -24).all())
+    assert bool(((y.sum(1, dtype=torch.float32) - 1).abs() < 0.01).all())
+
+
 @pytest.mark.parametrize("rows,length", [(64, 17), (65, 18), (1836, 17), (4096, 33), (12 * 161, 161), (513, 255), (70000, 31)])
 def test_short_packed_rows(rt, dev, rows, length):
     check(rt, dev, (rows, length), 1)

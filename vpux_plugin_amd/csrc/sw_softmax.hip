@@ -12,7 +12,8 @@
 //   rows_block : innermost axis of any length or alignment: one workgroup per row, three passes.
 //   slabs      : fp16 reduction over an outer axis of up to 1024 steps with contiguous inner
 //                dimensions: the whole [axis x columns] slab of a wave or a workgroup sits in registers.
-//   lines      : any other reduction over an outer (strided) axis: one lane per line, lanes adjacent
+//   cols       : longer axes over runs of 64 columns and more, padded axes, fp32: running maximum and sum per wave.
+//   lines      : any other reduction over an outer (strided) axis, tensors of more tiles than a launch holds among them: one lane per line, lanes adjacent
 //                along the innermost dimension so every step of the axis is a coalesced access.
 #include <type_traits>
 
@@ -1017,20 +1018,21 @@ int softmax_typed(const SoftmaxPlan& p, const T* in, T* out, hipStream_t s) {
                 vec = 2;
                 kw = len <= 16 ? 1 : (len <= 64 ? 4 : (len <= 256 ? 8 : 16));
             }
-            const int cols = (narrow ? 16 : 64) * vec, tpo = (int)((inner + cols - 1) / cols);
+            const int cols = (narrow ? 16 : 64) * vec;
+            const int64_t tpo = (inner + cols - 1) / cols;
             tiles = outer * tpo;
-            VPX_REQUIRE(tiles < (1ll << 31), VPX_RESULT_ERROR_UNSUPPORTED_FEATURE, "softmax: %lld tiles exceed the launch limit",
-                        (long long)tiles);
-            const half_t* hin = reinterpret_cast<const half_t*>(in);
-            half_t* hout = reinterpret_cast<half_t*>(out);
             const int L = (int)len, I = (int)inner, shares = kw * (narrow ? 4 : 1), steps = (L + shares - 1) / shares;
-            // rows that do not start on cache lines: neighbouring tiles share a line of every row, which one die's L2 puts
-            // together ([1,213,303,470] 41 -> 30 us).  Rows on lines share none, and dies far apart in a row of a power of two
-            // would meet on the same memory channels ([1,150,512,512] 28 -> 37 us): those keep the plain order.
-            bool lines = ((reinterpret_cast<uintptr_t>(in) | reinterpret_cast<uintptr_t>(out)) & 127) == 0 && in_as % 64 == 0 && out_as % 64 == 0;
-            for (int d = 0; d < om.nd; d++) lines = lines && om.in_stride[d] % 64 == 0 && om.out_stride[d] % 64 == 0;
-            const int by_die = lines ? 0 : 1;
-            const dim3 grid((unsigned)(kw == 1 ? (tiles + 3) / 4 : tiles)), block(kw == 1 ? 256 : 64 * kw);
+            const bool fits = (kw == 1 ? (tiles + 3) / 4 * 4 : tiles) * kw < (1ll << 26);  // 2^32 lanes in a launch
+            if (fits) {
+                const half_t* hin = reinterpret_cast<const half_t*>(in);
+                half_t* hout = reinterpret_cast<half_t*>(out);
+                // rows that do not start on cache lines: neighbouring tiles share a line of every row, which one die's L2 puts
+                // together ([1,213,303,470] 41 -> 30 us).  Rows on lines share none, and dies far apart in a row of a power of two
+                // would meet on the same memory channels ([1,150,512,512] 28 -> 37 us): those keep the plain order.
+                bool lines = ((reinterpret_cast<uintptr_t>(in) | reinterpret_cast<uintptr_t>(out)) & 127) == 0 && in_as % 64 == 0 && out_as % 64 == 0;
+                for (int d = 0; d < om.nd; d++) lines = lines && om.in_stride[d] % 64 == 0 && om.out_stride[d] % 64 == 0;
+                const int by_die = lines ? 0 : 1;
+                const dim3 grid((unsigned)(kw == 1 ? (tiles + 3) / 4 : tiles)), block(kw == 1 ? 256 : 64 * kw);
 #define VPX_SLAB_NT(VEC, KW, SMAX, CL, NT) \
     hipLaunchKernelGGL((softmax_slab_f16<VEC, KW, SMAX, CL, NT>), grid, block, 0, s, hin, hout, om, tiles, tpo, L, I, in_as, out_as, by_die)
 #define VPX_SLAB(VEC, KW, SMAX)                                      \
@@ -1038,24 +1040,25 @@ int softmax_typed(const SoftmaxPlan& p, const T* in, T* out, hipStream_t s) {
         if (small) VPX_SLAB_NT(VEC, KW, SMAX, 64, false);            \
         else VPX_SLAB_NT(VEC, KW, SMAX, 64, true);                   \
     } while (0)
-            if (narrow && kw == 1) VPX_SLAB_NT(2, 1, 4, 16, false);
-            else if (narrow && kw == 4) VPX_SLAB_NT(2, 4, 4, 16, false);
-            else if (narrow && kw == 8) VPX_SLAB_NT(2, 8, 8, 16, false);
-            else if (narrow) VPX_SLAB_NT(2, 16, 16, 16, false);
-            else if (kw == 1) { if (steps <= 4) VPX_SLAB(4, 1, 4); else VPX_SLAB(4, 1, 8); }
-            else if (kw == 2) VPX_SLAB(4, 2, 8);
-            else if (kw == 4) { if (steps <= 4) VPX_SLAB(2, 4, 4); else if (steps <= 8) VPX_SLAB(2, 4, 8); else VPX_SLAB(2, 4, 16); }
-            else if (kw == 8) {
-                if (steps <= 4) VPX_SLAB(2, 8, 4); else if (steps <= 8) VPX_SLAB(2, 8, 8); else if (steps <= 16) VPX_SLAB(2, 8, 16);
-                else if (steps <= 24) VPX_SLAB(2, 8, 24); else if (steps <= 32) VPX_SLAB(2, 8, 32); else VPX_SLAB(2, 8, 64);
-            } else {
-                if (steps <= 8) VPX_SLAB(2, 16, 8); else if (steps <= 16) VPX_SLAB(2, 16, 16); else if (steps <= 24) VPX_SLAB(2, 16, 24);
-                else if (steps <= 32) VPX_SLAB(2, 16, 32); else VPX_SLAB(2, 16, 64);
-            }
+                if (narrow && kw == 1) VPX_SLAB_NT(2, 1, 4, 16, false);
+                else if (narrow && kw == 4) VPX_SLAB_NT(2, 4, 4, 16, false);
+                else if (narrow && kw == 8) VPX_SLAB_NT(2, 8, 8, 16, false);
+                else if (narrow) VPX_SLAB_NT(2, 16, 16, 16, false);
+                else if (kw == 1) { if (steps <= 4) VPX_SLAB(4, 1, 4); else VPX_SLAB(4, 1, 8); }
+                else if (kw == 2) VPX_SLAB(4, 2, 8);
+                else if (kw == 4) { if (steps <= 4) VPX_SLAB(2, 4, 4); else if (steps <= 8) VPX_SLAB(2, 4, 8); else VPX_SLAB(2, 4, 16); }
+                else if (kw == 8) {
+                    if (steps <= 4) VPX_SLAB(2, 8, 4); else if (steps <= 8) VPX_SLAB(2, 8, 8); else if (steps <= 16) VPX_SLAB(2, 8, 16);
+                    else if (steps <= 24) VPX_SLAB(2, 8, 24); else if (steps <= 32) VPX_SLAB(2, 8, 32); else VPX_SLAB(2, 8, 64);
+                } else {
+                    if (steps <= 8) VPX_SLAB(2, 16, 8); else if (steps <= 16) VPX_SLAB(2, 16, 16); else if (steps <= 24) VPX_SLAB(2, 16, 24);
+                    else if (steps <= 32) VPX_SLAB(2, 16, 32); else VPX_SLAB(2, 16, 64);
+                }
 #undef VPX_SLAB_NT
 #undef VPX_SLAB
-            VPX_HIP_CHECK(hipGetLastError());
-            return VPX_RESULT_SUCCESS;
+                VPX_HIP_CHECK(hipGetLastError());
+                return VPX_RESULT_SUCCESS;
+            }
         }
     }
     // outer axis, contiguous inner run of at least 64 columns: wavefronts along the axis, lanes along the columns
@@ -1093,18 +1096,18 @@ int softmax_typed(const SoftmaxPlan& p, const T* in, T* out, hipStream_t s) {
                     break;
                 }
             const int64_t tpo = (inner + 64 * vec - 1) / (64 * vec);
-            VPX_REQUIRE(outer * tpo < (1ll << 31), VPX_RESULT_ERROR_UNSUPPORTED_FEATURE, "softmax: %lld tiles exceed the launch limit",
-                        (long long)(outer * tpo));
-            const dim3 grid((unsigned)(outer * tpo));
+            if (outer * tpo < (1ll << 22)) {  // 2^32 lanes in a launch
+                const dim3 grid((unsigned)(outer * tpo));
 #define VPX_COLS(V) hipLaunchKernelGGL((softmax_cols<T, V>), grid, dim3(1024), 0, s, in, out, om, (int)tpo, len, valid, inner, in_as, out_as)
-            if (vec == 8) {
-                if constexpr (sizeof(T) == 2) VPX_COLS(8);
-            } else if (vec == 4) VPX_COLS(4);
-            else if (vec == 2) VPX_COLS(2);
-            else VPX_COLS(1);
+                if (vec == 8) {
+                    if constexpr (sizeof(T) == 2) VPX_COLS(8);
+                } else if (vec == 4) VPX_COLS(4);
+                else if (vec == 2) VPX_COLS(2);
+                else VPX_COLS(1);
 #undef VPX_COLS
-            VPX_HIP_CHECK(hipGetLastError());
-            return VPX_RESULT_SUCCESS;
+                VPX_HIP_CHECK(hipGetLastError());
+                return VPX_RESULT_SUCCESS;
+            }
         }
     }
     const unsigned blocks = (unsigned)((rows + 255) / 256);
