@@ -36,6 +36,13 @@ def test_large(rt, dev, shape):
     check(rt, dev, shape, 1)
 
 
+@pytest.mark.parametrize("shape", [(5000, 2, 3), (20000, 8, 5), (3000, 9, 5), (10922, 16, 24), (31837, 17, 31), (700, 40, 7), (8000, 64, 33), (11185, 100, 15),
+                                   (90, 300, 3), (1900, 500, 63), (9709, 9, 79), (66052, 2, 127)])
+def test_short_runs(rt, dev, shape):
+    """Runs shorter than a tile, on either side of the rule between a slab and a lane per line."""
+    check(rt, dev, shape, 1)
+
+
 def test_more_slabs_than_a_launch_holds(rt, dev):
     """2^24 workgroups of four waves are 2^32 lanes."""
     import torch

@@ -13,10 +13,11 @@
 //   slabs      : fp16 reduction over an outer axis of up to 1024 steps with contiguous inner
 //                dimensions: the whole [axis x columns] slab of a wave or a workgroup sits in registers.
 //   cols       : longer axes over runs of 64 columns and more, padded axes, fp32: running maximum and sum per wave.
-//   lines      : any other reduction over an outer (strided) axis, tensors of more tiles than a launch holds among them: one lane per line, lanes adjacent
+//   lines      : any other reduction over an outer (strided) axis, runs too short for a tile and tensors of more tiles than a launch holds among them: one lane per line, lanes adjacent
 //                along the innermost dimension so every step of the axis is a coalesced access.
 #include <type_traits>
 
+#include <cmath>
 #include <cstdlib>
 
 #include "vpx_common.h"
@@ -829,6 +830,21 @@ void launch_rows_wave(const T* in, T* out, const RowMap& map, int64_t rows, int 
     hipLaunchKernelGGL((softmax_rows_wave<T, NV, ROWS>), dim3(blocks), dim3(256), 0, s, in, out, map, rows, len, valid);
 }
 
+// What the two kernels for an outer axis take, us: fitted to 1530 tensors of 2^16 ... 2^24 values in runs of 2 ... 127, axes of
+// 2 ... 1000 steps (its choice is within 10 % of the better one for all but 26 of them, at worst 49 % above it).
+// A slab tile: its `columns_x_waves` lanes' registers, half of them with a value; a partial vector goes value by value.
+double slab_microseconds(int64_t tiles, int columns_x_waves, int steps, bool partial) {
+    int held = 4;  // steps a wave has registers for
+    while (held < steps) held *= 2;
+    const double per_tile = 0.09 + (partial ? 0.079 : 0.05) * 0.25 * columns_x_waves * (held + steps);
+    return 2.9 + (partial ? 0.7 : 0.0) + 1e-3 * per_tile * (double)tiles;
+}
+// A lane per line: one step after the other, out of the caches or memory, or what the scattered accesses give.
+double line_microseconds(int64_t elements, int len) {
+    const double m = (double)elements, chain = (0.33 + 0.4 * (m < 16777216.0 ? m / 16777216.0 : 1.0)) * len, bytes = 2.3e-6 * m;
+    return 2.3 + std::sqrt(chain * chain + bytes * bytes);
+}
+
 template <typename T>
 int softmax_typed(const SoftmaxPlan& p, const T* in, T* out, hipStream_t s) {
     constexpr int N = VecTraits<T>::N;
@@ -1023,7 +1039,12 @@ int softmax_typed(const SoftmaxPlan& p, const T* in, T* out, hipStream_t s) {
             tiles = outer * tpo;
             const int L = (int)len, I = (int)inner, shares = kw * (narrow ? 4 : 1), steps = (L + shares - 1) / shares;
             const bool fits = (kw == 1 ? (tiles + 3) / 4 * 4 : tiles) * kw < (1ll << 26);  // 2^32 lanes in a launch
-            if (fits) {
+            // A run shorter than a tile leaves lanes idle, a run of 3 all but two: below 64 columns (128 where a tile ends in a
+            // partial vector, unless softmax_cols has such runs) the cheaper of the two.  Slab / line, us: [2796202,2,3] 1057 / 46,
+            // [31835,17,31] 73 / 40, [11184,100,15] 98 / 87, [5412,100,31] 55 / 88, [1285,17,3] 5.8 / 7.7, [5899,9,79] 15.2 / 9.9.
+            const bool pays = inner >= 128 || (inner >= 64 && (len >= 32 || inner % vec == 0)) ||
+                              slab_microseconds(tiles, kw * vec, steps, inner % vec != 0) <= line_microseconds(elements, L);
+            if (fits && pays) {
                 const half_t* hin = reinterpret_cast<const half_t*>(in);
                 half_t* hout = reinterpret_cast<half_t*>(out);
                 // rows that do not start on cache lines: neighbouring tiles share a line of every row, which one die's L2 puts
