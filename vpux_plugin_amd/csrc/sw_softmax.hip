@@ -13,8 +13,9 @@
 //   slabs      : fp16 reduction over an outer axis of up to 1024 steps with contiguous inner
 //                dimensions: the whole [axis x columns] slab of a wave or a workgroup sits in registers.
 //   cols       : longer axes over runs of 64 columns and more, padded axes, fp32: running maximum and sum per wave.
-//   lines      : any other reduction over an outer (strided) axis, runs too short for a tile and tensors of more tiles than a launch holds among them: one lane per line, lanes adjacent
-//                along the innermost dimension so every step of the axis is a coalesced access.
+//   lines      : any other reduction over an outer (strided) axis, runs too short for a tile and tensors of more tiles than a
+//                launch holds among them: one lane per line, lanes adjacent along the innermost dimension so every step of the
+//                axis is a coalesced access.
 #include <type_traits>
 
 #include <cmath>
