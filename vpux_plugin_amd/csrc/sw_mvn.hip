@@ -490,7 +490,7 @@ constexpr int kSyncStride = 64;            // words per group in the sync area: 
 // its own group's launch count
 constexpr size_t kSyncRecords = 4 * 1024;  // byte offset of the records in the sync area (the groups' counters before it)
 static_assert(kFusedMaxGroups * kSyncStride * sizeof(unsigned) <= kSyncRecords &&
-              kSyncRecords + sizeof(Record) * kFusedMaxGroups * kMergeInKernel <= kSyncBytes, "sync area layout");
+              kSyncRecords + sizeof(Record) * kFusedMaxGroups * kMergeInKernel <= kSyncCminor, "sync area layout");
 
 // A published slice: two 64-bit words, {mean, tag} and {M2, tag}, each written and read as one access that goes
 // through to memory (agent scope), so neither needs the other to be valid; the count of a slice follows from its index.

@@ -43,6 +43,9 @@ struct Geom {
 struct __attribute__((aligned(16))) Tagged {
     unsigned long long sum, sq;
 };
+static_assert(kSyncCminor + sizeof(unsigned) * kCountStride * (kMostGroups + kMostRowGroups) +
+                      sizeof(Tagged) * ((size_t)kMostGroups * kMostRecords + (size_t)kMostRowGroups * kMostRowRecords) <=
+                  kSyncBytes, "sync area layout");
 __device__ __forceinline__ unsigned long long tagged(float v, unsigned tag) {
     return (unsigned long long)__builtin_bit_cast(unsigned, v) | ((unsigned long long)tag << 32);
 }
