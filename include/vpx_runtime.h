@@ -237,8 +237,8 @@ VPX_API int vpx_nce_task(const vpx_nce_task_t* task, void* stream);
  * "VPX_CONV_KERNEL" (regw | tile | stream), "VPX_CONV_ROWS" (n), "VPX_CONV_COLS" (n), "VPX_CONV_WAVES" (4 | 8), "VPX_STREAM_KSPLIT" (off: the streamed-weights
  * convolution kernel gives every wave a 32 x 32 tile also on small planes, instead of splitting K over the waves of a group),
  * "VPX_MVN_FUSED" (off: long MVN groups take
- * the two-launch kernels; nowait: the one-launch kernel's workgroups do not wait for each other and each recomputes its
- * group's statistics, the path taken when they are not all resident), "VPX_CALIB_BLOCKS" (n: workgroups of
+ * the two-launch kernels and channel-minor tensors the three-launch ones; nowait: the one-launch kernels' workgroups do not
+ * wait for each other and each computes what it finds missing, the path taken when they are not all resident), "VPX_CALIB_BLOCKS" (n: workgroups of
  * vpx_calib_mfma_i8, by default one per compute unit); `value` NULL or "" restores the default.
  * Environment variables of the same names give the initial values; they are read once, at the first NCE task or the
  * first call of this function, never during a launch.  Process-wide; results do not depend on any of them. */

@@ -46,7 +46,7 @@ def test_shapes(rt, dev, shape, offset):
 
 
 def test_launch_after_launch(rt, dev):
-    """Launches of different geometry share the counters and the records."""
+    """Launches of different geometry share the launch counts and the records."""
     import torch
     sets = [make(dev, s) for s in ((1, 224, 224, 64), (2, 101, 99, 34), (16, 56, 56, 208), (2, 37, 55, 16), (4, 112, 112, 256))]
     firsts = []

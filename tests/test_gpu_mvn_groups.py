@@ -52,3 +52,60 @@ def test_images_without_waiting(rt, dev, shape):
     finally:
         rt.set_tuning("VPX_MVN_FUSED", None)
     assert torch.equal(y, z)
+
+
+# a group per image: 1 ... 16 groups, 2 ... 256 workgroups each
+SHAPES = [(1, 3, 64, 65), (16, 7, 49, 51), (3, 5, 63, 65), (1, 64, 257, 255), (1, 1, 65, 64), (2, 31, 201, 203), (7, 3, 50, 50)]
+
+
+def test_launch_after_launch(rt, dev):
+    """Launches of different geometry, waiting or not, share the launch counts and the records."""
+    import torch
+    sets = [run(rt, dev, s, True) for s in SHAPES]
+    for k in range(60):
+        x, y = sets[k * 3 % len(sets)]
+        z = torch.zeros_like(y)
+        rt.set_tuning("VPX_MVN_FUSED", "nowait" if k % 4 == 3 else None)
+        try:
+            rt.mvn(x, z, True, True, 1e-5, "NCHW")
+        finally:
+            rt.set_tuning("VPX_MVN_FUSED", None)
+        assert torch.equal(z, y), SHAPES[k * 3 % len(sets)]
+
+
+@pytest.mark.parametrize("shape,across,order", [((4, 256, 64, 64), True, "NCHW"), ((1, 3200, 128, 128), True, "NCHW"), ((1, 448, 448, 256), False, "NHWC"),
+                                                ((1, 900, 900, 17), False, "NHWC")])
+def test_beside_a_launch_that_holds_compute_units(rt, dev, shape, across, order):
+    """With 32 compute units left the workgroups start in eight rounds.  The first one waits 0.5 ms, computes what is missing
+    and publishes it; the others find it.  The time is bounded by that and some passes over the tensor (104 MB in 0.4 ms at the
+    rate of 32 compute units, both ways), not by a wait and the whole tensor for every workgroup (29 ms)."""
+    import time
+    import torch
+    g = torch.Generator(device="cuda").manual_seed(3)
+    x = (torch.rand(shape, device=dev, generator=g) * 16 - 8).half()
+    alone, beside = torch.empty_like(x), torch.empty_like(x)
+    src = torch.zeros((65536,), device=dev, dtype=torch.int8)
+    cus = torch.cuda.get_device_properties(0).multi_processor_count
+    sink = torch.empty((cus * 8192,), device=dev, dtype=torch.uint8)
+    torch.cuda.synchronize()
+    a, b = torch.cuda.Stream(), torch.cuda.Stream()
+    start, end = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+    rt.set_tuning("VPX_CALIB_BLOCKS", str(max(1, cus - 32)))
+    try:
+        with torch.cuda.stream(a):
+            rt.mvn(x, alone, across, True, 1e-5, order)
+        rt.calib_mfma_i8(src, sink, 200)
+        torch.cuda.synchronize()
+        with torch.cuda.stream(b):
+            rt.calib_mfma_i8(src, sink, 60000)  # about 26 ms
+        time.sleep(0.002)
+        with torch.cuda.stream(a):
+            start.record()
+            rt.mvn(x, beside, across, True, 1e-5, order)
+            end.record()
+        torch.cuda.synchronize()
+    finally:
+        rt.set_tuning("VPX_CALIB_BLOCKS", None)
+    assert torch.equal(alone, beside)
+    print("%s beside a launch on %d of %d compute units: %.3f ms" % (shape, cus - 32, cus, start.elapsed_time(end)))
+    assert start.elapsed_time(end) < 4.0

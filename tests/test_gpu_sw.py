@@ -969,10 +969,9 @@ def test_mvn_config_c3_full_size(rt, orc, dev):
 
 @pytest.mark.parametrize("shape", [(4, 64, 64, 64), (1, 3, 72, 200), (3, 5, 40, 104), (7, 2, 64, 40), (2, 33, 97, 8), (1, 128, 128, 128)])
 def test_mvn_one_launch_kernel_and_its_fallback(rt, orc, dev, shape):
-    """Long groups in one launch (workgroups of a group meet at the group's counter): against the oracle, bit for bit
-    against the same kernel when no workgroup waits for the others (each recomputes its group's moments, as a
-    workgroup does whose wait runs out), repeated launches (the counters are left at zero), and within tolerance
-    against the two-launch kernels."""
+    """Long groups in one launch (workgroups of a group meet at their records): against the oracle, bit for bit
+    against the same kernel when no workgroup waits for the others (each computes the slices it finds missing, as a
+    workgroup does whose wait runs out), repeated launches, and within tolerance against the two-launch kernels."""
     import torch
     rng = np.random.default_rng(sum(shape))
     x = (rng.uniform(-8, 8, shape) + rng.normal(0, 2, (1, shape[1], 1, 1))).astype(np.float32)
@@ -985,7 +984,7 @@ def test_mvn_one_launch_kernel_and_its_fallback(rt, orc, dev, shape):
     try:
         alone = _mvn(rt, dev, xb, True, True, 1e-9)
         rt.set_tuning("VPX_MVN_FUSED", None)
-        after = _mvn(rt, dev, xb, True, True, 1e-9)  # the counters were left clean by the launch that did not wait
+        after = _mvn(rt, dev, xb, True, True, 1e-9)  # a launch that did not wait leaves counts and records in order
         rt.set_tuning("VPX_MVN_FUSED", "off")
         two = _mvn(rt, dev, xb, True, True, 1e-9)
     finally:
@@ -997,7 +996,7 @@ def test_mvn_one_launch_kernel_and_its_fallback(rt, orc, dev, shape):
 def test_mvn_one_launch_kernel_beside_a_launch_that_holds_compute_units(rt, orc, dev):
     """Configuration 3's MVN on one stream while another stream runs a long launch on all but 32 compute units: only
     some of the MVN kernel's workgroups are resident at a time, those wait for records that cannot arrive, their
-    bounded wait runs out and they compute their group's moments themselves.  Every kernel exits, and the result is
+    bounded wait runs out and they compute the missing slices themselves.  Every kernel exits, and the result is
     the bits of the undisturbed run."""
     import time
     import torch
@@ -1040,8 +1039,8 @@ def test_mvn_one_launch_kernel_beside_a_launch_that_holds_compute_units(rt, orc,
 @pytest.mark.parametrize("shape", [(4, 64, 64, 64), (3, 5, 40, 104), (2, 3, 8, 8), (2, 70, 112, 112)])
 @pytest.mark.parametrize("fused", [None, "nowait"])
 def test_mvn_in_place(rt, orc, dev, shape, fused):
-    """Output tensor = input tensor.  Long groups then leave the one-launch kernel alone (a workgroup that recomputes
-    its group's moments would read slices other workgroups have already normalised): same bits as out of place."""
+    """Output tensor = input tensor.  Long groups then leave the one-launch kernel alone (a workgroup that computes
+    a missing slice would read what its owner may have normalised already): same bits as out of place."""
     import torch
     rng = np.random.default_rng(sum(shape) + 5)
     xb = orc.f32_to_f16((rng.uniform(-8, 8, shape) + rng.normal(0, 2, (1, shape[1], 1, 1))).astype(np.float32))

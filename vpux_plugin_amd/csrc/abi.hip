@@ -44,14 +44,14 @@ struct Scratch {
     void* ptr = nullptr;
     size_t size = 0;
     std::vector<void*> retired;  // outgrown blocks: work already queued may still use them, freed on release
-    void* sync = nullptr;        // kSyncBytes of counters for kernels whose workgroups meet inside one launch
+    void* sync = nullptr;        // kSyncBytes of launch counts and records for kernels whose workgroups meet inside one launch
 };
 std::mutex g_ws_mutex;
 std::map<std::pair<int, hipStream_t>, Scratch> g_ws;
 
 // The fixed scratch array.  Its name is a host-side handle, not a device address: host code uses the per-device
 // address that hipGetSymbolAddress returns (each device holds its own copy of the array).
-// (the counters of the allocation-free entry point sit behind the bytes get_workspace() hands out; device arrays
+// (the launch counts and records of the allocation-free entry point sit behind the bytes get_workspace() hands out; device arrays
 // start as zeros)
 static __device__ __align__(256) unsigned char scratch[VPX_NOALLOC_SCRATCH_BYTES + kSyncBytes];
 constexpr int kMaxDevices = 64;
@@ -122,9 +122,10 @@ int get_workspace(hipStream_t stream, size_t bytes, void** out) {
     return VPX_RESULT_SUCCESS;
 }
 
-// Counters that start as zeros and that every kernel using them leaves as zeros (the last workgroup through resets
-// them), so launches on one stream can share them without a clearing pass.  One area per (device, stream handle),
-// allocated and cleared on first need; nothing else is ever written there.
+// Launch counts and tagged records that start as zeros; a launch leaves its groups' counts moved on by one and its records
+// behind, which carry a tag that no later launch uses, so launches on one stream can share them without a clearing pass.
+// One area of kSyncBytes (8.6 MiB) per (device, stream handle), allocated and cleared on first need (the one-launch MVN
+// kernels, vpx_workspace_reserve); nothing else is ever written there.
 int get_sync_area(hipStream_t stream, void** out) {
     if (t_noalloc) {
         void* base = nullptr;

@@ -480,17 +480,20 @@ int mem_pos_of(uint64_t order, int nd, int logical) {
 // stores; the first wavefront then polls the records of ITS group (not of the whole grid) with loads that bypass the
 // caches until every tag names this launch, merges them in a fixed order and hands the result to the other wavefronts,
 // which normalise the slice from the registers.  No read-modify-write is involved: arrivals do not queue at a counter.
-// The tag is the group's launch count + 1; the count lives in the zero-initialised sync area.  The wait is bounded: a
-// workgroup that does not see its group complete in time (the others are not resident, e.g. the device is shared)
-// computes the group's moments itself, slice by slice with the same arithmetic, so the result is the same bits and
-// every wave exits.
+// The tag is the launch count + 1.  Every workgroup has counts of its own in the zero-initialised sync area (a run of the
+// group's kMergeInKernel, all of which a launch moves on, however many workgroups it has): nobody else writes them during a
+// launch, so a workgroup finds the launch's tag however late it starts, and no record of an earlier launch carries it.
+// The wait is bounded: a workgroup that does not see its group complete in time (the others are not resident: the device is
+// shared) computes missing slices with the same arithmetic and publishes them for their owners and for everyone else, one
+// at a time, each time one that nobody has published yet.  So the result is the same bits, the missing slices are computed
+// about once among those that wait, whoever starts later finds the group complete, and every wave exits: a workgroup
+// computes a slice at most once.  (Each computing all slices for itself took 29 ms for 52 M values beside a launch that held
+// 224 of 256 compute units, eight rounds of workgroups that wait and read the tensor 32 times; now 0.9: the wait, 0.1 for the missing slices, eight rounds.)
 constexpr int kFusedMaxVec = 52;           // 128-bit words per lane of 512, 208 of its 256 registers: the chip holds 54 M values
-constexpr int kSyncStride = 64;            // words per group in the sync area: the launch count at +0, alone in its cache lines
-// kFusedMaxGroups groups at most: each owns a fixed run of kMergeInKernel record slots, so a slot only ever carries tags of
-// its own group's launch count
-constexpr size_t kSyncRecords = 4 * 1024;  // byte offset of the records in the sync area (the groups' counters before it)
-static_assert(kFusedMaxGroups * kSyncStride * sizeof(unsigned) <= kSyncRecords &&
-              kSyncRecords + sizeof(Record) * kFusedMaxGroups * kMergeInKernel <= kSyncCminor, "sync area layout");
+constexpr int kSyncStride = 4;             // words between launch counts
+// kFusedMaxGroups groups at most: each owns a fixed run of kMergeInKernel launch counts and as many record slots
+constexpr size_t kSyncRecords = sizeof(unsigned) * kSyncStride * kFusedMaxGroups * kMergeInKernel;  // byte offset of the records
+static_assert(kSyncRecords + sizeof(Record) * kFusedMaxGroups * kMergeInKernel <= kSyncCminor, "sync area layout");
 
 // A published slice: two 64-bit words, {mean, tag} and {M2, tag}, each written and read as one access that goes
 // through to memory (agent scope), so neither needs the other to be valid; the count of a slice follows from its index.
@@ -582,17 +585,19 @@ __global__ __launch_bounds__(T) void mvn_fused_kernel(const half_t* __restrict__
                                                       uint32_t group_size, int wpg, uint32_t slice, unsigned* sync,
                                                       int normalize_variance, float eps, unsigned long long spin_ticks) {
     __shared__ Moments red[8];
-    __shared__ Moments others[kMergeInKernel];
     __shared__ Moments shared_total;
-    __shared__ int complete;
+    __shared__ int complete, pick;
+    __shared__ unsigned char helped[kMergeInKernel];
     const int64_t group = blockIdx.x / wpg;
     const int part = blockIdx.x % wpg;
     const int lane = threadIdx.x & 63;
-    unsigned* count = sync + group * kSyncStride;
-    Tagged* mine = reinterpret_cast<Tagged*>(reinterpret_cast<char*>(sync) + kSyncRecords) + group * kMergeInKernel;
+    // this workgroup's launch counts
+    unsigned* counts = sync + group * (kMergeInKernel * kSyncStride);
+    const int first_count = part * kMergeInKernel / wpg, end_count = (part + 1) * kMergeInKernel / wpg;
+    Tagged* records = reinterpret_cast<Tagged*>(reinterpret_cast<char*>(sync) + kSyncRecords) + group * kMergeInKernel;
     unsigned tag = 0;
     if (wpg > 1 && threadIdx.x < 64) {
-        tag = __hip_atomic_load(count, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) + 1u;
+        tag = __hip_atomic_load(counts + first_count * kSyncStride, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) + 1u;
         tag = tag == 0u ? 1u : tag;
     }
     const half_t* gin = in + group * group_size;
@@ -602,30 +607,30 @@ __global__ __launch_bounds__(T) void mvn_fused_kernel(const half_t* __restrict__
     load_slice<V, T>(gin, base, end, group_size, sl);
     Moments total = slice_moments<V, T>(sl, red);
     if (wpg > 1) {
-        if (threadIdx.x < 64) {  // the first wavefront
-            if (lane == 0) {
-                __hip_atomic_store(&mine[part].mean, tagged(total.mean, tag), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                __hip_atomic_store(&mine[part].m2, tagged(total.m2, tag), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            }
+        const auto publish = [&](int p, const Moments& m) {  // by one lane of the first wavefront
+            __hip_atomic_store(&records[p].mean, tagged(m.mean, tag), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            __hip_atomic_store(&records[p].m2, tagged(m.m2, tag), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        };
+        unsigned long long rm[kMergeInKernel / 64], rq[kMergeInKernel / 64];
+        const auto poll = [&](int k) {  // record k * 64 + lane; true if it is this launch's, or none
+            const int i = k * 64 + lane;
+            rm[k] = rq[k] = 0;
+            if (i >= wpg) return true;
+            rm[k] = __hip_atomic_load(&records[i].mean, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            rq[k] = __hip_atomic_load(&records[i].m2, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            return (unsigned)(rm[k] >> 32) == tag && (unsigned)(rq[k] >> 32) == tag;
+        };
+        const auto collect = [&](bool waits) {  // the first wavefront: reads the group's records and merges them
             const unsigned long long t0 = wall_clock64();
-            unsigned long long rm[kMergeInKernel / 64], rq[kMergeInKernel / 64];
             bool ok;
             for (;;) {
                 bool ready = true;
 #pragma unroll
-                for (int k = 0; k < kMergeInKernel / 64; k++) {
-                    const int i = k * 64 + lane;
-                    rm[k] = rq[k] = 0;
-                    if (i < wpg) {
-                        rm[k] = __hip_atomic_load(&mine[i].mean, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                        rq[k] = __hip_atomic_load(&mine[i].m2, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                        ready = ready && (unsigned)(rm[k] >> 32) == tag && (unsigned)(rq[k] >> 32) == tag;
-                    }
-                }
+                for (int k = 0; k < kMergeInKernel / 64; k++) ready &= poll(k);
                 ok = __builtin_amdgcn_ballot_w64(!ready) == 0;
-                if (ok || wall_clock64() - t0 >= spin_ticks) break;  // (pausing between polls measured slower)
+                if (ok || !waits || wall_clock64() - t0 >= spin_ticks) break;  // (pausing between polls measured slower)
             }
-            if (ok) {
+            if (ok || !waits) {
                 Moments acc{0.f, 0.f, 0.f};
 #pragma unroll
                 for (int k = 0; k < kMergeInKernel / 64; k++) {
@@ -639,37 +644,61 @@ __global__ __launch_bounds__(T) void mvn_fused_kernel(const half_t* __restrict__
                 const Moments t = wave_merge(acc);
                 if (lane == 0) shared_total = t;
             }
+            return ok;
+        };
+        if (threadIdx.x < 64) {
+            if (lane == 0) publish(part, total);
+            // (here and not behind the meeting: their way to memory then ends under the wait, 0.2 of 8.3 us at [4,256,64,64])
+            for (int i = first_count + lane; i < end_count; i += 64)
+                __hip_atomic_store(counts + i * kSyncStride, tag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            const bool ok = collect(true);
             if (lane == 0) complete = ok ? 1 : 0;
         }
         __syncthreads();
-        if (complete) {
-            total = shared_total;
-        } else {
-            for (int p = 0; p < wpg; p++) {
+        if (!complete) {
+            for (int i = threadIdx.x; i < wpg; i += T) helped[i] = 0;
+            __syncthreads();
+            for (int n = 0; n < wpg; n++) {
+                if (threadIdx.x < 64) {
+                    // of the slices that nobody has published: the one at this workgroup's place among them
+                    unsigned long long missing[kMergeInKernel / 64];
+                    int count = 0;
+#pragma unroll
+                    for (int k = 0; k < kMergeInKernel / 64; k++) {
+                        const bool there = poll(k) || helped[k * 64 + lane];
+                        missing[k] = __builtin_amdgcn_ballot_w64(!there);
+                        count += __builtin_popcountll(missing[k]);
+                    }
+                    int at = count ? part % count : 0, p = -1;
+#pragma unroll
+                    for (int k = 0; k < kMergeInKernel / 64; k++) {
+                        unsigned long long m = missing[k];
+                        const int c = __builtin_popcountll(m);
+                        if (p < 0 && at < c) {
+                            for (; at > 0; at--) m &= m - 1;
+                            p = k * 64 + __builtin_ctzll(m);
+                        }
+                        at -= c;
+                    }
+                    if (lane == 0) pick = p;
+                }
+                __syncthreads();
+                const int p = pick;
+                if (p < 0) break;
                 const uint32_t b = (uint32_t)p * slice;
-                const uint32_t e = p + 1 < wpg ? b + slice : group_size;
-                load_slice<V, T>(gin, b, e, group_size, sl);
+                load_slice<V, T>(gin, b, p + 1 < wpg ? b + slice : group_size, group_size, sl);
                 const Moments mp = slice_moments<V, T>(sl, red);
-                if (threadIdx.x == 0) others[p] = mp;
+                if (threadIdx.x == 0) {
+                    publish(p, mp);
+                    __threadfence();
+                    helped[p] = 1;
+                }
             }
+            if (threadIdx.x < 64) collect(false);
             load_slice<V, T>(gin, base, end, group_size, sl);  // its own again
             __syncthreads();
-            total = merge_partials([&](int i) { return others[i]; }, wpg);  // the order the first wavefront uses above
         }
-        // The group's first workgroup advances the launch count, and it alone: stores of many workgroups to one word
-        // queue up (64 of them cost 1.5 us here).  When its wait was met, every workgroup of the group has read the
-        // count already (a record carries the tag only after its writer has); when its wait ran out, a workgroup that
-        // starts even later reads the advanced count, publishes under the next tag, meets nobody and recomputes, like
-        // everyone else in a launch that far apart.  A workgroup whose wait ran out withdraws its record (tag 0 is
-        // never used), so that whichever tag the next launch uses, the slot is not taken for published until its
-        // owner writes it again.
-        if (threadIdx.x == 0) {
-            if (part == 0) __hip_atomic_store(count, tag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            if (!complete) {
-                __hip_atomic_store(&mine[part].mean, 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                __hip_atomic_store(&mine[part].m2, 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            }
-        }
+        total = shared_total;
     }
     const float mean = total.mean, inv = inv_std(total, normalize_variance, eps);
     half_t* gout = out + group * group_size;
@@ -693,14 +722,14 @@ __global__ __launch_bounds__(T) void mvn_fused_kernel(const half_t* __restrict__
 int launch_fused_groups(const half_t* in, half_t* out, int64_t groups, int64_t group_size, int nv, float eps, hipStream_t s,
                         bool* done) {
     *done = false;
-    const int mode = tuning_mvn_fused();  // 0: never, 1: default, 2: spin limit 0 (every workgroup recomputes)
+    const int mode = tuning_mvn_fused();  // 0: never, 1: default, 2: spin limit 0 (a workgroup computes what it finds missing at once)
     if (mode == 0) return VPX_RESULT_SUCCESS;
     int cus = 0;
     int rc = device_compute_units(&cus);
     if (rc) return rc;
     if (groups > cus || groups > kFusedMaxGroups) return VPX_RESULT_SUCCESS;
-    // In place (or any overlap of the two tensors): a workgroup whose wait runs out reads its whole group again, and by
-    // then other workgroups may have stored their normalised slices over it.  The two-launch kernels finish every
+    // In place (or any overlap of the two tensors): a workgroup whose wait runs out reads slices of others, which
+    // by then may have stored their normalised values over them.  The two-launch kernels finish every
     // read of the statistics before the first store, so overlapping tensors go there.
     {
         const uintptr_t ib = reinterpret_cast<uintptr_t>(in), ob = reinterpret_cast<uintptr_t>(out);

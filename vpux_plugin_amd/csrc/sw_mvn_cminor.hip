@@ -25,7 +25,8 @@ constexpr int kT = 512;
 constexpr int kMostWords = 50;        // words per lane: 200 of the 256 registers of a lane at two wavefronts per SIMD
 constexpr int kAhead = 12;            // words per lane under way: 96 KB a compute unit
 constexpr int kMostGroups = 128;      // groups of workgroups that exchange partial sums
-constexpr int kCountStride = 32;      // words between the groups' launch counts: a cache line each
+constexpr int kMostParts = 256;       // workgroups of a group
+constexpr int kCountStride = 4;       // words between launch counts
 constexpr int kMostRowGroups = 16;    // the same for the form that deals whole rows, with more records each
 constexpr int kMostRowRecords = 16384;
 constexpr int kMostRecords = 2048;    // partial sums a workgroup reads from the workgroups it shares channels with: four per lane
@@ -43,7 +44,7 @@ struct Geom {
 struct __attribute__((aligned(16))) Tagged {
     unsigned long long sum, sq;
 };
-static_assert(kSyncCminor + sizeof(unsigned) * kCountStride * (kMostGroups + kMostRowGroups) +
+static_assert(kSyncCminor + sizeof(unsigned) * kCountStride * kMostParts * (kMostGroups + kMostRowGroups) +
                       sizeof(Tagged) * ((size_t)kMostGroups * kMostRecords + (size_t)kMostRowGroups * kMostRowRecords) <=
                   kSyncBytes, "sync area layout");
 __device__ __forceinline__ unsigned long long tagged(float v, unsigned tag) {
@@ -59,15 +60,18 @@ __device__ __forceinline__ half_t round_f16(float v) {
     return (half_t)v;
 }
 
-// Tags.  The workgroups that share a block of channels of an image are a group with a launch count and a run of records of
-// its own, so that a record only ever carries tags of its own group's count; a launch's tag is the count + 1, and it is the
-// device that counts, as a replayed graph needs.  The group's first workgroup moves the count on: when its wait was met,
-// every workgroup of the group has read the count (a record carries the tag only after its writer has).  No
-// read-modify-write is involved: 192 arrivals at one counter took 1.5 us.
+// Tags.  The workgroups that share a block of channels of an image are a group with launch counts and a run of records of
+// its own, so that a record only ever carries tags of its own group's counts; a launch's tag is the count + 1, and it is the
+// device that counts, as a replayed graph needs.  Every workgroup has counts of its own (a run of the group's kMostParts, all
+// of which a launch moves on, however many workgroups it has): nobody else writes them during a launch, so a workgroup finds
+// the launch's tag however late it starts, and no record of an earlier launch carries it.  No read-modify-write is involved:
+// 192 arrivals at one counter took 1.5 us.
 // The wait is bounded: a workgroup whose partners do not show up in time (they are not resident: the device is shared)
-// computes their partial sums itself with the same arithmetic, so the result is the same bits and every wave exits.  It
-// withdraws its records (tag 0 is never used): a workgroup that starts later still reads the moved count, publishes under
-// the next tag, meets nobody and does the same, and no later launch takes either's records for its own.
+// computes missing partial sums with the same arithmetic and publishes them for their owners and for everyone else, part by
+// part, each time one that nobody has published yet.  So the result is the same bits, the missing parts are computed about
+// once among those that wait, whoever starts later finds its group complete, and every wave exits: a workgroup computes a
+// part at most once.  (Each computing all parts for itself took 6.5 ms for [1,448,448,256] beside a launch that held 224 of 256
+// compute units; now 1.4.)
 //
 // How the sums meet.  With whole words per position (OCTETS) ob is a power of two: lanes that own the same word are ob apart
 // in a wavefront and add up by rotations and swaps, and so do a channel's partial sums of other workgroups; eight wavefronts
@@ -112,11 +116,11 @@ __global__ __launch_bounds__(kT) void mvn_cminor_resident(const half_t* __restri
                                                           int normalize_variance, float eps, unsigned long long spin_ticks) {
     constexpr bool OCTETS = FORM != kRows;
     __shared__ float2 red[OCTETS ? 8 * 64 : kT * 8];  // [wavefront or slot][column] sums
-    __shared__ float2 others[OCTETS ? kMostRecords : kT];  // partial sums computed here, in the order they are added up
     __shared__ float2 folded[OCTETS ? 1 : kT];             // [group of lanes][channel]
     __shared__ float s_mean[OCTETS ? 64 : kT], s_inv[OCTETS ? 64 : kT];
     __shared__ float2 s_tail[8];
-    __shared__ unsigned s_tag;
+    __shared__ unsigned s_tag, s_pick;
+    __shared__ unsigned char helped[kMostParts];
 
     // the blocks of one part are neighbours on one die, whose L2 then holds the lines they share
     const uint32_t seq = blockIdx.x >> 3, b = seq % g.nb, u = seq / g.nb * 8 + (blockIdx.x & 7);
@@ -136,11 +140,14 @@ __global__ __launch_bounds__(kT) void mvn_cminor_resident(const half_t* __restri
     // of the channel whose statistics this lane finishes
     const float own_shift = (float)img[(uint32_t)t < nch && ch0 + t < g.C ? ch0 + t : 0];
     const uint32_t rem = OCTETS ? 0 : g.per_n % 8;  // values of the image's last, partial word
-    unsigned* launches = sync + (OCTETS ? n * g.nb + b : kMostGroups + n) * kCountStride;
-    Tagged* records = reinterpret_cast<Tagged*>(sync + (kMostGroups + kMostRowGroups) * kCountStride) +
-                      (OCTETS ? (size_t)(n * g.nb + b) * kMostRecords : (size_t)kMostGroups * kMostRecords + (size_t)n * kMostRowRecords);
+    const uint32_t group = OCTETS ? n * g.nb + b : kMostGroups + n;
+    // this workgroup's launch counts
+    unsigned* counts = sync + (size_t)group * (kMostParts * kCountStride);
+    const uint32_t first_count = part * kMostParts / g.parts, end_count = (part + 1) * kMostParts / g.parts;
+    Tagged* records = reinterpret_cast<Tagged*>(sync + (size_t)(kMostGroups + kMostRowGroups) * (kMostParts * kCountStride)) +
+                      (OCTETS ? (size_t)group * kMostRecords : (size_t)kMostGroups * kMostRecords + (size_t)n * kMostRowRecords);
     unsigned tag = 0;
-    if (g.parts > 1 && t == 0) tag = __hip_atomic_load(launches, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) + 1u;
+    if (g.parts > 1 && t == 0) tag = __hip_atomic_load(counts + first_count * kCountStride, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) + 1u;
 
     // sums are of x - x[first position of the channel]: no cancellation where a channel's mean is far from zero
     halfx8 first;
@@ -267,16 +274,21 @@ __global__ __launch_bounds__(kT) void mvn_cminor_resident(const half_t* __restri
     };
 
     float2 total = part_sums(part);
-    bool met = true;
     if (g.parts > 1) {
         if (t == 0) s_tag = tag == 0u ? 1u : tag;
         __syncthreads();
         tag = s_tag;
         const uint32_t count = g.parts * nch;
-        if ((uint32_t)t < nch) {
-            __hip_atomic_store(&records[part * nch + t].sum, tagged(total.x, tag), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            __hip_atomic_store(&records[part * nch + t].sq, tagged(total.y, tag), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        }
+        const auto publish = [&](uint32_t p, float2 v) {
+            if ((uint32_t)t < nch) {
+                __hip_atomic_store(&records[p * nch + t].sum, tagged(v.x, tag), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                __hip_atomic_store(&records[p * nch + t].sq, tagged(v.y, tag), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            }
+        };
+        publish(part, total);
+        // (here and not at the end: their way to memory then ends under the wait, 1.2 of 43 us at [16,112,112,256])
+        if (first_count + t < end_count)
+            __hip_atomic_store(counts + (first_count + t) * kCountStride, tag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         const unsigned long long began = wall_clock64();
         const auto poll = [&](uint32_t i, unsigned long long& rs, unsigned long long& rq) {
             rs = __hip_atomic_load(&records[i].sum, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -285,33 +297,71 @@ __global__ __launch_bounds__(kT) void mvn_cminor_resident(const half_t* __restri
         };
         constexpr int kAtOnce = 4;
         static_assert(kMostRecords == kAtOnce * kT, "records a workgroup reads at once");
-        float2 a{0.f, 0.f};
-        if (OCTETS) {
-            // a lane's records are all of channel t % nch
-            unsigned long long rs[kAtOnce], rq[kAtOnce];
-            bool ready;
-            do {
-                ready = true;
+        // adds up this lane's records in `a`; false if one of them was not this launch's when the wait ran out
+        float2 a;
+        const auto collect = [&](bool waits) {
+            a = float2{0.f, 0.f};
+            bool ready = true;
+            if (OCTETS) {
+                // a lane's records are all of channel t % nch
+                unsigned long long rs[kAtOnce], rq[kAtOnce];
+                do {
+                    ready = true;
+#pragma unroll
+                    for (int k = 0; k < kAtOnce; k++)
+                        if ((uint32_t)(k * kT + t) < count) ready &= poll(k * kT + t, rs[k], rq[k]);
+                } while (waits && __builtin_amdgcn_ballot_w64(!ready) != 0 && wall_clock64() - began < spin_ticks);
 #pragma unroll
                 for (int k = 0; k < kAtOnce; k++)
-                    if ((uint32_t)(k * kT + t) < count) ready &= poll(k * kT + t, rs[k], rq[k]);
-            } while (__builtin_amdgcn_ballot_w64(!ready) != 0 && wall_clock64() - began < spin_ticks);
-            met = __syncthreads_and(ready);
-            if (!met) {
-                for (uint32_t p = 0; p < g.parts; p++) {
-                    const float2 v = part_sums(p);
-                    if ((uint32_t)t < nch) others[p * nch + t] = v;
+                    if ((uint32_t)(k * kT + t) < count) {
+                        a.x += untagged(rs[k]);
+                        a.y += untagged(rq[k]);
+                    }
+            } else {
+                // lane (gi, c) adds up channel c of the parts gi, gi + G, ...
+                constexpr int kRowsAtOnce = V >= 32 ? 4 : 12;  // (more would not leave the words their registers)
+                for (uint32_t p = gi; p < g.parts && gi < G && ready; p += kRowsAtOnce * G) {
+                    unsigned long long rs[kRowsAtOnce], rq[kRowsAtOnce];
+                    do {
+                        ready = true;
+#pragma unroll
+                        for (int k = 0; k < kRowsAtOnce; k++) ready &= poll((p + k * G < g.parts ? p + k * G : p) * nch + c, rs[k], rq[k]);
+                    } while (waits && !ready && wall_clock64() - began < spin_ticks);
+#pragma unroll
+                    for (int k = 0; k < kRowsAtOnce; k++)
+                        if (p + k * G < g.parts) {
+                            a.x += untagged(rs[k]);
+                            a.y += untagged(rq[k]);
+                        }
                 }
-                part_sums(part);  // its own words again
+            }
+            return ready;
+        };
+        if (!__syncthreads_and(collect(true))) {
+            if (t < kMostParts) helped[t] = 0;
+            for (uint32_t k = 0; k < g.parts; k++) {
+                // of the parts that nobody has published: the first one from a place of this workgroup's own on
+                const uint32_t from = (part * 2654435761u >> 8) % g.parts;
+                if (t == 0) s_pick = g.parts;
+                __syncthreads();
+                for (uint32_t i = t; i < count; i += kT) {
+                    unsigned long long rs, rq;
+                    const uint32_t p = i / nch;
+                    if (!poll(i, rs, rq) && !helped[p]) atomicMin(&s_pick, (p + g.parts - from) % g.parts);
+                }
+                __syncthreads();
+                const uint32_t pick = s_pick, p = (from + pick) % g.parts;
+                if (pick == g.parts) break;
+                publish(p, part_sums(p));
+                __threadfence();
+                if (t == 0) helped[p] = 1;
                 __syncthreads();
             }
-#pragma unroll
-            for (int k = 0; k < kAtOnce; k++)
-                if ((uint32_t)(k * kT + t) < count) {
-                    const float2 v = met ? float2{untagged(rs[k]), untagged(rq[k])} : others[OCTETS ? k * kT + t : 0];
-                    a.x += v.x;
-                    a.y += v.y;
-                }
+            collect(false);
+            part_sums(part);  // its own words again
+            __syncthreads();
+        }
+        if (OCTETS) {
             float both[2] = {a.x, a.y};
             stride_sums(both, nch);
             if (nch <= 16) {
@@ -333,39 +383,6 @@ __global__ __launch_bounds__(kT) void mvn_cminor_resident(const half_t* __restri
                 }
             }
         } else {
-            // lane (gi, c) adds up channel c of the parts gi, gi + G, ...
-            bool ready = true;
-            constexpr int kRowsAtOnce = V >= 32 ? 4 : 12;  // (more would not leave the words their registers)
-            for (uint32_t p = gi; p < g.parts && gi < G && ready; p += kRowsAtOnce * G) {
-                unsigned long long rs[kRowsAtOnce], rq[kRowsAtOnce];
-                do {
-                    ready = true;
-#pragma unroll
-                    for (int k = 0; k < kRowsAtOnce; k++) ready &= poll((p + k * G < g.parts ? p + k * G : p) * nch + c, rs[k], rq[k]);
-                } while (!ready && wall_clock64() - began < spin_ticks);
-#pragma unroll
-                for (int k = 0; k < kRowsAtOnce; k++)
-                    if (p + k * G < g.parts) {
-                        a.x += untagged(rs[k]);
-                        a.y += untagged(rq[k]);
-                    }
-            }
-            met = __syncthreads_and(ready);
-            if (!met) {
-                others[t] = float2{0.f, 0.f};
-                __syncthreads();
-                for (uint32_t p = 0; p < g.parts; p++) {
-                    const float2 v = part_sums(p);
-                    if ((uint32_t)t < nch) {
-                        float2& o = others[p % G * nch + t];
-                        o.x += v.x;
-                        o.y += v.y;
-                    }
-                }
-                part_sums(part);  // its own words again
-                __syncthreads();
-                a = others[t];
-            }
             folded[t] = a;
             __syncthreads();
             total = float2{0.f, 0.f};
@@ -411,13 +428,6 @@ __global__ __launch_bounds__(kT) void mvn_cminor_resident(const half_t* __restri
         const uint32_t f = g.per_n - rem + t, ch = f % g.C;
         oimg[f] = round_f16(((float)img[f] - s_mean[ch]) * s_inv[ch]);
     }
-    if (g.parts > 1) {
-        if (t == 0 && part == 0) __hip_atomic_store(launches, tag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        if (!met && (uint32_t)t < nch) {
-            __hip_atomic_store(&records[part * nch + t].sum, 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            __hip_atomic_store(&records[part * nch + t].sq, 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        }
-    }
 }
 
 uint32_t ceil_div(uint64_t a, uint64_t b) {
@@ -460,6 +470,7 @@ int launch_mvn_cminor_resident(const void* in, void* out, int64_t N, int64_t S, 
     // partial sums than there are records.
     const auto most_parts = [&](uint32_t ob, uint32_t blocks, uint32_t records) {
         uint32_t parts = (uint32_t)cus / blocks;
+        if (parts > kMostParts) parts = kMostParts;
         if (parts > rows / (2 * (kT / ob))) parts = rows / (2 * (kT / ob));
         return parts < records ? parts : records;
     };
@@ -478,8 +489,8 @@ int launch_mvn_cminor_resident(const void* in, void* out, int64_t N, int64_t S, 
         for (uint32_t div = 1; div <= 4 && parts / div > 1 && N <= kMostRowGroups; div *= 2) consider(true, words, 0, 1, parts / div);
     }
     if (best_v == 0) return VPX_RESULT_SUCCESS;
-    // In place, a workgroup that has to read its partners' values again could find results there: those launches take
-    // the kernels that finish all reads first.  (A workgroup alone with its channels reads everything before it writes.)
+    // In place, a workgroup that computes a partner's partial sums could find results there: those launches take the
+    // kernels that finish all reads first.  (A workgroup alone with its channels reads everything before it writes.)
     if (best.parts > 1 && in == out) return VPX_RESULT_SUCCESS;
     // A launch holds fewer than 2^32 lanes; small images of many channels ask for more from N * nb = 2^23 on.
     const uint64_t blocks = ((uint64_t)best.units + 7) / 8 * best.nb * 8;

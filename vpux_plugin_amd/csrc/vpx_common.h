@@ -88,8 +88,8 @@ int get_workspace(hipStream_t stream, size_t bytes, void** out);
 // A small area, zero at first, per (device, stream handle) for kernels whose workgroups meet inside a launch: each such
 // kernel has a part of its own and keeps its counters and tagged records there from launch to launch.
 constexpr size_t kSyncCminor = 128 * 1024;  // the channel-minor MVN's part: 128 groups of 2048 records of 16 bytes and 16 of
-                                            // 16384, a launch count in a line of its own for each
-constexpr size_t kSyncBytes = kSyncCminor + 128 * (128 + 2048 * 16) + 16 * (128 + 16384 * 16);
+                                            // 16384, 256 launch counts of 16 bytes for each group
+constexpr size_t kSyncBytes = kSyncCminor + (128 + 16) * (256 * 16) + 128 * (2048 * 16) + 16 * (16384 * 16);
 int get_sync_area(hipStream_t stream, void** out);
 // Compute units of the current device (cached per device).
 int device_compute_units(int* out);
@@ -105,8 +105,8 @@ int calib_coissue(int valu_kind, int wide_mfma, int mode, int iters, void* sink,
 
 // Dispatch override for tests and tuning (knob names are those of the VPX_* environment variables, read once).
 int set_tuning(const char* knob, const char* value);
-// VPX_MVN_FUSED: 0 = never take the one-launch MVN kernel, 1 = default, 2 = its workgroups do not wait for each other
-// (every one recomputes the group's moments: the path a workgroup takes when the others are not resident)
+// VPX_MVN_FUSED: 0 = never take the one-launch MVN kernels, 1 = default, 2 = their workgroups do not wait for each other
+// (each computes and publishes what it finds missing: the path a workgroup takes when the others are not resident)
 int tuning_mvn_fused();
 // VPX_CALIB_BLOCKS: workgroups of the MFMA calibration loop (0: one per compute unit); fewer leave compute units free
 // for whatever another stream launches beside it
