@@ -262,9 +262,8 @@ VPX_API int vpx_calib_mfma_i8(const void* operands, void* sink, int iters, int f
  * memory per compute unit.  The caller times the launch; time / iters is the length of a round. */
 VPX_API int vpx_calib_coissue(int valu_kind, int wide_mfma, int mode, int iters, void* sink, void* stream);
 
-/* Name of the kernel family the last successful vpx_nce_task on this thread dispatched to ("" before the first); for tests
- * and profiles.  A family's small layers run its staging-free form, the device kernel nce_direct; the name is "nce_direct" where
- * VPX_NCE_DIRECT asks for that form. */
+/* Name of the device kernel that the last successful vpx_nce_task on this thread ran ("" before the first); for tests and
+ * profiles. */
 VPX_API const char* vpx_nce_last_kernel(void);
 
 #ifdef __cplusplus

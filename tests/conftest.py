@@ -26,6 +26,15 @@ def rt():
     return runtime
 
 
+@pytest.fixture
+def without_nce_direct(rt):
+    """Layers that are over before a tile is staged run nce_direct; without it they run the kernel that serves their family at
+    larger sizes, which is what a test that names one is about."""
+    rt.set_tuning("VPX_NCE_DIRECT", "off")
+    yield
+    rt.set_tuning("VPX_NCE_DIRECT", None)
+
+
 @pytest.fixture(scope="session")
 def dev():
     import torch

@@ -5,7 +5,7 @@ import os
 import numpy as np
 import pytest
 
-pytestmark = pytest.mark.gpu
+pytestmark = [pytest.mark.gpu, pytest.mark.usefixtures("without_nce_direct")]
 
 
 def dev_t(a, dev):
@@ -287,10 +287,12 @@ def test_negative_multipliers(rt, orc, dev, geom, kernel, mode):
     assert np.array_equal(got, want), "%s %s: %d mismatches" % (kernel, mode, int((got != want).sum()))
 
 
+@pytest.mark.parametrize("direct", [None, "off"])
 @pytest.mark.parametrize("seed,weight_zp", [(1234, False), (99, False), (7, True), (8, True)])
-def test_conv_random_geometries(rt, orc, dev, seed, weight_zp):
-    """Thirty seeded draws of shape, kernel, stride, padding, types, zero points and PPE mode, whichever kernel they select;
-    the last two seeds also draw the weight storage type and a weight zero point."""
+def test_conv_random_geometries(rt, orc, dev, seed, weight_zp, direct):
+    """Thirty seeded draws of shape, kernel, stride, padding, types, zero points and PPE mode, whichever kernel they select,
+    and whichever staged one; the last two seeds also draw the weight storage type and a weight zero point."""
+    rt.set_tuning("VPX_NCE_DIRECT", direct)
     rng = np.random.default_rng(seed)
     for i in range(30):
         IC = int(rng.choice([16, 32, 48, 64, 64, 96, 128, 128, 192, 256, 320, 512]))

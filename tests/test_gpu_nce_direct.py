@@ -30,6 +30,13 @@ def test_tiles_and_waves(rt, orc, dev, layer, shape):
         assert run_views(rt, orc, dev, rng, LAYERS[layer], *kinds, tuning=(("VPX_NCE_DIRECT", shape),), **kw) == "nce_direct"
 
 
+@pytest.mark.parametrize("family", ["gemm_stride2", "tile", "tile5x5", "stream", "stream_ksplit", "rows16", "rows16_48"])
+def test_small_layers_take_it_by_themselves_and_say_so(rt, orc, dev, family):
+    g, force, tuning, _ = FAMILIES[family]
+    rng = np.random.default_rng(seed("auto", family))
+    assert run_views(rt, orc, dev, rng, g, "window_chan", "chan_odd", force=force, tuning=tuning) == "nce_direct"
+
+
 @pytest.mark.parametrize("family", sorted(FAMILIES))
 def test_families_without_it(rt, orc, dev, family):
     g, force, tuning, kernel = FAMILIES[family]

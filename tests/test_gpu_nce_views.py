@@ -7,7 +7,7 @@ import zlib
 import numpy as np
 import pytest
 
-pytestmark = pytest.mark.gpu
+pytestmark = [pytest.mark.gpu, pytest.mark.usefixtures("without_nce_direct")]
 
 GUARD = 77
 
