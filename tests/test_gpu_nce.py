@@ -536,10 +536,10 @@ def test_matmul_weights_in_registers_weight_zero_points(rt, orc, dev, regb_on, M
 
 
 def test_matmul_weights_in_registers_leaves_ragged_rows_to_the_tile_kernel(rt, orc, dev, regb_on):
-    """Channel counts that are not a multiple of 16 (rows of the result that do not end on a 16-byte piece) and a K it
-    does not serve."""
+    """Channel counts that are not a multiple of 16 (rows of the result that do not end on a 16-byte piece) and a K beyond
+    the one whose weights the registers hold."""
     rng = np.random.default_rng(185)
-    for M, K, N in ((300, 64, 77), (300, 192, 128)):
+    for M, K, N in ((300, 64, 77), (300, 320, 128)):
         a = rng.integers(-128, 128, (M, K)).astype(np.int8)
         b = rng.integers(-127, 128, (N, K)).astype(np.int8)
         got, want, name = run_task(rt, orc, dev, a.reshape(1, M, 1, K), b.reshape(N, 1, 1, K), rng.integers(2 ** 14, 2 ** 15, N),

@@ -9,7 +9,7 @@ pytestmark = pytest.mark.gpu
 
 
 @pytest.mark.parametrize("OC", [16, 32, 48, 80, 96, 144, 208, 256])
-@pytest.mark.parametrize("IC", [16, 32, 48, 80, 96, 112, 144, 208, 240])
+@pytest.mark.parametrize("IC", [16, 32, 48, 80, 96, 112, 144, 192, 208, 240])
 def test_row_lengths(rt, orc, dev, IC, OC):
     rng = np.random.default_rng(seed("regb", IC, OC))
     g = dict(N=1, H=int(rng.integers(1, 90)), W=7, IC=IC, OC=OC, KY=1, KX=1)
