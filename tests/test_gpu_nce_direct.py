@@ -37,6 +37,14 @@ def test_small_layers_take_it_by_themselves_and_say_so(rt, orc, dev, family):
     assert run_views(rt, orc, dev, rng, g, "window_chan", "chan_odd", force=force, tuning=tuning) == "nce_direct"
 
 
+@pytest.mark.parametrize("family,knob,value", [("stream_ksplit", "VPX_STREAM_KSPLIT", "off"), ("stream", "VPX_CONV_ROWS", 2), ("tile", "VPX_CONV_WAVES", 4),
+                                               ("rows16", "VPX_CONV_COLS", 7), ("gemm_stride2", "VPX_GEMM_TILE", 128), ("gemm_stride2", "VPX_GEMM_WAVES", 4)])
+def test_a_knob_of_a_family_keeps_its_kernel(rt, orc, dev, family, knob, value):
+    g, force, tuning, kernel = FAMILIES[family]
+    rng = np.random.default_rng(seed("knob", family))
+    assert run_views(rt, orc, dev, rng, g, "dense", "dense", force=force, tuning=tuple(tuning) + ((knob, value),)) == kernel
+
+
 @pytest.mark.parametrize("family", sorted(FAMILIES))
 def test_families_without_it(rt, orc, dev, family):
     g, force, tuning, kernel = FAMILIES[family]
