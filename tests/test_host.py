@@ -94,6 +94,29 @@ def test_a_tile_that_no_kernel_has_is_refused(rt, value):
         rt.set_tuning("VPX_NCE_DIRECT", good)
 
 
+def test_operator_functions_refuse_what_does_not_fit(rt):
+    """Wrong counts and types are named before anything is launched (the tensors hold nothing that could be)."""
+    import types
+    import torch
+    stream = types.SimpleNamespace(cuda_stream=0)
+    inp, out = torch.empty((0, 4, 4, 16), dtype=torch.uint8), torch.empty((0, 4, 4, 16), dtype=torch.uint8)
+    w, wt = torch.zeros((16, 1, 1, 16), dtype=torch.int8), torch.zeros((16, 4), dtype=torch.int32)
+    ppe = rt.PpeInt(rt.PPE_NOOP, 0, 255, 1, 0)
+    for strides in ((1, 1, 1), (1,), ()):
+        with pytest.raises(ValueError):
+            rt.nce_task(inp, w, wt, out, ppe, strides=strides, stream=stream)
+    with pytest.raises(IndexError):
+        rt.nce_task(inp, w, wt, out, ppe, pads=(0, 0, 0), stream=stream)
+    same_size = np.zeros(len(bytes(ppe)), np.uint8)
+    for other in (same_size, bytes(ppe), bytearray(bytes(ppe)), 5, None):
+        with pytest.raises(TypeError):
+            rt.nce_task(inp, w, wt, out, other, stream=stream)
+        with pytest.raises(TypeError):
+            rt.nce_eltwise(inp, inp, out, other, stream=stream)
+        with pytest.raises(TypeError):
+            rt.nce_matmul(torch.empty((0, 16), dtype=torch.int8), w.view(16, 16), wt, torch.empty((0, 16), dtype=torch.int8), other, stream=stream)
+
+
 def test_half_conversion_matches_oracle(rt, orc):
     L = rt.lib()
     rng = np.random.default_rng(11)

@@ -17,6 +17,7 @@
 namespace {
 
 PyObject* g_orders = nullptr;  // name of a layout -> its code (runtime.ORDER)
+PyObject* g_ppe = nullptr;     // the type of a task's ppe (runtime.PpeInt)
 
 // What a Python error leaves behind: the exception is set, the call returns null.
 struct Raised {};
@@ -318,25 +319,43 @@ PyObject* py_quantize(PyObject*, PyObject* const* a, Py_ssize_t n) {
     });
 }
 
+// A PpeInt, or a tuple of its fields.
 void read_ppe(PyObject* o, vpx_ppe_int_t* ppe) {
+    PyObject* made = nullptr;
+    if (PyTuple_Check(o)) {
+        o = made = PyObject_CallObject(g_ppe, o);
+        if (!made) throw Raised{};
+    } else {
+        const int is = PyObject_IsInstance(o, g_ppe);
+        if (is < 0) throw Raised{};
+        if (!is) {
+            PyErr_Format(PyExc_TypeError, "ppe must be a PpeInt, got %s", Py_TYPE(o)->tp_name);
+            throw Raised{};
+        }
+    }
     Py_buffer view;
-    if (PyObject_GetBuffer(o, &view, PyBUF_SIMPLE) < 0) throw Raised{};
-    const bool fits = view.len == (Py_ssize_t)sizeof(*ppe);
+    const int rc = PyObject_GetBuffer(o, &view, PyBUF_SIMPLE);
+    const bool fits = rc == 0 && view.len == (Py_ssize_t)sizeof(*ppe);
     if (fits) std::memcpy(ppe, view.buf, sizeof(*ppe));
-    PyBuffer_Release(&view);
-    if (!fits) raise(PyExc_TypeError, "ppe must be a PpeInt");
+    if (rc == 0) PyBuffer_Release(&view);
+    Py_XDECREF(made);
+    if (rc < 0) throw Raised{};
+    if (!fits) raise(PyExc_TypeError, "a PpeInt of another size");
 }
 
 void require(bool ok, const char* text) {
     if (!ok) raise(PyExc_AssertionError, text);
 }
 
-void read_pair(PyObject* o, int32_t* v, Py_ssize_t n) {
+// The first n values of a sequence; `exactly`: which has no others.
+void read_values(PyObject* o, int32_t* v, Py_ssize_t n, bool exactly) {
     PyObject* f = PySequence_Fast(o, "expected a sequence of integers");
     if (!f) throw Raised{};
-    if (PySequence_Fast_GET_SIZE(f) < n) {
+    const Py_ssize_t size = PySequence_Fast_GET_SIZE(f);
+    if (size < n || (exactly && size > n)) {
         Py_DECREF(f);
-        raise(PyExc_ValueError, "too few values");
+        PyErr_Format(exactly ? PyExc_ValueError : PyExc_IndexError, "expected %zd values, got %zd", n, size);
+        throw Raised{};
     }
     for (Py_ssize_t i = 0; i < n; i++) {
         const long x = PyLong_AsLong(PySequence_Fast_GET_ITEM(f, i));
@@ -399,8 +418,8 @@ PyObject* py_conv(PyObject*, PyObject* const* a, Py_ssize_t n) {
         t.kernel_size[0] = (int32_t)w.size(-3);
         t.kernel_size[1] = (int32_t)w.size(-2);
         require(t.IC == w.size(-1), "input and weights have different channel counts");
-        read_pair(a[8], t.kernel_strides, 2);
-        read_pair(a[9], t.kernel_padding, 4);
+        read_values(a[8], t.kernel_strides, 2, true);
+        read_values(a[9], t.kernel_padding, 4, false);
         t.zp_in = integer32(a[5]);
         t.zp_w = integer32(a[6]);
         t.zp_out = integer32(a[7]);
@@ -503,6 +522,16 @@ PyObject* py_set_orders(PyObject*, PyObject* orders) {
     Py_RETURN_NONE;
 }
 
+PyObject* py_set_ppe(PyObject*, PyObject* type) {
+    if (!PyType_Check(type)) {
+        PyErr_SetString(PyExc_TypeError, "expected the type of a ppe");
+        return nullptr;
+    }
+    Py_INCREF(type);
+    Py_XSETREF(g_ppe, type);
+    Py_RETURN_NONE;
+}
+
 #define FAST(f) (PyCFunction)(void (*)(void)) f
 PyMethodDef kMethods[] = {
     {"launch", FAST(py_launch), METH_FASTCALL, "software kernel on tensors"},
@@ -516,6 +545,7 @@ PyMethodDef kMethods[] = {
     {"eltwise", FAST(py_eltwise), METH_FASTCALL, "NCE eltwise task"},
     {"stream", py_stream, METH_O, "handle of a stream, or of the current one"},
     {"set_orders", py_set_orders, METH_O, "names of the layouts"},
+    {"set_ppe", py_set_ppe, METH_O, "type of a ppe"},
     {nullptr, nullptr, 0, nullptr}};
 PyModuleDef kModule = {PyModuleDef_HEAD_INIT, "_binding", "operator calls on torch tensors through libvpx_amd.so", -1, kMethods,
                        nullptr, nullptr, nullptr, nullptr};

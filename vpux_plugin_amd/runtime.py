@@ -173,6 +173,7 @@ def _bind():
         module = importlib.util.module_from_spec(spec)
         spec.loader.exec_module(module)
         module.set_orders(ORDER)
+        module.set_ppe(PpeInt)
         _binding = module
     return _binding
 
