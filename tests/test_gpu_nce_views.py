@@ -203,9 +203,18 @@ def test_matmul_on_a_column_block_of_a_wider_matrix(rt, orc, dev):
     torch.cuda.synchronize()
     assert rt.nce_last_kernel() == "nce_gemm_mfma"
     want = orc.nce_matmul(np.ascontiguousarray(big_a[:, 32:32 + K]), b, wt, orc.ppe(1638, 14, 0, -128, 127), zp_a=3)
+    # ... and as matrices; the result with a leading dimension of one or with its rows in two, the ppe as a tuple of its fields
+    for shape in (None, (1, M, N), (2, M // 2, N)):
+        got = big_out.cpu().numpy()
+        assert np.array_equal(got[:, 16:16 + N], want)
+        assert (got[:, :16] == GUARD).all() and (got[:, 16 + N:] == GUARD).all()
+        big_out.fill_(GUARD)
+        block = big_out[:, 16:16 + N]
+        rt.nce_matmul(ta[:, 32:32 + K], dev_t(b, dev), dev_t(wt, dev), block if shape is None else block.unflatten(0, shape[:2]),
+                      (rt.PPE_LPRELU, -128, 127, 1638, 14), zp_a=3)
+        torch.cuda.synchronize()
     got = big_out.cpu().numpy()
     assert np.array_equal(got[:, 16:16 + N], want)
-    assert (got[:, :16] == GUARD).all() and (got[:, 16 + N:] == GUARD).all()
 
 
 @pytest.mark.parametrize("out_f16", [False, True])

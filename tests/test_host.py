@@ -115,6 +115,8 @@ def test_operator_functions_refuse_what_does_not_fit(rt):
             rt.nce_eltwise(inp, inp, out, other, stream=stream)
         with pytest.raises(TypeError):
             rt.nce_matmul(torch.empty((0, 16), dtype=torch.int8), w.view(16, 16), wt, torch.empty((0, 16), dtype=torch.int8), other, stream=stream)
+    with pytest.raises(ValueError):
+        rt.nce_matmul(torch.empty((0, 1), dtype=torch.int8), torch.zeros(16, dtype=torch.int8), wt, torch.empty((0, 16), dtype=torch.int8), ppe, stream=stream)
 
 
 def test_half_conversion_matches_oracle(rt, orc):

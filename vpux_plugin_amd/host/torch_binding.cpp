@@ -441,7 +441,8 @@ PyObject* py_matmul(PyObject*, PyObject* const* a, Py_ssize_t n) {
         expect_count(n, 9, 9);
         const at::Tensor &x = tensor(a[0]), &b = tensor(a[1]), &table = tensor(a[2]), &out = tensor(a[3]);
         const bool grouped = x.dim() == 3;
-        if ((x.dim() != 2 && !grouped) || b.dim() < (grouped ? 2 : 1)) raise(PyExc_ValueError, "a is a matrix, or three-dimensional (groups first)");
+        if ((x.dim() != 2 && !grouped) || (grouped ? b.dim() < 2 : b.dim() != 2))
+            raise(PyExc_ValueError, "a and b are matrices, or three-dimensional (groups first)");
         const int64_t M = x.size(-2), K = x.size(-1), N = b.size(grouped ? 1 : 0), G = grouped ? x.size(0) : 1;
         if (b.numel() != G * N * K || out.numel() != G * M * N) raise(PyExc_RuntimeError, "a [M,K], b [N,K] and out [M,N] do not fit each other");
         require(b.is_contiguous() && table.is_contiguous(), "b and the weight table are dense");
@@ -462,18 +463,9 @@ PyObject* py_matmul(PyObject*, PyObject* const* a, Py_ssize_t n) {
             require(x.is_contiguous() && out.is_contiguous(), "the operands of a grouped matmul are dense");
             t.groups = (int32_t)G;
         } else {
-            // a matrix that is a view of a larger one, as [1, rows, 1, columns]
-            const auto rows = [](int64_t* field, const at::Tensor& m) {
-                if (m.is_contiguous()) return;
-                if (m.dim() != 2) raise(PyExc_RuntimeError, "an operand that is no matrix must be dense");
-                field[0] = m.size(0) * m.stride(0);
-                field[1] = m.stride(0);
-                field[2] = m.size(1) * m.stride(1);
-                field[3] = m.stride(1);
-            };
-            if (!out.is_contiguous() && out.dim() == 2 && out.size(0) != M) raise(PyExc_RuntimeError, "out has another shape than [M,N]");
-            rows(t.input_strides, x);
-            rows(t.output_strides, out);
+            // a matrix that is a view of a larger one (out with any dimensions that make one), as [1, rows, 1, columns]
+            if (!x.is_contiguous()) view_strides(t.input_strides, x.view({1, M, 1, K}));
+            if (!out.is_contiguous()) view_strides(t.output_strides, out.view({1, M, 1, N}));
         }
         const int rc = run_task(t, a[8]);
         if (rc) return PyLong_FromLong(rc);
