@@ -94,6 +94,25 @@ def test_a_tile_that_no_kernel_has_is_refused(rt, value):
         rt.set_tuning("VPX_NCE_DIRECT", good)
 
 
+def test_the_c_library_is_built_without_python_headers(monkeypatch, tmp_path, capsys):
+    import sysconfig
+    from vpux_plugin_amd import build as b
+    made = []
+    monkeypatch.setattr(b, "BINDING", str(tmp_path / "_binding.so"))
+    monkeypatch.setattr(b.subprocess, "Popen", lambda cmd, **kw: made.append(cmd[-1]))
+    monkeypatch.setattr(b.subprocess, "check_call", lambda cmd: made.append(cmd[cmd.index("-o") + 1]))
+    monkeypatch.setattr(b, "_drain", lambda procs, verbose: procs.clear())
+    monkeypatch.setattr(b.os, "makedirs", lambda *a, **kw: None)
+    b.build(verbose=False)
+    assert made[-3:] == [b.LIB, os.path.join(b.HERE, "examples", "c_abi_host"), b.BINDING]
+    made.clear()
+    open(b.BINDING, "w").close()  # of an earlier build
+    monkeypatch.setattr(sysconfig, "get_paths", lambda: {"include": str(tmp_path)})
+    b.build(verbose=False)
+    assert made[-2:] == [b.LIB, os.path.join(b.HERE, "examples", "c_abi_host")]
+    assert not os.path.exists(b.BINDING) and "Python.h" in capsys.readouterr().err
+
+
 def test_operator_functions_refuse_what_does_not_fit(rt):
     """Wrong counts and types are named before anything is launched (the tensors hold nothing that could be)."""
     import types

@@ -44,7 +44,6 @@ def build(verbose=True, jobs=8):
     if verbose:
         print(" ".join(cmd), flush=True)
     subprocess.check_call(cmd)
-    build_binding(verbose)
     # the C++ host example: the C ABI driven without Python; it links the HIP runtime itself
     exe = os.path.join(HERE, "examples", "c_abi_host")
     cmd = [hipcc, "--offload-arch=gfx950", "-O2", "-std=c++17", "-I", os.path.join(ROOT, "include"), os.path.join(HERE, "examples", "c_abi_host.cpp"),
@@ -52,25 +51,39 @@ def build(verbose=True, jobs=8):
     if verbose:
         print(" ".join(cmd), flush=True)
     subprocess.check_call(cmd)
+    build_binding(verbose)
     return LIB
 
 
 def build_binding(verbose=True):
     """The CPython module runtime.py calls the library through: host code against torch's C++ headers.  torch's own
-    libraries are in the process before it is loaded; libvpx_amd.so lies beside it."""
+    libraries are in the process before it is loaded; libvpx_amd.so lies beside it.  A host that has only the C library to
+    build lacks torch or the headers: it is told so, False is returned and the operator functions of runtime.py raise."""
     import sysconfig
-    import torch
-    top = os.path.dirname(torch.__file__)
+    if os.path.exists(BINDING):
+        os.remove(BINDING)  # (one of another build would call this library)
+    python = sysconfig.get_paths()["include"]
+    try:
+        import torch
+        top = os.path.dirname(torch.__file__)
+        needs = [os.path.join(python, "Python.h"), os.path.join(top, "include", "torch", "csrc", "autograd", "python_variable.h")]
+        absent = [h for h in needs if not os.path.exists(h)]
+    except ImportError:
+        absent = ["torch"]
+    if absent:
+        sys.stderr.write("%s is not built: %s not found (the C library and its hosts do not need it)\n" % (os.path.basename(BINDING), ", ".join(absent)))
+        return False
     rocm = os.environ.get("ROCM_PATH", "/opt/rocm")
     cmd = [os.environ.get("CXX", "g++"), "-O2", "-std=c++17", "-fPIC", "-shared", "-fvisibility=hidden", "-Wall", "-D__HIP_PLATFORM_AMD__", "-DUSE_ROCM",
            "-D_GLIBCXX_USE_CXX11_ABI=%d" % torch._C._GLIBCXX_USE_CXX11_ABI, "-I", os.path.join(ROOT, "include")]
-    for d in (os.path.join(top, "include"), os.path.join(rocm, "include"), sysconfig.get_paths()["include"]):
+    for d in (os.path.join(top, "include"), os.path.join(rocm, "include"), python):
         cmd += ["-isystem", d]
     cmd += [os.path.join(HERE, "host", "torch_binding.cpp"), "-o", BINDING, "-L", HERE, "-lvpx_amd", "-Wl,-rpath,$ORIGIN",
             "-L", os.path.join(top, "lib"), "-lc10", "-lc10_hip", "-ltorch_cpu", "-ltorch_python"]
     if verbose:
         print(" ".join(cmd), flush=True)
     subprocess.check_call(cmd)
+    return True
 
 
 def _drain(procs, verbose):
