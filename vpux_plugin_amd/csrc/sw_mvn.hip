@@ -2,20 +2,19 @@
 // square root) or x - mean; group = (C,H,W) of one batch element when across_channels, else (H,W)
 // of one channel (VPU.MVN, src/vpux_compiler/tblgen/vpux/compiler/dialect/VPU/ops.td:3600-3652).
 //
-// Statistics are fp32.  Each workgroup owns one 4096-element chunk of a group, keeps it in
-// registers, computes the chunk's mean and centred sum of squares exactly in two register passes
-// and publishes {count, mean, M2}.  Chunks of a group are merged with the pairwise update of
-// Chan et al. in a fixed tree order, so results do not depend on scheduling.  This is the
+// Statistics are fp32: mean and centred sum of squares in two passes over values that stay on chip.  Where a group is more
+// than one workgroup's, each publishes {count, mean, M2} of its part and the parts are merged with the pairwise update of
+// Chan et al. in a fixed order, so results do not depend on scheduling.  This is the
 // decomposition the compiler itself uses when a group does not fit local memory
 // (MVN1Sum -> MVN1MeanVar -> MVN1Normalize,
 // src/vpux_compiler/src/NPU37XX/dialect/VPU/transforms/passes/decompose_mvn.cpp:82-129), with
 // centred partial sums instead of raw sum / sum of squares.
 //
-// Two launches on purpose.  A single launch whose workgroups keep their chunk in registers and
-// meet at a device-wide barrier (arrival counter + bounded wait) was built and measured: on this
-// part the barrier alone costs about 30 us (device-scope atomics from 1024 workgroups on 8 dies
-// meet in memory, not in a cache), against about 3 us for a launch boundary, and the second read
-// of the input comes from L2 / Infinity Cache anyway.
+// Groups that one wavefront or workgroup holds (registers or LDS) take one launch without any exchange.  Up to 16 longer
+// groups that the chip's registers hold take one launch whose workgroups exchange their moments (mvn_fused_kernel): tagged
+// records that each polls for its own group, 2.9 us, where an arrival counter for the whole device took about 30.  What is
+// left -- more or longer groups, input and output in one place -- takes two launches over 4096-element chunks, the second
+// of which reads the tensor again.
 #include <atomic>
 
 #include "vpx_common.h"
