@@ -81,9 +81,9 @@ VPX_API int vpx_sw_kernel_launch(const char* entry, const void* params, size_t p
  * reference.  Kernels that need scratch memory (mvn1 / mvn6 chunk moments, the MVN-1 decomposition's partial sums,
  * dynamic_quantize's range pass, per-axis quantize / dequantize tables) take it from one fixed array of
  * VPX_NOALLOC_SCRATCH_BYTES in device memory that the library holds on every device it runs on; a launch that
- * would need more returns VPX_RESULT_ERROR_OUT_OF_MEMORY and enqueues nothing (the library keeps a further 128 KiB of
- * counters behind it for kernels whose workgroups meet inside one launch).  The call performs no hipMalloc /
- * hipFree.  All calls on one device share that array and it keeps the previous call's contents: calls through
+ * would need more returns VPX_RESULT_ERROR_OUT_OF_MEMORY and enqueues nothing (behind it the library keeps a further
+ * 8.7 MiB of launch counts and records for kernels whose workgroups meet inside one launch: 12.7 MiB per device in
+ * all).  The call performs no hipMalloc / hipFree.  All calls on one device share that array and it keeps the previous call's contents: calls through
  * this entry point that may overlap on one device (different streams, or different threads) race; order them on
  * one stream.  Arguments, results and errors are otherwise those of vpx_sw_kernel_launch. */
 #define VPX_NOALLOC_SCRATCH_BYTES (4u << 20)
@@ -95,14 +95,16 @@ VPX_API int vpx_sw_kernel_launch_noalloc(const char* entry, const void* params, 
  * grows it with hipMalloc when a launch needs more: mvn1 / mvn6 / mvn1_sum with several chunks per group (12 bytes
  * per 4096 values), dynamic_quantize, per-axis quantize / dequantize tables, and an NCE task with a non-zero
  * activation zero point, unsigned weights or a weight zero point (4 bytes per output channel and per output
- * position, plus a signed copy of unsigned weights).  A launch on a capturing stream that would have to grow the
- * block returns VPX_RESULT_ERROR_UNSUPPORTED_FEATURE instead.
+ * position, plus a signed copy of unsigned weights).  The first one-launch mvn1 on a stream (few long groups, or
+ * per-channel statistics on a channel-minor layout) and vpx_workspace_reserve also allocate the 8.7 MiB of launch counts
+ * and records that its workgroups meet at.  A launch on a capturing stream that would have to allocate either
+ * returns VPX_RESULT_ERROR_UNSUPPORTED_FEATURE instead.
  * vpx_workspace_reserve grows the block of `stream` on the current device to at least `bytes` ahead of time (before
  * a capture, or to keep hipMalloc out of a serving loop).  vpx_workspace_release waits for the stream, then frees
  * its block, the blocks it outgrew and the per-axis tables cached for it; the next launch allocates afresh.
  * Blocks are keyed by the stream HANDLE: release before destroying a stream (a new stream may get the same
  * handle), and do not run one handle's work concurrently from several threads' per-thread streams.  A graph captured
- * on a stream records the addresses of that stream's block, counter area and cached tables: destroy such graphs
+ * on a stream records the addresses of that stream's block, launch counts and cached tables: destroy such graphs
  * before releasing the stream's workspace (and replay them on no other stream).  Every block is freed even when one
  * hipFree fails; the first failure is what the call returns. */
 VPX_API int vpx_workspace_reserve(void* stream, size_t bytes);
@@ -230,9 +232,11 @@ VPX_API int vpx_nce_task(const vpx_nce_task_t* task, void* stream);
 /* Testing and tuning hook (no counterpart in the reference): overrides how vpx_nce_task picks its device kernel.
  * `knob` is one of "VPX_NCE_KERNEL" (naive | gather | conv), "VPX_GEMM_TILE" (128 | 256), "VPX_GEMM_WAVES" (4 | 8),
  * "VPX_GEMM_REGB" (on | wide | off: the weights-in-registers matmul for every K up to 256 that is a multiple of 16, which by
- * itself serves layers of many rows; wide: with as many channel blocks per wave as it otherwise takes from some hundreds of thousands of rows on),
+ * itself serves layers of many rows; wide: with as many channel blocks per wave as it otherwise takes from some hundreds of
+ * thousands of rows on),
  * "VPX_NCE_DIRECT" (off | tm,tn,waves: never, or always with tiles of 16 tm channels x 16 tn positions and K over that many waves,
- * the form that stages nothing, which by itself serves layers that are over before a tile is staged),
+ * the form that stages nothing, which by itself serves layers that are over before a tile is staged; 1,1 / 2,1 / 2,2 with one to
+ * eight waves, 2,4 / 4,4 with one, others are refused),
  * "VPX_GEMM_PINGPONG" (on: the two waves of a SIMD take turns at the MFMAs of the large matmul tile; measured slower, off by default),
  * "VPX_CONV_KERNEL" (regw | tile | stream), "VPX_CONV_ROWS" (n), "VPX_CONV_COLS" (n), "VPX_CONV_WAVES" (4 | 8), "VPX_STREAM_KSPLIT" (off: the streamed-weights
  * convolution kernel gives every wave a 32 x 32 tile also on small planes, instead of splitting K over the waves of a group),

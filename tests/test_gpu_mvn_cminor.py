@@ -61,7 +61,8 @@ def test_launch_after_launch(rt, dev):
         assert torch.equal(y, firsts[(k * 3) % len(sets)])
 
 
-@pytest.mark.parametrize("shape", [(2, 37, 55, 16), (1, 100, 101, 20), (5, 53, 61, 17), (2, 130, 105, 176), (3, 79, 98, 215), (1, 64, 66, 509), (2, 101, 99, 34), (4, 112, 112, 256)])
+@pytest.mark.parametrize("shape", [(2, 37, 55, 16), (1, 100, 101, 20), (5, 53, 61, 17), (2, 130, 105, 176), (3, 79, 98, 215), (1, 64, 66, 509), (2, 101, 99, 34), (4, 112, 112, 256),
+                                   (16, 112, 112, 256), (1, 448, 448, 256), (1, 900, 900, 17)])
 def test_without_waiting(rt, dev, shape):
     import torch
     x, _, y = make(dev, shape)

@@ -41,7 +41,7 @@ def test_images(rt, dev, shape, offset):
     run(rt, dev, shape, True, offset)
 
 
-@pytest.mark.parametrize("shape", [(2, 31, 101, 103), (3, 64, 181, 183)])
+@pytest.mark.parametrize("shape", [(2, 31, 101, 103), (3, 64, 181, 183), (1, 96, 512, 512), (2, 399, 255, 257)])
 def test_images_without_waiting(rt, dev, shape):
     import torch
     x, y = run(rt, dev, shape, True)

@@ -124,7 +124,7 @@ int get_workspace(hipStream_t stream, size_t bytes, void** out) {
 
 // Launch counts and tagged records that start as zeros; a launch leaves its groups' counts moved on by one and its records
 // behind, which carry a tag that no later launch uses, so launches on one stream can share them without a clearing pass.
-// One area of kSyncBytes (8.6 MiB) per (device, stream handle), allocated and cleared on first need (the one-launch MVN
+// One area of kSyncBytes (8.7 MiB) per (device, stream handle), allocated and cleared on first need (the one-launch MVN
 // kernels, vpx_workspace_reserve); nothing else is ever written there.
 int get_sync_area(hipStream_t stream, void** out) {
     if (t_noalloc) {
@@ -140,7 +140,7 @@ int get_sync_area(hipStream_t stream, void** out) {
     Scratch& sc = g_ws[std::make_pair(dev, stream)];
     if (!sc.sync) {
         VPX_REQUIRE(!stream_is_capturing(stream), VPX_RESULT_ERROR_UNSUPPORTED_FEATURE,
-                    "the stream is capturing and has no counter area yet: call vpx_workspace_reserve before the capture, "
+                    "the stream is capturing and has no area for launch counts and records yet: call vpx_workspace_reserve before the capture, "
                     "or use vpx_sw_kernel_launch_noalloc");
         void* p = nullptr;
         VPX_HIP_CHECK(hipMalloc(&p, kSyncBytes));
