@@ -42,7 +42,7 @@ constexpr int regb_waves_per_simd(bool same_f, int ks, int cbw, int nt) {
 template <bool SAME_F, int KS, int CBW, int GW, int NT>
 __global__ __launch_bounds__(64 * kRegbWaves) __attribute__((amdgpu_waves_per_eu(regb_waves_per_simd(SAME_F, KS, CBW, NT)))) void nce_gemm_regb(
     const int8_t* __restrict__ A, const int8_t* __restrict__ B, const int32_t* __restrict__ wt, uint8_t* __restrict__ out, int64_t M, int N,
-    int chunks, int64_t lda, int64_t ldc, GemmPpe ppe, int supers, int sign_flip) {
+    int chunks, int64_t lda, int64_t ldc, GemmPpe ppe, int supers, int sign_flip, int past_cache) {
     constexpr int BCH = 16 * NT, NCH = CBW * BCH, RSW = kRegbWaves / GW, TCH = GW * NCH;
     static_assert(TCH <= 64 * kRegbWaves, "one thread prepares one channel");
     constexpr int kPrefetch = KS * CBW >= 4 ? (KS == 1 ? 2 : 1) : (KS == 1 ? 3 : 2);  // row blocks ahead; (kPrefetch + 1) x KS x 4 registers
@@ -148,9 +148,6 @@ __global__ __launch_bounds__(64 * kRegbWaves) __attribute__((amdgpu_waves_per_eu
     constexpr int kTileStride = NCH + 32, PPR = NCH / 16;
     __shared__ __attribute__((aligned(16))) uint8_t s_tile[kRegbWaves][16 * kTileStride];
     uint8_t* const tile_w = &s_tile[w][n16 * kTileStride + c4 * (4 * NT)];
-    // (pieces of rows that do not begin and end at 64-byte boundaries share cache lines with the next wave's: they are left
-    // to the cache to put together)
-    const bool whole = NCH % 64 == 0 && (ldc & 63) == 0;
     auto write_out = [&](int b) {
 #pragma unroll
         for (int p = lane; p < 16 * PPR; p += 64) {
@@ -160,8 +157,13 @@ __global__ __launch_bounds__(64 * kRegbWaves) __attribute__((amdgpu_waves_per_eu
             const int col = n0 + piece * 16;
             i32x4* const dst = reinterpret_cast<i32x4*>(out + (m * ldc + col));
             if (m < M && col < N) {
-                if (whole) __builtin_nontemporal_store(v, dst);
-                else *dst = v;
+                if (past_cache) {
+                    __builtin_nontemporal_store(v, dst);
+                } else {
+                    asm volatile("");  // (without the two, both stores are compiled to one plain one)
+                    *dst = v;
+                    asm volatile("");
+                }
             }
         }
     };
@@ -291,10 +293,19 @@ int launch_gemm_regb(const GemmLaunch& a, const RegbShape& r, int workgroups, hi
     const bool same_f = a.ppe.prelu_mult == 1 && a.ppe.prelu_shift == 0;
     const int ks = (int)((a.K + 63) / 64);
     const int sign_flip = a.in_u8 ? (int)0x80808080 : 0;
+    // Stores go past the cache where the waves of a workgroup fill whole 128-byte lines and the result is up to 16 MB.  Through
+    // the cache / past it, us, alone: [25088 x 64] . [64 x 256] 6.0 / 5.2, [100352 x 64] . [64 x 128] 9.2 / 7.4, [25088 x 128] . [128
+    // x 512] 12.3 / 10.5; with the eltwise that reads the result 11.4 / 10.9, 18.7 / 17.6, 21.7 / 21.2.  A larger one is found in the
+    // Infinity Cache by the next call, which gains what the store lost: [100352 x 64] . [64 x 256] 13.7 / 10.7 alone, but in a
+    // residual block (three convolutions and the eltwise) 46.0 / 46.7; [401408 x 64] . [64 x 256] 39.3 / 36.3, with the eltwise 84 / 87.
+    // Rows that begin inside a line share it with their neighbours and are left to the cache to put together ([100352 x 64] .
+    // [64 x 192] 11.8 / 11.8, with the eltwise 23.6 / 24.3).
+    const int nch = 16 * r.nt * r.cbw;
+    const int past_cache = nch % 64 == 0 && ((a.dst.sw & 127) == 0 || a.dst.sw == nch) && a.M * a.N <= (16ll << 20) ? 1 : 0;
     if (supers < 1 || workgroups % supers != 0 || a.K % 16 != 0) return VPX_RESULT_ERROR_UNKNOWN;
     const auto launch = [&](auto kernel) {
         hipLaunchKernelGGL(kernel, dim3((unsigned)workgroups), dim3(64 * kRegbWaves), 0, s, a.A, a.B, a.wt, a.out, a.M, (int)a.N, (int)(a.K / 16),
-                           a.rows.lda, a.dst.sw, a.ppe, supers, sign_flip);
+                           a.rows.lda, a.dst.sw, a.ppe, supers, sign_flip, past_cache);
     };
     bool known = true;
     const auto by_groups = [&](auto same_c, auto ks_c, auto cbw_c, auto nt_c) {
