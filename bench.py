@@ -35,11 +35,11 @@ METRIC = "int8 conv/matmul TOPS (% MFMA peak); SW-kernel GB/s (% HBM peak)"
 # WRITE_SIZE counters of an earlier run of the same workload, scaled by a plain copy of known size
 # (profiles/<workload>__*.md hold those runs and their commands); the JSON line labels them as such.
 MEASURED_TRAFFIC = {
-    "c1_fake_quantize": 888450, "c2_softmax": 134261983, "c3_mvn": 17043564, "c4_conv": 14905457,
+    "c1_fake_quantize": 888450, "c2_softmax": 134261983, "c3_mvn": 17093583, "c4_conv": 14905457,
     "c5_matmul": 339731998, "c5_dequantize": 135262411, "c5_eltwise_add": 270552950, "c5_nce_eltwise": 135260008,
     "calib_copy": 134217728, "calib_int_mm": 534882288, "x_mvn6_layernorm": 268523883, "x_activation_hswish": 180471319,
     "x_mvn1_three_steps": 25341653, "x_stem_conv": 67131551, "x_small_plane_conv": 20886567, "x_large_conv": 54593192,
-    "x_wide_conv": 58724921, "x_pointwise_conv": 36744405, "x_softmax_outer_axis": 402620437, "x_mvn_nhwc_per_channel": 212575560,
+    "x_wide_conv": 58724921, "x_pointwise_conv": 32407905, "x_softmax_outer_axis": 402620437, "x_mvn_nhwc_per_channel": 212576856,
 }
 
 
