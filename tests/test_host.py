@@ -138,6 +138,17 @@ def test_operator_functions_refuse_what_does_not_fit(rt):
         rt.nce_matmul(torch.empty((0, 1), dtype=torch.int8), torch.zeros(16, dtype=torch.int8), wt, torch.empty((0, 16), dtype=torch.int8), ppe, stream=stream)
 
 
+def test_the_native_module_by_itself(rt):
+    """What its entry points index with is checked where they are called, not by their callers alone."""
+    import torch
+    x = torch.zeros(4, dtype=torch.float16)
+    for inputs in (-1, -2 ** 31, 3):
+        with pytest.raises(ValueError):
+            rt._bind().launch(b"convert", inputs, None, b"", None, False, x, x)
+    with pytest.raises(KeyError):
+        rt._bind().launch(b"convert", 1, "NOPE", b"", None, False, x, x)
+
+
 def test_half_conversion_matches_oracle(rt, orc):
     L = rt.lib()
     rng = np.random.default_rng(11)

@@ -102,6 +102,7 @@ uint64_t order_code(PyObject* order, int64_t rank) {
         return code;
     }
     if (PyUnicode_Check(order)) {
+        if (!g_orders) raise(PyExc_RuntimeError, "set_orders was not called");
         PyObject* code = PyDict_GetItemWithError(g_orders, order);
         if (!code) {
             if (!PyErr_Occurred()) PyErr_SetObject(PyExc_KeyError, order);
@@ -163,7 +164,7 @@ constexpr int kMostTensors = 16, kMostAxes = 32;
 // order: one layout for all tensors, or a tuple with one each.
 PyObject* launch_tensors(const char* entry, int n_in, int n, PyObject* const* objects, PyObject* order, const void* attrs, size_t attrs_size,
                          PyObject* stream, bool noalloc) {
-    if (n > kMostTensors || n_in > n) raise(PyExc_ValueError, "too many operands");
+    if (n > kMostTensors || n_in < 0 || n_in > n) raise(PyExc_ValueError, "a number of operands that no launch has");
     if (PyTuple_Check(order) && PyTuple_GET_SIZE(order) != n) raise(PyExc_ValueError, "one layout per operand, or one for all");
     const at::Tensor* t[kMostTensors];
     Blob b = Blob::fresh();
@@ -321,6 +322,7 @@ PyObject* py_quantize(PyObject*, PyObject* const* a, Py_ssize_t n) {
 
 // A PpeInt, or a tuple of its fields.
 void read_ppe(PyObject* o, vpx_ppe_int_t* ppe) {
+    if (!g_ppe) raise(PyExc_RuntimeError, "set_ppe was not called");
     PyObject* made = nullptr;
     if (PyTuple_Check(o)) {
         o = made = PyObject_CallObject(g_ppe, o);
