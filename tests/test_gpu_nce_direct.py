@@ -52,3 +52,32 @@ def test_families_without_it(rt, orc, dev, family):
     for in_kind, out_kind, in_u8 in (("dense", "dense", True), ("window_chan", "window", False)):
         assert run_views(rt, orc, dev, rng, g, in_kind, out_kind, in_u8=in_u8, out_signed=not in_u8, force=force,
                          tuning=tuple(tuning) + (("VPX_NCE_DIRECT", "off"),)) == kernel
+
+
+@pytest.mark.parametrize("shape,depth", [("1,1,1", 8), ("1,1,8", 8), ("2,1,1", 6), ("2,1,8", 6), ("2,2,1", 4), ("2,2,8", 4), ("2,4,1", 3), ("4,4,1", 2)])
+@pytest.mark.parametrize("taps", [1, 3])
+def test_walks_around_the_steps_asked_for_at_once(rt, orc, dev, shape, depth, taps):
+    """K of one step less than a wave asks for, as many, one more, twice as many; taps per step (64 channels) and per lane (48);
+    scales below 1/2 (the epilogue without clipping), both signs of the multiplier, odd rows of bytes."""
+    import torch
+    waves = int(shape.split(",")[2])
+    rng = np.random.default_rng(seed("walk", shape, taps))
+    for steps in (depth - 1, depth, depth + 1, 2 * depth - 1, 2 * depth):
+        for unit in ((64, 48) if taps == 3 else (64,)):
+            IC = unit if taps == 3 else 64 * steps * waves
+            KY = max(1, steps * waves * 64 // (unit * taps)) if taps == 3 else 1
+            N, H, W, OC = 2, KY + 2, 9, 37
+            inp = rng.integers(0, 256, (N, H, W, IC), dtype=np.uint8)
+            w = rng.integers(-127, 128, (OC, KY, taps, IC)).astype(np.int8)
+            mults, shifts = rng.integers(2 ** 13, 2 ** 15, OC) * rng.choice([-1, 1], OC), rng.integers(23, 26, OC)
+            wt = rt.make_weights_table(mults, shifts, rng.integers(-2 ** 15, 2 ** 15, OC).astype(np.int32), KY * taps * IC)
+            pads = (1, 1, 1, 1) if taps == 3 else (0, 0, 0, 0)
+            want = orc.nce_conv(inp, w, wt, orc.ppe(1638, 14, 4, 0, 255), zp_in=101, pads=pads)
+            out = torch.zeros(want.shape, dtype=torch.uint8, device=dev)
+            rt.set_tuning("VPX_NCE_DIRECT", shape)
+            try:
+                rt.nce_task(*(torch.from_numpy(a).to(dev) for a in (inp, w, wt)), out, rt.PpeInt(rt.PPE_LPRELU, 0, 255, 1638, 14), zp_in=101, zp_out=4, pads=pads)
+            finally:
+                rt.set_tuning("VPX_NCE_DIRECT", None)
+            assert rt.nce_last_kernel() == "nce_direct"
+            assert np.array_equal(out.cpu().numpy(), want), (steps, unit)
