@@ -8,6 +8,7 @@
 //   nce_direct.hip      nce_direct: small layers of every kind, nothing staged
 //   nce_conv_patch.hip  nce_conv_regw / nce_conv_tile / nce_conv_stream: input rows of a tile in LDS
 //   nce_conv_rows.hip   nce_conv_rows16: channel counts that are a multiple of 16 only
+//   nce_conv_strips.hip nce_conv_strips: the same with a patch per wave
 //   nce_conv_gather.hip nce_conv_mfma / nce_conv_mfma16 / nce_conv_naive: the general fallbacks
 //   nce_eltwise.hip     task type ELTWISE
 //
@@ -33,6 +34,7 @@ namespace nce {
 
 typedef int32_t i32x4 __attribute__((ext_vector_type(4)));
 typedef int32_t i32x16 __attribute__((ext_vector_type(16)));
+typedef i32x4 i32x4_any __attribute__((aligned(1)));  // (the hardware takes wide accesses at any address)
 
 struct Ppe {
     int prelu_mult, prelu_shift, zp_out, clamp_lo, clamp_hi;
@@ -589,6 +591,24 @@ struct RowsGeom {
     FastDiv tiles_y, ow, rc, cpp, kc, fm, rin;  // tiles per image, OW, row_chunks, chunks per pixel, 2 * S, m, chunks per kernel row
 };
 
+// Tiles of the row-patch kernel with a patch per wave.  (Offsets inside an image fit 32 bits.)
+struct StripGeom {
+    int64_t isn, osn;      // from image to image
+    int ish, isw, osh, osw;
+    int H, W, OH, OW, OC;
+    int SY, SX, PT, PL;
+    int R, cw_log;         // output rows per tile; its columns: 16 or 32
+    int PH, RB;            // patch rows: (R - 1) * SY + KY; bytes per patch row in LDS: m planes of `plane` chunks
+    int row_chunks;        // 16-byte chunks per patch row, 128 at most
+    int m, plane;          // chunks between neighbouring output positions; chunks per plane
+    int patch_bytes;       // per wave
+    int PW;                // input columns under a tile
+    int nchunks, S, WS;    // K / 16; MFMA steps; bytes per weight row in LDS
+    int every, more;       // tiles a wave walks; waves that walk one more
+    int pad32;             // the padding byte, four times
+    FastDiv tiles_x, tiles_y, cpp, kc, fm, rin;  // as in RowsGeom
+};
+
 // TN: channel tiles of 32 per workgroup (1 for layers of up to 32 output channels; 4, with TM = 2, for short-K layers of
 // many output channels, whose input rows are then staged by half as many workgroups).  MULTI: some workgroup takes more
 
@@ -620,6 +640,7 @@ struct Tuning {
     std::atomic<int> conv_cols{0};          // VPX_CONV_COLS = n: output columns per tile of the row-patch kernel
     std::atomic<int> conv_waves{0};         // VPX_CONV_WAVES = 4 | 8
     std::atomic<int> stream_ksplit{1};      // VPX_STREAM_KSPLIT = off: the streamed-weights kernel never splits K over its waves
+    std::atomic<int> conv_strips{0};        // VPX_CONV_STRIPS = off | 16 | 32: never / with tiles of that many columns the row-patch kernel with a patch per wave (-1, 16, 32; 0: by size)
     std::atomic<int> direct{0};             // VPX_NCE_DIRECT = off | tm,tn,waves: never / always (with that tile) the kernel that stages nothing (-1, tm << 16 | tn << 8 | waves; 0: by size)
     std::atomic<int> mvn_fused{1};          // VPX_MVN_FUSED = off | nowait (see tuning_mvn_fused)
     std::atomic<int> calib_blocks{0};       // VPX_CALIB_BLOCKS = n: workgroups of the MFMA calibration loop (0: one per compute unit)
@@ -731,6 +752,21 @@ struct RowsLaunch {
     size_t lds;
 };
 int launch_conv_rows16(const RowsLaunch& a, hipStream_t s);
+
+// nce_conv_strips.hip: 64 channels per workgroup of kStripWaves waves.
+constexpr int kStripWaves = 8;
+struct StripLaunch {
+    const int8_t* in;
+    const int8_t* w;
+    const int32_t* wt;
+    uint8_t* out;
+    StripGeom sg;
+    GemmPpe ppe;
+    bool in_u8;
+    dim3 grid;
+    size_t lds;
+};
+int launch_conv_strips(const StripLaunch& a, hipStream_t s);
 
 // nce_conv_gather.hip
 int launch_fold(const int8_t* w, const int32_t* wt, ChanPrep* prep, int64_t OC, int64_t K, int corr, const Ppe& ppe, int shift_sub,

@@ -31,7 +31,6 @@ namespace {
 constexpr int kMaxWaves = 8;
 
 typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
-typedef i32x4 i32x4_any __attribute__((aligned(1)));
 typedef u32x2 u32x2_any __attribute__((aligned(1)));
 typedef uint32_t u32_any __attribute__((aligned(1)));
 
