@@ -20,6 +20,14 @@
 // rows, neighbouring lanes neighbouring 16-byte pieces (measured at [401408 x 64] . [64 x 256]: 64-byte pieces of
 // 256-byte rows, one per lane quarter, 34 us; a row per sixteen lanes 28 us).
 //
+// The set-up was half of a launch: weights (each wave its own copy, sixteen rows a load), then the weight table behind two barriers,
+// then the first rows' way from memory, one after the other.  All are asked for at once now, a wave's first row block first; four
+// waves with the same channels and a K beyond 64 deal one contiguous fetch out through LDS; channel sums come from MFMAs against
+// ones.  us in a HIP graph over rotating buffers, before / after: [100352 x 256] . [256 x 64] 12.9 / 9.8, [34848 x 256] . [256 x 64] 9.5 / 6.7,
+// [100352 x 128] . [128 x 32] 8.1 / 6.6, [100352 x 64] . [64 x 256] 14.3 / 13.2, [401408 x 64] . [64 x 256] 38.5 / 33.6, [16854 x 192] . [192 x 48] 5.0 / 4.2,
+// [9000 x 32] . [32 x 128] 4.0 / 3.2.  (More blocks asked for ahead of the weights hold up the set-up: 11.1 at K = 256.)
+// What is left at K = 64: a SIMD's vector instructions (115 a block of 16 x 64, 64 of them the PPE) as long as its memory time.
+//
 // Work is dealt by wave.  The four waves of a workgroup serve GW different groups of CBW channel blocks (4 / GW row
 // streams each): with GW > 1 the waves that share a row block are neighbours, so its rows come from memory once.  A
 // workgroup's index modulo the number of its kind picks the channels; wave s of those that share them takes row blocks
@@ -45,7 +53,7 @@ __global__ __launch_bounds__(64 * kRegbWaves) __attribute__((amdgpu_waves_per_eu
     int chunks, int64_t lda, int64_t ldc, GemmPpe ppe, int supers, int sign_flip, int past_cache) {
     constexpr int BCH = 16 * NT, NCH = CBW * BCH, RSW = kRegbWaves / GW, TCH = GW * NCH;
     static_assert(TCH <= 64 * kRegbWaves, "one thread prepares one channel");
-    constexpr int kPrefetch = KS * CBW >= 4 ? (KS == 1 ? 2 : 1) : (KS == 1 ? 3 : 2);  // row blocks ahead; (kPrefetch + 1) x KS x 4 registers
+    constexpr int kPrefetch = KS == 4 ? 1 : (KS == 1 && CBW < 4 ? 3 : 2);  // row blocks ahead; (kPrefetch + 1) x KS x 4 registers
     const int tid = threadIdx.x, lane = tid & 63;
     const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int gw = w / RSW, super = (int)blockIdx.x % supers;
@@ -55,50 +63,101 @@ __global__ __launch_bounds__(64 * kRegbWaves) __attribute__((amdgpu_waves_per_eu
     const int tb = gw * NCH;                 // ... and its place in the workgroup's tables
 
     const bool tail = (KS - 1) * 4 + c4 < chunks;  // the last fragment's chunk of this lane exists
-    // ---- this wave's weights and their column sums.  Fragment (cbl, j): row n16 of tile j of block cbl, 16 of K per quarter.
+    const int nblk = (int)((M + 15) >> 4);
+    const int tail_at = tail ? (KS - 1) * 64 + c4 * 16 : 0;
+    auto fetch = [&](int b, i32x4 (&a)[KS]) {
+        int64_t row = (int64_t)b * 16 + n16;
+        row = row < M ? row : M - 1;
+        const int8_t* src = A + row * lda;
+#pragma unroll
+        for (int ks = 0; ks < KS; ks++) a[ks] = *reinterpret_cast<const i32x4*>(src + (ks < KS - 1 ? c4 * 16 + ks * 64 : tail_at));
+    };
+    // ---- everything the set-up waits for is asked for at once, the longest way first: the first row blocks (from memory; past the
+    // last one its last row), this thread's words of the weight table, the weights (from the caches: every workgroup reads them)
+    i32x4 a[kPrefetch + 1][KS];
+    fetch(stream, a[0]);
+    const auto fetch_ahead = [&]() __attribute__((always_inline)) {
+#pragma unroll
+        for (int p = 1; p < kPrefetch; p++) fetch(stream + p * streams, a[p]);
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    int2 words = int2{0, 0};
+    if (tid < TCH) {
+        const int ch = super * TCH + tid;
+        words = *reinterpret_cast<const int2*>(wt + (int64_t)(ch < N ? ch : N - 1) * 4 + 2);
+    }
+    // Fragment (cbl, j) of the weights: row n16 of tile j of block cbl, 16 of K per quarter.  Where the four waves serve the same channels
+    // and K is long, the workgroup fetches them once, a contiguous piece, and deals them out through LDS.
     i32x4 wb[CBW][NT][KS];
-    int colsum[CBW][NT];
+    constexpr bool SHARE = GW == 1 && KS >= 2;
+    if constexpr (SHARE) {
+        constexpr int ROW = KS * 64 + 16, PIECES = NCH * KS * 4, PER = (PIECES + 64 * kRegbWaves - 1) / (64 * kRegbWaves);
+        __shared__ __attribute__((aligned(16))) uint8_t s_w[NCH * ROW];
+        i32x4 v[PER];
 #pragma unroll
-    for (int cbl = 0; cbl < CBW; cbl++)
-#pragma unroll
-        for (int j = 0; j < NT; j++) {
-            int ch = n0 + cbl * BCH + (n16 >> 2) * (4 * NT) + j * 4 + (n16 & 3);
-            ch = ch < N ? ch : N - 1;  // channels past the end repeat the last one (never stored)
-            int sum = 0;
-#pragma unroll
-            for (int ks = 0; ks < KS; ks++) {
-                const bool real = ks < KS - 1 || tail;
-                wb[cbl][j][ks] = *reinterpret_cast<const i32x4*>(B + ((int64_t)ch * chunks + (real ? ks * 4 + c4 : 0)) * 16);
-#pragma unroll
-                for (int q = 0; q < 4; q++) wb[cbl][j][ks][q] = real ? wb[cbl][j][ks][q] : 0;
-#pragma unroll
-                for (int q = 0; q < 4; q++) sum = __builtin_amdgcn_sdot4(wb[cbl][j][ks][q], 0x01010101, sum, false);
-            }
-            if (ppe.corr != 0) {  // the four lanes that hold a channel's K sit 16 lanes apart
-                sum += __shfl_xor(sum, 16);
-                sum += __shfl_xor(sum, 32);
-            }
-            colsum[cbl][j] = sum;  // of row n16 of tile j
+        for (int u = 0; u < PER; u++) {
+            const int q0 = u * 64 * kRegbWaves + tid, q = q0 < PIECES ? q0 : PIECES - 1, row = q / (KS * 4), c = q % (KS * 4);
+            const int ch = n0 + row < N ? n0 + row : N - 1;  // channels past the end repeat the last one (never stored)
+            v[u] = *reinterpret_cast<const i32x4*>(B + ((int64_t)ch * chunks + (c < chunks ? c : 0)) * 16);
         }
-
-    // ---- PPE parameters: thread t prepares channel t of the workgroup's TCH into tables in LDS
-    __shared__ double s_fpos[TCH], s_fneg[TCH];
-    __shared__ __attribute__((aligned(16))) int s_bias[TCH];
-    __shared__ int s_w2[TCH], s_sum[TCH];
-    if (ppe.corr != 0 && c4 == 0) {  // (waves that serve the same channels write the same sums)
+        fetch_ahead();
+#pragma unroll
+        for (int u = 0; u < PER; u++) {
+            const int q0 = u * 64 * kRegbWaves + tid, q = q0 < PIECES ? q0 : PIECES - 1, row = q / (KS * 4), c = q % (KS * 4);
+            *reinterpret_cast<i32x4*>(s_w + row * ROW + c * 16) = v[u];
+        }
+        __syncthreads();
 #pragma unroll
         for (int cbl = 0; cbl < CBW; cbl++)
 #pragma unroll
-            for (int j = 0; j < NT; j++) s_sum[tb + cbl * BCH + (n16 >> 2) * (4 * NT) + j * 4 + (n16 & 3)] = colsum[cbl][j];
+            for (int j = 0; j < NT; j++)
+#pragma unroll
+                for (int ks = 0; ks < KS; ks++)
+                    wb[cbl][j][ks] = *reinterpret_cast<const i32x4*>(s_w + (cbl * BCH + (n16 >> 2) * (4 * NT) + j * 4 + (n16 & 3)) * ROW + ks * 64 + c4 * 16);
+    } else {
+#pragma unroll
+        for (int cbl = 0; cbl < CBW; cbl++)
+#pragma unroll
+            for (int j = 0; j < NT; j++) {
+                int ch = n0 + cbl * BCH + (n16 >> 2) * (4 * NT) + j * 4 + (n16 & 3);
+                ch = ch < N ? ch : N - 1;
+#pragma unroll
+                for (int ks = 0; ks < KS; ks++)
+                    wb[cbl][j][ks] = *reinterpret_cast<const i32x4*>(B + ((int64_t)ch * chunks + (ks < KS - 1 || tail ? ks * 4 + c4 : 0)) * 16);
+            }
+        fetch_ahead();
     }
-    __syncthreads();
+#pragma unroll
+    for (int cbl = 0; cbl < CBW; cbl++)
+#pragma unroll
+        for (int j = 0; j < NT; j++)
+#pragma unroll
+            for (int q = 0; q < 4; q++) wb[cbl][j][KS - 1][q] = tail ? wb[cbl][j][KS - 1][q] : 0;
+
+    // ---- PPE parameters: thread t prepares channel t of the workgroup's TCH into tables in LDS
+    __shared__ double s_fpos[TCH], s_fneg[TCH];
+    __shared__ __attribute__((aligned(16))) int s_bias[TCH], s_sum[TCH];
+    __shared__ int s_w2[TCH], s_general[kRegbWaves];
+    if (ppe.corr != 0) {
+        // the column sums by MFMAs against ones: a lane's four of a tile are four channels (waves that serve the same channels write the same)
+        const i32x4 ones = {0x01010101, 0x01010101, 0x01010101, 0x01010101};
+#pragma unroll
+        for (int cbl = 0; cbl < CBW; cbl++)
+#pragma unroll
+            for (int j = 0; j < NT; j++) {
+                i32x4 sum = i32x4{0, 0, 0, 0};
+#pragma unroll
+                for (int ks = 0; ks < KS; ks++) sum = __builtin_amdgcn_mfma_i32_16x16x64_i8(wb[cbl][j][ks], ones, sum, 0, 0, 0);
+                if (n16 == 0) *reinterpret_cast<i32x4*>(&s_sum[tb + cbl * BCH + c4 * (4 * NT) + j * 4]) = sum;
+            }
+        __syncthreads();
+    }
+    const PpePack pk = make_ppe_pack(ppe.zp_out, ppe.lo, ppe.hi, ppe.out_signed != 0);
     bool clip = false;
     if (tid < TCH) {
-        int ch = super * TCH + tid;
-        ch = ch < N ? ch : N - 1;
         const int sum = ppe.corr != 0 ? s_sum[tid] : 0;
-        const uint32_t w2 = (uint32_t)wt[ch * 4 + 2];
-        const ChanPrep c = ppe_prepare((int)(int16_t)(w2 >> 16), (int)((w2 >> 8) & 0xffu), (int)((unsigned)wt[ch * 4 + 3] + (unsigned)(ppe.corr * sum)),
+        const uint32_t w2 = (uint32_t)words.x;
+        const ChanPrep c = ppe_prepare((int)(int16_t)(w2 >> 16), (int)((w2 >> 8) & 0xffu), (int)((unsigned)words.y + (unsigned)(ppe.corr * sum)),
                                        ppe.prelu_mult, ppe.prelu_shift);
         clip = c.bmax_pos != 0x7fffffff || c.bmax_neg != 0x7fffffff;
         s_fpos[tid] = c.f_pos;
@@ -106,27 +165,15 @@ __global__ __launch_bounds__(64 * kRegbWaves) __attribute__((amdgpu_waves_per_eu
         s_bias[tid] = c.bias;
         s_w2[tid] = (int)w2;
     }
-    __shared__ int s_general;
-    if (tid == 0) s_general = 0;
-    __syncthreads();
-    const PpePack pk = make_ppe_pack(ppe.zp_out, ppe.lo, ppe.hi, ppe.out_signed != 0);
     // the short PPE serves slopes in [0, 1] (ReLU, LeakyReLU), an even zero-point offset and scales up to 1/2
     const bool slope_ok = SAME_F || (ppe.prelu_mult >= 0 && (ppe.prelu_shift >= 31 || ppe.prelu_mult <= (1 << ppe.prelu_shift)));
-    if ((__builtin_amdgcn_ballot_w64(clip) != 0 || pk.odd != 0 || !slope_ok) && lane == 0) s_general = 1;
+    const bool special = __builtin_amdgcn_ballot_w64(clip) != 0 || pk.odd != 0 || !slope_ok;
+    if (lane == 0) s_general[w] = special ? 1 : 0;
     __syncthreads();
-    const bool general = s_general != 0;  // (one answer for the workgroup)
+    const bool general = (s_general[0] | s_general[1] | s_general[2] | s_general[3]) != 0;  // (one answer for the workgroup)
     if (n0 >= N) return;  // (a wave past the last block)
     const int32_t* const rt = ppe.rowterm;
-    const int nblk = (int)((M + 15) >> 4);
 
-    const int last = tail ? (KS - 1) * 64 + c4 * 16 : 0;
-    auto fetch = [&](int b, i32x4 (&a)[KS]) {
-        int64_t row = (int64_t)b * 16 + n16;
-        row = row < M ? row : M - 1;
-        const int8_t* src = A + row * lda;
-#pragma unroll
-        for (int ks = 0; ks < KS; ks++) a[ks] = *reinterpret_cast<const i32x4*>(src + (ks < KS - 1 ? c4 * 16 + ks * 64 : last));
-    };
     // the sums of channel block cbl of a row block: from the bias (short PPE) or from zero, the row term added
     auto multiply = [&](int cbl, const i32x4 (&f)[KS], int rowterm, i32x4 (&acc)[NT], bool from_bias) {
 #pragma unroll
@@ -216,15 +263,10 @@ __global__ __launch_bounds__(64 * kRegbWaves) __attribute__((amdgpu_waves_per_eu
     };
     if (general) {  // (nothing fetched ahead)
         for (int b = stream; b < nblk; b += streams) {
-            i32x4 a[KS];
-            fetch(b, a);
-            one_block(b, a, std::true_type{});
+            fetch(b, a[0]);
+            one_block(b, a[0], std::true_type{});
         }
     } else {
-        i32x4 a[kPrefetch + 1][KS];
-#pragma unroll
-        for (int p = 0; p < kPrefetch; p++)
-            if (stream + p * streams < nblk) fetch(stream + p * streams, a[p]);
         for (int b = stream; b < nblk; b += (kPrefetch + 1) * streams) {
 #pragma unroll
             for (int p = 0; p <= kPrefetch; p++) {
