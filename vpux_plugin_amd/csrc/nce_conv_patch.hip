@@ -258,7 +258,10 @@ __global__ __launch_bounds__(64 * NW, NW == 8 ? 1 : (TMW <= 4 ? 2 : 1)) void nce
 // (On this part the vector ALU work of one wave does not run under the MFMAs of the other wave of its SIMD, and
 // interleaving the PPE of block b-1 with the MFMAs of block b inside a wave needs a second set of accumulators,
 // which at two waves per SIMD spills: measured, a pipelined four-wave form with 32x32x32 MFMAs took 10.7 us where
-// this one takes 9.6 us at [32,56,56,64] -> 64.)
+// the form of its time took 9.6 us at [32,56,56,64] -> 64.)
+// A launch of one tile per compute unit is mostly set-up: the first wave asks for its words of the weight table before anything
+// else and prepares the 64 channels once, under the patch rows' flight -- every wave asking for its own after the staging put a
+// trip to memory behind it, 9.5 -> 8.3 us at [32,56,56,64] -> 64, 8.1 -> 7.0 at [32,46,46,64], 24.0 -> 22.6 at [128,56,56,64].
 //
 // Channel order inside a block: column n of MFMA tile j is output channel 16*(n/4) + 4*j + n%4.  After the 4x4 byte
 // transpose a lane then holds channels 16*q .. 16*q+15 of one position in its four result dwords (tile j -> dword j),
@@ -274,9 +277,10 @@ __global__ __launch_bounds__(512) void nce_conv_regw(const int8_t* __restrict__ 
     constexpr int BN = 64, IC = 64, PS = IC + 32, NW = 8, NT = 64 * NW, TAPS = KY * KX, Ktot = TAPS * IC, WS = Ktot + 32;
     static_assert((PS / 16) % 4 == 2 && (WS / 16) % 4 == 2, "conflict-free fragment reads");
     extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
-    uint8_t* const wlds = smem;             // [64][Ktot + 32], rows in tile order
-    uint8_t* const patch = smem + BN * WS;  // [PH*PW][IC + 32]
-    __shared__ int csum[BN];                // weight sums, by LDS row
+    ChanPrep* const sprep = reinterpret_cast<ChanPrep*>(smem);       // [64], by row of `wlds`
+    int* const sgeneral = reinterpret_cast<int*>(smem + BN * sizeof(ChanPrep));
+    uint8_t* const wlds = smem + kRegwTables;                        // [64][Ktot + 32], rows in tile order
+    uint8_t* const patch = wlds + BN * WS;                           // [PH*PW][IC + 32]
 
     // A launch of a few microseconds is bound by instructions as much as by anything else: all index arithmetic below
     // is 32-bit, on offsets from a few 64-bit bases that are the same for the whole wave.
@@ -290,6 +294,16 @@ __global__ __launch_bounds__(512) void nce_conv_regw(const int8_t* __restrict__ 
     // ---- weights and patch -> LDS.  All loads are issued up front, weights first: they come from L2 and are back
     // before the patch rows are, so the waves copy their weight fragments to registers while the patch is on its way.
     const int n16 = lane & 15, c4 = lane >> 4;
+    const PpePack pk = make_ppe_pack(ppe.zp_out, ppe.lo, ppe.hi, ppe.out_signed != 0);
+    // the short PPE serves slopes in [0, 1] (ReLU, LeakyReLU), an even zero-point offset and scales up to 1/2
+    const bool slope_ok = SAME_F || (ppe.prelu_mult >= 0 && (ppe.prelu_shift >= 31 || ppe.prelu_mult <= (1 << ppe.prelu_shift)));
+    // The first wave prepares the channels, lane l that of weight row l of the LDS copy, while the patch rows are on their way; its words
+    // of the weight table are asked for before anything else.
+    int2 words = int2{0, 0};
+    if (wave == 0) {
+        const int n = oc0 + (n16 >> 2) * 16 + c4 * 4 + (n16 & 3);
+        words = *reinterpret_cast<const int2*>(wt + (n < OC ? n : OC - 1) * 4 + 2);
+    }
     i32x4 wb[TAPS][4];
     {
         constexpr int cpr = Ktot / 16;                 // 16-byte chunks per weight row
@@ -358,18 +372,23 @@ __global__ __launch_bounds__(512) void nce_conv_regw(const int8_t* __restrict__ 
         for (int t = 0; t < TAPS; t++)
 #pragma unroll
             for (int j = 0; j < 4; j++) wb[t][j] = *reinterpret_cast<const i32x4*>(wlds + (j * 16 + n16) * WS + t * IC + c4 * 16);
-        // the sums of the weight rows where the zero-point term needs them
-        if (ppe.corr != 0 && tid < 256) {
-            const int row = tid >> 2, part = tid & 3;
-            int sum = 0;
-            for (int c = part; c < Ktot / 16; c += 4) {
-                const i32x4 q = *reinterpret_cast<const i32x4*>(wlds + row * WS + c * 16);
+        if (wave == 0) {
+            int sum = 0;  // of the weight row, for the zero-point term
+            if (ppe.corr != 0) {
+#pragma unroll 6
+                for (int c = 0; c < Ktot / 16; c++) {
+                    const i32x4 q = *reinterpret_cast<const i32x4*>(wlds + lane * WS + c * 16);
 #pragma unroll
-                for (int j = 0; j < 4; j++) sum = __builtin_amdgcn_sdot4(q[j], 0x01010101, sum, false);
+                    for (int j = 0; j < 4; j++) sum = __builtin_amdgcn_sdot4(q[j], 0x01010101, sum, false);
+                }
             }
-            sum += (int)dpp_u32<0xB1>((unsigned)sum);
-            sum += (int)dpp_u32<0x4E>((unsigned)sum);
-            if (part == 0) csum[row] = sum;
+            const uint32_t w2 = (uint32_t)words.x;
+            const ChanPrep c = ppe_prepare((int)(int16_t)(w2 >> 16), (int)((w2 >> 8) & 0xffu), (int)((unsigned)words.y + (unsigned)(ppe.corr * sum)),
+                                           ppe.prelu_mult, ppe.prelu_shift);
+            sprep[lane] = c;
+            const bool clip = c.bmax_pos != 0x7fffffff || c.bmax_neg != 0x7fffffff;
+            const bool special = __builtin_amdgcn_ballot_w64(clip) != 0 || pk.odd != 0 || !slope_ok;
+            if (lane == 0) sgeneral[0] = special ? 1 : 0;
         }
         store_patch();
         for (int u0 = NW * UP; u0 < units; u0 += NW * UP) {  // tall patches: the rest, a round trip each
@@ -379,24 +398,14 @@ __global__ __launch_bounds__(512) void nce_conv_regw(const int8_t* __restrict__ 
     }
     __syncthreads();
 
-    // ---- per-channel PPE parameters of the lane's four channels
+    // ---- PPE parameters of the lane's four channels
     ChanPrep cp[4];
-    bool clip = false;
 #pragma unroll
     for (int j = 0; j < 4; j++) {
-        int n = oc0 + (n16 >> 2) * 16 + j * 4 + (n16 & 3);
-        n = n < OC ? n : OC - 1;
-        const int cs = ppe.corr != 0 ? csum[j * 16 + n16] : 0;
-        const uint32_t w2 = (uint32_t)wt[n * 4 + 2];
-        cp[j] = ppe_prepare((int)(int16_t)(w2 >> 16), (int)((w2 >> 8) & 0xffu),
-                            (int)((unsigned)wt[n * 4 + 3] + (unsigned)(ppe.corr * cs)), ppe.prelu_mult, ppe.prelu_shift);
-        clip = clip || cp[j].bmax_pos != 0x7fffffff || cp[j].bmax_neg != 0x7fffffff;
+        cp[j] = sprep[j * 16 + n16];
         asm volatile("" : "+v"(cp[j].f_pos), "+v"(cp[j].f_neg));
     }
-    const PpePack pk = make_ppe_pack(ppe.zp_out, ppe.lo, ppe.hi, ppe.out_signed != 0);
-    // the short PPE serves slopes in [0, 1] (ReLU, LeakyReLU), an even zero-point offset and scales up to 1/2
-    const bool slope_ok = SAME_F || (ppe.prelu_mult >= 0 && (ppe.prelu_shift >= 31 || ppe.prelu_mult <= (1 << ppe.prelu_shift)));
-    const bool general = __builtin_amdgcn_ballot_w64(clip) != 0 || pk.odd != 0 || !slope_ok;
+    const bool general = __builtin_amdgcn_readfirstlane(sgeneral[0]) != 0;
     const QuadTranspose transpose(lane);
 
     const int rows_here = OH - oy0 < pg.R ? OH - oy0 : pg.R;
