@@ -230,7 +230,7 @@ typedef struct vpx_nce_task_t {
 VPX_API int vpx_nce_task(const vpx_nce_task_t* task, void* stream);
 
 /* Testing and tuning hook (no counterpart in the reference): overrides how vpx_nce_task picks its device kernel.
- * `knob` is one of "VPX_NCE_KERNEL" (naive | gather | conv), "VPX_GEMM_TILE" (128 | 256), "VPX_GEMM_WAVES" (4 | 8),
+ * `knob` is one of "VPX_NCE_KERNEL" (naive | gather | conv), "VPX_GEMM_TILE" (64 | 128 | 256), "VPX_GEMM_WAVES" (4 | 8),
  * "VPX_GEMM_REGB" (on | wide | off: the weights-in-registers matmul for every K up to 256 that is a multiple of 16, which by
  * itself serves layers of many rows; wide: with as many channel blocks per wave as it otherwise takes from some hundreds of
  * thousands of rows on),

@@ -632,7 +632,7 @@ int set_dyn_lds(KernelT kernel, size_t bytes) {
 enum { NCE_AUTO = 0, NCE_NAIVE, NCE_GATHER, NCE_CONV };
 struct Tuning {
     std::atomic<int> nce_kernel{NCE_AUTO};  // VPX_NCE_KERNEL = naive | gather | conv: restrict the choice to slower, more general paths
-    std::atomic<int> gemm_tile{0};          // VPX_GEMM_TILE = 128 | 256 (0: chosen from the shape)
+    std::atomic<int> gemm_tile{0};          // VPX_GEMM_TILE = 64 | 128 | 256 (0: chosen from the shape)
     std::atomic<int> gemm_waves{0};         // VPX_GEMM_WAVES = 4 | 8
     std::atomic<int> gemm_regb{0};          // VPX_GEMM_REGB = on | wide | off: weights-in-registers matmul, K up to 256 (1, 2: with the most channel blocks per wave, -1; 0: chosen from the shape)
     std::atomic<int> gemm_pingpong{0};      // VPX_GEMM_PINGPONG = on | off: the waves of a SIMD take turns at the MFMAs
@@ -667,7 +667,8 @@ struct GemmLaunch {
     const int32_t* wt;
     uint8_t* out;
     int64_t M, N, K, G;
-    int tile, waves;
+    int tile, waves;  // waves: of the 256 tile
+    int stages;       // panel buffers of the 64 and 128 tiles
     bool shortk, in_u8, pingpong;
     int out_kind;  // OutKind
     GemmPpe ppe;

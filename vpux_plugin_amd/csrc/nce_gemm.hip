@@ -1,6 +1,6 @@
 // nce_gemm_mfma: 1x1 kernel, no padding (this is how NCE.MatMul arrives; a stride picks rows from the input): a plain
-// A[M][K] x B[N][K]^T GEMM.  256 x 256 (or 128 x 128) output tile per workgroup, v_mfma_i32_32x32x32_i8, K panels from
-// global memory straight into XOR-swizzled LDS (global_load_lds, no register staging), four buffers, the integer PPE
+// A[M][K] x B[N][K]^T GEMM.  256 x 256, 128 x 128 or 64 x 64 output tile per workgroup, v_mfma_i32_32x32x32_i8, K panels from
+// global memory straight into XOR-swizzled LDS (global_load_lds, no register staging), a ring of buffers, the integer PPE
 // fused into the epilogue.
 #include "nce_common.h"
 
@@ -25,7 +25,18 @@ namespace {
 // fragment reads of its next panel, its four panel loads, the column sums -- and at a workgroup barrier they swap,
 // twice per panel.  (With both waves running the same interleaved stream their loads and reads fall on the same
 // moments and the MFMA pipe waits for both.)
-template <bool IN_U8, int OUT, int NW, int TILE = 256, bool SHORTK = false, bool PP = false>
+//
+// WIDE (the 128 tile with eight waves of 64 x 32, the 64 tile with four of 32 x 32; K of more than three panels of 64): panels of
+// 128 bytes, whole cache lines -- of 64-byte pieces the second of a line came after the first had left the first-level cache, and
+// every line was read from the second level twice -- with one barrier each, between the panel's halves.  The loads of a panel
+// stand in line far ahead and nobody waits for them; a tile of 128 takes about 850 clocks for a panel whose MFMAs take 512,
+// bound by the LDS (96 KiB of fragments and 32 KiB of loads), one of 64 about 400, bound likewise.  Four waves of 64 x 64 on
+// panels of 64, 24.5 us at [2080 x 3456] . [3456 x 608] whether or not fragments were read a panel ahead or twice the
+// panels were in flight, now take 20.2, 16.2 with the 64 tile; [512 x 4096] . [4096 x 4096] 26.9, now 22.0 and 20.7;
+// [1024 x 1024] . [1024 x 1024] 9.7, now 8.6 and 6.2.  (Eight waves of 64 x 64 with K split over two groups read a third less
+// but hand 64 KiB of sums over: 21.3 at the first.)  Summing the columns in one row of waves only cost 260 clocks a panel
+// on the SIMDs that held them; now the waves that share columns take a half of each panel each.
+template <bool IN_U8, int OUT, int NW, int TILE = 256, bool SHORTK = false, bool PP = false, int NS = 4>
 __global__ __launch_bounds__(64 * NW) void nce_gemm_mfma(const int8_t* __restrict__ A, const int8_t* __restrict__ B,
                                                      const int32_t* __restrict__ wt, const int32_t* __restrict__ colsum,
                                                      uint8_t* __restrict__ out,
@@ -33,15 +44,15 @@ __global__ __launch_bounds__(64 * NW) void nce_gemm_mfma(const int8_t* __restric
                                                      GemmPpe ppe, GemmRows rows, GemmOut dst) {
     // NW = 4: waves 2 x 2, 128 x 128 each, one per SIMD.  NW = 8: waves 2 x 4, 128 x 64 each, two per SIMD,
     // so that one wave's loads and address arithmetic issue while the other's MFMAs run.
-    // TILE = 128 (four waves of 64 x 64, 64 KiB of LDS, two workgroups per CU) serves problems with too few 256 x 256 tiles.
+    // TILE = 128 and 64 serve problems with too few 256 x 256 tiles.
     // SHORTK (K <= 192, three panels at most): all panels are fetched up front, nothing is pipelined and no panel buffer
     // is reused, so the workgroup asks only for the LDS it touches and more of them fit a CU (a matmul this short is
     // bound by its epilogue and stores, not by the MFMAs).
-    constexpr int BM = TILE, BN = TILE, BK = 64, WM = BM / 2, WN = BN / (NW / 2), TM = WM / 32, TN = WN / 32;
-    constexpr int MFMA_PER_DMA = TM * TN / (BM * BK / 1024 / NW);  // MFMAs between two DMA instructions of a sub-step
-    static_assert(TM * TN >= TM + TN && MFMA_PER_DMA >= 1, "fragment reads and DMA instructions are interleaved with the MFMAs");
+    constexpr bool WIDE = (TILE == 128 && NW == 8) || TILE == 64;
+    constexpr int BM = TILE, BN = TILE, BK = WIDE ? 128 : 64, WM = BM / 2, WN = BN / (NW / 2), TM = WM / 32, TN = WN / 32;
+    constexpr int MFMA_PER_DMA = WIDE ? 1 : TM * TN / (BM * BK / 1024 / NW);  // MFMAs between two DMA instructions of a sub-step
+    static_assert(WIDE || (TM * TN >= TM + TN && MFMA_PER_DMA >= 1), "fragment reads and DMA instructions are interleaved with the MFMAs");
     constexpr int NT = 64 * NW;
-    constexpr int NS = 4;                             // LDS panel buffers
     constexpr int CPR = BK / 16;                      // 16-byte chunks per tile row
     constexpr int RPI = 64 / CPR;                     // tile rows one 1 KiB DMA instruction covers
     constexpr int DMA_PER_WAVE = BM * BK / 1024 / NW;  // per operand, per panel
@@ -103,16 +114,20 @@ __global__ __launch_bounds__(64 * NW) void nce_gemm_mfma(const int8_t* __restric
     const int8_t* abase = rows.strided ? A : A + m0 * rows.lda;
     const int8_t* bbase = B + n0 * K;
     const unsigned lds0 = lds_address(smem);
-    const int nk = (int)(K / BK);
+    const int nk = (int)((K + BK - 1) / BK);
+    const bool half = WIDE && (K & 64) != 0;  // the last panel is half a panel
+    const unsigned past_half = WIDE && (((lane % CPR) ^ lds_swz<BK>(wave * RPI + lane / CPR)) & 4) != 0 ? 64u : 0u;
     // d-th DMA instruction (first half A, second half B) of panel p.  Panels past the end keep the number of loads
     // in flight the same in every iteration: every lane re-fetches the tile's first 16 bytes (one cache line for
     // the whole instruction) into a buffer nobody reads.
     auto dma_one = [&](auto known_real, int p, int d) {
-        const unsigned base = lds0 + (unsigned)((p & (NS - 1)) * STAGE);
+        const unsigned base = lds0 + (unsigned)((p % NS) * STAGE);
         const bool real = decltype(known_real)::value || p < nk;  // (known: no select instructions in the loop body)
         const int64_t k0 = real ? (int64_t)p * BK : 0;
-        if (d < DMA_PER_WAVE) dma16(abase + k0, real ? oa[d] : 0u, base + (unsigned)((wave + NW * d) * 1024));
-        else dma16(bbase + k0, real ? ob[d - DMA_PER_WAVE] : 0u, base + (unsigned)(BM * BK + (wave + NW * (d - DMA_PER_WAVE)) * 1024));
+        unsigned off = d < DMA_PER_WAVE ? oa[d] : ob[d - DMA_PER_WAVE];
+        if (WIDE && !decltype(known_real)::value && half && p == nk - 1) off -= past_half;  // (its second half: the first again, not multiplied)
+        if (d < DMA_PER_WAVE) dma16(abase + k0, real ? off : 0u, base + (unsigned)((wave + NW * d) * 1024));
+        else dma16(bbase + k0, real ? off : 0u, base + (unsigned)(BM * BK + (wave + NW * (d - DMA_PER_WAVE)) * 1024));
     };
 
     i32x16 acc[TM][TN];
@@ -140,6 +155,7 @@ __global__ __launch_bounds__(64 * NW) void nce_gemm_mfma(const int8_t* __restric
     for (int hi = 0; hi < 2; hi++)
 #pragma unroll
         for (int kk = 0; kk < 2; kk++) {
+            if (WIDE) continue;
             const int chunk = kk * 2 + (lane >> 5);
             frag_base[hi][0][kk] = (lds_bytes_t)(smem + hi * 2 * STAGE + lds_offset<BK>(wm0 + (lane & 31), chunk));
             frag_base[hi][1][kk] = (lds_bytes_t)(smem + hi * 2 * STAGE + BM * BK + lds_offset<BK>(wn0 + (lane & 31), chunk));
@@ -149,9 +165,9 @@ __global__ __launch_bounds__(64 * NW) void nce_gemm_mfma(const int8_t* __restric
         constexpr int stage = decltype(stage_c)::value;
         constexpr int imm = (stage & 1) * STAGE;
         // rows 32 apart are 32 * BK bytes apart and share their swizzle
-        if (n == 0) fa[slot][0] = *(lds_v4_t)(frag_base[stage >> 1][0][kk] + imm);
-        else if (n <= TN) fb[slot][n - 1] = *(lds_v4_t)(frag_base[stage >> 1][1][kk] + imm + (n - 1) * 32 * BK);
-        else fa[slot][n - TN] = *(lds_v4_t)(frag_base[stage >> 1][0][kk] + imm + (n - TN) * 32 * BK);
+        if (n == 0) fa[slot][0] = *(lds_v4_t)(frag_base[(stage >> 1) & 1][0][kk] + imm);
+        else if (n <= TN) fb[slot][n - 1] = *(lds_v4_t)(frag_base[(stage >> 1) & 1][1][kk] + imm + (n - 1) * 32 * BK);
+        else fa[slot][n - TN] = *(lds_v4_t)(frag_base[(stage >> 1) & 1][0][kk] + imm + (n - TN) * 32 * BK);
     };
     // One sub-step: the TM x TN MFMAs on fragment slot `cur`; between them, the TM + TN fragment reads of the
     // next sub-step (panel at pnext, sub-step knext) into the other slot and this wave's DMA instructions
@@ -209,11 +225,85 @@ __global__ __launch_bounds__(64 * NW) void nce_gemm_mfma(const int8_t* __restric
         w2r[j] = wt[n * 4 + 2];
         w3r[j] = wt[n * 4 + 3];
     }
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // keeps the count of loads in flight below exact
+    // (Nobody waits for these words here: they are the oldest loads in flight, so every count waited for below covers them.)
 
     constexpr std::integral_constant<int, -1> kDynamicStage{};
     auto main_loop = [&](auto sum_c) {
-        if (SHORTK) {
+        if constexpr (WIDE) {
+            // The fragments of half a panel are read under the MFMAs of the half before it; behind the barrier between the two
+            // everybody is through with the panel's buffer, which panel k + NS is then asked into.
+            constexpr int HALF = decltype(sum_c)::value;  // the half of each panel whose column sums this wave takes, or neither (2)
+            i32x4 pa[2][2][TM], pb[2][2];
+            int cs1 = 0;
+            lds_bytes_t base[2][4];  // [operand][sub-step of a panel]
+#pragma unroll
+            for (int o = 0; o < 2; o++)
+#pragma unroll
+                for (int kk = 0; kk < 4; kk++) {
+                    base[o][kk] = (lds_bytes_t)(smem + o * BM * BK + lds_offset<BK>((o ? wn0 : wm0) + (lane & 31), kk * 2 + (lane >> 5)));
+                    asm volatile("" : "+v"(base[o][kk]));
+                }
+            auto read_half = [&](int stage, auto h_c) {
+                constexpr int h = decltype(h_c)::value;
+#pragma unroll
+                for (int kk = 0; kk < 2; kk++) {
+                    pb[h][kk] = *(lds_v4_t)(base[1][h * 2 + kk] + stage * STAGE);
+#pragma unroll
+                    for (int i = 0; i < TM; i++) pa[h][kk][i] = *(lds_v4_t)(base[0][h * 2 + kk] + stage * STAGE + i * 32 * BK);
+                }
+                __builtin_amdgcn_sched_barrier(0);
+            };
+            auto mfma_half = [&](auto h_c, auto real_c, int p) {
+                constexpr int h = decltype(h_c)::value;
+#pragma unroll
+                for (int kk = 0; kk < 2; kk++)
+#pragma unroll
+                    for (int i = 0; i < TM; i++) {
+                        i32x4 a = pa[h][kk][i];
+                        if (IN_U8) a ^= (int32_t)0x80808080;  // u8 -> s8 (value - 128)
+                        acc[i][0] = __builtin_amdgcn_mfma_i32_32x32x32_i8(a, pb[h][kk], acc[i][0], 0, 0, 0);
+                        if (h == 1) {
+#pragma unroll
+                            for (int d = 0; d < DMA_PER_WAVE / TM; d++) dma_one(real_c, p, (kk * TM + i) * (DMA_PER_WAVE / TM) + d);
+                        }
+                        if (h == HALF && kk == 1 && i == 0) {  // (two chains: an instruction need not wait for the one before it)
+#pragma unroll
+                            for (int d = 0; d < 4; d++) {
+                                cs[0] = __builtin_amdgcn_sdot4(pb[h][0][d], 0x01010101, cs[0], false);
+                                cs1 = __builtin_amdgcn_sdot4(pb[h][1][d], 0x01010101, cs1, false);
+                            }
+                        }
+                        __builtin_amdgcn_sched_barrier(0);
+                    }
+            };
+            static_assert(!WIDE || (DMA_PER_WAVE % TM == 0 && TN == 1), "the same number of loads behind each MFMA of a second half");
+            constexpr std::integral_constant<int, 0> first{};
+            constexpr std::integral_constant<int, 1> second{};
+            auto one_panel = [&](int u, auto real_c, int k) {
+                read_half(u, second);
+                mfma_half(first, real_c, 0);
+                asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"((NS - 2) * 2 * DMA_PER_WAVE) : "memory");  // panel k + 1 is in
+                read_half((u + 1) % NS, first);
+                if (decltype(real_c)::value || k + 1 < nk || !half) mfma_half(second, real_c, k + NS);
+            };
+#pragma unroll
+            for (int p = 0; p < NS; p++)
+#pragma unroll
+                for (int d = 0; d < 2 * DMA_PER_WAVE; d++) dma_one(std::false_type{}, p, d);
+            asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"((NS - 1) * 2 * DMA_PER_WAVE) : "memory");  // panel 0 is in
+            read_half(0, first);
+            int kt = 0;
+            for (; kt + 2 * NS < nk; kt += NS) {  // (every panel asked for whole)
+#pragma unroll
+                for (int u = 0; u < NS; u++) one_panel(u, std::true_type{}, kt + u);
+            }
+            for (; kt < nk; kt += NS) {  // the last panels, at most two rounds
+#pragma unroll
+                for (int u = 0; u < NS; u++)
+                    if (kt + u < nk) one_panel(u, std::false_type{}, kt + u);
+            }
+            cs[0] += cs1;
+        } else if constexpr (SHORTK) {
 #pragma unroll
             for (int p = 0; p < NS - 1; p++)
                 if (p < nk) {
@@ -349,20 +439,28 @@ __global__ __launch_bounds__(64 * NW) void nce_gemm_mfma(const int8_t* __restric
         pingpong_loop();
     } else {
         // (a matmul of at most three panels is all epilogue: there every wave sums its own columns and nothing is handed over)
-        if (SHORTK || wm0 == 0) main_loop(std::true_type{});
-        else main_loop(std::false_type{});
+        if constexpr (WIDE) {  // (of the two waves on the same columns each sums half of every panel)
+            if (ppe.corr == 0) main_loop(std::integral_constant<int, 2>{});
+            else if (wm0 == 0) main_loop(std::integral_constant<int, 0>{});
+            else main_loop(std::integral_constant<int, 1>{});
+        } else {
+            if (ppe.corr != 0 && (SHORTK || wm0 == 0)) main_loop(std::true_type{});
+            else main_loop(std::false_type{});
+        }
     }
 #pragma unroll
     for (int j = 0; j < TN; j++) {
         csr[j] = cs[j] + __shfl_xor(cs[j], 32, 64);  // every lane takes part
-        if (!SHORTK && wm0 == 0 && lane < 32) colsums[wn0 + j * 32 + lane] = csr[j];
+        if (!SHORTK && (WIDE || wm0 == 0) && lane < 32) colsums[(WIDE && wm0 != 0 ? TILE : 0) + wn0 + j * 32 + lane] = csr[j];
     }
     dma_wait_all_and_barrier();  // every wave is done with the panels: LDS becomes the output staging tile
     if (!SHORTK) {
 #pragma unroll
-        for (int j = 0; j < TN; j++) csr[j] = colsums[wn0 + j * 32 + (lane & 31)];  // sum_k B[n][k] of column n of block j
+        for (int j = 0; j < TN; j++) {
+            csr[j] = colsums[wn0 + j * 32 + (lane & 31)];  // sum_k B[n][k] of column n of block j
+            if (WIDE) csr[j] += colsums[TILE + wn0 + j * 32 + (lane & 31)];
+        }
     }
-
     // Epilogue.  Accumulator register r of lane l is C[8*(r/4) + 4*(l/32) + r%4][l%32] of its 32x32 tile.
     if constexpr (OUT == OUT_F16) {
         // fp16 output: through the staging tile like the bytes below, half of a 256-row tile at a time (128 rows x 544
@@ -493,60 +591,60 @@ __global__ __launch_bounds__(64 * NW) void nce_gemm_mfma(const int8_t* __restric
 }  // namespace
 
 int launch_gemm_mfma(const GemmLaunch& a, hipStream_t s) {
-    const int tile = a.tile, nw = tile == 128 ? 4 : a.waves;
+    const int tile = a.tile, nw = tile == 64 ? 4 : (tile == 128 ? (a.shortk ? 4 : 8) : a.waves);
     const bool out_f16 = a.out_kind == OUT_F16;
     const int tiles_m = (int)((a.M + tile - 1) / tile), tiles_n = (int)((a.N + tile - 1) / tile);
     const int per_xcd = (tiles_m * tiles_n + 7) / 8;
-    const dim3 grid((unsigned)(per_xcd * 8), (unsigned)a.G), block(64 * nw);
+    const dim3 grid((unsigned)(per_xcd * 8), (unsigned)a.G);
     const int64_t nk = a.K / 64;
     const bool shortk = a.shortk;
     size_t lds = 4 * (size_t)(tile + tile) * 64;  // four K panels; the output staging tile reuses them
     if (shortk) {
         lds = (size_t)nk * (tile + tile) * 64;  // only the panels there are ...
         if (lds < (size_t)tile * kOutStride) lds = (size_t)tile * kOutStride;  // ... or the staging tile
+    } else if (tile < 256) {
+        lds = (size_t)a.stages * (tile + tile) * 128;
     }
     lds += kGemmLdsHead;
     const int32_t* colsum = nullptr;  // the kernel sums the columns of B itself, from the fragments it reads
     int rc = VPX_RESULT_SUCCESS;
     // the form in which the waves of a SIMD take turns: K a whole number of panel-buffer rounds
     const bool pingpong = a.pingpong && tile == 256 && nw == 8 && nk % 4 == 0 && nk >= 4 && !out_f16;
-#define VPX_GEMM_W(U8, SGN, NW, TILE, SHORTK)                                                                        \
+#define VPX_GEMM_K(...)                                                                                              \
     do {                                                                                                             \
-        auto kern = nce_gemm_mfma<U8, SGN, NW, TILE, SHORTK>;                                                        \
+        auto kern = nce_gemm_mfma<__VA_ARGS__>;                                                                      \
         rc = set_dyn_lds(kern, lds);                                                                                 \
         if (rc) return rc;                                                                                           \
-        hipLaunchKernelGGL(kern, grid, dim3(64 * NW), lds, s, a.A, a.B, a.wt, colsum, a.out, a.M, a.N, a.K, tiles_m,  \
+        hipLaunchKernelGGL(kern, grid, dim3(64 * nw), lds, s, a.A, a.B, a.wt, colsum, a.out, a.M, a.N, a.K, tiles_m,  \
                            tiles_n, a.ppe, a.rows, a.dst);                                                           \
     } while (0)
-#define VPX_GEMM_PP(U8, SGN)                                                                                         \
+    // the tiles of 64 and 128, any kind of output
+#define VPX_GEMM_SMALL(U8, SGN)                                                                                      \
     do {                                                                                                             \
-        auto kern = nce_gemm_mfma<U8, SGN, 8, 256, false, true>;                                                     \
-        rc = set_dyn_lds(kern, lds);                                                                                 \
-        if (rc) return rc;                                                                                           \
-        hipLaunchKernelGGL(kern, grid, dim3(512), lds, s, a.A, a.B, a.wt, colsum, a.out, a.M, a.N, a.K, tiles_m,      \
-                           tiles_n, a.ppe, a.rows, a.dst);                                                           \
+        if (tile == 64) VPX_GEMM_K(U8, SGN, 4, 64, false, false, 4);                                                 \
+        else if (a.stages == 3) VPX_GEMM_K(U8, SGN, 8, 128, false, false, 3);                                        \
+        else VPX_GEMM_K(U8, SGN, 8, 128, false, false, 2);                                                           \
     } while (0)
 #define VPX_GEMM(U8, SGN)                                                                                            \
     do {                                                                                                             \
-        if (shortk) VPX_GEMM_W(U8, SGN, 4, 128, true);                                                               \
-        else if (tile == 128) VPX_GEMM_W(U8, SGN, 4, 128, false);                                                    \
-        else if (nw == 4) VPX_GEMM_W(U8, SGN, 4, 256, false);                                                        \
-        else if (pingpong) VPX_GEMM_PP(U8, SGN);                                                                     \
-        else VPX_GEMM_W(U8, SGN, 8, 256, false);                                                                     \
+        if (shortk) VPX_GEMM_K(U8, SGN, 4, 128, true);                                                               \
+        else if (tile < 256) VPX_GEMM_SMALL(U8, SGN);                                                                \
+        else if (nw == 4) VPX_GEMM_K(U8, SGN, 4, 256);                                                               \
+        else if (pingpong) VPX_GEMM_K(U8, SGN, 8, 256, false, true);                                                 \
+        else VPX_GEMM_K(U8, SGN, 8, 256);                                                                            \
     } while (0)
     if (out_f16) {
-        // fp16 output: the eight-wave 256-tile and the four-wave 128-tile forms only (the host passes waves = 8)
-        if (a.in_u8) { if (tile == 128) VPX_GEMM_W(true, OUT_F16, 4, 128, false); else VPX_GEMM_W(true, OUT_F16, 8, 256, false); }
-        else { if (tile == 128) VPX_GEMM_W(false, OUT_F16, 4, 128, false); else VPX_GEMM_W(false, OUT_F16, 8, 256, false); }
+        // fp16 output: of the large tile the eight-wave form only (the host passes waves = 8)
+        if (a.in_u8) { if (tile < 256) VPX_GEMM_SMALL(true, OUT_F16); else VPX_GEMM_K(true, OUT_F16, 8, 256); }
+        else { if (tile < 256) VPX_GEMM_SMALL(false, OUT_F16); else VPX_GEMM_K(false, OUT_F16, 8, 256); }
     }
     else if (a.in_u8 && a.out_kind == OUT_I8) VPX_GEMM(true, OUT_I8);
     else if (a.in_u8) VPX_GEMM(true, OUT_U8);
     else if (a.out_kind == OUT_I8) VPX_GEMM(false, OUT_I8);
     else VPX_GEMM(false, OUT_U8);
 #undef VPX_GEMM
-#undef VPX_GEMM_PP
-#undef VPX_GEMM_W
-    (void)block;
+#undef VPX_GEMM_SMALL
+#undef VPX_GEMM_K
     VPX_HIP_CHECK(hipGetLastError());
     return VPX_RESULT_SUCCESS;
 }
