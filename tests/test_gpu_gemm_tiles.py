@@ -1,4 +1,4 @@
-"""The matmul kernel's 64 and 128 tiles (panels of 128 bytes, the last one halved where K is an odd multiple of 64; column sums
+"""The matmul kernel's tiles (panels of 128 bytes, the last one halved where K is an odd multiple of 64; column sums
 shared between the waves of a column) against the oracle, where the panels, the ring of buffers and the tiles end."""
 import numpy as np
 import pytest
@@ -27,7 +27,7 @@ def run(rt, orc, dev, rng, M, K, N, tile, in_u8, zp_in, zp_w, out_f16, shift=20)
     return rt.nce_last_kernel()
 
 
-@pytest.mark.parametrize("tile", [64, 128])
+@pytest.mark.parametrize("tile", [64, 128, 256])
 @pytest.mark.parametrize("K", [64, 128, 192, 256, 320, 384, 448, 512, 576, 704, 1088])
 def test_every_end_of_the_panels(rt, orc, dev, tile, K):
     """fewer panels than buffers, one more, half of one; tiles of one row, full, and one past full; sums on and off"""
@@ -38,7 +38,7 @@ def test_every_end_of_the_panels(rt, orc, dev, tile, K):
             assert name == "nce_gemm_mfma"
 
 
-@pytest.mark.parametrize("tile", [None, 64, 128])
+@pytest.mark.parametrize("tile", [None, 64, 128, 256])
 @pytest.mark.parametrize("M,K,N", [(1100, 320, 208), (2180, 448, 2070)])
 def test_outputs_and_zero_points(rt, orc, dev, tile, M, K, N):
     """fp16 outputs, a weight zero point (the per-row term), scales that clip; more tiles than compute units and fewer"""

@@ -11,14 +11,14 @@ namespace {
 
 // A[M][K] x B[N][K]^T with the PPE fused; see the file header.  K must be a multiple of 64.
 //
-// Pipeline.  K is walked in panels of 64 bytes; a panel of A and B (32 KiB) goes from global memory
-// straight into one of four LDS buffers.  In iteration kt the waves multiply panel kt, fetch panel
-// kt+3 (8 DMA instructions per wave, spread between the MFMAs) and read the fragments one sub-step
-// ahead; the only wait is for panel kt+1, which was requested two iterations earlier, and it sits
+// Pipeline of the forms below that walk K in panels of 64 bytes (K <= 192, and two that are only run when asked for: the 256 tile
+// with four waves, and PP): a panel of A and B (32 KiB of the 256 tile) goes from global memory straight into one of four LDS
+// buffers.  In iteration kt the waves multiply panel kt, fetch panel kt+3 (DMA instructions spread between the MFMAs) and read
+// the fragments one sub-step ahead; the only wait is for panel kt+1, which was requested two iterations earlier, and it sits
 // with the workgroup barrier in the middle of the iteration, between the two sub-steps,
-// so that the MFMAs of the second sub-step cover the first fragment reads of panel kt+1.  The column sums of B that the zero-point
-// term needs come from nce_colsum_kernel (only when that term is not zero), and the per-column PPE
-// parameters are unpacked from the weight table in the epilogue.
+// so that the MFMAs of the second sub-step cover the first fragment reads of panel kt+1.  The column sums of B that the
+// zero-point term needs are taken from the fragments as they pass, and the per-column PPE parameters are unpacked from the
+// weight table in the epilogue.
 //
 // PP (eight waves, large tile, K a multiple of four panels): the two waves of a SIMD take turns.  While one runs the
 // sixteen MFMAs of a panel back to back at raised priority, the other issues everything else it has to -- the twelve
@@ -26,11 +26,14 @@ namespace {
 // twice per panel.  (With both waves running the same interleaved stream their loads and reads fall on the same
 // moments and the MFMA pipe waits for both.)
 //
-// WIDE (the 128 tile with eight waves of 64 x 32, the 64 tile with four of 32 x 32; K of more than three panels of 64): panels of
+// WIDE (the 256 tile with eight waves of 128 x 64, the 128 tile with eight of 64 x 32, the 64 tile with four of 32 x 32): panels of
 // 128 bytes, whole cache lines -- of 64-byte pieces the second of a line came after the first had left the first-level cache, and
-// every line was read from the second level twice -- with one barrier each, between the panel's halves.  The loads of a panel
-// stand in line far ahead and nobody waits for them; a tile of 128 takes about 850 clocks for a panel whose MFMAs take 512,
-// bound by the LDS (96 KiB of fragments and 32 KiB of loads), one of 64 about 400, bound likewise.  Four waves of 64 x 64 on
+// every line was read from the second level twice -- with one barrier each.  The 256 tile has LDS for two such panels, and asks
+// for one whenever it has read the last fragment of the one before the last: its panel's MFMAs take 2 048 clocks, and between
+// 192.4 us (panels of 64 bytes, four buffers) and 172.0 at [4096 x 4096] . [4096 x 11008], 497 and 451 at 8192^3, 71.3
+// and 63.8 at 4096^3 lies only the order of its loads.  The smaller tiles' loads stand in line far ahead and nobody
+// waits for them; a tile of 128 takes about 850 clocks for a panel whose MFMAs take 512, bound by the LDS (96 KiB of
+// fragments and 32 KiB of loads), one of 64 about 400, bound likewise.  Four waves of 64 x 64 on
 // panels of 64, 24.5 us at [2080 x 3456] . [3456 x 608] whether or not fragments were read a panel ahead or twice the
 // panels were in flight, now take 20.2, 16.2 with the 64 tile; [512 x 4096] . [4096 x 4096] 26.9, now 22.0 and 20.7;
 // [1024 x 1024] . [1024 x 1024] 9.7, now 8.6 and 6.2.  (Eight waves of 64 x 64 with K split over two groups read a third less
@@ -48,7 +51,8 @@ __global__ __launch_bounds__(64 * NW) void nce_gemm_mfma(const int8_t* __restric
     // SHORTK (K <= 192, three panels at most): all panels are fetched up front, nothing is pipelined and no panel buffer
     // is reused, so the workgroup asks only for the LDS it touches and more of them fit a CU (a matmul this short is
     // bound by its epilogue and stores, not by the MFMAs).
-    constexpr bool WIDE = (TILE == 128 && NW == 8) || TILE == 64;
+    constexpr bool WIDE = (TILE == 128 && NW == 8) || TILE == 64 || (TILE == 256 && NS == 2);
+    constexpr bool SPLIT_RINGS = WIDE && TILE == 256;  // a ring of buffers per operand, so that an instruction's offset reaches both of its buffers
     constexpr int BM = TILE, BN = TILE, BK = WIDE ? 128 : 64, WM = BM / 2, WN = BN / (NW / 2), TM = WM / 32, TN = WN / 32;
     constexpr int MFMA_PER_DMA = WIDE ? 1 : TM * TN / (BM * BK / 1024 / NW);  // MFMAs between two DMA instructions of a sub-step
     static_assert(WIDE || (TM * TN >= TM + TN && MFMA_PER_DMA >= 1), "fragment reads and DMA instructions are interleaved with the MFMAs");
@@ -121,13 +125,14 @@ __global__ __launch_bounds__(64 * NW) void nce_gemm_mfma(const int8_t* __restric
     // in flight the same in every iteration: every lane re-fetches the tile's first 16 bytes (one cache line for
     // the whole instruction) into a buffer nobody reads.
     auto dma_one = [&](auto known_real, int p, int d) {
-        const unsigned base = lds0 + (unsigned)((p % NS) * STAGE);
+        const unsigned base = lds0 + (unsigned)((p % NS) * (SPLIT_RINGS ? BM * BK : STAGE));
+        constexpr unsigned B0 = SPLIT_RINGS ? NS * BM * BK : BM * BK;  // of the first B panel
         const bool real = decltype(known_real)::value || p < nk;  // (known: no select instructions in the loop body)
         const int64_t k0 = real ? (int64_t)p * BK : 0;
         unsigned off = d < DMA_PER_WAVE ? oa[d] : ob[d - DMA_PER_WAVE];
         if (WIDE && !decltype(known_real)::value && half && p == nk - 1) off -= past_half;  // (its second half: the first again, not multiplied)
         if (d < DMA_PER_WAVE) dma16(abase + k0, real ? off : 0u, base + (unsigned)((wave + NW * d) * 1024));
-        else dma16(bbase + k0, real ? off : 0u, base + (unsigned)(BM * BK + (wave + NW * (d - DMA_PER_WAVE)) * 1024));
+        else dma16(bbase + k0, real ? off : 0u, base + B0 + (unsigned)((wave + NW * (d - DMA_PER_WAVE)) * 1024));
     };
 
     i32x16 acc[TM][TN];
@@ -229,7 +234,83 @@ __global__ __launch_bounds__(64 * NW) void nce_gemm_mfma(const int8_t* __restric
 
     constexpr std::integral_constant<int, -1> kDynamicStage{};
     auto main_loop = [&](auto sum_c) {
-        if constexpr (WIDE) {
+        if constexpr (WIDE && TILE == 256) {
+            constexpr int HALF = decltype(sum_c)::value;  // the half of each panel whose column sums this wave takes, or neither (2)
+            i32x4 pa[2][TM], pb[2][TN];
+            lds_bytes_t base[2][4];  // [operand][sub-step of a panel]
+#pragma unroll
+            for (int o = 0; o < 2; o++)
+#pragma unroll
+                for (int kk = 0; kk < 4; kk++) {
+                    base[o][kk] = (lds_bytes_t)(smem + o * NS * BM * BK + lds_offset<BK>((o ? wn0 : wm0) + (lane & 31), kk * 2 + (lane >> 5)));
+                    asm volatile("" : "+v"(base[o][kk]));
+                }
+            auto read_one = [&](int stage, int kk, int slot, int n) {
+                if (n == 0) pa[slot][0] = *(lds_v4_t)(base[0][kk] + stage * BM * BK);
+                else if (n <= TN) pb[slot][n - 1] = *(lds_v4_t)(base[1][kk] + stage * BN * BK + (n - 1) * 32 * BK);
+                else pa[slot][n - TN] = *(lds_v4_t)(base[0][kk] + stage * BM * BK + (n - TN) * 32 * BK);
+            };
+            // Sub-step kk of a panel; the next one's fragments come from `stage`.  Panel p is asked for in the last sub-step of panel
+            // p - 2, all of it: with half its loads in the next sub-step [4096 x 4096] . [4096 x 11008] takes 186 us, not 176.
+            auto step = [&](auto kk_c, int stage, auto real_c, int p) {
+                constexpr int kk = decltype(kk_c)::value, slot = kk & 1;
+#pragma unroll
+                for (int i = 0; i < TM; i++) {
+                    i32x4 a = pa[slot][i];
+                    if (IN_U8) a ^= (int32_t)0x80808080;  // u8 -> s8 (value - 128)
+#pragma unroll
+                    for (int j = 0; j < TN; j++) {
+                        const int idx = i * TN + j;
+                        acc[i][j] = __builtin_amdgcn_mfma_i32_32x32x32_i8(a, pb[slot][j], acc[i][j], 0, 0, 0);
+                        constexpr int FH = (TM + TN + 1) / 2;
+                        if (idx == 0) {
+#pragma unroll
+                            for (int n = 0; n < FH; n++) read_one(stage, (kk + 1) & 3, slot ^ 1, n);
+                        } else if (idx == 1) {
+#pragma unroll
+                            for (int n = FH; n < TM + TN; n++) read_one(stage, (kk + 1) & 3, slot ^ 1, n);
+                        }
+                        if (kk == 3) dma_one(real_c, p, idx);
+                        if (kk / 2 == HALF && idx == TM * TN - 1) {
+#pragma unroll
+                            for (int d = 0; d < 4; d++)
+#pragma unroll
+                                for (int c = 0; c < TN; c++) cs[c] = __builtin_amdgcn_sdot4(pb[slot][c][d], 0x01010101, cs[c], false);
+                        }
+                        __builtin_amdgcn_sched_barrier(0);
+                    }
+                }
+            };
+            constexpr std::integral_constant<int, 0> s0{};
+            constexpr std::integral_constant<int, 1> s1{};
+            constexpr std::integral_constant<int, 2> s2{};
+            constexpr std::integral_constant<int, 3> s3{};
+            static_assert(TILE != 256 || !WIDE || 2 * DMA_PER_WAVE == TM * TN, "a load behind each MFMA of a panel's last sub-step");
+            auto one_panel = [&](int u, auto real_c, int k) {
+                step(s0, u, real_c, 0);
+                step(s1, u, real_c, 0);
+                if (!decltype(real_c)::value && half && k == nk - 1) return;
+                step(s2, u, real_c, 0);
+                asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");  // panel k + 1 is in, panel k has been read
+                step(s3, u ^ 1, real_c, k + 2);
+            };
+#pragma unroll
+            for (int p = 0; p < 2; p++)
+#pragma unroll
+                for (int d = 0; d < 2 * DMA_PER_WAVE; d++) dma_one(std::false_type{}, p, d);
+            asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"(2 * DMA_PER_WAVE) : "memory");  // panel 0 is in
+#pragma unroll
+            for (int n = 0; n < TM + TN; n++) read_one(0, 0, 0, n);
+            int kt = 0;
+            for (; kt + 4 < nk; kt += 2) {  // (every panel asked for whole)
+                one_panel(0, std::true_type{}, kt);
+                one_panel(1, std::true_type{}, kt + 1);
+            }
+            for (; kt < nk; kt += 2) {
+                one_panel(0, std::false_type{}, kt);
+                if (kt + 1 < nk) one_panel(1, std::false_type{}, kt + 1);
+            }
+        } else if constexpr (WIDE) {
             // The fragments of half a panel are read under the MFMAs of the half before it; behind the barrier between the two
             // everybody is through with the panel's buffer, which panel k + NS is then asked into.
             constexpr int HALF = decltype(sum_c)::value;  // the half of each panel whose column sums this wave takes, or neither (2)
@@ -276,7 +357,7 @@ __global__ __launch_bounds__(64 * NW) void nce_gemm_mfma(const int8_t* __restric
                         __builtin_amdgcn_sched_barrier(0);
                     }
             };
-            static_assert(!WIDE || (DMA_PER_WAVE % TM == 0 && TN == 1), "the same number of loads behind each MFMA of a second half");
+            static_assert(!WIDE || TILE == 256 || (DMA_PER_WAVE % TM == 0 && TN == 1), "the same number of loads behind each MFMA of a second half");
             constexpr std::integral_constant<int, 0> first{};
             constexpr std::integral_constant<int, 1> second{};
             auto one_panel = [&](int u, auto real_c, int k) {
@@ -631,12 +712,12 @@ int launch_gemm_mfma(const GemmLaunch& a, hipStream_t s) {
         else if (tile < 256) VPX_GEMM_SMALL(U8, SGN);                                                                \
         else if (nw == 4) VPX_GEMM_K(U8, SGN, 4, 256);                                                               \
         else if (pingpong) VPX_GEMM_K(U8, SGN, 8, 256, false, true);                                                 \
-        else VPX_GEMM_K(U8, SGN, 8, 256);                                                                            \
+        else VPX_GEMM_K(U8, SGN, 8, 256, false, false, 2);                                                           \
     } while (0)
     if (out_f16) {
         // fp16 output: of the large tile the eight-wave form only (the host passes waves = 8)
-        if (a.in_u8) { if (tile < 256) VPX_GEMM_SMALL(true, OUT_F16); else VPX_GEMM_K(true, OUT_F16, 8, 256); }
-        else { if (tile < 256) VPX_GEMM_SMALL(false, OUT_F16); else VPX_GEMM_K(false, OUT_F16, 8, 256); }
+        if (a.in_u8) { if (tile < 256) VPX_GEMM_SMALL(true, OUT_F16); else VPX_GEMM_K(true, OUT_F16, 8, 256, false, false, 2); }
+        else { if (tile < 256) VPX_GEMM_SMALL(false, OUT_F16); else VPX_GEMM_K(false, OUT_F16, 8, 256, false, false, 2); }
     }
     else if (a.in_u8 && a.out_kind == OUT_I8) VPX_GEMM(true, OUT_I8);
     else if (a.in_u8) VPX_GEMM(true, OUT_U8);
