@@ -1225,36 +1225,48 @@ template <int TEAM, int VPT, int RPT = 1, bool WORDS = true>  // RPT: consecutiv
 __global__ __launch_bounds__(kThreads) void mvn6_rows_kernel(const half_t* __restrict__ in, half_t* __restrict__ out,
                                                              const half_t* __restrict__ sc, const half_t* __restrict__ bi,
                                                              Mvn6Geom g, int normalize_variance, int eps_mode, float eps) {
-    __shared__ float red[8];
-    static_assert(TEAM != 256 || RPT == 1, "the workgroup-wide sums have slots for one row");
+    __shared__ float red[RPT > 1 ? 16 : 8];
     const int t = (int)(threadIdx.x % TEAM);
     const int64_t row0 = ((int64_t)blockIdx.x * (kThreads / TEAM) + threadIdx.x / TEAM) * RPT;
-    // scale and bias that run along the row (and do not depend on it): loaded once for the RPT rows
+    // The words of a row are asked for all at once, and before they are used the scale and the bias that run along it: asked for
+    // where they are needed, behind both sums, they cost a trip to the caches per row ([16384 x 4096] 56.7 -> 51.9 us, [16384 x
+    // 1024] 17.1 -> 15.9, [1 x 4096] 3.2 -> 2.7).  They stay late where nothing is gained, of one word per lane of a workgroup or
+    // of half a wavefront, and where their registers cost a wavefront per SIMD, from three words of half a wavefront or four of
+    // one on ([16384 x 768] 11.2 us late, 13.1 early, [8192 x 2048] 14.2 and 17.2).
+    constexpr bool EARLY = RPT > 1 || (TEAM == 64 ? VPT <= 3 : VPT == 2);
+    const auto fetch = [&](const RowBase& at, bool real, u32x4(&w)[VPT]) {
+#pragma unroll
+        for (int j = 0; j < VPT; j++) {
+            const uint32_t e0 = (uint32_t)(j * TEAM + t) * 8;
+            if (real && e0 < g.row_len) w[j] = row_word<WORDS>(in + at.in, e0, g.row_len);
+        }
+    };
+    bool live = row0 < g.rows;  // uniform per team; dead teams skip memory only
+    RowBase b = row_base(g, live ? row0 : 0);
+    u32x4 words[VPT];
+    fetch(b, live, words);
+    // scale and bias that run along the row, asked for beside it; with RPT > 1 they do not depend on it and are loaded once
     u32x4 scv[VPT], biv[VPT];
-    if (RPT > 1) {
+    if (EARLY) {
 #pragma unroll
         for (int j = 0; j < VPT; j++) {
             const uint32_t e0 = (uint32_t)(j * TEAM + t) * 8;
             if (e0 < g.row_len) {
-                if (sc) scv[j] = row_word<WORDS>(sc, e0, g.row_len);
-                if (bi) biv[j] = row_word<WORDS>(bi, e0, g.row_len);
+                if (sc && g.sc_along_row) scv[j] = row_word<WORDS>(sc + b.sc, e0, g.row_len);
+                if (bi && g.bi_along_row) biv[j] = row_word<WORDS>(bi + b.bi, e0, g.row_len);
             }
         }
     }
 #pragma unroll 1
     for (int rr = 0; rr < RPT; rr++) {
-    int64_t row = row0 + rr;
-    const bool live = row < g.rows;  // uniform per team; dead teams skip memory only
-    if (!live) row = 0;
-    const RowBase b = row_base(g, row);
+    float* const slots = red + (RPT > 1 ? (rr & 1) * 8 : 0);  // (a row's slots are written again two rows on, behind that row's barriers)
     float x[VPT][8];
     float sum = 0.f;
 #pragma unroll
     for (int j = 0; j < VPT; j++) {
         const uint32_t e0 = (uint32_t)(j * TEAM + t) * 8;
         if (live && e0 < g.row_len) {
-            const u32x4 q = row_word<WORDS>(in + b.in, e0, g.row_len);
-            const half_t* p = reinterpret_cast<const half_t*>(&q);
+            const half_t* p = reinterpret_cast<const half_t*>(&words[j]);
             const int again = row_again<WORDS>(e0, g.row_len);
 #pragma unroll
             for (int k = 0; k < 8; k++) {
@@ -1266,8 +1278,15 @@ __global__ __launch_bounds__(kThreads) void mvn6_rows_kernel(const half_t* __res
             for (int k = 0; k < 8; k++) x[j][k] = 0.f;
         }
     }
+    const RowBase here = b;
+    const bool real = live;
+    if (RPT > 1 && rr + 1 < RPT) {  // the next row is on its way while this one is summed and stored
+        live = row0 + rr + 1 < g.rows;
+        b = row_base(g, live ? row0 + rr + 1 : 0);
+        fetch(b, live, words);
+    }
     const float n = (float)g.row_len;
-    const float mean = team_sum<TEAM>(sum, red) / n;
+    const float mean = team_sum<TEAM>(sum, slots) / n;
     float q = 0.f;
 #pragma unroll
     for (int j = 0; j < VPT; j++) {
@@ -1279,20 +1298,20 @@ __global__ __launch_bounds__(kThreads) void mvn6_rows_kernel(const half_t* __res
             q += (WORDS ? e0 < g.row_len : k >= again) ? d * d : 0.f;
         }
     }
-    const float var = team_sum<TEAM>(q, red + 4) / n;
+    const float var = team_sum<TEAM>(q, slots + 4) / n;
     const float inv = mvn6_inv(var, normalize_variance, eps_mode, eps);
-    const float sc_row = sc && !g.sc_along_row ? (float)sc[b.sc] : 1.0f;
-    const float bi_row = bi && !g.bi_along_row ? (float)bi[b.bi] : 0.0f;
+    const float sc_row = sc && !g.sc_along_row ? (float)sc[here.sc] : 1.0f;
+    const float bi_row = bi && !g.bi_along_row ? (float)bi[here.bi] : 0.0f;
 #pragma unroll
     for (int j = 0; j < VPT; j++) {
         const uint32_t e0 = (uint32_t)(j * TEAM + t) * 8;
-        if (!(live && e0 < g.row_len)) continue;
+        if (!(real && e0 < g.row_len)) continue;
         float y[8];
 #pragma unroll
         for (int k = 0; k < 8; k++) y[k] = (x[j][k] - mean) * inv;
         if (sc) {
             if (g.sc_along_row) {
-                const u32x4 v = RPT > 1 ? scv[j] : row_word<WORDS>(sc + b.sc, e0, g.row_len);
+                const u32x4 v = EARLY ? scv[j] : row_word<WORDS>(sc + here.sc, e0, g.row_len);
                 const half_t* p = reinterpret_cast<const half_t*>(&v);
 #pragma unroll
                 for (int k = 0; k < 8; k++) y[k] *= (float)p[k];
@@ -1303,7 +1322,7 @@ __global__ __launch_bounds__(kThreads) void mvn6_rows_kernel(const half_t* __res
         }
         if (bi) {
             if (g.bi_along_row) {
-                const u32x4 v = RPT > 1 ? biv[j] : row_word<WORDS>(bi + b.bi, e0, g.row_len);
+                const u32x4 v = EARLY ? biv[j] : row_word<WORDS>(bi + here.bi, e0, g.row_len);
                 const half_t* p = reinterpret_cast<const half_t*>(&v);
 #pragma unroll
                 for (int k = 0; k < 8; k++) y[k] += (float)p[k];
@@ -1316,8 +1335,8 @@ __global__ __launch_bounds__(kThreads) void mvn6_rows_kernel(const half_t* __res
         half_t* po = reinterpret_cast<half_t*>(&o);
 #pragma unroll
         for (int k = 0; k < 8; k++) po[k] = (half_t)y[k];
-        if (WORDS) __builtin_nontemporal_store(o, reinterpret_cast<u32x4*>(out + b.out + e0));
-        else *reinterpret_cast<u32x4_any*>(out + b.out + row_at(e0, g.row_len)) = o;
+        if (WORDS) __builtin_nontemporal_store(o, reinterpret_cast<u32x4*>(out + here.out + e0));
+        else *reinterpret_cast<u32x4_any*>(out + here.out + row_at(e0, g.row_len)) = o;
     }
     }
 }
