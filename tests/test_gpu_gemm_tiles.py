@@ -30,16 +30,17 @@ def run(rt, orc, dev, rng, M, K, N, tile, in_u8, zp_in, zp_w, out_f16, shift=20)
 @pytest.mark.parametrize("tile", [64, 128, 256])
 @pytest.mark.parametrize("K", [64, 128, 192, 256, 320, 384, 448, 512, 576, 704, 1088])
 def test_every_end_of_the_panels(rt, orc, dev, tile, K):
-    """fewer panels than buffers, one more, half of one; tiles of one row, full, and one past full; sums on and off"""
+    """fewer panels than buffers, one more, half of one; tiles of one row, full, and one past full; rows that start at any byte and
+    end in part of a word, also the first of a tile; sums on and off"""
     rng = np.random.default_rng(K + tile)
-    for M, N in ((1200, 144), (tile, tile), (tile + 1, 3 * tile + 2), (1000, 49)):
+    for M, N in ((1200, 144), (tile, tile), (tile + 1, 3 * tile + 2), (67, tile + 21), (1000, 49)):
         for in_u8, zp_in in ((True, 128), (True, 7), (False, -5)):
             name = run(rt, orc, dev, rng, M, K, N, tile, in_u8, zp_in, 0, False)
             assert name == "nce_gemm_mfma"
 
 
 @pytest.mark.parametrize("tile", [None, 64, 128, 256])
-@pytest.mark.parametrize("M,K,N", [(1100, 320, 208), (2180, 448, 2070)])
+@pytest.mark.parametrize("M,K,N", [(1100, 320, 209), (2180, 448, 2070)])
 def test_outputs_and_zero_points(rt, orc, dev, tile, M, K, N):
     """fp16 outputs, a weight zero point (the per-row term), scales that clip; more tiles than compute units and fewer"""
     rng = np.random.default_rng(M)
