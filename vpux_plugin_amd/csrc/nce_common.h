@@ -3,7 +3,7 @@
 // the LDS and store helpers, and the launchers each kernel family's translation unit exports.
 //
 //   nce.hip             the dispatcher (vpx_nce_task -> kernel), tuning knobs, operand views, preparation kernels
-//   nce_gemm.hip        nce_gemm_mfma: 1x1 layers and NCE.MatMul
+//   nce_gemm.hip        nce_gemm_mfma: 1x1 layers and NCE.MatMul; nce_conv_gemm: middling convolutions on its small tiles
 //   nce_gemm_regb.hip   nce_gemm_regb: the same with a short K and many rows, weights in registers
 //   nce_direct.hip      nce_direct: small layers of every kind, nothing staged
 //   nce_conv_patch.hip  nce_conv_regw / nce_conv_tile / nce_conv_stream: input rows of a tile in LDS
@@ -359,7 +359,7 @@ __device__ __forceinline__ int out_align(unsigned bits) {
 // LDS tile of ROWS x BK bytes; the 16-byte chunk c of row r is kept at chunk slot c ^ swz(r) so
 // that the lanes served together by a 128-bit LDS read hit different bank groups.
 template <int BK>
-__device__ __forceinline__ int lds_swz(int row) {
+__host__ __device__ constexpr __forceinline__ int lds_swz(int row) {
     constexpr int CPR = BK / 16;   // chunks per row
     constexpr int RPW = 16 / CPR;  // rows per 256-byte bank wrap
     return (row / RPW) % CPR;
@@ -376,6 +376,10 @@ __device__ __forceinline__ int lds_offset(int row, int chunk) {
 // The source is a wave-uniform base plus a 32-bit per-lane byte offset.
 __device__ __forceinline__ void dma16(const void* gbase, unsigned goff, unsigned lds_addr) {
     asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds_addr), "v"(goff), "s"(gbase) : "memory");
+}
+// the same from an address per lane
+__device__ __forceinline__ void dma16_at(const void* from, unsigned lds_addr) {
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(lds_addr), "v"(from) : "memory");
 }
 __device__ __forceinline__ void dma_wait_all_and_barrier() {
     asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
@@ -636,7 +640,7 @@ struct Tuning {
     std::atomic<int> gemm_waves{0};         // VPX_GEMM_WAVES = 4 | 8
     std::atomic<int> gemm_regb{0};          // VPX_GEMM_REGB = on | wide | off: weights-in-registers matmul, K up to 256 (1, 2: with the most channel blocks per wave, -1; 0: chosen from the shape)
     std::atomic<int> gemm_pingpong{0};      // VPX_GEMM_PINGPONG = on | off: the waves of a SIMD take turns at the MFMAs
-    std::atomic<int> conv_stream{0};        // VPX_CONV_KERNEL = regw | tile | stream: start the choice of LDS-patch kernel at this one (-1, 1, 2; 0: by size)
+    std::atomic<int> conv_stream{0};        // VPX_CONV_KERNEL = regw | tile | stream: start the choice of LDS-patch kernel at this one (-1, 1, 2; 0: by size); gemm (-2): as a matmul
     std::atomic<int> conv_rows{0};          // VPX_CONV_ROWS = n: cap on the output rows per workgroup of the LDS-patch kernels
     std::atomic<int> conv_cols{0};          // VPX_CONV_COLS = n: output columns per tile of the row-patch kernel
     std::atomic<int> conv_waves{0};         // VPX_CONV_WAVES = 4 | 8
@@ -661,6 +665,13 @@ int operand_view(const int64_t st[4], int64_t N, int64_t H, int64_t W, int64_t C
 
 // nce_gemm.hip.  `tile` 128 | 256, `waves` 4 | 8 (8 with the large tile only), `shortk`: K of at most three panels on
 // the small tile; G groups on the grid's second dimension.
+// A convolution as a matmul: row m is output position (image, oy, ox), byte k of it byte k % (16 cpt) of tap k / (16 cpt).
+struct GemmConv {
+    int H, W, isn, ish, isw;  // of the input, strides in bytes
+    int ow, ohow, SY, SX, PT, PL, KX;
+    int cpt;  // 16-byte chunks per tap
+    int pad;  // the byte of a tap outside the image
+};
 struct GemmLaunch {
     const int8_t* A;
     const int8_t* B;
@@ -674,6 +685,8 @@ struct GemmLaunch {
     GemmPpe ppe;
     GemmRows rows;
     GemmOut dst;
+    bool is_conv = false;  // tiles of 64 and 128, one group, byte outputs, at least four chunks per tap
+    GemmConv conv{};
 };
 int launch_gemm_mfma(const GemmLaunch& a, hipStream_t s);
 // nce_gemm_regb.hip: K up to 256 in multiples of 16, rows of A and of the result at a fixed pitch, 16-byte aligned, N a

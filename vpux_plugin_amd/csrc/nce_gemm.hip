@@ -1,4 +1,5 @@
-// nce_gemm_mfma: 1x1 kernel, no padding (this is how NCE.MatMul arrives; a stride picks rows from the input): a plain
+// nce_gemm_mfma: 1x1 kernel, no padding (this is how NCE.MatMul arrives; a stride picks rows from the input), and as nce_conv_gemm
+// convolutions of 64 channels and more that fill the chip a few times at most: a plain
 // A[M][K] x B[N][K]^T GEMM.  256 x 256, 128 x 128 or 64 x 64 output tile per workgroup, v_mfma_i32_32x32x32_i8, K panels from
 // global memory straight into XOR-swizzled LDS (global_load_lds, no register staging), a ring of buffers, the integer PPE
 // fused into the epilogue.
@@ -8,6 +9,15 @@ namespace vpx {
 namespace nce {
 namespace {
 
+// Sixteen bytes of every value, for the taps of a convolution that lie outside the image.
+struct PadTable {
+    uint8_t bytes[256][16];
+    constexpr PadTable() : bytes{} {
+        for (int v = 0; v < 256; v++)
+            for (int i = 0; i < 16; i++) bytes[v][i] = (uint8_t)v;
+    }
+};
+__device__ const PadTable g_pads{};
 
 // A[M][K] x B[N][K]^T with the PPE fused; see the file header.  K must be a multiple of 64.
 //
@@ -39,12 +49,18 @@ namespace {
 // [1024 x 1024] . [1024 x 1024] 9.7, now 8.6 and 6.2.  (Eight waves of 64 x 64 with K split over two groups read a third less
 // but hand 64 KiB of sums over: 21.3 at the first.)  Summing the columns in one row of waves only cost 260 clocks a panel
 // on the SIMDs that held them; now the waves that share columns take a half of each panel each.
-template <bool IN_U8, int OUT, int NW, int TILE = 256, bool SHORTK = false, bool PP = false, int NS = 4>
+//
+// CONV (WIDE, 64 and 128 tiles): a convolution as a matmul over (tap, channel) with nothing laid out for it: row m is an output
+// position, and a lane keeps where its 16 bytes of the next panel lie -- tap, chunk of the tap, offset -- and steps them by a panel,
+// seven vector instructions; what lies outside the image it fetches from sixteen bytes of padding, what lies past the end of
+// K, of the weights, from sixteen zeros.  A panel costs a fifth more than the matmul's ([2000 x 2880] . [2880 x 320] 9.3 us,
+// [20,10,10,320] -> 320 3x3 11.0), bound by the LDS as there.
+template <bool IN_U8, int OUT, int NW, int TILE = 256, bool SHORTK = false, bool PP = false, int NS = 4, bool CONV = false>
 __global__ __launch_bounds__(64 * NW) void nce_gemm_mfma(const int8_t* __restrict__ A, const int8_t* __restrict__ B,
                                                      const int32_t* __restrict__ wt, const int32_t* __restrict__ colsum,
                                                      uint8_t* __restrict__ out,
                                                      int64_t M, int64_t N, int64_t K, int tiles_m, int tiles_n,
-                                                     GemmPpe ppe, GemmRows rows, GemmOut dst) {
+                                                     GemmPpe ppe, GemmRows rows, GemmOut dst, GemmConv cv) {
     // NW = 4: waves 2 x 2, 128 x 128 each, one per SIMD.  NW = 8: waves 2 x 4, 128 x 64 each, two per SIMD,
     // so that one wave's loads and address arithmetic issue while the other's MFMAs run.
     // TILE = 128 and 64 serve problems with too few 256 x 256 tiles.
@@ -67,7 +83,7 @@ __global__ __launch_bounds__(64 * NW) void nce_gemm_mfma(const int8_t* __restric
     uint8_t* const smem = smem_raw + kGemmLdsHead;          // the panel buffers, later the output staging tile
 
     // Grouped matmul: blockIdx.y is the group; every operand holds the groups one after the other.
-    if (const int64_t grp = blockIdx.y) {
+    if (const int64_t grp = CONV ? 0 : blockIdx.y) {
         A += grp * M * K;
         B += grp * N * K;
         wt += grp * N * 4;
@@ -100,6 +116,7 @@ __global__ __launch_bounds__(64 * NW) void nce_gemm_mfma(const int8_t* __restric
     // [q*1024, q*1024+1024) of the operand's tile = rows q*RPI .. ; the lane sitting at chunk slot p
     // of row r fetches source chunk p ^ swz(r), which is what puts the swizzle in place.
     unsigned oa[DMA_PER_WAVE], ob[DMA_PER_WAVE];  // byte offsets from the tile's first row
+    [[maybe_unused]] int iy[DMA_PER_WAVE], ix[DMA_PER_WAVE];  // CONV: the row's first tap
 #pragma unroll
     for (int i = 0; i < DMA_PER_WAVE; i++) {
         const int q = wave + NW * i;
@@ -108,6 +125,14 @@ __global__ __launch_bounds__(64 * NW) void nce_gemm_mfma(const int8_t* __restric
         int64_t m = m0 + r, n = n0 + r;
         m = m < M ? m : M - 1;  // rows past the edge repeat the last one; their outputs are not stored
         n = n < N ? n : N - 1;
+        if constexpr (CONV) {
+            const unsigned mm = (unsigned)m, img = mm / (unsigned)cv.ohow, rem = mm - img * (unsigned)cv.ohow, oy = rem / (unsigned)cv.ow, ox = rem - oy * (unsigned)cv.ow;
+            iy[i] = (int)oy * cv.SY - cv.PT;
+            ix[i] = (int)ox * cv.SX - cv.PL;
+            oa[i] = (unsigned)((int)img * cv.isn + iy[i] * cv.ish + ix[i] * cv.isw);  // (of a pixel that may lie outside the image)
+            ob[i] = (unsigned)((n - n0) * K + c * 16);
+            continue;
+        }
         oa[i] = (unsigned)((m - m0) * rows.lda + c * 16);
         if (rows.strided) {  // (offsets from the tensor's first byte; the host has checked that they fit 32 bits)
             const int mm = (int)m, img = mm / rows.ohow, rem = mm - img * rows.ohow, oy = rem / rows.ow, ox = rem - oy * rows.ow;
@@ -115,18 +140,60 @@ __global__ __launch_bounds__(64 * NW) void nce_gemm_mfma(const int8_t* __restric
         }
         ob[i] = (unsigned)((n - n0) * K + c * 16);
     }
-    const int8_t* abase = rows.strided ? A : A + m0 * rows.lda;
+    const int8_t* abase = CONV || rows.strided ? A : A + m0 * rows.lda;
     const int8_t* bbase = B + n0 * K;
     const unsigned lds0 = lds_address(smem);
     const int nk = (int)((K + BK - 1) / BK);
-    const bool half = WIDE && (K & 64) != 0;  // the last panel is half a panel
+    const bool half = WIDE && !CONV && (K & 64) != 0;  // the last panel is half a panel
     const unsigned past_half = WIDE && (((lane % CPR) ^ lds_swz<BK>(wave * RPI + lane / CPR)) & 4) != 0 ? 64u : 0u;
+    // CONV: the chunk of K this lane fetches of the panel asked for next, the same for all its rows (their swizzle is): the chunk
+    // of the tap's channels, the tap, and its offset from the row's first tap.
+    [[maybe_unused]] int cc = 0, ky = 0, kx = 0, koff = 0;
+    [[maybe_unused]] const int kc = ((lane % CPR) ^ lds_swz<BK>(wave * RPI + lane / CPR)) * 16;  // byte of the panel
+    if constexpr (CONV) {
+        static_assert(!CONV || (lds_swz<BK>(NW * RPI) == lds_swz<BK>(0)), "a lane's rows share their swizzle");
+        const int tap = (kc / 16) / cv.cpt;
+        cc = kc / 16 - tap * cv.cpt;
+        ky = tap / cv.KX;
+        kx = tap - ky * cv.KX;
+        koff = ky * cv.ish + kx * cv.isw + cc * 16;
+    }
+    [[maybe_unused]] const int8_t* const pad16 = reinterpret_cast<const int8_t*>(g_pads.bytes[CONV ? cv.pad : 0]);
+    [[maybe_unused]] const int8_t* const zero16 = reinterpret_cast<const int8_t*>(g_pads.bytes[0]);
+    [[maybe_unused]] const auto next_tap = [&]() {
+        const bool wrap = cc >= cv.cpt;
+        cc -= wrap ? cv.cpt : 0;
+        koff += wrap ? cv.isw - cv.cpt * 16 : 0;
+        kx += wrap ? 1 : 0;
+        const bool down = kx == cv.KX;
+        kx = down ? 0 : kx;
+        ky += down ? 1 : 0;
+        koff += down ? cv.ish - cv.KX * cv.isw : 0;
+    };
+    [[maybe_unused]] const auto next_panel = [&]() {
+        cc += CPR;
+        koff += CPR * 16;
+        next_tap();
+        if (cv.cpt < CPR) next_tap();  // (a tap is at least half a panel)
+    };
     // d-th DMA instruction (first half A, second half B) of panel p.  Panels past the end keep the number of loads
     // in flight the same in every iteration: every lane re-fetches the tile's first 16 bytes (one cache line for
     // the whole instruction) into a buffer nobody reads.
     auto dma_one = [&](auto known_real, int p, int d) {
         const unsigned base = lds0 + (unsigned)((p % NS) * (SPLIT_RINGS ? BM * BK : STAGE));
         constexpr unsigned B0 = SPLIT_RINGS ? NS * BM * BK : BM * BK;  // of the first B panel
+        if constexpr (CONV) {
+            if (d < DMA_PER_WAVE) {  // (past the end of K the walk goes on, on pixels inside the image or on padding)
+                const bool in = (unsigned)(iy[d] + ky) < (unsigned)cv.H && (unsigned)(ix[d] + kx) < (unsigned)cv.W;
+                dma16_at(in ? A + (int64_t)(int)(oa[d] + (unsigned)koff) : pad16, base + (unsigned)((wave + NW * d) * 1024));
+                if (d == DMA_PER_WAVE - 1) next_panel();
+            } else {
+                const int8_t* from = bbase + (int64_t)p * BK + ob[d - DMA_PER_WAVE];
+                if (!decltype(known_real)::value && (int64_t)p * BK + kc >= K) from = zero16;
+                dma16_at(from, base + (unsigned)(BM * BK + (wave + NW * (d - DMA_PER_WAVE)) * 1024));
+            }
+            return;
+        }
         const bool real = decltype(known_real)::value || p < nk;  // (known: no select instructions in the loop body)
         const int64_t k0 = real ? (int64_t)p * BK : 0;
         unsigned off = d < DMA_PER_WAVE ? oa[d] : ob[d - DMA_PER_WAVE];
@@ -708,7 +775,7 @@ int launch_gemm_mfma(const GemmLaunch& a, hipStream_t s) {
         rc = set_dyn_lds(kern, lds);                                                                                 \
         if (rc) return rc;                                                                                           \
         hipLaunchKernelGGL(kern, grid, dim3(64 * nw), lds, s, a.A, a.B, a.wt, colsum, a.out, a.M, a.N, a.K, tiles_m,  \
-                           tiles_n, a.ppe, a.rows, a.dst);                                                           \
+                           tiles_n, a.ppe, a.rows, a.dst, a.conv);                                                   \
     } while (0)
     // the tiles of 64 and 128, any kind of output
 #define VPX_GEMM_SMALL(U8, SGN)                                                                                      \
@@ -716,6 +783,13 @@ int launch_gemm_mfma(const GemmLaunch& a, hipStream_t s) {
         if (tile == 64) VPX_GEMM_K(U8, SGN, 4, 64, false, false, 4);                                                 \
         else if (a.stages == 3) VPX_GEMM_K(U8, SGN, 8, 128, false, false, 3);                                        \
         else VPX_GEMM_K(U8, SGN, 8, 128, false, false, 2);                                                           \
+    } while (0)
+    // a convolution: byte outputs
+#define VPX_GEMM_CONV(U8, SGN)                                                                                       \
+    do {                                                                                                             \
+        if (tile == 64) VPX_GEMM_K(U8, SGN, 4, 64, false, false, 4, true);                                           \
+        else if (a.stages == 3) VPX_GEMM_K(U8, SGN, 8, 128, false, false, 3, true);                                  \
+        else VPX_GEMM_K(U8, SGN, 8, 128, false, false, 2, true);                                                     \
     } while (0)
 #define VPX_GEMM(U8, SGN)                                                                                            \
     do {                                                                                                             \
@@ -725,7 +799,12 @@ int launch_gemm_mfma(const GemmLaunch& a, hipStream_t s) {
         else if (pingpong) VPX_GEMM_K(U8, SGN, 8, 256, false, true);                                                 \
         else VPX_GEMM_K(U8, SGN, 8, 256, false, false, 2);                                                           \
     } while (0)
-    if (out_f16) {
+    if (a.is_conv) {
+        if (a.in_u8 && a.out_kind == OUT_I8) VPX_GEMM_CONV(true, OUT_I8);
+        else if (a.in_u8) VPX_GEMM_CONV(true, OUT_U8);
+        else if (a.out_kind == OUT_I8) VPX_GEMM_CONV(false, OUT_I8);
+        else VPX_GEMM_CONV(false, OUT_U8);
+    } else if (out_f16) {
         // fp16 output: of the large tile the eight-wave form only (the host passes waves = 8)
         if (a.in_u8) { if (tile < 256) VPX_GEMM_SMALL(true, OUT_F16); else VPX_GEMM_K(true, OUT_F16, 8, 256, false, false, 2); }
         else { if (tile < 256) VPX_GEMM_SMALL(false, OUT_F16); else VPX_GEMM_K(false, OUT_F16, 8, 256, false, false, 2); }
@@ -736,6 +815,7 @@ int launch_gemm_mfma(const GemmLaunch& a, hipStream_t s) {
     else VPX_GEMM(false, OUT_U8);
 #undef VPX_GEMM
 #undef VPX_GEMM_SMALL
+#undef VPX_GEMM_CONV
 #undef VPX_GEMM_K
     VPX_HIP_CHECK(hipGetLastError());
     return VPX_RESULT_SUCCESS;
