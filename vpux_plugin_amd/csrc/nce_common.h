@@ -665,11 +665,20 @@ int operand_view(const int64_t st[4], int64_t N, int64_t H, int64_t W, int64_t C
 
 // nce_gemm.hip.  `tile` 128 | 256, `waves` 4 | 8 (8 with the large tile only), `shortk`: K of at most three panels on
 // the small tile; G groups on the grid's second dimension.
+// n / d for any n and d of 32 bits: with magic = floor((2^32 - 1) / d), which lies less than one below 2^32 / d, the high half of n * magic is
+// the quotient or one less.
+inline unsigned quotient_magic(unsigned d) { return 0xffffffffu / d; }
+__device__ __forceinline__ unsigned quotient(unsigned n, unsigned d, unsigned magic) {
+    const unsigned q = __umulhi(n, magic);
+    return q + (n - q * d >= d ? 1u : 0u);
+}
+
 // A convolution as a matmul: row m is output position (image, oy, ox), byte k of it byte k % (16 cpt) of tap k / (16 cpt).
 struct GemmConv {
     int H, W, isn, ish, isw;  // of the input, strides in bytes
     int ow, ohow, SY, SX, PT, PL, KX;
     int cpt;  // 16-byte chunks per tap
+    unsigned ow_magic, ohow_magic;  // quotient_magic(ow), (ohow)
     int pad;  // the byte of a tap outside the image
 };
 struct GemmLaunch {

@@ -59,7 +59,7 @@ template <bool IN_U8, int OUT, int NW, int TILE = 256, bool SHORTK = false, bool
 __global__ __launch_bounds__(64 * NW) void nce_gemm_mfma(const int8_t* __restrict__ A, const int8_t* __restrict__ B,
                                                      const int32_t* __restrict__ wt, const int32_t* __restrict__ colsum,
                                                      uint8_t* __restrict__ out,
-                                                     int64_t M, int64_t N, int64_t K, int tiles_m, int tiles_n,
+                                                     int64_t M, int64_t N, int64_t K, int tiles_m, int tiles_n, unsigned group_magic,
                                                      GemmPpe ppe, GemmRows rows, GemmOut dst, GemmConv cv) {
     // NW = 4: waves 2 x 2, 128 x 128 each, one per SIMD.  NW = 8: waves 2 x 4, 128 x 64 each, two per SIMD,
     // so that one wave's loads and address arithmetic issue while the other's MFMAs run.
@@ -95,17 +95,18 @@ __global__ __launch_bounds__(64 * NW) void nce_gemm_mfma(const int8_t* __restric
     // Workgroup ids are dealt round-robin to the 8 XCDs.  Give each XCD a contiguous run of tile
     // ids and walk tiles in groups of 4 tile-rows, so that workgroups resident on one XCD at the
     // same time share A and B panels in that XCD's L2.
-    const int total = tiles_m * tiles_n;
-    const int per_xcd = (total + 7) / 8;
-    const int id = (int)(blockIdx.x % 8) * per_xcd + (int)(blockIdx.x / 8);
+    // (Everything up to the first load is a chain of instructions fetched for the first time: no division, 32 bits where they do.)
+    const unsigned total = (unsigned)tiles_m * (unsigned)tiles_n;
+    const unsigned per_xcd = (total + 7) / 8;
+    const unsigned id = (blockIdx.x % 8) * per_xcd + blockIdx.x / 8;
     if (id >= total) return;
     constexpr int GM = 4;
-    const int group = id / (GM * tiles_n);
-    const int gm0 = group * GM;
+    const unsigned group = quotient(id, GM * (unsigned)tiles_n, group_magic);
+    const int gm0 = (int)group * GM;
     const int gsz = tiles_m - gm0 < GM ? tiles_m - gm0 : GM;
-    const int in_group = id - group * GM * tiles_n;
-    const int tm = gm0 + in_group % gsz;
-    const int tn = in_group / gsz;
+    const unsigned in_group = id - group * (GM * (unsigned)tiles_n);
+    const unsigned tn = gsz == 4 ? in_group / 4 : (gsz == 3 ? in_group / 3 : (gsz == 2 ? in_group / 2 : in_group));
+    const unsigned tm = (unsigned)gm0 + (in_group - tn * (unsigned)gsz);
     const int64_t m0 = (int64_t)tm * BM, n0 = (int64_t)tn * BN;
 
     const int tid = threadIdx.x, lane = tid & 63;
@@ -115,6 +116,7 @@ __global__ __launch_bounds__(64 * NW) void nce_gemm_mfma(const int8_t* __restric
     // Source addresses of this lane's DMA chunks.  Instruction q of a panel fills LDS bytes
     // [q*1024, q*1024+1024) of the operand's tile = rows q*RPI .. ; the lane sitting at chunk slot p
     // of row r fetches source chunk p ^ swz(r), which is what puts the swizzle in place.
+    const int mrows = (int)(M - m0 < BM ? M - m0 : BM), nrows = (int)(N - n0 < BN ? N - n0 : BN);
     unsigned oa[DMA_PER_WAVE], ob[DMA_PER_WAVE];  // byte offsets from the tile's first row
     [[maybe_unused]] int iy[DMA_PER_WAVE], ix[DMA_PER_WAVE];  // CONV: the row's first tap
 #pragma unroll
@@ -122,23 +124,26 @@ __global__ __launch_bounds__(64 * NW) void nce_gemm_mfma(const int8_t* __restric
         const int q = wave + NW * i;
         const int r = q * RPI + lane / CPR, p = lane % CPR;
         const int c = p ^ lds_swz<BK>(r);
-        int64_t m = m0 + r, n = n0 + r;
-        m = m < M ? m : M - 1;  // rows past the edge repeat the last one; their outputs are not stored
-        n = n < N ? n : N - 1;
+        const unsigned rm = (unsigned)(r < mrows ? r : mrows - 1);  // rows past the edge repeat the last one; their outputs are not stored
+        const unsigned rn = (unsigned)(r < nrows ? r : nrows - 1);
+        ob[i] = rn * (unsigned)K + (unsigned)(c * 16);
         if constexpr (CONV) {
-            const unsigned mm = (unsigned)m, img = mm / (unsigned)cv.ohow, rem = mm - img * (unsigned)cv.ohow, oy = rem / (unsigned)cv.ow, ox = rem - oy * (unsigned)cv.ow;
+            const unsigned mm = (unsigned)m0 + rm, img = quotient(mm, (unsigned)cv.ohow, cv.ohow_magic), rem = mm - img * (unsigned)cv.ohow;
+            const unsigned oy = quotient(rem, (unsigned)cv.ow, cv.ow_magic), ox = rem - oy * (unsigned)cv.ow;
             iy[i] = (int)oy * cv.SY - cv.PT;
             ix[i] = (int)ox * cv.SX - cv.PL;
             oa[i] = (unsigned)((int)img * cv.isn + iy[i] * cv.ish + ix[i] * cv.isw);  // (of a pixel that may lie outside the image)
-            ob[i] = (unsigned)((n - n0) * K + c * 16);
-            continue;
+        } else {
+            oa[i] = rm * (unsigned)rows.lda + (unsigned)(c * 16);
         }
-        oa[i] = (unsigned)((m - m0) * rows.lda + c * 16);
-        if (rows.strided) {  // (offsets from the tensor's first byte; the host has checked that they fit 32 bits)
-            const int mm = (int)m, img = mm / rows.ohow, rem = mm - img * rows.ohow, oy = rem / rows.ow, ox = rem - oy * rows.ow;
+    }
+    if (!CONV && rows.strided) {  // (offsets from the tensor's first byte; the host has checked that they fit 32 bits)
+#pragma unroll
+        for (int i = 0; i < DMA_PER_WAVE; i++) {
+            const int r = (wave + NW * i) * RPI + lane / CPR, c = (lane % CPR) ^ lds_swz<BK>(r);
+            const int mm = (int)m0 + (r < mrows ? r : mrows - 1), img = mm / rows.ohow, rem = mm - img * rows.ohow, oy = rem / rows.ow, ox = rem - oy * rows.ow;
             oa[i] = (unsigned)img * rows.pimg + (unsigned)oy * rows.py + (unsigned)ox * rows.px + (unsigned)(c * 16);
         }
-        ob[i] = (unsigned)((n - n0) * K + c * 16);
     }
     const int8_t* abase = CONV || rows.strided ? A : A + m0 * rows.lda;
     const int8_t* bbase = B + n0 * K;
@@ -291,11 +296,11 @@ __global__ __launch_bounds__(64 * NW) void nce_gemm_mfma(const int8_t* __restric
     int w2r[TN], w3r[TN], csr[TN];
 #pragma unroll
     for (int j = 0; j < TN; j++) {
-        int64_t n = n0 + wn0 + j * 32 + (lane & 31);
-        n = n < N ? n : N - 1;
+        const int r = wn0 + j * 32 + (lane & 31);
+        const int2 words = *reinterpret_cast<const int2*>(wt + n0 * 4 + (unsigned)((r < nrows ? r : nrows - 1) * 4 + 2));
         csr[j] = 0;
-        w2r[j] = wt[n * 4 + 2];
-        w3r[j] = wt[n * 4 + 3];
+        w2r[j] = words.x;
+        w3r[j] = words.y;
     }
     // (Nobody waits for these words here: they are the oldest loads in flight, so every count waited for below covers them.)
 
@@ -775,7 +780,7 @@ int launch_gemm_mfma(const GemmLaunch& a, hipStream_t s) {
         rc = set_dyn_lds(kern, lds);                                                                                 \
         if (rc) return rc;                                                                                           \
         hipLaunchKernelGGL(kern, grid, dim3(64 * nw), lds, s, a.A, a.B, a.wt, colsum, a.out, a.M, a.N, a.K, tiles_m,  \
-                           tiles_n, a.ppe, a.rows, a.dst, a.conv);                                                   \
+                           tiles_n, quotient_magic(4 * (unsigned)tiles_n), a.ppe, a.rows, a.dst, a.conv);                                                   \
     } while (0)
     // the tiles of 64 and 128, any kind of output
 #define VPX_GEMM_SMALL(U8, SGN)                                                                                      \
