@@ -381,7 +381,7 @@ __global__ __launch_bounds__(256) void softmax_lines(const T* __restrict__ in, T
 // two-byte alignment only (7.8 TB/s on cached data where they fall on 16 bytes, 6.9 where not), and the run's last, partial
 // vector goes value by value.  NT: a tensor beyond the L2 is stored past it; one of a few megabytes is 0.3 us faster
 // through it.
-// CL: lanes along the columns; with 16 of them the wave's four quarters are four more shares of the axis (small tensors,
+// CL: lanes along the columns; with 16 (or 32) of them the wave's four quarters (its halves) are more shares of the axis (small tensors,
 // whose few tiles of 64 lanes would put all the exponentials on a few compute units: [1,500,20,24] 10.9 -> 5.9 us).
 template <int VEC, int KW, int SMAX, int CL, bool NT>
 __global__ __launch_bounds__(KW == 1 ? 256 : 64 * KW) void softmax_slab_f16(const half_t* __restrict__ in,
@@ -429,10 +429,10 @@ __global__ __launch_bounds__(KW == 1 ? 256 : 64 * KW) void softmax_slab_f16(cons
     }
 #pragma unroll
     for (int i = 0; i < SMAX; i++) m = __builtin_elementwise_max(m, h[i]);
-    if constexpr (CL == 16) {
-        static_assert(VEC == 2, "one register of maxima crosses the quarters");
+    if constexpr (CL < 64) {
+        static_assert(VEC == 2, "one register of maxima crosses the wave's parts");
 #pragma unroll
-        for (int o = 16; o < 64; o *= 2)
+        for (int o = CL; o < 64; o *= 2)
             m = __builtin_elementwise_max(m, __builtin_bit_cast(hvec, __shfl_xor(__builtin_bit_cast(int, m), o, 64)));
     }
     if (KW > 1) {
@@ -451,9 +451,9 @@ __global__ __launch_bounds__(KW == 1 ? 256 : 64 * KW) void softmax_slab_f16(cons
     for (int i = 0; i < SMAX; i++)
 #pragma unroll
         for (int k = 0; k < VEC; k++) sum[k] += __builtin_amdgcn_exp2f(__builtin_fmaf((float)h[i][k], kLog2e, nmb[k]));
-    if constexpr (CL == 16) {
+    if constexpr (CL < 64) {
 #pragma unroll
-        for (int o = 16; o < 64; o *= 2)
+        for (int o = CL; o < 64; o *= 2)
 #pragma unroll
             for (int k = 0; k < VEC; k++) sum[k] += __shfl_xor(sum[k], o, 64);
     }
@@ -1015,9 +1015,9 @@ int softmax_typed(const SoftmaxPlan& p, const T* in, T* out, hipStream_t s) {
         const int64_t in_as = p.in_stride[ax], out_as = p.out_stride[ax];
         if (ok && inner < (1ll << 31)) {
             // Small tensors want waves (a wave's steps follow one another), large ones pieces of 256 and 512 bytes of a row:
-            // up to 8 steps a wave alone; to 16 two of them; to 64 four (eight where the tensor is small); to 512 eight --
-            // sixteen while tiles are fewer than two and a half per compute unit ([5,185,41,357] 16.8 against 22.4 us, but
-            // [32,256,56,56] 22.1 against 20.1 and [2,300,300,170] 45 against 32 from three on).
+            // up to 8 steps a wave alone; to 16 two of them; to 64 four (eight where the tensor is small); to 512 eight, beyond
+            // sixteen, of which one workgroup or two fit a compute unit ([1,300,200,201], 315 tiles, 16.1 us with eight, 27.0 with
+            // sixteen, [1,96,200,333], 521, 9.2 and 12.0, [1,302,237,321], 595, 29.1 and 49.5).
             // [4,21,513,513] 44.8 -> 17.1 us (the lane-per-line kernel served odd planes), [1,31,66,123] 8.4 -> 2.9,
             // [32,256,56,56] 22.4 -> 20.1, [2,14,494,640] 10.2 -> 8.5.
             const int64_t elements = outer * inner * len;
@@ -1028,17 +1028,25 @@ int softmax_typed(const SoftmaxPlan& p, const T* in, T* out, hipStream_t s) {
             int vec = len <= 8 || (len <= 16 && !small) ? 4 : 2;
             int kw = len <= 8 ? 1 : (len <= 16 ? (small ? 4 : 2) : (len <= 64 ? (small ? 8 : 4) : 8));
             int64_t tiles = outer * ((inner + 64 * vec - 1) / (64 * vec));
-            if (len > 512 || (len > 64 && 2 * tiles < 5 * cus)) kw = 16;
+            const bool few = len > 64 && tiles * 20 < 11 * (int64_t)cus;
+            if (len > 512 || few) kw = 16;
             // fewer waves than SIMDs (with a short axis: than compute units): columns of 16 lanes, four shares of the axis a wave
             const bool narrow = tiles * kw < (len > 16 ? 4 : 1) * cus;
             if (narrow) {
                 vec = 2;
                 kw = len <= 16 ? 1 : (len <= 64 ? 4 : (len <= 256 ? 8 : 16));
             }
-            const int cols = (narrow ? 16 : 64) * vec;
+            // few tiles of many steps: columns of 32 lanes, two shares of the axis a wave, twice the tiles ([1,185,41,357], 115 tiles,
+            // 8.6 -> 7.3 us, [1,200,130,91] 7.8 -> 6.3, [1,512,90,101] 13.3 -> 10.2; at 158 tiles, [1,300,100,201], 11.8 against 10.9)
+            const bool half = few && !narrow;
+            if (half) {
+                vec = 2;
+                kw = len <= 256 ? 8 : 16;
+            }
+            const int cols = (narrow ? 16 : (half ? 32 : 64)) * vec;
             const int64_t tpo = (inner + cols - 1) / cols;
             tiles = outer * tpo;
-            const int L = (int)len, I = (int)inner, shares = kw * (narrow ? 4 : 1), steps = (L + shares - 1) / shares;
+            const int L = (int)len, I = (int)inner, shares = kw * (narrow ? 4 : (half ? 2 : 1)), steps = (L + shares - 1) / shares;
             const bool fits = (kw == 1 ? (tiles + 3) / 4 * 4 : tiles) * kw < (1ll << 26);  // 2^32 lanes in a launch
             // A run shorter than a tile leaves lanes idle, a run of 3 all but two: below 64 columns (128 where a tile ends in a
             // partial vector, unless softmax_cols has such runs) the cheaper of the two.  Slab / line, us: [2796202,2,3] 1057 / 46,
@@ -1062,7 +1070,15 @@ int softmax_typed(const SoftmaxPlan& p, const T* in, T* out, hipStream_t s) {
         if (small) VPX_SLAB_NT(VEC, KW, SMAX, 64, false);            \
         else VPX_SLAB_NT(VEC, KW, SMAX, 64, true);                   \
     } while (0)
-                if (narrow && kw == 1) VPX_SLAB_NT(2, 1, 4, 16, false);
+#define VPX_SLAB_HALF(KW, SMAX) VPX_SLAB_NT(2, KW, SMAX, 32, true)
+                // Eight waves a tile and 33 to 48 steps: three workgroups a compute unit fit, with registers for 64 steps two; whichever
+                // has the fewer tiles one after another on a unit ([1,302,237,321], 595 tiles, three: 29.1 us, two: 35.6; [1,320,311,330],
+                // 802 tiles: 44.3 and 39.8).
+                const int64_t rounds3 = (tiles + 3 * cus - 1) / (3 * cus), rounds2 = (tiles + 2 * cus - 1) / (2 * cus);
+                const bool three = tiles <= 2 * cus || 3 * rounds3 <= 2 * rounds2;  // (one round either way: the fewer idle steps)
+                if (half && kw == 8) { if (steps <= 8) VPX_SLAB_HALF(8, 8); else VPX_SLAB_HALF(8, 16); }
+                else if (half) { if (steps <= 16) VPX_SLAB_HALF(16, 16); else VPX_SLAB_HALF(16, 32); }
+                else if (narrow && kw == 1) VPX_SLAB_NT(2, 1, 4, 16, false);
                 else if (narrow && kw == 4) VPX_SLAB_NT(2, 4, 4, 16, false);
                 else if (narrow && kw == 8) VPX_SLAB_NT(2, 8, 8, 16, false);
                 else if (narrow) VPX_SLAB_NT(2, 16, 16, 16, false);
@@ -1071,12 +1087,12 @@ int softmax_typed(const SoftmaxPlan& p, const T* in, T* out, hipStream_t s) {
                 else if (kw == 4) { if (steps <= 4) VPX_SLAB(2, 4, 4); else if (steps <= 8) VPX_SLAB(2, 4, 8); else VPX_SLAB(2, 4, 16); }
                 else if (kw == 8) {
                     if (steps <= 4) VPX_SLAB(2, 8, 4); else if (steps <= 8) VPX_SLAB(2, 8, 8); else if (steps <= 16) VPX_SLAB(2, 8, 16);
-                    else if (steps <= 24) VPX_SLAB(2, 8, 24); else if (steps <= 32) VPX_SLAB(2, 8, 32); else VPX_SLAB(2, 8, 64);
-                } else {
-                    if (steps <= 8) VPX_SLAB(2, 16, 8); else if (steps <= 16) VPX_SLAB(2, 16, 16); else if (steps <= 24) VPX_SLAB(2, 16, 24);
-                    else if (steps <= 32) VPX_SLAB(2, 16, 32); else VPX_SLAB(2, 16, 64);
-                }
+                    else if (steps <= 24) VPX_SLAB(2, 8, 24); else if (steps <= 32) VPX_SLAB(2, 8, 32);
+                    else if (steps <= 40 && three) VPX_SLAB(2, 8, 40); else if (steps <= 48 && three) VPX_SLAB(2, 8, 48); else VPX_SLAB(2, 8, 64);
+                } else if (steps <= 48) VPX_SLAB(2, 16, 48);  // (from 33 on)
+                else VPX_SLAB(2, 16, 64);
 #undef VPX_SLAB_NT
+#undef VPX_SLAB_HALF
 #undef VPX_SLAB
                 VPX_HIP_CHECK(hipGetLastError());
                 return VPX_RESULT_SUCCESS;
