@@ -1228,12 +1228,16 @@ __global__ __launch_bounds__(kThreads) void mvn6_rows_kernel(const half_t* __res
     __shared__ float red[RPT > 1 ? 16 : 8];
     const int t = (int)(threadIdx.x % TEAM);
     const int64_t row0 = ((int64_t)blockIdx.x * (kThreads / TEAM) + threadIdx.x / TEAM) * RPT;
-    // The words of a row are asked for all at once, and before they are used the scale and the bias that run along it: asked for
+    // The words of a row are asked for all at once (but see AHEAD), and before they are used the scale and the bias that run along it: asked for
     // where they are needed, behind both sums, they cost a trip to the caches per row ([16384 x 4096] 56.7 -> 51.9 us, [16384 x
     // 1024] 17.1 -> 15.9, [1 x 4096] 3.2 -> 2.7).  They stay late where nothing is gained, of one word per lane of a workgroup or
     // of half a wavefront, and where their registers cost a wavefront per SIMD, from three words of half a wavefront or four of
     // one on ([16384 x 768] 11.2 us late, 13.1 early, [8192 x 2048] 14.2 and 17.2).
     constexpr bool EARLY = RPT > 1 || (TEAM == 64 ? VPT <= 3 : VPT == 2);
+    // Three to five words per lane of a workgroup are converted each as it comes: all asked for first they gain from memory
+    // ([800 x 6480] 7.83 -> 6.98 us) what they lose from the cache that the writer of the rows left them in ([1280 x 4324] 8.51 ->
+    // 8.76 us, [800 x 8100] 9.12 -> 9.57); from six on there is a gain in both ([512 x 12544] 9.53 -> 7.45 and 8.01 -> 7.70).
+    constexpr bool AHEAD = RPT > 1 || TEAM != 256 || VPT <= 2 || VPT >= 6;
     const auto fetch = [&](const RowBase& at, bool real, u32x4(&w)[VPT]) {
 #pragma unroll
         for (int j = 0; j < VPT; j++) {
@@ -1244,7 +1248,7 @@ __global__ __launch_bounds__(kThreads) void mvn6_rows_kernel(const half_t* __res
     bool live = row0 < g.rows;  // uniform per team; dead teams skip memory only
     RowBase b = row_base(g, live ? row0 : 0);
     u32x4 words[VPT];
-    fetch(b, live, words);
+    if (AHEAD) fetch(b, live, words);
     // scale and bias that run along the row, asked for beside it; with RPT > 1 they do not depend on it and are loaded once
     u32x4 scv[VPT], biv[VPT];
     if (EARLY) {
@@ -1266,7 +1270,8 @@ __global__ __launch_bounds__(kThreads) void mvn6_rows_kernel(const half_t* __res
     for (int j = 0; j < VPT; j++) {
         const uint32_t e0 = (uint32_t)(j * TEAM + t) * 8;
         if (live && e0 < g.row_len) {
-            const half_t* p = reinterpret_cast<const half_t*>(&words[j]);
+            const u32x4 q = AHEAD ? words[j] : row_word<WORDS>(in + b.in, e0, g.row_len);
+            const half_t* p = reinterpret_cast<const half_t*>(&q);
             const int again = row_again<WORDS>(e0, g.row_len);
 #pragma unroll
             for (int k = 0; k < 8; k++) {
