@@ -64,6 +64,8 @@ def test_taps_and_padding(rt, orc, dev, case, tile):
     (30, 14, 96, "nce_conv_gemm"), (30, 14, 192, "nce_conv_gemm"),  # 92 and 276 tiles of 64
     (16, 30, 160, "nce_conv_gemm"),                                  # 226 tiles of 128
     (2, 30, 128, "nce_conv_tile"),                                   # 58 tiles of 64: a family's
+    (40, 8, 256, "nce_conv_stream"), (16, 7, 512, "nce_conv_stream"),  # small planes, K split over waves, in one round
+    (40, 7, 512, "nce_conv_gemm"), (32, 7, 384, "nce_conv_gemm"),    # in two rounds; without the split
     (32, 28, 48, "nce_conv_rows16"),                                 # taps of less than half a panel
     (40, 16, 64, "nce_conv_regw"),                                   # 3x3 taps of 64 channels
 ])
