@@ -35,11 +35,11 @@ METRIC = "int8 conv/matmul TOPS (% MFMA peak); SW-kernel GB/s (% HBM peak)"
 # WRITE_SIZE counters of an earlier run of the same workload, scaled by a plain copy of known size
 # (profiles/<workload>__*.md hold those runs and their commands); the JSON line labels them as such.
 MEASURED_TRAFFIC = {
-    "c1_fake_quantize": 888450, "c2_softmax": 134261983, "c3_mvn": 17093583, "c4_conv": 14905457,
-    "c5_matmul": 339731998, "c5_dequantize": 135262411, "c5_eltwise_add": 270552950, "c5_nce_eltwise": 135260008,
-    "calib_copy": 134217728, "calib_int_mm": 534882288, "x_mvn6_layernorm": 268523883, "x_activation_hswish": 180471319,
-    "x_mvn1_three_steps": 25341653, "x_stem_conv": 67131551, "x_small_plane_conv": 20886567, "x_large_conv": 54593192,
-    "x_wide_conv": 58724921, "x_pointwise_conv": 32407905, "x_softmax_outer_axis": 402620437, "x_mvn_nhwc_per_channel": 212576856,
+    "c1_fake_quantize": 888450, "c2_softmax": 134261983, "c3_mvn": 17093583, "c4_conv": 14913796,
+    "c5_matmul": 339794672, "c5_dequantize": 135262411, "c5_eltwise_add": 270552950, "c5_nce_eltwise": 135260008,
+    "calib_copy": 134217728, "calib_int_mm": 534882288, "x_mvn6_layernorm": 268564672, "x_activation_hswish": 180471319,
+    "x_mvn1_three_steps": 25341653, "x_stem_conv": 54509346, "x_small_plane_conv": 20886567, "x_large_conv": 54601720,
+    "x_wide_conv": 58733750, "x_pointwise_conv": 32401682, "x_softmax_outer_axis": 402620437, "x_mvn_nhwc_per_channel": 212576856,
 }
 
 
@@ -273,7 +273,7 @@ def make_stem(rt):
     step.keep = (inp, w, wt, out, task)
     ops = 2 * N * (H // 2) * (H // 2) * OC * K * K * IC
     return Workload("x_stem_conv", "int8 Conv 7x7 s2 p3 NHWC [32,224,224,16] u8 zp128 x [64,7,7,16] i8, ReLU (not a BASELINE config)",
-                    step, inp.numel() + out.numel() + w.numel() + wt.numel() * 4, ops, "mfma", "int8", "nce_conv_rows16")
+                    step, inp.numel() + out.numel() + w.numel() + wt.numel() * 4, ops, "mfma", "int8", "nce_conv_strips")
 
 
 def make_small_plane_conv(rt):
