@@ -73,3 +73,24 @@ def test_where_the_rule_takes_it(rt, orc, dev, N, P, C, kernel):
     rng = np.random.default_rng(P + C)
     case = (N, P, P, C, C, 3, 3, (1, 1), (1, 1, 1, 1))
     assert run(rt, orc, dev, rng, case, None, 5, 0, True, False, 20, kernel=None) == kernel
+
+
+@pytest.mark.parametrize("zp,kernel", [(128, "nce_conv_stream"), (5, "nce_conv_gemm")])
+def test_small_planes_near_the_direct_form_take_no_scratch(rt, dev, zp, kernel):
+    import torch
+    g = torch.Generator(device="cuda").manual_seed(zp)
+    x = torch.randint(0, 256, (32, 7, 7, 256), dtype=torch.uint8, device="cuda", generator=g)
+    w = torch.randint(-127, 128, (256, 3, 3, 256), dtype=torch.int8, device="cuda", generator=g)
+    rng = np.random.default_rng(zp)
+    wt = torch.from_numpy(rt.make_weights_table(rng.integers(2**14, 2**15, 256), rng.integers(30, 32, 256),
+                                                rng.integers(-2**15, 2**15, 256).astype(np.int32), 2304)).cuda()
+    out, ref = torch.empty_like(x), torch.empty_like(x)
+    ppe = rt.PpeInt(rt.PPE_LRELU, 0, 255, 1, 0)
+    rt.nce_task(x, w, wt, out, ppe, zp_in=zp, pads=(1, 1, 1, 1))
+    assert rt.nce_last_kernel() == kernel
+    rt.set_tuning("VPX_NCE_KERNEL", "naive")
+    try:
+        rt.nce_task(x, w, wt, ref, ppe, zp_in=zp, pads=(1, 1, 1, 1))
+    finally:
+        rt.set_tuning("VPX_NCE_KERNEL", None)
+    assert torch.equal(out, ref) and ref.unique().numel() > 16
