@@ -46,3 +46,34 @@ def test_outputs_and_zero_points(rt, orc, dev, tile, M, K, N):
     rng = np.random.default_rng(M)
     for in_u8, zp_in, zp_w, out_f16, shift in ((True, 7, 31, False, 20), (False, 3, 0, True, 24), (True, 128, 128, False, 20), (False, 0, 0, False, 9)):
         assert run(rt, orc, dev, rng, M, K, N, tile, in_u8, zp_in, zp_w, out_f16, shift) == "nce_gemm_mfma"
+
+
+@pytest.mark.parametrize("out_f16", [False, True])
+@pytest.mark.parametrize("K", [320, 384, 448, 640, 4096])
+def test_large_tiles_fill_the_chip(rt, dev, K, out_f16):
+    """342 tiles of 256, more than one for a compute unit, so that panels arrive late and the waves of a tile drift apart: the tables of
+    column sums keep to themselves whichever buffer the last panel lies in (bit for bit what tiles of 128 give)"""
+    import torch
+    M, N = 4600, 4700
+    g = torch.Generator(device="cuda").manual_seed(K)
+    b = torch.randint(-127, 128, (N, 1, 1, K), dtype=torch.int8, device="cuda", generator=g)
+    rng = np.random.default_rng(K)
+    wt = torch.from_numpy(rt.make_weights_table(rng.integers(2 ** 14, 2 ** 15, N), rng.integers(20, 23, N), rng.integers(-2 ** 15, 2 ** 15, N).astype(np.int32), K)).cuda()
+    lo, hi, zp_out = (-(2 ** 31), 2 ** 31 - 1, 0) if out_f16 else (0, 255, 3)
+    ppe = rt.PpeInt(rt.PPE_LPRELU, lo, hi, 1638, 14)
+    dt = torch.float16 if out_f16 else torch.uint8
+    inputs = [torch.randint(0, 256, (1, M, 1, K), dtype=torch.uint8, device="cuda", generator=g) for _ in range(3)]
+    outs = {}
+    try:
+        for tile in (256, 128):
+            rt.set_tuning("VPX_GEMM_TILE", tile)
+            outs[tile] = [torch.empty((1, M, 1, N), dtype=dt, device="cuda") for _ in inputs]
+            for x, out in zip(inputs, outs[tile]):
+                rt.nce_task(x, b, wt, out, ppe, zp_in=7, zp_out=zp_out)
+            assert rt.nce_last_kernel() == "nce_gemm_mfma"
+    finally:
+        rt.set_tuning("VPX_GEMM_TILE", None)
+    torch.cuda.synchronize()
+    for large, small in zip(outs[256], outs[128]):
+        assert torch.equal(large, small), (K, out_f16, int((large != small).sum()))
+        assert large.unique().numel() > 16

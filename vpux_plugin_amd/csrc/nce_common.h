@@ -450,7 +450,7 @@ __device__ __forceinline__ int row_align(const void* base, int64_t row_bytes) {
 }
 
 constexpr int kOutStride = 288;  // bytes per row of the 256-column output staging tile in LDS
-constexpr int kGemmLdsHead = 1024;  // bytes in front of the matmul kernel's panel buffers (column sums of B)
+constexpr int kGemmLdsHead = 2048;  // bytes in front of the matmul kernel's panel buffers (column sums of B: up to two tables of 256)
 
 struct GemmPpe {
     int prelu_mult, prelu_shift;  // applied to negative scaled values (1,0 = none; 0,0 = ReLU)

@@ -19,6 +19,24 @@ struct PadTable {
 };
 __device__ const PadTable g_pads{};
 
+// What a form of the kernel keeps in LDS: the tables of column sums in the head, behind them the panel buffers, which the staging tile
+// reuses.  The tables share no byte with the rest: the waves write and read them while panels are still arriving, and while
+// faster waves already fill the staging tile.
+template <bool IN_U8, int OUT, int NW, int TILE = 256, bool SHORTK = false, bool PP = false, int NS = 4, bool CONV = false>
+struct GemmLds {
+    // panels of 128 bytes (see WIDE below); else of 64
+    static constexpr bool kWide = (TILE == 128 && NW == 8) || TILE == 64 || (TILE == 256 && NS == 2);
+    static constexpr int kSumTables = kWide ? 2 : 1;  // one per row of waves that sums columns
+    static constexpr int kPanel = 2 * TILE * (kWide ? 128 : 64);
+    static constexpr int kStaging = OUT == OUT_F16 ? (TILE == 256 ? 128 : TILE) * (2 * TILE + 32) : TILE * kOutStride;
+    static_assert(kSumTables * TILE * (int)sizeof(int) <= kGemmLdsHead, "the column sums end in front of the panel buffers");
+    static_assert(SHORTK || kStaging <= NS * kPanel, "the staging tile fits the panel buffers");
+    static size_t bytes(int64_t K) {  // of a launch; a short K asks for the panels there are or for the staging tile
+        const size_t panels = SHORTK ? (size_t)(K / 64) * kPanel : (size_t)NS * kPanel;
+        return kGemmLdsHead + (panels > kStaging ? panels : (size_t)kStaging);
+    }
+};
+
 // A[M][K] x B[N][K]^T with the PPE fused; see the file header.  K must be a multiple of 64.
 //
 // Pipeline of the forms below that walk K in panels of 64 bytes (K <= 192, and two that are only run when asked for: the 256 tile
@@ -67,7 +85,8 @@ __global__ __launch_bounds__(64 * NW) void nce_gemm_mfma(const int8_t* __restric
     // SHORTK (K <= 192, three panels at most): all panels are fetched up front, nothing is pipelined and no panel buffer
     // is reused, so the workgroup asks only for the LDS it touches and more of them fit a CU (a matmul this short is
     // bound by its epilogue and stores, not by the MFMAs).
-    constexpr bool WIDE = (TILE == 128 && NW == 8) || TILE == 64 || (TILE == 256 && NS == 2);
+    using Lds = GemmLds<IN_U8, OUT, NW, TILE, SHORTK, PP, NS, CONV>;
+    constexpr bool WIDE = Lds::kWide;
     constexpr bool SPLIT_RINGS = WIDE && TILE == 256;  // a ring of buffers per operand, so that an instruction's offset reaches both of its buffers
     constexpr int BM = TILE, BN = TILE, BK = WIDE ? 128 : 64, WM = BM / 2, WN = BN / (NW / 2), TM = WM / 32, TN = WN / 32;
     constexpr int MFMA_PER_DMA = WIDE ? 1 : TM * TN / (BM * BK / 1024 / NW);  // MFMAs between two DMA instructions of a sub-step
@@ -77,9 +96,10 @@ __global__ __launch_bounds__(64 * NW) void nce_gemm_mfma(const int8_t* __restric
     constexpr int RPI = 64 / CPR;                     // tile rows one 1 KiB DMA instruction covers
     constexpr int DMA_PER_WAVE = BM * BK / 1024 / NW;  // per operand, per panel
     constexpr int STAGE = (BM + BN) * BK;
+    static_assert(STAGE == Lds::kPanel, "the launch asks for the panels there are");
 
     extern __shared__ __attribute__((aligned(16))) uint8_t smem_raw[];
-    int* const colsums = reinterpret_cast<int*>(smem_raw);  // TILE column sums of B, handed from the upper waves to the lower
+    int* const colsums = reinterpret_cast<int*>(smem_raw);  // [Lds::kSumTables][TILE] column sums of B, handed from wave to wave
     uint8_t* const smem = smem_raw + kGemmLdsHead;          // the panel buffers, later the output staging tile
 
     // Grouped matmul: blockIdx.y is the group; every operand holds the groups one after the other.
@@ -620,7 +640,7 @@ __global__ __launch_bounds__(64 * NW) void nce_gemm_mfma(const int8_t* __restric
         // bytes), so that the tile leaves in whole rows of 16-byte stores (two-byte stores straight from the registers,
         // 64 bytes of a row per half-wavefront, cost the [4096 x 4096] . [4096 x 11008] matmul 60 us).
         constexpr int PASSES = TILE == 256 ? 2 : 1, ROWS = BM / PASSES, STR = BN * 2 + 32;
-        static_assert(ROWS * STR <= NS * STAGE, "the fp16 staging tile fits the panel buffers");
+        static_assert(ROWS * STR == Lds::kStaging, "the fp16 staging tile is what the launch has room for");
         uint16_t* out16 = reinterpret_cast<uint16_t*>(out);
         if (ppe.rowterm) {  // (padded past the last row: edge tiles may read ahead)
 #pragma unroll
@@ -762,14 +782,6 @@ int launch_gemm_mfma(const GemmLaunch& a, hipStream_t s) {
     const dim3 grid((unsigned)(per_xcd * 8), (unsigned)a.G);
     const int64_t nk = a.K / 64;
     const bool shortk = a.shortk;
-    size_t lds = 4 * (size_t)(tile + tile) * 64;  // four K panels; the output staging tile reuses them
-    if (shortk) {
-        lds = (size_t)nk * (tile + tile) * 64;  // only the panels there are ...
-        if (lds < (size_t)tile * kOutStride) lds = (size_t)tile * kOutStride;  // ... or the staging tile
-    } else if (tile < 256) {
-        lds = (size_t)a.stages * (tile + tile) * 128;
-    }
-    lds += kGemmLdsHead;
     const int32_t* colsum = nullptr;  // the kernel sums the columns of B itself, from the fragments it reads
     int rc = VPX_RESULT_SUCCESS;
     // the form in which the waves of a SIMD take turns: K a whole number of panel-buffer rounds
@@ -777,6 +789,7 @@ int launch_gemm_mfma(const GemmLaunch& a, hipStream_t s) {
 #define VPX_GEMM_K(...)                                                                                              \
     do {                                                                                                             \
         auto kern = nce_gemm_mfma<__VA_ARGS__>;                                                                      \
+        const size_t lds = GemmLds<__VA_ARGS__>::bytes(a.K);                                                         \
         rc = set_dyn_lds(kern, lds);                                                                                 \
         if (rc) return rc;                                                                                           \
         hipLaunchKernelGGL(kern, grid, dim3(64 * nw), lds, s, a.A, a.B, a.wt, colsum, a.out, a.M, a.N, a.K, tiles_m,  \
