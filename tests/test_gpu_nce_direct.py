@@ -81,3 +81,56 @@ def test_walks_around_the_steps_asked_for_at_once(rt, orc, dev, shape, depth, ta
                 rt.set_tuning("VPX_NCE_DIRECT", None)
             assert rt.nce_last_kernel() == "nce_direct"
             assert np.array_equal(out.cpu().numpy(), want), (steps, unit)
+
+
+@pytest.mark.parametrize("N,H,W,IC,OC,k,s,p,zp", [
+    # beside the stream kernel, whose sums of a zero point take scratch: small planes, narrow outputs, inputs that a stride skips lines of
+    (54, 5, 5, 512, 176, (3, 3), 1, 1, 5), (17, 6, 6, 512, 400, (3, 3), 1, 1, 5), (86, 4, 26, 768, 128, (2, 2), 2, 0, -3),
+    (101, 48, 48, 256, 16, (1, 1), 2, 0, 5), (5, 85, 85, 896, 16, (1, 1), 1, 0, 5), (14, 32, 32, 1664, 64, (1, 3), 2, 0, 5),
+    (27, 9, 59, 1664, 109, (1, 3), 3, 0, 5),
+    # beside the gather kernel, whose prepared channels do
+    (3, 178, 178, 1792, 16, (1, 1), 1, 0, 128), (6, 167, 167, 960, 16, (2, 2), 2, 1, 128), (37, 37, 102, 2048, 16, (1, 1), 2, 0, 5),
+    (26, 56, 278, 384, 123, (2, 1), 3, 0, -3),
+])
+def test_layers_near_the_end_of_its_range_take_no_scratch(rt, dev, N, H, W, IC, OC, k, s, p, zp):
+    """captured on a stream that has no scratch block, which a kernel that needs one refuses"""
+    import torch
+    g = torch.Generator(device="cuda").manual_seed(OC)
+    x = torch.randint(0, 256, (N, H, W, IC), dtype=torch.uint8, device="cuda", generator=g)
+    if zp < 0:
+        x = x.view(torch.int8)
+    w = torch.randint(-127, 128, (OC,) + k + (IC,), dtype=torch.int8, device="cuda", generator=g)
+    rng = np.random.default_rng(OC)
+    K = k[0] * k[1] * IC
+    shift = int(round(np.log2(5400.0 * np.sqrt(K) * 24576.0 / 60)))
+    wt = torch.from_numpy(rt.make_weights_table(rng.integers(2 ** 14, 2 ** 15, OC), rng.integers(shift, shift + 2, OC), rng.integers(-2 ** 15, 2 ** 15, OC).astype(np.int32), K)).cuda()
+    shape = (N, (H + 2 * p - k[0]) // s + 1, (W + 2 * p - k[1]) // s + 1, OC)
+    out, ref = torch.empty(shape, dtype=torch.uint8, device="cuda"), torch.empty(shape, dtype=torch.uint8, device="cuda")
+    ppe = rt.PpeInt(rt.PPE_LRELU, 0, 255, 1, 0)
+
+    def layer(y):
+        rt.nce_task(x, w, wt, y, ppe, zp_in=zp, strides=(s, s), pads=(p, p, p, p))
+
+    rt.set_tuning("VPX_NCE_KERNEL", "naive")
+    try:
+        layer(ref)
+    finally:
+        rt.set_tuning("VPX_NCE_KERNEL", None)
+    stream, graph = torch.cuda.Stream(), torch.cuda.CUDAGraph()
+    rt.workspace_release(stream=stream)
+    refused = []
+    torch.cuda.synchronize()
+    with torch.cuda.stream(stream):
+        with torch.cuda.graph(graph, stream=stream):
+            try:
+                layer(out)
+            except rt.VpxError as err:
+                refused.append(err)
+            ref.add_(0)  # (the capture is ended normally either way)
+    assert not refused, str(refused[0])
+    assert rt.nce_last_kernel() in ("nce_direct", "nce_conv_gemm")
+    for _ in range(2):
+        out.fill_(77)
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out, ref) and ref.unique().numel() > 16

@@ -737,6 +737,7 @@ struct DirectShape {
     int tm, tn, waves;
     double us;  // what the launch is expected to take
 };
+constexpr double kDirectPerMByte = 0.141;  // the share of that time for each million bytes of operands and result
 DirectShape direct_shape(int64_t P, int64_t OC, int64_t K, int64_t in_bytes, int cus);
 
 // nce_conv_patch.hip: one workgroup per tile of `pg.R` output rows x 64 channels.

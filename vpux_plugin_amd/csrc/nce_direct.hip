@@ -362,7 +362,7 @@ DirectShape direct_shape(int64_t P, int64_t OC, int64_t K, int64_t in_bytes, int
         const double rounds = std::ceil(simd_waves / (c.tm * c.tn <= 4 ? 4.0 : 2.0));
         const double us = 2.2 + (split ? 0.484 : 0.0) + 0.491 * (rounds - 1.0) + 0.0066 * (double)tiles / cus * (double)steps * (c.tm + c.tn) +
                           0.07 * (double)((share + depth - 1) / depth) + 0.126 * (double)share + 0.0174 * simd_waves * (double)share * c.tm * (c.tn + 1) +
-                          values * (split ? 0.0122 + 0.0295 * (double)S : 0.0259) + 0.141 * mbytes + mout * (c.tm == 1 ? 0.913 : (c.tm == 2 ? 0.18 : 0.0));
+                          values * (split ? 0.0122 + 0.0295 * (double)S : 0.0259) + kDirectPerMByte * mbytes + mout * (c.tm == 1 ? 0.913 : (c.tm == 2 ? 0.18 : 0.0));
         if (best.tm == 0 || us < best.us) best = DirectShape{c.tm, c.tn, c.waves, us};
     }
     return best;
