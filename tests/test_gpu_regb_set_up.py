@@ -1,5 +1,5 @@
 """The weights-in-registers matmul's set-up: weights dealt out through LDS where one block of channels is all a workgroup has,
-channel sums by matrix instructions, rows asked for before the weights; against the oracle at every length of K."""
+channel sums by matrix instructions, rows asked for ahead; against the oracle at every length of K."""
 import numpy as np
 import pytest
 

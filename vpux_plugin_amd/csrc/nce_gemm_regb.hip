@@ -20,12 +20,14 @@
 // rows, neighbouring lanes neighbouring 16-byte pieces (measured at [401408 x 64] . [64 x 256]: 64-byte pieces of
 // 256-byte rows, one per lane quarter, 34 us; a row per sixteen lanes 28 us).
 //
-// The set-up was half of a launch: weights (each wave its own copy, sixteen rows a load), then the weight table behind two barriers,
-// then the first rows' way from memory, one after the other.  All are asked for at once now, a wave's first row block first; four
-// waves with the same channels and a K beyond 64 deal one contiguous fetch out through LDS; channel sums come from MFMAs against
-// ones.  us in a HIP graph over rotating buffers, before / after: [100352 x 256] . [256 x 64] 12.9 / 9.8, [34848 x 256] . [256 x 64] 9.5 / 6.7,
-// [100352 x 128] . [128 x 32] 8.1 / 6.6, [100352 x 64] . [64 x 256] 14.3 / 13.2, [401408 x 64] . [64 x 256] 38.5 / 33.6, [16854 x 192] . [192 x 48] 5.0 / 4.2,
-// [9000 x 32] . [32 x 128] 4.0 / 3.2.  (More blocks asked for ahead of the weights hold up the set-up: 11.1 at K = 256.)
+// The set-up is half of a launch.  Weights, then the words of the weight table, are asked for together, and the rows behind the barriers:
+// asked for in front, they stand between every workgroup and its weights ([3380 x 128] . [128 x 512], a block of rows for each wave, 5.25 us
+// on one set of buffers, now 4.69; 4.84 with the words behind a barrier of their own).  Four waves with the same channels and a K beyond 64
+// have few weights and deal one contiguous fetch out through LDS: there the first rows' way begins before it.  Channel sums come from MFMAs
+// against ones.  us in a HIP graph over rotating buffers, with the words behind the sums and a copy of the weights for each wave / now:
+// [100352 x 256] . [256 x 64] 12.6 / 9.0, [20216 x 256] . [256 x 64] 7.9 / 5.3, [100352 x 128] . [128 x 32] 8.3 / 6.0, [100352 x 64] . [64 x
+// 256] 14.2 / 13.1, [401408 x 64] . [64 x 256] 39.0 / 33.6, [18928 x 192] . [192 x 48] 5.1 / 4.1, [2890 x 192] . [192 x 768] 6.0 / 5.7,
+// [5547 x 32] . [32 x 128] 4.1 / 2.9.
 // What is left at K = 64: a SIMD's vector instructions (115 a block of 16 x 64, 64 of them the PPE) as long as its memory time.
 //
 // Work is dealt by wave.  The four waves of a workgroup serve GW different groups of CBW channel blocks (4 / GW row
@@ -72,24 +74,28 @@ __global__ __launch_bounds__(64 * kRegbWaves) __attribute__((amdgpu_waves_per_eu
 #pragma unroll
         for (int ks = 0; ks < KS; ks++) a[ks] = *reinterpret_cast<const i32x4*>(src + (ks < KS - 1 ? c4 * 16 + ks * 64 : tail_at));
     };
-    // ---- everything the set-up waits for is asked for at once, the longest way first: the first row blocks (from memory; past the
-    // last one its last row), this thread's words of the weight table, the weights (from the caches: every workgroup reads them)
+    // ---- what the set-up waits for, asked for in the order it is used: the weights (from the caches: every workgroup reads them), this
+    // thread's words of the weight table, then the rows.  (No branch around the words: at its end the compiler waits for what was asked for
+    // inside, which cost a trip to memory in front of the weights.)
+    constexpr bool SHARE = GW == 1 && KS >= 2;  // the four waves serve the same channels and K is long
     i32x4 a[kPrefetch + 1][KS];
-    fetch(stream, a[0]);
-    const auto fetch_ahead = [&]() __attribute__((always_inline)) {
+    const auto fetch_ahead = [&](int from) __attribute__((always_inline)) {  // (blocks that there are: repeating the last row for the others cost 2 %)
 #pragma unroll
-        for (int p = 1; p < kPrefetch; p++) fetch(stream + p * streams, a[p]);
-        __builtin_amdgcn_sched_barrier(0);
+        for (int p = 0; p < kPrefetch; p++)
+            if (p >= from && (p == 0 || stream + p * streams < nblk)) fetch(stream + p * streams, a[p]);
     };
-    int2 words = int2{0, 0};
-    if (tid < TCH) {
-        const int ch = super * TCH + tid;
+    int2 words;
+    const auto fetch_words = [&]() __attribute__((always_inline)) {
+        const int ch = super * TCH + (tid < TCH ? tid : 0);
         words = *reinterpret_cast<const int2*>(wt + (int64_t)(ch < N ? ch : N - 1) * 4 + 2);
+    };
+    if (SHARE) {  // (their weights are few: the first rows' longer way begins before)
+        fetch(stream, a[0]);
+        fetch_words();
     }
-    // Fragment (cbl, j) of the weights: row n16 of tile j of block cbl, 16 of K per quarter.  Where the four waves serve the same channels
-    // and K is long, the workgroup fetches them once, a contiguous piece, and deals them out through LDS.
+    // Fragment (cbl, j) of the weights: row n16 of tile j of block cbl, 16 of K per quarter.  SHARE: the workgroup fetches them once, a
+    // contiguous piece, and deals them out through LDS.
     i32x4 wb[CBW][NT][KS];
-    constexpr bool SHARE = GW == 1 && KS >= 2;
     if constexpr (SHARE) {
         constexpr int ROW = KS * 64 + 16, PIECES = NCH * KS * 4, PER = (PIECES + 64 * kRegbWaves - 1) / (64 * kRegbWaves);
         __shared__ __attribute__((aligned(16))) uint8_t s_w[NCH * ROW];
@@ -100,7 +106,6 @@ __global__ __launch_bounds__(64 * kRegbWaves) __attribute__((amdgpu_waves_per_eu
             const int ch = n0 + row < N ? n0 + row : N - 1;  // channels past the end repeat the last one (never stored)
             v[u] = *reinterpret_cast<const i32x4*>(B + ((int64_t)ch * chunks + (c < chunks ? c : 0)) * 16);
         }
-        fetch_ahead();
 #pragma unroll
         for (int u = 0; u < PER; u++) {
             const int q0 = u * 64 * kRegbWaves + tid, q = q0 < PIECES ? q0 : PIECES - 1, row = q / (KS * 4), c = q % (KS * 4);
@@ -125,7 +130,7 @@ __global__ __launch_bounds__(64 * kRegbWaves) __attribute__((amdgpu_waves_per_eu
                 for (int ks = 0; ks < KS; ks++)
                     wb[cbl][j][ks] = *reinterpret_cast<const i32x4*>(B + ((int64_t)ch * chunks + (ks < KS - 1 || tail ? ks * 4 + c4 : 0)) * 16);
             }
-        fetch_ahead();
+        fetch_words();
     }
 #pragma unroll
     for (int cbl = 0; cbl < CBW; cbl++)
@@ -171,6 +176,7 @@ __global__ __launch_bounds__(64 * kRegbWaves) __attribute__((amdgpu_waves_per_eu
     if (lane == 0) s_general[w] = special ? 1 : 0;
     __syncthreads();
     const bool general = (s_general[0] | s_general[1] | s_general[2] | s_general[3]) != 0;  // (one answer for the workgroup)
+    fetch_ahead(SHARE ? 1 : 0);
     if (n0 >= N) return;  // (a wave past the last block)
     const int32_t* const rt = ppe.rowterm;
 
