@@ -34,6 +34,8 @@
 // streams each): with GW > 1 the waves that share a row block are neighbours, so its rows come from memory once.  A
 // workgroup's index modulo the number of its kind picks the channels; wave s of those that share them takes row blocks
 // s, s + S, ...
+#include <algorithm>
+
 #include "nce_common.h"
 
 namespace vpx {
@@ -296,9 +298,9 @@ __global__ __launch_bounds__(64 * kRegbWaves) __attribute__((amdgpu_waves_per_eu
 // per store -- where the rows are many enough for units of that size to fill the waves evenly (about six row blocks per
 // wave: [401408 x 64] . [64 x 256] 30.5 us with four blocks per wave, 34.1 with one; [100352 x 64] . [64 x 256] 11.8
 // against 10.2 us); else one.
-// us: what the launch should take, fitted (non-negative least squares, median error 5 %) to 250 layers of 300 ... 120 000
-// rows, K 16 ... 256, 16 ... 1024 channels: the launch and the weights, the busiest wave's walk, the compute unit's share
-// of the arithmetic and of the row loads.
+// us: what the launch should take, fitted (non-negative least squares, median error 5 %, one tenth beyond 15) to 986 layers of 200 ...
+// 30 000 rows, K 16 ... 256, 16 ... 1024 channels, the mean of one set of buffers and of rotating ones: the launch and the weights, the busiest
+// wave's walk, the compute unit's share of the arithmetic, of the row loads and of the weight loads, memory.
 RegbShape gemm_regb_shape(int64_t M, int64_t N, int64_t K, int cus, bool same_f, bool widest) {
     const int ks = (int)((K + 63) / 64);
     const int64_t nblk = (M + 15) / 16;
@@ -306,8 +308,11 @@ RegbShape gemm_regb_shape(int64_t M, int64_t N, int64_t K, int cus, bool same_f,
         const int64_t tiles = (int64_t)r.nt * r.cbw, per = 16 * tiles * r.gw, supers = (N + per - 1) / per, blocks = supers * r.gw;
         const int64_t wgs = ((int64_t)cus * regb_waves_per_simd(same_f, ks, r.cbw, r.nt) + supers - 1) / supers * supers;
         const int64_t streams = wgs / supers * (kRegbWaves / r.gw), walks = (nblk + streams - 1) / streams;
-        r.us = 2.84 + 0.05 * (double)(ks * tiles) + (double)walks * (0.031 * ks + 0.074 * (double)tiles) +
-               (double)(nblk * blocks) / cus * (0.02 * (double)tiles + 0.025 * ks / r.gw);
+        const int64_t per_cu = (std::min(wgs, (nblk + kRegbWaves / r.gw - 1) / (kRegbWaves / r.gw) * supers) + cus - 1) / cus;
+        const bool shared = r.gw == 1 && ks >= 2;  // (SHARE above)
+        r.us = 2.13 + 0.036 * (double)(ks * tiles) + (double)walks * (0.059 * ks + 0.061 * (double)tiles) +
+               (double)(nblk * blocks) / cus * (0.0165 * (double)tiles + 0.028 * ks / r.gw) + 0.0125 * (double)(per_cu * ks * tiles * (shared ? 1 : 4)) +
+               0.035e-6 * (double)(M * (K + N));
         return r;
     };
     const int64_t cb_total = (N + 63) / 64;
