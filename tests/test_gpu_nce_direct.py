@@ -134,3 +134,13 @@ def test_layers_near_the_end_of_its_range_take_no_scratch(rt, dev, N, H, W, IC, 
         graph.replay()
         torch.cuda.synchronize()
         assert torch.equal(out, ref) and ref.unique().numel() > 16
+
+
+@pytest.mark.parametrize("N,P,IC,OC,p,kernel", [
+    (51, 12, 96, 96, 0, "nce_direct"), (26, 6, 144, 544, 1, "nce_direct"), (14, 15, 144, 144, 1, "nce_direct"),  # taps that end inside a line
+    (32, 14, 192, 192, 1, "nce_conv_gemm"), (61, 16, 144, 144, 0, "nce_conv_gemm"),
+])
+def test_beside_the_matmul_form_of_convolutions(rt, orc, dev, N, P, IC, OC, p, kernel):
+    rng = np.random.default_rng(IC + N)
+    g = dict(N=N, H=P, W=P, IC=IC, OC=OC, KY=3, KX=3, pads=(p, p, p, p))
+    assert run_views(rt, orc, dev, rng, g, "dense", "dense", mode="LRELU", zp_in=5) == kernel
