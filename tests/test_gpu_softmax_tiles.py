@@ -13,6 +13,7 @@ pytestmark = pytest.mark.gpu
     (1, 70, 8100), (3, 300, 2000), (1, 1000, 4000),                                                                    # fewer: 16 lanes
     (1, 65, 18100), (1, 264, 40003), (1, 320, 18001), (1, 321, 100001), (1, 384, 40001), (1, 385, 18111), (1, 512, 18003),  # more: 64 lanes, 8 waves
     (1, 513, 18001), (1, 768, 18050), (1, 769, 18002),                                                                 # 16 waves
+    (1, 129, 100001), (1, 185, 30002), (1, 192, 90001),                                                                # 8 waves of 17 to 24
 ])
 def test_every_shape_of_a_tile(rt, orc, dev, outer, L, inner):
     rng = np.random.default_rng(L + inner)

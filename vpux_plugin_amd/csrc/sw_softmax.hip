@@ -390,6 +390,8 @@ __global__ __launch_bounds__(KW == 1 ? 256 : 64 * KW) void softmax_slab_f16(cons
                                                                            int64_t in_as, int64_t out_as, int by_die) {
     typedef _Float16 hvec __attribute__((ext_vector_type(VEC)));
     typedef hvec hvec_any __attribute__((aligned(2)));
+    typedef uint32_t words __attribute__((ext_vector_type(VEC / 2)));  // a lane's VEC columns of a step
+    typedef words words_any __attribute__((aligned(2)));
     typedef float fvec __attribute__((ext_vector_type(VEC)));
     constexpr int SHARES = KW * (64 / CL);
     __shared__ hvec smax[KW == 1 ? 1 : KW][CL];
@@ -410,25 +412,29 @@ __global__ __launch_bounds__(KW == 1 ? 256 : 64 * KW) void softmax_slab_f16(cons
     const half_t* src = in + ioff + col;
     half_t* dst = out + ooff + col;
 
-    hvec h[SMAX];
+    words h[SMAX];  // (whole words: halves the compiler took apart between the loads for some SMAX and waited for each, [1,175,169,153] 12.0 us, now 8.5)
+    const auto halves = [](words w) { return __builtin_bit_cast(hvec, w); };
     hvec m;
 #pragma unroll
     for (int k = 0; k < VEC; k++) m[k] = (half_t)-INFINITY;
 #pragma unroll
     for (int i = 0; i < SMAX; i++) {
         const int a = kw + SHARES * i;
-        h[i] = m;  // -inf
-        if (live && a < L) h[i] = *reinterpret_cast<const hvec_any*>(src + a * in_as);
+        h[i] = __builtin_bit_cast(words, m);  // -inf
+        if (live && a < L) h[i] = *reinterpret_cast<const words_any*>(src + a * in_as);
     }
     if (VEC > 1 && left > 0 && !live) {
 #pragma unroll
-        for (int i = 0; i < SMAX; i++)
+        for (int i = 0; i < SMAX; i++) {
+            hvec v = halves(h[i]);
 #pragma unroll
             for (int k = 0; k + 1 < VEC; k++)
-                if (k < left && kw + SHARES * i < L) h[i][k] = src[(kw + SHARES * i) * in_as + k];
+                if (k < left && kw + SHARES * i < L) v[k] = src[(kw + SHARES * i) * in_as + k];
+            h[i] = __builtin_bit_cast(words, v);
+        }
     }
 #pragma unroll
-    for (int i = 0; i < SMAX; i++) m = __builtin_elementwise_max(m, h[i]);
+    for (int i = 0; i < SMAX; i++) m = __builtin_elementwise_max(m, halves(h[i]));
     if constexpr (CL < 64) {
         static_assert(VEC == 2, "one register of maxima crosses the wave's parts");
 #pragma unroll
@@ -450,7 +456,7 @@ __global__ __launch_bounds__(KW == 1 ? 256 : 64 * KW) void softmax_slab_f16(cons
 #pragma unroll
     for (int i = 0; i < SMAX; i++)
 #pragma unroll
-        for (int k = 0; k < VEC; k++) sum[k] += __builtin_amdgcn_exp2f(__builtin_fmaf((float)h[i][k], kLog2e, nmb[k]));
+        for (int k = 0; k < VEC; k++) sum[k] += __builtin_amdgcn_exp2f(__builtin_fmaf((float)halves(h[i])[k], kLog2e, nmb[k]));
     if constexpr (CL < 64) {
 #pragma unroll
         for (int o = CL; o < 64; o *= 2)
@@ -480,7 +486,7 @@ __global__ __launch_bounds__(KW == 1 ? 256 : 64 * KW) void softmax_slab_f16(cons
             hvec r;
 #pragma unroll
             for (int k = 0; k < VEC; k++)
-                r[k] = (half_t)(__builtin_amdgcn_exp2f(__builtin_fmaf((float)h[i][k], kLog2e, nmb[k])) * inv[k]);
+                r[k] = (half_t)(__builtin_amdgcn_exp2f(__builtin_fmaf((float)halves(h[i])[k], kLog2e, nmb[k])) * inv[k]);
             if (live) {
                 if (NT) __builtin_nontemporal_store(r, reinterpret_cast<hvec_any*>(dst + a * out_as));
                 else *reinterpret_cast<hvec_any*>(dst + a * out_as) = r;
