@@ -13,6 +13,8 @@ pytestmark = pytest.mark.gpu
     (1, 70, 8100), (3, 300, 2000), (1, 1000, 4000),                                                                    # fewer: 16 lanes
     (1, 65, 18100), (1, 264, 40003), (1, 320, 18001), (1, 321, 100001), (1, 384, 40001), (1, 385, 18111), (1, 512, 18003),  # more: 64 lanes, 8 waves
     (1, 513, 18001), (1, 768, 18050), (1, 769, 18002),                                                                 # 16 waves
+    (1, 67, 30001), (2, 192, 15001), (1, 256, 45001), (1, 383, 30001),                                                 # odd rows, 32 lanes beyond 140 tiles
+    (1, 193, 64001), (1, 256, 70001), (1, 385, 60001), (1, 512, 64003), (1, 400, 20002),                               # 16 waves of 13 to 16, 25 to 32 steps
     (1, 129, 100001), (1, 185, 30002), (1, 192, 90001),                                                                # 8 waves of 17 to 24
 ])
 def test_every_shape_of_a_tile(rt, orc, dev, outer, L, inner):

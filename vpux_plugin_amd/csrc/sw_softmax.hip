@@ -1035,7 +1035,12 @@ int softmax_typed(const SoftmaxPlan& p, const T* in, T* out, hipStream_t s) {
             int kw = len <= 8 ? 1 : (len <= 16 ? (small ? 4 : 2) : (len <= 64 ? (small ? 8 : 4) : 8));
             int64_t tiles = outer * ((inner + 64 * vec - 1) / (64 * vec));
             const bool few = len > 64 && tiles * 20 < 11 * (int64_t)cus;
-            if (len > 512 || few) kw = 16;
+            // Rows of an odd length want sixteen where eight would hold 32 or 64 steps a lane, up to two and a half tiles a compute unit ([6,221,101,
+            // 99], 474 tiles, 14.4 us, 17.1 with eight, [3,449,127,133], 396, 30.1 and 35.2); others only where eight would hold 64, up to
+            // three quarters of a tile.
+            const bool odd = inner % 2 != 0, hold64 = len > 384 && len <= 512, hold32 = len > 192 && len <= 256;
+            const bool sixteen = odd ? (hold32 || hold64) && tiles * 2 <= 5 * (int64_t)cus : hold64 && tiles * 4 <= 3 * (int64_t)cus;
+            if (len > 512 || few || sixteen) kw = 16;
             // fewer waves than SIMDs (with a short axis: than compute units): columns of 16 lanes, four shares of the axis a wave
             const bool narrow = tiles * kw < (len > 16 ? 4 : 1) * cus;
             if (narrow) {
@@ -1043,8 +1048,11 @@ int softmax_typed(const SoftmaxPlan& p, const T* in, T* out, hipStream_t s) {
                 kw = len <= 16 ? 1 : (len <= 64 ? 4 : (len <= 256 ? 8 : 16));
             }
             // few tiles of many steps: columns of 32 lanes, two shares of the axis a wave, twice the tiles ([1,185,41,357], 115 tiles,
-            // 8.6 -> 7.3 us, [1,200,130,91] 7.8 -> 6.3, [1,512,90,101] 13.3 -> 10.2; at 158 tiles, [1,300,100,201], 11.8 against 10.9)
-            const bool half = few && !narrow;
+            // 8.6 -> 7.3 us, [1,200,130,91] 7.8 -> 6.3, [1,512,90,101] 13.3 -> 10.2; at 158 tiles, [1,300,100,201], 11.8 against 10.9).
+            // Rows of an odd length, every other one off the words' alignment, want them for longer: up to one and a half tiles a compute
+            // unit (shorter by 5 ... 30 % than columns of 64 lanes), one beyond 256 steps (22 ... 42 %: [1,175,169,153], 202 tiles, 8.5 -> 7.6).
+            const bool half = !narrow && len > 64 && len <= 512 &&
+                              (few || (odd && len <= 384 && tiles * 2 <= (len <= 256 ? 3 : 2) * (int64_t)cus));
             if (half) {
                 vec = 2;
                 kw = len <= 256 ? 8 : 16;
@@ -1095,7 +1103,9 @@ int softmax_typed(const SoftmaxPlan& p, const T* in, T* out, hipStream_t s) {
                     if (steps <= 4) VPX_SLAB(2, 8, 4); else if (steps <= 8) VPX_SLAB(2, 8, 8); else if (steps <= 16) VPX_SLAB(2, 8, 16);
                     else if (steps <= 24) VPX_SLAB(2, 8, 24); else if (steps <= 32) VPX_SLAB(2, 8, 32);
                     else if (steps <= 40 && three) VPX_SLAB(2, 8, 40); else if (steps <= 48 && three) VPX_SLAB(2, 8, 48); else VPX_SLAB(2, 8, 64);
-                } else if (steps <= 48) VPX_SLAB(2, 16, 48);  // (from 33 on)
+                } else if (steps <= 16) VPX_SLAB(2, 16, 16);  // (13 to 16, 25 to 32, from 33 on)
+                else if (steps <= 32) VPX_SLAB(2, 16, 32);
+                else if (steps <= 48) VPX_SLAB(2, 16, 48);
                 else VPX_SLAB(2, 16, 64);
 #undef VPX_SLAB_NT
 #undef VPX_SLAB_HALF
