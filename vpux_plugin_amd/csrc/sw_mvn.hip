@@ -1225,7 +1225,8 @@ template <int TEAM, int VPT, int RPT = 1, bool WORDS = true>  // RPT: consecutiv
 __global__ __launch_bounds__(kThreads) void mvn6_rows_kernel(const half_t* __restrict__ in, half_t* __restrict__ out,
                                                              const half_t* __restrict__ sc, const half_t* __restrict__ bi,
                                                              Mvn6Geom g, int normalize_variance, int eps_mode, float eps) {
-    __shared__ float red[RPT > 1 ? 16 : 8];
+    __shared__ float red[8];
+    static_assert(TEAM != 256 || RPT == 1, "the workgroup-wide sums have slots for one row");
     const int t = (int)(threadIdx.x % TEAM);
     const int64_t row0 = ((int64_t)blockIdx.x * (kThreads / TEAM) + threadIdx.x / TEAM) * RPT;
     // The words of a row are asked for all at once (but see AHEAD), and before they are used the scale and the bias that run along it: asked for
@@ -1263,7 +1264,6 @@ __global__ __launch_bounds__(kThreads) void mvn6_rows_kernel(const half_t* __res
     }
 #pragma unroll 1
     for (int rr = 0; rr < RPT; rr++) {
-    float* const slots = red + (RPT > 1 ? (rr & 1) * 8 : 0);  // (a row's slots are written again two rows on, behind that row's barriers)
     float x[VPT][8];
     float sum = 0.f;
 #pragma unroll
@@ -1291,7 +1291,7 @@ __global__ __launch_bounds__(kThreads) void mvn6_rows_kernel(const half_t* __res
         fetch(b, live, words);
     }
     const float n = (float)g.row_len;
-    const float mean = team_sum<TEAM>(sum, slots) / n;
+    const float mean = team_sum<TEAM>(sum, red) / n;
     float q = 0.f;
 #pragma unroll
     for (int j = 0; j < VPT; j++) {
@@ -1303,7 +1303,7 @@ __global__ __launch_bounds__(kThreads) void mvn6_rows_kernel(const half_t* __res
             q += (WORDS ? e0 < g.row_len : k >= again) ? d * d : 0.f;
         }
     }
-    const float var = team_sum<TEAM>(q, slots + 4) / n;
+    const float var = team_sum<TEAM>(q, red + 4) / n;
     const float inv = mvn6_inv(var, normalize_variance, eps_mode, eps);
     const float sc_row = sc && !g.sc_along_row ? (float)sc[here.sc] : 1.0f;
     const float bi_row = bi && !g.bi_along_row ? (float)bi[here.bi] : 0.0f;
