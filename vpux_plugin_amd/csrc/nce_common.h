@@ -663,10 +663,8 @@ struct View {
 };
 int operand_view(const int64_t st[4], int64_t N, int64_t H, int64_t W, int64_t C, const char* what, View* v);
 
-// nce_gemm.hip.  `tile` 128 | 256, `waves` 4 | 8 (8 with the large tile only), `shortk`: K of at most three panels on
-// the small tile; G groups on the grid's second dimension.
-// n / d for any n and d of 32 bits: with magic = floor((2^32 - 1) / d), which lies less than one below 2^32 / d, the high half of n * magic is
-// the quotient or one less.
+// n / d for any n and d of 32 bits: magic = floor((2^32 - 1) / d) lies at most one below 2^32 / d (one where d is a power of two), so n * magic
+// falls short of 2^32 * n / d by at most n < 2^32, and its high half is the quotient or one less.
 inline unsigned quotient_magic(unsigned d) { return 0xffffffffu / d; }
 __device__ __forceinline__ unsigned quotient(unsigned n, unsigned d, unsigned magic) {
     const unsigned q = __umulhi(n, magic);
@@ -681,6 +679,8 @@ struct GemmConv {
     unsigned ow_magic, ohow_magic;  // quotient_magic(ow), (ohow)
     int pad;  // the byte of a tap outside the image
 };
+// nce_gemm.hip.  `tile` 64 | 128 | 256, `waves` 4 | 8 (of the large tile), `shortk`: K of at most three panels of 64 bytes on
+// the small tiles; G groups on the grid's second dimension.
 struct GemmLaunch {
     const int8_t* A;
     const int8_t* B;
