@@ -13,6 +13,7 @@ EDGE = 4096  # output positions x blocks of 64 channels from which the kernel is
     (3, 27, 26, 70, (1, 1)),                                                # two blocks of channels, the last of six
     (2, 91, 93, 130, (2, 2)),                                               # a stride, three blocks, tiles past the last row
     (7, 25, 24, 16, (1, 1)),                                                # a quarter of the block's channels
+    (43, 153, 37, 52, (2, 2)),                                              # tiles of 16 rows, 158.7 KiB of the 159.5 that a workgroup may have
 ])
 @pytest.mark.parametrize("zp,shift,lrelu", [(128, 20, None), (0, 20, (1638, 14)), (7, 12, (1638, 14)), (131, 3, None), (128, 20, (3, 0))])
 def test_sizes_around_the_edge(rt, orc, dev, N, H, W, OC, strides, zp, shift, lrelu):

@@ -532,7 +532,6 @@ __device__ __forceinline__ int64_t tile_out_pos(const ConvGeom& g, int p, FastDi
 }
 
 constexpr int kPatchMaxMT = 14;
-constexpr int kRegwTables = 64 * sizeof(ChanPrep) + 32;  // bytes in front of nce_conv_regw's weights: its prepared channels, a flag
 constexpr int kPatchOutStride = 80;  // bytes per output position in the staging tile
 constexpr int kPatchOutStrideF16 = 144;  // the same for an fp16 output
 

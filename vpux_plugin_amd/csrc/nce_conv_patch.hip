@@ -261,7 +261,8 @@ __global__ __launch_bounds__(64 * NW, NW == 8 ? 1 : (TMW <= 4 ? 2 : 1)) void nce
 // the form of its time took 9.6 us at [32,56,56,64] -> 64.)
 // A launch of one tile per compute unit is mostly set-up: the first wave asks for its words of the weight table before anything
 // else and prepares the 64 channels once, under the patch rows' flight -- every wave asking for its own after the staging put a
-// trip to memory behind it, 9.5 -> 8.3 us at [32,56,56,64] -> 64, 8.1 -> 7.0 at [32,46,46,64], 24.0 -> 22.6 at [128,56,56,64].
+// trip to memory behind it, 9.5 -> 8.3 us at [32,56,56,64] -> 64, 8.1 -> 7.0 at [32,46,46,64], 24.0 -> 22.6 at [128,56,56,64].  The
+// prepared channels lie in the 32 bytes between the weight rows: two KiB of their own cost tall tiles a row, and with it a round.
 //
 // Channel order inside a block: column n of MFMA tile j is output channel 16*(n/4) + 4*j + n%4.  After the 4x4 byte
 // transpose a lane then holds channels 16*q .. 16*q+15 of one position in its four result dwords (tile j -> dword j),
@@ -276,11 +277,11 @@ __global__ __launch_bounds__(512) void nce_conv_regw(const int8_t* __restrict__ 
     // (96 and 608 bytes; measured: 80 or 592 bytes take twice as long per read)
     constexpr int BN = 64, IC = 64, PS = IC + 32, NW = 8, NT = 64 * NW, TAPS = KY * KX, Ktot = TAPS * IC, WS = Ktot + 32;
     static_assert((PS / 16) % 4 == 2 && (WS / 16) % 4 == 2, "conflict-free fragment reads");
+    static_assert(Ktot + sizeof(ChanPrep) <= WS, "a channel behind its weights");
     extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
-    ChanPrep* const sprep = reinterpret_cast<ChanPrep*>(smem);       // [64], by row of `wlds`
-    int* const sgeneral = reinterpret_cast<int*>(smem + BN * sizeof(ChanPrep));
-    uint8_t* const wlds = smem + kRegwTables;                        // [64][Ktot + 32], rows in tile order
-    uint8_t* const patch = wlds + BN * WS;                           // [PH*PW][IC + 32]
+    uint8_t* const wlds = smem;             // [64][Ktot + 32], rows in tile order; behind a row's weights lies its prepared channel
+    __shared__ int sgeneral;
+    uint8_t* const patch = smem + BN * WS;  // [PH*PW][IC + 32]
 
     // A launch of a few microseconds is bound by instructions as much as by anything else: all index arithmetic below
     // is 32-bit, on offsets from a few 64-bit bases that are the same for the whole wave.
@@ -385,10 +386,10 @@ __global__ __launch_bounds__(512) void nce_conv_regw(const int8_t* __restrict__ 
             const uint32_t w2 = (uint32_t)words.x;
             const ChanPrep c = ppe_prepare((int)(int16_t)(w2 >> 16), (int)((w2 >> 8) & 0xffu), (int)((unsigned)words.y + (unsigned)(ppe.corr * sum)),
                                            ppe.prelu_mult, ppe.prelu_shift);
-            sprep[lane] = c;
+            *reinterpret_cast<ChanPrep*>(wlds + lane * WS + Ktot) = c;
             const bool clip = c.bmax_pos != 0x7fffffff || c.bmax_neg != 0x7fffffff;
             const bool special = __builtin_amdgcn_ballot_w64(clip) != 0 || pk.odd != 0 || !slope_ok;
-            if (lane == 0) sgeneral[0] = special ? 1 : 0;
+            if (lane == 0) sgeneral = special ? 1 : 0;
         }
         store_patch();
         for (int u0 = NW * UP; u0 < units; u0 += NW * UP) {  // tall patches: the rest, a round trip each
@@ -402,10 +403,10 @@ __global__ __launch_bounds__(512) void nce_conv_regw(const int8_t* __restrict__ 
     ChanPrep cp[4];
 #pragma unroll
     for (int j = 0; j < 4; j++) {
-        cp[j] = sprep[j * 16 + n16];
+        cp[j] = *reinterpret_cast<const ChanPrep*>(wlds + (j * 16 + n16) * WS + Ktot);
         asm volatile("" : "+v"(cp[j].f_pos), "+v"(cp[j].f_neg));
     }
-    const bool general = __builtin_amdgcn_readfirstlane(sgeneral[0]) != 0;
+    const bool general = __builtin_amdgcn_readfirstlane(sgeneral) != 0;
     const QuadTranspose transpose(lane);
 
     const int rows_here = OH - oy0 < pg.R ? OH - oy0 : pg.R;
