@@ -74,7 +74,7 @@ struct GemmLds {
 // K, of the weights, from sixteen zeros.  A panel costs a fifth more than the matmul's ([2000 x 2880] . [2880 x 320] 9.3 us,
 // [20,10,10,320] -> 320 3x3 11.0), bound by the LDS as there.
 template <bool IN_U8, int OUT, int NW, int TILE = 256, bool SHORTK = false, bool PP = false, int NS = 4, bool CONV = false>
-__global__ __launch_bounds__(64 * NW) void nce_gemm_mfma(const int8_t* __restrict__ A, const int8_t* __restrict__ B,
+__global__ __launch_bounds__(64 * NW, SHORTK ? 3 : 1) void nce_gemm_mfma(const int8_t* __restrict__ A, const int8_t* __restrict__ B,
                                                      const int32_t* __restrict__ wt, const int32_t* __restrict__ colsum,
                                                      uint8_t* __restrict__ out,
                                                      int64_t M, int64_t N, int64_t K, int tiles_m, int tiles_n, unsigned group_magic,
@@ -84,7 +84,8 @@ __global__ __launch_bounds__(64 * NW) void nce_gemm_mfma(const int8_t* __restric
     // TILE = 128 and 64 serve problems with too few 256 x 256 tiles.
     // SHORTK (K <= 192, three panels at most): all panels are fetched up front, nothing is pipelined and no panel buffer
     // is reused, so the workgroup asks only for the LDS it touches and more of them fit a CU (a matmul this short is
-    // bound by its epilogue and stores, not by the MFMAs).
+    // bound by its epilogue and stores, not by the MFMAs).  Three waves a SIMD are asked for: left to itself the compiler keeps the
+    // sums in accumulation registers beside 124 others, two waves, and [15514 x 64] . [64 x 584] took 10.1 us, now 8.6.
     using Lds = GemmLds<IN_U8, OUT, NW, TILE, SHORTK, PP, NS, CONV>;
     constexpr bool WIDE = Lds::kWide;
     constexpr bool SPLIT_RINGS = WIDE && TILE == 256;  // a ring of buffers per operand, so that an instruction's offset reaches both of its buffers
