@@ -6,7 +6,7 @@ import pytest
 pytestmark = pytest.mark.gpu
 
 
-def run(rt, orc, dev, rng, M, K, N, tile, in_u8, zp_in, zp_w, out_f16, shift=20):
+def run(rt, orc, dev, rng, M, K, N, tile, in_u8, zp_in, zp_w, out_f16, shift=20, direct="off"):
     import torch
     a = rng.integers(0, 256, (1, M, 1, K), dtype=np.uint8) if in_u8 else rng.integers(-128, 128, (1, M, 1, K)).astype(np.int8)
     b = rng.integers(0, 256, (N, 1, 1, K), dtype=np.uint8) if zp_w else rng.integers(-127, 128, (N, 1, 1, K)).astype(np.int8)
@@ -15,7 +15,7 @@ def run(rt, orc, dev, rng, M, K, N, tile, in_u8, zp_in, zp_w, out_f16, shift=20)
     want = orc.nce_conv(a, b, wt, orc.ppe(1638, 14, zp_out, lo, hi), zp_in=zp_in, zp_w=zp_w, out_f16=out_f16)
     out = torch.full((1, M, 1, N), 77, dtype=torch.float16 if out_f16 else torch.uint8, device=dev)
     rt.set_tuning("VPX_GEMM_TILE", tile)
-    rt.set_tuning("VPX_NCE_DIRECT", "off")
+    rt.set_tuning("VPX_NCE_DIRECT", direct)
     rt.set_tuning("VPX_GEMM_REGB", "off")
     try:
         rt.nce_task(*(torch.from_numpy(x).to(dev) for x in (a, b, wt)), out, rt.PpeInt(rt.PPE_LPRELU, lo, hi, 1638, 14), zp_in=zp_in, zp_w=zp_w, zp_out=zp_out)
@@ -77,3 +77,12 @@ def test_large_tiles_fill_the_chip(rt, dev, K, out_f16):
     for large, small in zip(outs[256], outs[128]):
         assert torch.equal(large, small), (K, out_f16, int((large != small).sum()))
         assert large.unique().numel() > 16
+
+
+@pytest.mark.parametrize("M,K,N,kernel", [
+    (4009, 64, 904, "nce_gemm_mfma"), (6294, 128, 424, "nce_gemm_mfma"), (256, 128, 8848, "nce_gemm_mfma"),  # a short K, tiles of 64 x 64 of the other form
+    (294, 384, 5632, "nce_gemm_mfma"), (700, 512, 900, "nce_gemm_mfma"),                                    # 440 and 165 tiles of 64
+    (200, 128, 600, "nce_direct"), (100, 512, 500, "nce_direct"), (4, 4096, 1024, "nce_direct"),
+])
+def test_beside_the_form_that_stages_nothing(rt, orc, dev, M, K, N, kernel):
+    assert run(rt, orc, dev, np.random.default_rng(M + N), M, K, N, None, True, 7, 0, False, direct=None) == kernel
