@@ -234,7 +234,7 @@ VPX_API int vpx_nce_task(const vpx_nce_task_t* task, void* stream);
  * "VPX_GEMM_REGB" (on | wide | off: the weights-in-registers matmul for every K up to 256 that is a multiple of 16, which by
  * itself serves layers of many rows; wide: with as many channel blocks per wave as it otherwise takes from some hundreds of
  * thousands of rows on),
- * "VPX_CONV_STRIPS" (off | 16 | 32: never, or always with tiles of that many output columns, the row-patch convolution with a patch per wave),
+ * "VPX_CONV_STRIPS" (off | 8 | 16 | 32: never, or always with tiles of that many output columns, the row-patch convolution with a patch per wave),
  * "VPX_NCE_DIRECT" (off | tm,tn,waves: never, or always with tiles of 16 tm channels x 16 tn positions and K over that many waves,
  * the form that stages nothing, which by itself serves layers that are over before a tile is staged; 1,1 / 2,1 / 2,2 with one to
  * eight waves, 2,4 / 4,4 with one, others are refused),

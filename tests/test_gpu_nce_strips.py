@@ -12,15 +12,15 @@ LAYERS = [
     dict(N=2, H=30, W=37, IC=16, OC=64, KY=7, KX=7, strides=(2, 2), pads=(3, 3, 3, 3)),
     # more rows under a tile than travel ahead; different strides; K of an odd number of chunks
     dict(N=1, H=41, W=33, IC=16, OC=70, KY=11, KX=3, strides=(2, 1), pads=(1, 0, 5, 4)),
-    # rows of more than 64 chunks; six or three chunks a pixel
-    dict(N=2, H=9, W=40, IC={16: 96, 32: 48}, OC=48, KY=3, KX=3, pads=(1, 1, 1, 1)),
+    # rows of more than 64 chunks (60 under 8 columns); six or three chunks a pixel
+    dict(N=2, H=9, W=40, IC={8: 96, 16: 96, 32: 48}, OC=48, KY=3, KX=3, pads=(1, 1, 1, 1)),
     # more tiles than waves, one and two blocks of channels; walks of unequal length that cross columns and images
     dict(N=23, H=70, W=129, IC=16, OC=48, KY=2, KX=2),
     dict(N=11, H=64, W=130, IC=32, OC=130, KY=1, KX=3, pads=(1, 1, 0, 0)),
 ]
 
 
-@pytest.mark.parametrize("cols", [16, 32])
+@pytest.mark.parametrize("cols", [8, 16, 32])
 @pytest.mark.parametrize("layer", range(len(LAYERS)))
 def test_tiles_and_walks(rt, orc, dev, layer, cols):
     rng = np.random.default_rng(seed("strips", layer, cols))
@@ -46,3 +46,25 @@ def test_short_ppe_and_the_rule(rt, orc, dev, mode, slope):
     rt.nce_task(*(torch.from_numpy(a).to(dev) for a in (inp, w, wt)), out, rt.PpeInt(getattr(rt, "PPE_" + mode), 0, 255, 1638, 14), zp_in=100, zp_out=4, pads=(2, 2, 2, 2))
     assert rt.nce_last_kernel() == "nce_conv_strips"
     assert np.array_equal(out.cpu().numpy(), want)
+
+
+@pytest.mark.parametrize("W", [17, 20, 24, 25, 37, 48])
+def test_narrow_planes(rt, dev, W):
+    """planes that fall into fewer tiles of 8 columns than of 16, and planes that do not, against the row-patch kernel"""
+    import torch
+    N, H, IC, OC = 30, 160, 16, 64
+    gen = torch.Generator().manual_seed(W)
+    inp, w = torch.randint(0, 256, (N, H, W, IC), dtype=torch.uint8, generator=gen).to(dev), torch.randint(-127, 128, (OC, 3, 3, IC), dtype=torch.int8, generator=gen).to(dev)
+    rng = np.random.default_rng(W)
+    wt = torch.from_numpy(rt.make_weights_table(rng.integers(2 ** 14, 2 ** 15, OC), rng.integers(24, 27, OC), rng.integers(-2 ** 15, 2 ** 15, OC).astype(np.int32), 9 * IC)).to(dev)
+    outs = []
+    for knob, kernel in ((None, "nce_conv_strips"), ("off", "nce_conv_rows16")):
+        out = torch.zeros((N, H, W, OC), dtype=torch.uint8, device=dev)
+        rt.set_tuning("VPX_CONV_STRIPS", knob)
+        try:
+            rt.nce_task(inp, w, wt, out, rt.PpeInt(rt.PPE_NOOP, 0, 255), zp_in=100, zp_out=4, pads=(1, 1, 1, 1))
+        finally:
+            rt.set_tuning("VPX_CONV_STRIPS", None)
+        assert rt.nce_last_kernel() == kernel
+        outs.append(out)
+    assert torch.equal(*outs)

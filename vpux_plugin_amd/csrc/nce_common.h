@@ -644,7 +644,7 @@ struct Tuning {
     std::atomic<int> conv_cols{0};          // VPX_CONV_COLS = n: output columns per tile of the row-patch kernel
     std::atomic<int> conv_waves{0};         // VPX_CONV_WAVES = 4 | 8
     std::atomic<int> stream_ksplit{1};      // VPX_STREAM_KSPLIT = off: the streamed-weights kernel never splits K over its waves
-    std::atomic<int> conv_strips{0};        // VPX_CONV_STRIPS = off | 16 | 32: never / with tiles of that many columns the row-patch kernel with a patch per wave (-1, 16, 32; 0: by size)
+    std::atomic<int> conv_strips{0};        // VPX_CONV_STRIPS = off | 8 | 16 | 32: never / with tiles of that many columns the row-patch kernel with a patch per wave (-1, 8, 16, 32; 0: by size)
     std::atomic<int> direct{0};             // VPX_NCE_DIRECT = off | tm,tn,waves: never / always (with that tile) the kernel that stages nothing (-1, tm << 16 | tn << 8 | waves; 0: by size)
     std::atomic<int> mvn_fused{1};          // VPX_MVN_FUSED = off | nowait (see tuning_mvn_fused)
     std::atomic<int> calib_blocks{0};       // VPX_CALIB_BLOCKS = n: workgroups of the MFMA calibration loop (0: one per compute unit)

@@ -3,7 +3,7 @@
 // patches fit LDS together.
 //
 // There the eight waves of a workgroup share one patch and go through load, MFMA loop, PPE and stores in step, two barriers a
-// tile; MFMA loops were half of a stem's time.  Here a wave owns a tile of 64 positions (16 columns x 4 rows, or 32 x 2) with
+// tile; MFMA loops were half of a stem's time.  Here a wave owns a tile of 64 positions (16 columns x 4 rows, 8 x 8, or 32 x 2) with
 // the input rows under it, walks its own run of tiles down a column of tiles and meets nobody after the weights are staged, so
 // that one wave's MFMAs cover the other's PPE, stores and row writes.  The next tile's rows travel in registers while a tile
 // is computed (a row per load: its first byte is a scalar, the lane's offset the same for every row and tile).
