@@ -94,3 +94,33 @@ def test_small_planes_near_the_direct_form_take_no_scratch(rt, dev, zp, kernel):
     finally:
         rt.set_tuning("VPX_NCE_KERNEL", None)
     assert torch.equal(out, ref) and ref.unique().numel() > 16
+
+
+@pytest.mark.parametrize("N,H,W,IC,OC,k,kernel", [
+    (10, 34, 218, 224, 64, 3, "nce_conv_gemm"),    # 580 tiles of 128, a round of two a compute unit and some
+    (4, 121, 150, 288, 48, 4, "nce_conv_gemm"),    # 576, 568 full
+    (27, 43, 137, 288, 64, 3, "nce_direct"),       # 1243, the form that stages nothing on tiles of 64 x 64
+    (3, 122, 260, 112, 16, 5, "nce_conv_rows16"),  # K of 2800 whose weights fit LDS beside their rows
+    (5, 130, 131, 624, 16, 2, "nce_direct"),       # rows that do not
+])
+def test_many_tiles_beside_the_gather_kernels(rt, dev, N, H, W, IC, OC, k, kernel):
+    """channels that are no multiple of 64 and weights that the row kernels have no room for: which of the forms takes them, and that it agrees with the general kernel"""
+    import torch
+    g = torch.Generator(device="cuda").manual_seed(IC + k)
+    x = torch.randint(0, 256, (N, H, W, IC), dtype=torch.uint8, device="cuda", generator=g)
+    w = torch.randint(-127, 128, (OC, k, k, IC), dtype=torch.int8, device="cuda", generator=g)
+    rng = np.random.default_rng(IC + k)
+    K = k * k * IC
+    wt = torch.from_numpy(rt.make_weights_table(rng.integers(2**14, 2**15, OC), rng.integers(30, 32, OC), rng.integers(-2**15, 2**15, OC).astype(np.int32), K)).cuda()
+    shape = (N, H + 2 * (k // 2) - k + 1, W + 2 * (k // 2) - k + 1, OC)
+    out, ref = (torch.empty(shape, dtype=torch.uint8, device="cuda") for _ in range(2))
+    pads = (k // 2,) * 4
+    rt.nce_task(x, w, wt, out, rt.PpeInt(rt.PPE_NOOP, 0, 255), zp_in=5, zp_out=128, pads=pads)
+    took = rt.nce_last_kernel()
+    rt.set_tuning("VPX_NCE_KERNEL", "naive")
+    try:
+        rt.nce_task(x, w, wt, ref, rt.PpeInt(rt.PPE_NOOP, 0, 255), zp_in=5, zp_out=128, pads=pads)
+    finally:
+        rt.set_tuning("VPX_NCE_KERNEL", None)
+    assert torch.equal(out, ref) and ref.unique().numel() > 16
+    assert took == kernel
