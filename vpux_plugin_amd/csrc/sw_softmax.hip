@@ -391,7 +391,8 @@ __global__ __launch_bounds__(KW == 1 ? 256 : 64 * KW) void softmax_slab_f16(cons
     typedef _Float16 hvec __attribute__((ext_vector_type(VEC)));
     typedef hvec hvec_any __attribute__((aligned(2)));
     typedef uint32_t words __attribute__((ext_vector_type(VEC / 2)));  // a lane's VEC columns of a step
-    typedef words words_any __attribute__((aligned(2)));
+    typedef std::conditional_t<(SMAX > 8), words, hvec> held;  // (see h)
+    typedef held held_any __attribute__((aligned(2)));
     typedef float fvec __attribute__((ext_vector_type(VEC)));
     constexpr int SHARES = KW * (64 / CL);
     __shared__ hvec smax[KW == 1 ? 1 : KW][CL];
@@ -412,16 +413,18 @@ __global__ __launch_bounds__(KW == 1 ? 256 : 64 * KW) void softmax_slab_f16(cons
     const half_t* src = in + ioff + col;
     half_t* dst = out + ooff + col;
 
-    words h[SMAX];  // (whole words: halves the compiler took apart between the loads for some SMAX and waited for each, [1,175,169,153] 12.0 us, now 8.5)
-    const auto halves = [](words w) { return __builtin_bit_cast(hvec, w); };
+    // Whole words where there are many: halves the compiler took apart between the loads and waited for each, [1,175,169,153] 12.0 us, now 8.5.
+    // Up to eight it does not, and halves are a little shorter ([4,21,513,513] 16.8 us, words 17.0).
+    held h[SMAX];
+    const auto halves = [](held w) { return __builtin_bit_cast(hvec, w); };
     hvec m;
 #pragma unroll
     for (int k = 0; k < VEC; k++) m[k] = (half_t)-INFINITY;
 #pragma unroll
     for (int i = 0; i < SMAX; i++) {
         const int a = kw + SHARES * i;
-        h[i] = __builtin_bit_cast(words, m);  // -inf
-        if (live && a < L) h[i] = *reinterpret_cast<const words_any*>(src + a * in_as);
+        h[i] = __builtin_bit_cast(held, m);  // -inf
+        if (live && a < L) h[i] = *reinterpret_cast<const held_any*>(src + a * in_as);
     }
     if (VEC > 1 && left > 0 && !live) {
 #pragma unroll
@@ -430,7 +433,7 @@ __global__ __launch_bounds__(KW == 1 ? 256 : 64 * KW) void softmax_slab_f16(cons
 #pragma unroll
             for (int k = 0; k + 1 < VEC; k++)
                 if (k < left && kw + SHARES * i < L) v[k] = src[(kw + SHARES * i) * in_as + k];
-            h[i] = __builtin_bit_cast(words, v);
+            h[i] = __builtin_bit_cast(held, v);
         }
     }
 #pragma unroll
