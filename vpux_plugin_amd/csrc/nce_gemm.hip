@@ -59,7 +59,7 @@ struct GemmLds {
 // every line was read from the second level twice -- with one barrier each.  The 256 tile has LDS for two such panels, and asks
 // for one whenever it has read the last fragment of the one before the last: its panel's MFMAs take 2 048 clocks, and between
 // 192.4 us (panels of 64 bytes, four buffers) and 172.0 at [4096 x 4096] . [4096 x 11008], 497 and 451 at 8192^3, 71.3
-// and 63.8 at 4096^3 lies only the order of its loads.  The smaller tiles' loads stand in line far ahead and nobody
+// and 63.8 at 4096^3 lies only the order of its loads (back to back, the clock settled; beside a dequantize and an add a program sees 243 and 234 in all).  The smaller tiles' loads stand in line far ahead and nobody
 // waits for them; a tile of 128 takes about 850 clocks for a panel whose MFMAs take 512, bound by the LDS (96 KiB of
 // fragments and 32 KiB of loads), one of 64 about 400, bound likewise.  Four waves of 64 x 64 on
 // panels of 64, 24.5 us at [2080 x 3456] . [3456 x 608] whether or not fragments were read a panel ahead or twice the
