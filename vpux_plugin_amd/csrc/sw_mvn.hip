@@ -243,12 +243,11 @@ __global__ __launch_bounds__(kThreads) void mvn_merge_kernel(const Record* parti
     if (threadIdx.x == 0) merged[group] = Record{total.n, total.mean, total.m2, 0.f};
 }
 
-// Many short groups that follow one another in memory (per-channel statistics of small planes, 14 x 14 or 7 x 7; rows
-// of a few hundred values): a workgroup takes a run of whole groups of about kSmallChunk values, moves it between
+// Many short groups that follow one another in memory (per-channel statistics of small planes, 15 x 15 or 7 x 7; rows
+// of a few hundred values): a workgroup takes a run of whole groups of at most kSmallChunk values, moves it between
 // global memory and LDS in aligned 128-bit words whatever the group length (the values of neighbouring groups that
 // share its first and last word are read too, but never written), and half-wavefronts normalise one group each in LDS:
-// sum, centred sum of squares, scale -- three passes over at most kSmallGroup values.
-constexpr int kSmallGroup = 1024;   // longest group this form takes
+// sum, centred sum of squares, scale -- three passes over at most 512 values.
 constexpr int kSmallChunk = 4096;   // values per workgroup, at most
 __device__ __forceinline__ float half_wave_sum(float v) {
     v += dppf<0xB1>(v);
@@ -447,20 +446,30 @@ static int launch_tiny_groups(const half_t* in, half_t* out, int64_t groups, int
     return VPX_RESULT_SUCCESS;
 }
 
-// Whether the short-group form applies, and its launch.
+// Groups a workgroup takes: what its eight half-wavefronts walk one after another.  As many as fill kSmallChunk, 37 of 110 values, left a small
+// tensor to a few workgroups with a long walk each and a large one waiting for it too (us, that many / these): [512 x 7] 24.6 / 3.3,
+// [16384 x 21] 12.9 / 4.4, [65536 x 110] 12.1 / 9.6, [65536 x 361] 22.8 / 19.7, [131072 x 49] 16.5 / 12.6.
+static int small_groups_run(int64_t groups, int64_t len) {
+    const int64_t fits = kSmallChunk / len, most = len <= 64 ? (groups < 16384 ? 8 : 32) : len > 128 ? 8 : groups < (1 << 18) ? 16 : fits;
+    return (int)(fits < most ? fits : most);
+}
+// Whether the short-group form applies, and its launch.  It serves what the registers of mvn6_rows_kernel do not, groups of fewer than eight
+// values, and many groups of up to 512 that are no whole number of words: a row of those leaves most of a team's lanes idle or ends in a word that
+// two lanes take.  us in a HIP graph, that kernel / this one: [448 x 110] 3.2 / 3.3, [1024 x 390] 3.3 / 4.2, [8192 x 361] 5.85 / 5.83,
+// [65536 x 110] 12.3 / 9.6, [131072 x 390] 25.6 / 20.6 a half of them, [131072 x 49] 20.0 / 12.6; but [16384 x 675] 11.6 / 13.7, [16384 x 784] 10.1 / 14.2.
 static bool small_groups_ok(const half_t* in, const half_t* out, int64_t groups, int64_t len) {
-    return len >= 1 && len <= kSmallGroup && groups >= 64 && ((reinterpret_cast<uintptr_t>(in) | reinterpret_cast<uintptr_t>(out)) & 15) == 0 &&
-           (groups + (kSmallChunk / len) - 1) / (kSmallChunk / len) < (1ll << 31);
+    const int64_t run = len >= 1 ? small_groups_run(groups, len) : 1;
+    return len >= 1 && groups >= 64 && (len < 8 || (groups > 8192 && len <= 512 && len % 8 != 0)) &&
+           ((reinterpret_cast<uintptr_t>(in) | reinterpret_cast<uintptr_t>(out)) & 15) == 0 && (groups + run - 1) / run < (1ll << 31);
 }
 static int launch_small_groups(const half_t* in, half_t* out, int64_t groups, int64_t len, int nv, int eps_mode, float eps, hipStream_t s) {
-    const int per_wg = (int)(kSmallChunk / len);
+    const int per_wg = small_groups_run(groups, len);
     const unsigned blocks = (unsigned)((groups + per_wg - 1) / per_wg);
 #define VPX_SMALL(K) hipLaunchKernelGGL(mvn_small_groups_kernel<K>, dim3(blocks), dim3(kThreads), 0, s, in, out, groups, (int)len, per_wg, nv, eps_mode, eps)
     if (len <= 64) VPX_SMALL(2);
     else if (len <= 128) VPX_SMALL(4);
     else if (len <= 256) VPX_SMALL(8);
-    else if (len <= 512) VPX_SMALL(16);
-    else VPX_SMALL(32);
+    else VPX_SMALL(16);
 #undef VPX_SMALL
     VPX_HIP_CHECK(hipGetLastError());
     return VPX_RESULT_SUCCESS;
@@ -1195,10 +1204,16 @@ __device__ __forceinline__ float team_sum(float v, float* smem) {
     }
     v = wave_sum(v);
     if (TEAM == 64) return v;
-    // one barrier: each sum of a workgroup's lifetime has four slots of its own
+    // one barrier: each sum of a workgroup's lifetime has slots of its own
     if ((threadIdx.x & 63) == 0) smem[threadIdx.x >> 6] = v;
     __syncthreads();
-    return (smem[0] + smem[1]) + (smem[2] + smem[3]);
+    if (TEAM == 256) return (smem[0] + smem[1]) + (smem[2] + smem[3]);
+    constexpr int WAVES = TEAM / 64;  // 8 or 16, one per lane of a row of 16
+    v = smem[threadIdx.x & (WAVES - 1)];
+    v += dppf<0xB1>(v);
+    v += dppf<0x4E>(v);
+    v += dppf<0x141>(v);
+    return WAVES == 16 ? v + dppf<0x140>(v) : v;
 }
 
 // Rows that are contiguous in memory: the row lives in the registers of half a wavefront (TEAM = 32, eight rows per
@@ -1221,20 +1236,22 @@ __device__ __forceinline__ int row_again(uint32_t e0, uint32_t row_len) {
     return WORDS ? 0 : e0 >= row_len ? 8 : (int)(e0 - row_at(e0, row_len));
 }
 constexpr int kMvn6MaxRegRow = 16384;  // longest row a workgroup keeps in registers (64 values per lane)
+constexpr int team_threads(int team) { return team > kThreads ? team : kThreads; }
 template <int TEAM, int VPT, int RPT = 1, bool WORDS = true>  // RPT: consecutive rows a team walks, keeping a scale / bias that runs along the row in registers
-__global__ __launch_bounds__(kThreads) void mvn6_rows_kernel(const half_t* __restrict__ in, half_t* __restrict__ out,
+__global__ __launch_bounds__(team_threads(TEAM)) void mvn6_rows_kernel(const half_t* __restrict__ in, half_t* __restrict__ out,
                                                              const half_t* __restrict__ sc, const half_t* __restrict__ bi,
                                                              Mvn6Geom g, int normalize_variance, int eps_mode, float eps) {
-    __shared__ float red[8];
-    static_assert(TEAM != 256 || RPT == 1, "the workgroup-wide sums have slots for one row");
+    constexpr int T = team_threads(TEAM);
+    __shared__ float red[32];
+    static_assert(TEAM < 256 || RPT == 1, "the workgroup-wide sums have slots for one row");
     const int t = (int)(threadIdx.x % TEAM);
-    const int64_t row0 = ((int64_t)blockIdx.x * (kThreads / TEAM) + threadIdx.x / TEAM) * RPT;
+    const int64_t row0 = ((int64_t)blockIdx.x * (T / TEAM) + threadIdx.x / TEAM) * RPT;
     // The words of a row are asked for all at once (but see AHEAD), and before they are used the scale and the bias that run along it: asked for
     // where they are needed, behind both sums, they cost a trip to the caches per row ([16384 x 4096] 56.7 -> 51.9 us, [16384 x
     // 1024] 17.1 -> 15.9, [1 x 4096] 3.2 -> 2.7).  They stay late where nothing is gained, of one word per lane of a workgroup or
     // of half a wavefront, and where their registers cost a wavefront per SIMD, from three words of half a wavefront or four of
     // one on ([16384 x 768] 11.2 us late, 13.1 early, [8192 x 2048] 14.2 and 17.2).
-    constexpr bool EARLY = RPT > 1 || (TEAM == 64 ? VPT <= 3 : VPT == 2);
+    constexpr bool EARLY = RPT > 1 || (TEAM == 64 ? VPT <= 3 : TEAM == 512 ? VPT <= 2 : VPT == 2);
     // Three to five words per lane of a workgroup are converted each as it comes: all asked for first they gain from memory
     // ([800 x 6480] 7.83 -> 6.98 us) what they lose from the cache that the writer of the rows left them in ([1280 x 4324] 8.51 ->
     // 8.76 us, [800 x 8100] 9.12 -> 9.57); from six on there is a gain in both ([512 x 12544] 9.53 -> 7.45 and 8.01 -> 7.70).
@@ -1303,7 +1320,7 @@ __global__ __launch_bounds__(kThreads) void mvn6_rows_kernel(const half_t* __res
             q += (WORDS ? e0 < g.row_len : k >= again) ? d * d : 0.f;
         }
     }
-    const float var = team_sum<TEAM>(q, red + 4) / n;
+    const float var = team_sum<TEAM>(q, red + 16) / n;
     const float inv = mvn6_inv(var, normalize_variance, eps_mode, eps);
     const float sc_row = sc && !g.sc_along_row ? (float)sc[here.sc] : 1.0f;
     const float bi_row = bi && !g.bi_along_row ? (float)bi[here.bi] : 0.0f;
@@ -1467,12 +1484,13 @@ int launch_rows(const half_t* pi, half_t* po, const half_t* ps, const half_t* pb
     const int rpt = !shared_rows ? 1 : team_rows >= 4 * 4096 ? 4 : team_rows >= 2 * 4096 ? 2 : 1;
 #define VPX_MVN6_ROWS_R(TEAM, VPT, RPT)                                                                                      \
     do {                                                                                                                     \
-        const dim3 grid((unsigned)((g.rows + RPT * kThreads / TEAM - 1) / (RPT * kThreads / TEAM)));                         \
+        constexpr int T = team_threads(TEAM), PER = RPT * (T / TEAM);                                                        \
+        const dim3 grid((unsigned)((g.rows + PER - 1) / PER));                                                               \
         if (words)                                                                                                           \
-            hipLaunchKernelGGL((mvn6_rows_kernel<TEAM, VPT, RPT, true>), grid, dim3(kThreads), 0, s, pi, po, ps, pb, g, nv,  \
+            hipLaunchKernelGGL((mvn6_rows_kernel<TEAM, VPT, RPT, true>), grid, dim3(T), 0, s, pi, po, ps, pb, g, nv,         \
                                eps_mode, eps);                                                                               \
         else                                                                                                                 \
-            hipLaunchKernelGGL((mvn6_rows_kernel<TEAM, VPT, RPT, false>), grid, dim3(kThreads), 0, s, pi, po, ps, pb, g, nv, \
+            hipLaunchKernelGGL((mvn6_rows_kernel<TEAM, VPT, RPT, false>), grid, dim3(T), 0, s, pi, po, ps, pb, g, nv,        \
                                eps_mode, eps);                                                                               \
     } while (0)
 #define VPX_MVN6_ROWS(TEAM, VPT) VPX_MVN6_ROWS_R(TEAM, VPT, 1)
@@ -1486,7 +1504,19 @@ int launch_rows(const half_t* pi, half_t* po, const half_t* ps, const half_t* pb
     // place of up to six one after another ([1024 x 2752] 7.5 -> 5.0 us, [2048 x 2304] 7.9 -> 6.4, [64 x 1280] 4.4 -> 3.3;
     // with twice the rows the wavefront form is ahead again, 6.7 against 7.6 us for [4096 x 1280]).
     const bool few = row_len > 640 && g.rows <= (row_len > 1024 ? 2048 : 1024);
-    if (few && row_len <= 2048) VPX_MVN6_ROWS(256, 1);
+    // A row or less per compute unit: 512 lanes take it, at most half as many words each ([128 x 8640] 4.53 -> 4.03 us in a HIP graph, [9 x
+    // 9216] 4.33 -> 3.79; with scale and bias [16 x 2050] 3.88 -> 3.59, [256 x 3136] 3.94 -> 3.79, [1 x 1088] 3.20 -> 3.11; of up to 2048 values without them
+    // nothing is gained, [128 x 1200] 3.47 / 3.52).  With two rows a unit it is even ([512 x 4096] 3.97 / 4.01), with four slower ([1024 x 4096] 4.73 / 5.20);
+    // 1024 lanes are behind 512 but for [512 x 16384] (8.17 / 7.80, 1024 rows 11.7 / 12.9).
+    int cus = 0;
+    const int rc = device_compute_units(&cus);
+    if (rc) return rc;
+    const bool wide = g.rows <= cus && row_len > (ps || pb ? 640 : 2048);
+    if (wide && row_len <= 4096) VPX_MVN6_ROWS(512, 1);
+    else if (wide && row_len <= 8192) VPX_MVN6_ROWS(512, 2);
+    else if (wide && row_len <= 12288) VPX_MVN6_ROWS(512, 3);
+    else if (wide) VPX_MVN6_ROWS(512, 4);
+    else if (few && row_len <= 2048) VPX_MVN6_ROWS(256, 1);
     else if (few && row_len <= 4096) VPX_MVN6_ROWS(256, 2);
     else if (row_len <= 256) VPX_MVN6_SHORT(32, 1);
     else if (row_len <= 512) VPX_MVN6_SHORT(64, 1);
