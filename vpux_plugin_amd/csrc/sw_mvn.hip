@@ -16,6 +16,7 @@
 // left -- more or longer groups, input and output in one place -- takes two launches over 4096-element chunks, the second
 // of which reads the tensor again.
 #include <atomic>
+#include <type_traits>
 
 #include "vpx_common.h"
 
@@ -77,6 +78,30 @@ __device__ __forceinline__ float wave_sum(float v) {
     v += dppf<0x140>(v);
     v += swz16(v);
     return lane_bcast(v, 0) + lane_bcast(v, 32);
+}
+// The same bits with a lane of each row of 16 read instead of the trip through LDS: shorter where a workgroup waits for its sum ([3,144,82,56] across
+// channels 6.93 -> 6.54 us, layer norm [25 x 3008] 3.74 -> 3.54), more vector instructions where many wavefronts hide the trip ([6052 x 576] 6.10 -> 6.37).
+__device__ __forceinline__ float wave_sum_soon(float v) {
+    v += dppf<0xB1>(v);
+    v += dppf<0x4E>(v);
+    v += dppf<0x141>(v);
+    v += dppf<0x140>(v);
+    return (lane_bcast(v, 0) + lane_bcast(v, 16)) + (lane_bcast(v, 32) + lane_bcast(v, 48));
+}
+
+// a / n where 1 / n, correctly rounded, was at hand before a was: two fused operations behind the product in place of the dozen of a division, whose
+// result this is.  An infinite a stays infinite.
+__device__ __forceinline__ float over(float a, float n, float inv_n) {
+    const float q = a * inv_n;
+    return __builtin_fabsf(q) < __builtin_inff() ? __builtin_fmaf(__builtin_fmaf(-q, n, a), inv_n, q) : q;
+}
+
+// 1 / sqrt(v): the hardware's approximation and one Newton step, within an ulp as a rounded root and a rounded quotient are, in a fifth of their
+// instructions.  Outside the normal numbers those.
+__device__ __forceinline__ float inv_root(float v) {
+    if (!(v >= 0x1p-126f && v < __builtin_inff())) return 1.0f / __builtin_sqrtf(v);
+    const float y = __builtin_amdgcn_rsqf(v);
+    return __builtin_fmaf(0.5f * y, __builtin_fmaf(-v * y, y, 1.0f), y);
 }
 
 template <class Shuffle>
@@ -488,8 +513,8 @@ int mem_pos_of(uint64_t order, int nd, int logical) {
 // stores; the first wavefront then polls the records of ITS group (not of the whole grid) with loads that bypass the
 // caches until every tag names this launch, merges them in a fixed order and hands the result to the other wavefronts,
 // which normalise the slice from the registers.  No read-modify-write is involved: arrivals do not queue at a counter.
-// The tag is the launch count + 1.  Every workgroup has counts of its own in the zero-initialised sync area (a run of the
-// group's kMergeInKernel, all of which a launch moves on, however many workgroups it has): nobody else writes them during a
+// The tag is the launch count + 1.  Every workgroup has counts of its own in the zero-initialised sync area (the group's kMergeInKernel
+// are dealt out in turn, and a launch moves all of them on, however many workgroups it has): nobody else writes them during a
 // launch, so a workgroup finds the launch's tag however late it starts, and no record of an earlier launch carries it.
 // The wait is bounded: a workgroup that does not see its group complete in time (the others are not resident: the device is
 // shared) computes missing slices with the same arithmetic and publishes them for their owners and for everyone else, one
@@ -497,6 +522,9 @@ int mem_pos_of(uint64_t order, int nd, int logical) {
 // about once among those that wait, whoever starts later finds the group complete, and every wave exits: a workgroup
 // computes a slice at most once.  (Each computing all slices for itself took 29 ms for 52 M values beside a launch that held
 // 224 of 256 compute units, eight rounds of workgroups that wait and read the tensor 32 times; now 0.9: the wait, 0.1 for the missing slices, eight rounds.)
+// What bounds a small tensor is the chain of trips to memory: arguments, slice, tag, publication, the others' records; in between nothing waits for a
+// division by a count that was known before, and moments meet all at once.  us in a HIP graph, with the tag in front of the slice, records
+// polled a round of 64 at a time and pairwise merges / now: [1,128,57,73] 7.1 / 5.6, [4,256,64,64] 6.5 / 5.9, [16,16,142,176] 6.6 / 6.0.
 constexpr int kFusedMaxVec = 52;           // 128-bit words per lane of 512, 208 of its 256 registers: the chip holds 54 M values
 constexpr int kSyncStride = 4;             // words between launch counts
 // kFusedMaxGroups groups at most: each owns a fixed run of kMergeInKernel launch counts and as many record slots
@@ -520,6 +548,7 @@ struct Slice {
     int have;    // words of this lane
     float last;  // its value of the partial word
     bool has_last;
+    float wave_count, count;  // values of the wavefront, of the slice
 };
 
 template <int V, int T>
@@ -538,6 +567,9 @@ __device__ __forceinline__ void load_slice(const half_t* __restrict__ g, uint32_
     const uint32_t rest = base + words * 8 + threadIdx.x;
     sl.has_last = rest < end && threadIdx.x < 8;
     sl.last = sl.has_last ? (float)g[rest] : 0.f;
+    const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)), more = (int)(words % T) - 64 * wave;
+    sl.count = (float)(end - base);
+    sl.wave_count = (float)(8 * (64 * (int)(words / T) + (more < 0 ? 0 : more < 64 ? more : 64)) + (wave == 0 ? (int)(end - base - words * 8) : 0));
 }
 
 // The eight values of a word in single precision (the conversion is exact).  KEEP: both passes of the moments and the
@@ -564,8 +596,8 @@ __device__ __forceinline__ Moments slice_moments(Slice<V>& sl, Moments* red) {
         for (int k = 0; k < 8; k++) sum += f[k];
         if (!KEEP) asm volatile("" : "+v"(sum));
     }
-    const float n = wave_sum((float)(8 * sl.have + (sl.has_last ? 1 : 0)));
-    const float mean = n > 0.f ? wave_sum(sum) / n : 0.f;
+    const float n = sl.wave_count, inv_n = 1.f / n;  // (of loads that are still on their way)
+    const float mean = n > 0.f ? over(wave_sum_soon(sum), n, inv_n) : 0.f;
     float q = sl.has_last ? (sl.last - mean) * (sl.last - mean) : 0.f;
 #pragma unroll
     for (int j = 0; j < V; j++) {
@@ -579,13 +611,25 @@ __device__ __forceinline__ Moments slice_moments(Slice<V>& sl, Moments* red) {
         q += j < sl.have ? qj : 0.f;
         if (!KEEP) asm volatile("" : "+v"(q));
     }
-    q = wave_sum(q);
+    q = wave_sum_soon(q);
     __syncthreads();  // the previous use of `red` is over
     if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = Moments{n, mean, q};
     __syncthreads();
-    Moments m = merge(merge(red[0], red[1]), merge(red[2], red[3]));
-    if (T == 512) m = merge(m, merge(merge(red[4], red[5]), merge(red[6], red[7])));
-    return m;
+    // all at once, about the first one's mean: a tree of pairwise merges is three reciprocals in a row
+    Moments w[T / 64];
+#pragma unroll
+    for (int k = 0; k < T / 64; k++) w[k] = red[k];
+    const float count = sl.count, inv_count = 1.f / count;
+    float shift = 0.f, m2 = 0.f;
+#pragma unroll
+    for (int k = 0; k < T / 64; k++) shift += w[k].n * (w[k].mean - w[0].mean);
+    shift = over(shift, count, inv_count);
+#pragma unroll
+    for (int k = 0; k < T / 64; k++) {
+        const float d = (w[k].mean - w[0].mean) - shift;
+        m2 += w[k].m2 + w[k].n * d * d;
+    }
+    return Moments{count, w[0].mean + shift, m2};
 }
 
 template <int V, int T>
@@ -596,25 +640,26 @@ __global__ __launch_bounds__(T) void mvn_fused_kernel(const half_t* __restrict__
     __shared__ Moments shared_total;
     __shared__ int complete, pick;
     __shared__ unsigned char helped[kMergeInKernel];
-    const int64_t group = blockIdx.x / wpg;
-    const int part = blockIdx.x % wpg;
+    const int64_t group = blockIdx.y;
+    const int part = (int)blockIdx.x;
     const int lane = threadIdx.x & 63;
-    // this workgroup's launch counts
+    // this workgroup's launch counts: every wpg-th of the group's, from its own place on
     unsigned* counts = sync + group * (kMergeInKernel * kSyncStride);
-    const int first_count = part * kMergeInKernel / wpg, end_count = (part + 1) * kMergeInKernel / wpg;
     Tagged* records = reinterpret_cast<Tagged*>(reinterpret_cast<char*>(sync) + kSyncRecords) + group * kMergeInKernel;
-    unsigned tag = 0;
-    if (wpg > 1 && threadIdx.x < 64) {
-        tag = __hip_atomic_load(counts + first_count * kSyncStride, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) + 1u;
-        tag = tag == 0u ? 1u : tag;
-    }
     const half_t* gin = in + group * group_size;
     const uint32_t base = (uint32_t)part * slice;
     const uint32_t end = part + 1 < wpg ? base + slice : group_size;
     Slice<V> sl;
     load_slice<V, T>(gin, base, end, group_size, sl);
+    // The launch's tag, asked for behind the slice: loads return in order, and this one goes through to memory.  (In front of them, in a branch that
+    // works with it at once or moved to a scalar register as uniform, every launch paid its way, 0.6 of 6.7 us at [3,48,76,60].)
+    int here = 0;
+    asm("" : "+v"(here));
+    const unsigned counted = __hip_atomic_load(counts + part * kSyncStride + here, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    const float group_count = (float)group_size, inv_count = 1.f / group_count;
     Moments total = slice_moments<V, T>(sl, red);
     if (wpg > 1) {
+        const unsigned tag = counted + 1u == 0u ? 1u : counted + 1u;
         const auto publish = [&](int p, const Moments& m) {  // by one lane of the first wavefront
             __hip_atomic_store(&records[p].mean, tagged(m.mean, tag), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
             __hip_atomic_store(&records[p].m2, tagged(m.m2, tag), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -631,33 +676,50 @@ __global__ __launch_bounds__(T) void mvn_fused_kernel(const half_t* __restrict__
         const auto collect = [&](bool waits) {  // the first wavefront: reads the group's records and merges them
             const unsigned long long t0 = wall_clock64();
             bool ok;
-            for (;;) {
+            // (records asked for together, places past the last one reading that again: a branch around each round waits for it)
+            const auto poll_rounds = [&](auto rounds_c) {
+                constexpr int ROUNDS = decltype(rounds_c)::value;
+#pragma unroll
+                for (int k = 0; k < ROUNDS; k++) {
+                    const Tagged* r = &records[k * 64 + lane < wpg ? k * 64 + lane : wpg - 1];
+                    rm[k] = __hip_atomic_load(&r->mean, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                    rq[k] = __hip_atomic_load(&r->m2, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                }
                 bool ready = true;
 #pragma unroll
-                for (int k = 0; k < kMergeInKernel / 64; k++) ready &= poll(k);
-                ok = __builtin_amdgcn_ballot_w64(!ready) == 0;
+                for (int k = 0; k < ROUNDS; k++) ready &= (unsigned)(rm[k] >> 32) == tag && (unsigned)(rq[k] >> 32) == tag;
+                return __builtin_amdgcn_ballot_w64(!ready) == 0;
+            };
+            constexpr int kRounds = kMergeInKernel / 64;
+            for (;;) {
+                if (wpg <= 64) ok = poll_rounds(std::integral_constant<int, 1>{});
+                else if (wpg <= 128) ok = poll_rounds(std::integral_constant<int, 2>{});
+                else ok = poll_rounds(std::integral_constant<int, kRounds>{});
                 if (ok || !waits || wall_clock64() - t0 >= spin_ticks) break;  // (pausing between polls measured slower)
             }
             if (ok || !waits) {
-                Moments acc{0.f, 0.f, 0.f};
+                // all at once, about the first slice's mean, in a fixed order (a butterfly of pairwise merges: six reciprocals in a row)
+                const float first = lane_bcast(__builtin_bit_cast(float, (unsigned)rm[0]), 0);
+                float shift = 0.f, m2 = 0.f;
+                const auto count = [&](int i) { return i >= wpg ? 0.f : i + 1 < wpg ? (float)slice : (float)(group_size - (uint32_t)i * slice); };
+                const auto off = [&](int k) { return k * 64 + lane < wpg ? __builtin_bit_cast(float, (unsigned)rm[k]) - first : 0.f; };
+#pragma unroll
+                for (int k = 0; k < kMergeInKernel / 64; k++) shift += count(k * 64 + lane) * off(k);
+                shift = over(wave_sum_soon(shift), group_count, inv_count);
 #pragma unroll
                 for (int k = 0; k < kMergeInKernel / 64; k++) {
-                    const int i = k * 64 + lane;
-                    if (i < wpg) {
-                        const uint32_t b = (uint32_t)i * slice;
-                        const uint32_t cnt = i + 1 < wpg ? slice : group_size - b;
-                        acc = merge(acc, Moments{(float)cnt, __builtin_bit_cast(float, (unsigned)rm[k]), __builtin_bit_cast(float, (unsigned)rq[k])});
-                    }
+                    const float d = off(k) - shift;
+                    m2 += k * 64 + lane < wpg ? __builtin_bit_cast(float, (unsigned)rq[k]) + count(k * 64 + lane) * d * d : 0.f;
                 }
-                const Moments t = wave_merge(acc);
-                if (lane == 0) shared_total = t;
+                m2 = wave_sum_soon(m2);
+                if (lane == 0) shared_total = Moments{group_count, first + shift, m2};
             }
             return ok;
         };
         if (threadIdx.x < 64) {
             if (lane == 0) publish(part, total);
             // (here and not behind the meeting: their way to memory then ends under the wait, 0.2 of 8.3 us at [4,256,64,64])
-            for (int i = first_count + lane; i < end_count; i += 64)
+            for (int i = part + lane * wpg; i < kMergeInKernel; i += 64 * wpg)
                 __hip_atomic_store(counts + i * kSyncStride, tag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
             const bool ok = collect(true);
             if (lane == 0) complete = ok ? 1 : 0;
@@ -708,7 +770,7 @@ __global__ __launch_bounds__(T) void mvn_fused_kernel(const half_t* __restrict__
         }
         total = shared_total;
     }
-    const float mean = total.mean, inv = inv_std(total, normalize_variance, eps);
+    const float mean = total.mean, inv = normalize_variance ? inv_root(over(total.m2, group_count, inv_count) + eps) : 1.0f;
     half_t* gout = out + group * group_size;
     uint32_t at = base + threadIdx.x * 8;
 #pragma unroll
@@ -758,7 +820,7 @@ int launch_fused_groups(const half_t* in, half_t* out, int64_t groups, int64_t g
     rc = get_sync_area(s, &sync);
     if (rc) return rc;
     const unsigned long long spin = mode == 2 ? 0ull : 50000ull;  // 0.5 ms of the 100 MHz counter
-    const dim3 grid((unsigned)(groups * wpg));
+    const dim3 grid((unsigned)wpg, (unsigned)groups);
 #define VPX_FUSED(V, T)                                                                                                        \
     hipLaunchKernelGGL((mvn_fused_kernel<V, T>), grid, dim3(T), 0, s, in, out, (uint32_t)group_size, (int)wpg, (uint32_t)slice, \
                        (unsigned*)sync, nv, eps, spin)
@@ -1187,9 +1249,21 @@ __device__ __forceinline__ RowBase row_base(const Mvn6Geom& g, int64_t row) {
     return b;
 }
 
+// The same with at most one kept dimension: what a launch says fits two lines of its argument block, read at once.  (Mvn6Geom's eleven lines are read
+// one after another as the walk over its dimensions comes to them, each a trip to memory in front of the first row.)
+struct FlatGeom {
+    int64_t in, out, sc, bi;  // from row to row
+    int64_t rows;
+    uint32_t row_len;
+    int sc_along_row, bi_along_row;
+};
+__device__ __forceinline__ RowBase row_base(const FlatGeom& g, int64_t row) {
+    return RowBase{row * g.in, row * g.out, row * g.sc, row * g.bi};
+}
+
 __device__ __forceinline__ float mvn6_inv(float var, int normalize_variance, int eps_mode, float eps) {
     if (!normalize_variance) return 1.0f;
-    return eps_mode == 0 ? 1.0f / __builtin_sqrtf(var + eps) : 1.0f / (__builtin_sqrtf(var) + eps);
+    return eps_mode == 0 ? inv_root(var + eps) : 1.0f / (__builtin_sqrtf(var) + eps);
 }
 
 // Sum over the TEAM lanes that share a row: half a wavefront, a wavefront, or the whole workgroup.
@@ -1202,8 +1276,8 @@ __device__ __forceinline__ float team_sum(float v, float* smem) {
         v += dppf<0x140>(v);
         return v + swz16(v);
     }
-    v = wave_sum(v);
-    if (TEAM == 64) return v;
+    if (TEAM == 64) return wave_sum(v);
+    v = wave_sum_soon(v);
     // one barrier: each sum of a workgroup's lifetime has slots of its own
     if ((threadIdx.x & 63) == 0) smem[threadIdx.x >> 6] = v;
     __syncthreads();
@@ -1237,10 +1311,15 @@ __device__ __forceinline__ int row_again(uint32_t e0, uint32_t row_len) {
 }
 constexpr int kMvn6MaxRegRow = 16384;  // longest row a workgroup keeps in registers (64 values per lane)
 constexpr int team_threads(int team) { return team > kThreads ? team : kThreads; }
-template <int TEAM, int VPT, int RPT = 1, bool WORDS = true>  // RPT: consecutive rows a team walks, keeping a scale / bias that runs along the row in registers
-__global__ __launch_bounds__(team_threads(TEAM)) void mvn6_rows_kernel(const half_t* __restrict__ in, half_t* __restrict__ out,
+// Wavefronts a SIMD that the registers are cut for: the words and their values, with RPT > 1 a scale and a bias beside them.  (Left to itself the compiler
+// takes 250 registers for eight words: [3808 x 10640] 45 us in place of 35.)
+constexpr int row_waves(int vpt, int rpt) {
+    return rpt > 1 ? (vpt == 1 ? 8 : vpt == 2 ? 5 : vpt == 3 ? 4 : vpt == 4 ? 3 : 2) : vpt <= 2 ? 8 : vpt <= 4 ? 7 : vpt == 5 ? 6 : vpt == 6 ? 5 : 4;
+}
+template <class GEOM, int TEAM, int VPT, int RPT = 1, bool WORDS = true>  // RPT: consecutive rows a team walks, keeping a scale / bias that runs along the row in registers
+__global__ __launch_bounds__(team_threads(TEAM)) __attribute__((amdgpu_waves_per_eu(row_waves(VPT, RPT)))) void mvn6_rows_kernel(const half_t* __restrict__ in, half_t* __restrict__ out,
                                                              const half_t* __restrict__ sc, const half_t* __restrict__ bi,
-                                                             Mvn6Geom g, int normalize_variance, int eps_mode, float eps) {
+                                                             GEOM g, int normalize_variance, int eps_mode, float eps) {
     constexpr int T = team_threads(TEAM);
     __shared__ float red[32];
     static_assert(TEAM < 256 || RPT == 1, "the workgroup-wide sums have slots for one row");
@@ -1279,6 +1358,7 @@ __global__ __launch_bounds__(team_threads(TEAM)) void mvn6_rows_kernel(const hal
             }
         }
     }
+    const float n = (float)g.row_len, inv_n = 1.0f / n;  // (under the loads)
 #pragma unroll 1
     for (int rr = 0; rr < RPT; rr++) {
     float x[VPT][8];
@@ -1307,8 +1387,7 @@ __global__ __launch_bounds__(team_threads(TEAM)) void mvn6_rows_kernel(const hal
         b = row_base(g, live ? row0 + rr + 1 : 0);
         fetch(b, live, words);
     }
-    const float n = (float)g.row_len;
-    const float mean = team_sum<TEAM>(sum, red) / n;
+    const float mean = over(team_sum<TEAM>(sum, red), n, inv_n);
     float q = 0.f;
 #pragma unroll
     for (int j = 0; j < VPT; j++) {
@@ -1320,7 +1399,7 @@ __global__ __launch_bounds__(team_threads(TEAM)) void mvn6_rows_kernel(const hal
             q += (WORDS ? e0 < g.row_len : k >= again) ? d * d : 0.f;
         }
     }
-    const float var = team_sum<TEAM>(q, red + 16) / n;
+    const float var = over(team_sum<TEAM>(q, red + 16), n, inv_n);
     const float inv = mvn6_inv(var, normalize_variance, eps_mode, eps);
     const float sc_row = sc && !g.sc_along_row ? (float)sc[here.sc] : 1.0f;
     const float bi_row = bi && !g.bi_along_row ? (float)bi[here.bi] : 0.0f;
@@ -1470,14 +1549,10 @@ __global__ __launch_bounds__(kThreads) void mvn6_generic_kernel(const half_t* __
 
 
 // Contiguous rows of 8 ... kMvn6MaxRegRow values (see mvn6_rows_kernel); words: the rows are whole, aligned 128-bit words.
-int launch_rows(const half_t* pi, half_t* po, const half_t* ps, const half_t* pb, const Mvn6Geom& g, bool words, int nv, int eps_mode,
-                float eps, hipStream_t s) {
+template <class GEOM>
+int launch_rows_of(const half_t* pi, half_t* po, const half_t* ps, const half_t* pb, const GEOM& g, bool shared_rows, bool words, int nv, int eps_mode,
+                   float eps, hipStream_t s) {
     const int64_t row_len = g.row_len;
-    // A scale / bias shared by all rows stays in registers while a team walks 2 or 4 consecutive rows, as long
-    // as that leaves 4096 workgroups (two rounds of the chip) or more.
-    bool shared_rows = (ps && g.sc_along_row) || (pb && g.bi_along_row);
-    for (int d = 0; d < g.nk; d++)
-        if ((ps && g.sc_along_row && g.k_sc[d] != 0) || (pb && g.bi_along_row && g.k_bi[d] != 0)) shared_rows = false;
     const bool half768 = shared_rows && row_len == 768;  // 32 lanes x 3 words, none idle: pays with scale / bias
     const int team = row_len <= 256 || half768 ? 32 : 64;
     const int64_t team_rows = g.rows / (kThreads / team);
@@ -1487,10 +1562,10 @@ int launch_rows(const half_t* pi, half_t* po, const half_t* ps, const half_t* pb
         constexpr int T = team_threads(TEAM), PER = RPT * (T / TEAM);                                                        \
         const dim3 grid((unsigned)((g.rows + PER - 1) / PER));                                                               \
         if (words)                                                                                                           \
-            hipLaunchKernelGGL((mvn6_rows_kernel<TEAM, VPT, RPT, true>), grid, dim3(T), 0, s, pi, po, ps, pb, g, nv,         \
+            hipLaunchKernelGGL((mvn6_rows_kernel<GEOM, TEAM, VPT, RPT, true>), grid, dim3(T), 0, s, pi, po, ps, pb, g, nv,         \
                                eps_mode, eps);                                                                               \
         else                                                                                                                 \
-            hipLaunchKernelGGL((mvn6_rows_kernel<TEAM, VPT, RPT, false>), grid, dim3(T), 0, s, pi, po, ps, pb, g, nv,        \
+            hipLaunchKernelGGL((mvn6_rows_kernel<GEOM, TEAM, VPT, RPT, false>), grid, dim3(T), 0, s, pi, po, ps, pb, g, nv,        \
                                eps_mode, eps);                                                                               \
     } while (0)
 #define VPX_MVN6_ROWS(TEAM, VPT) VPX_MVN6_ROWS_R(TEAM, VPT, 1)
@@ -1540,18 +1615,33 @@ int launch_rows(const half_t* pi, half_t* po, const half_t* ps, const half_t* pb
     return VPX_RESULT_SUCCESS;
 }
 
+// rows of a tensor with any kept dimensions
+int launch_rows(const half_t* pi, half_t* po, const half_t* ps, const half_t* pb, const Mvn6Geom& g, bool words, int nv, int eps_mode,
+                float eps, hipStream_t s) {
+    // A scale / bias shared by all rows stays in registers while a team walks 2 or 4 consecutive rows, as long
+    // as that leaves 4096 workgroups (two rounds of the chip) or more.
+    bool shared_rows = (ps && g.sc_along_row) || (pb && g.bi_along_row);
+    for (int d = 0; d < g.nk; d++)
+        if ((ps && g.sc_along_row && g.k_sc[d] != 0) || (pb && g.bi_along_row && g.k_bi[d] != 0)) shared_rows = false;
+    // kept dimensions that every operand walks as one
+    int nk = g.nk > 0 ? 1 : 0;
+    for (; nk < g.nk; nk++) {
+        const int64_t n = g.kdim[nk - 1];
+        if (g.k_in[nk] != n * g.k_in[nk - 1] || g.k_out[nk] != n * g.k_out[nk - 1] || (ps && g.k_sc[nk] != n * g.k_sc[nk - 1]) ||
+            (pb && g.k_bi[nk] != n * g.k_bi[nk - 1]))
+            break;
+    }
+    if (nk < g.nk) return launch_rows_of(pi, po, ps, pb, g, shared_rows, words, nv, eps_mode, eps, s);
+    const bool kept = g.nk > 0;
+    const FlatGeom f{kept ? g.k_in[0] : 0, kept ? g.k_out[0] : 0, kept && ps ? g.k_sc[0] : 0, kept && pb ? g.k_bi[0] : 0, g.rows, g.row_len,
+                     g.sc_along_row, g.bi_along_row};
+    return launch_rows_of(pi, po, ps, pb, f, shared_rows, words, nv, eps_mode, eps, s);
+}
+
 // mvn1 over groups that follow one another in memory, as rows
 int launch_group_rows(const half_t* in, half_t* out, int64_t groups, int64_t len, int nv, float eps, hipStream_t s) {
-    Mvn6Geom g{};
-    g.nk = g.nr = 1;
-    g.kdim[0] = (int32_t)groups;
-    g.rdim[0] = (int32_t)len;
-    g.k_in[0] = g.k_out[0] = len;
-    g.r_in[0] = g.r_out[0] = 1;
-    g.rows = groups;
-    g.row_len = (uint32_t)len;
     const bool words = len % 8 == 0 && ((reinterpret_cast<uintptr_t>(in) | reinterpret_cast<uintptr_t>(out)) & 15) == 0;
-    return launch_rows(in, out, nullptr, nullptr, g, words, nv, 0, eps, s);
+    return launch_rows_of(in, out, nullptr, nullptr, FlatGeom{len, len, 0, 0, groups, (uint32_t)len, 0, 0}, false, words, nv, 0, eps, s);
 }
 
 // mvn1 with per-channel statistics on a channel-minor layout: shifted partial sums over spatial ranges,
