@@ -524,7 +524,7 @@ int mem_pos_of(uint64_t order, int nd, int logical) {
 // 224 of 256 compute units, eight rounds of workgroups that wait and read the tensor 32 times; now 0.9: the wait, 0.1 for the missing slices, eight rounds.)
 // What bounds a small tensor is the chain of trips to memory: arguments, slice, tag, publication, the others' records; in between nothing waits for a
 // division by a count that was known before, and moments meet all at once.  us in a HIP graph, with the tag in front of the slice, records
-// polled a round of 64 at a time and pairwise merges / now: [1,128,57,73] 7.1 / 5.6, [4,256,64,64] 6.5 / 5.9, [16,16,142,176] 6.6 / 6.0.
+// polled a round of 64 at a time and pairwise merges / now: [1,128,57,73] 7.1 / 5.6, [1,16,142,176] 6.6 / 5.1, [4,256,64,64] among other calls 6.5 / 6.0.
 constexpr int kFusedMaxVec = 52;           // 128-bit words per lane of 512, 208 of its 256 registers: the chip holds 54 M values
 constexpr int kSyncStride = 4;             // words between launch counts
 // kFusedMaxGroups groups at most: each owns a fixed run of kMergeInKernel launch counts and as many record slots
