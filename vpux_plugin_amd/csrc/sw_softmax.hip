@@ -307,6 +307,75 @@ __global__ __launch_bounds__(256) void softmax_rows_f16(const half_t* __restrict
     }
 }
 
+// fp16 rows one after another in memory, of any length from eight values on at any address: TEAM adjacent lanes hold a row, VPT words of 128 bits
+// each.  The lane with the row's last, partial word takes the row's last eight values, lanes past the end the same: what they hold
+// again stays out of the sum, and whoever shares a value stores it alike.  No branch stands around a load, and the four arguments
+// are one read.  What bounds it is the launch, for large tensors memory with lines that two rows share.  us in a HIP graph, through LDS or as aligned
+// words with masked ends / here: [40 x 197] 3.4 / 2.7, [5000 x 231] 5.0 / 3.3, [30000 x 48] 5.9 / 3.3, [150000 x 17] 12.7 / 5.2, [30000 x 403] 13.0 / 10.9.
+typedef half8_t half8_any __attribute__((aligned(2)));
+template <int TEAM, int VPT, bool READ_ONCE>
+__global__ __launch_bounds__(256) void softmax_packed_rows(const half_t* __restrict__ in, half_t* __restrict__ out, uint32_t rows, uint32_t len) {
+    const uint32_t t = threadIdx.x % TEAM;
+    const uint32_t mine = TEAM == 64 ? (uint32_t)__builtin_amdgcn_readfirstlane((int)(threadIdx.x / 64)) : threadIdx.x / TEAM;
+    const uint32_t row = blockIdx.x * (256 / TEAM) + mine;
+    if (row >= rows) return;  // a row's lanes leave together
+    const uint64_t base = (uint64_t)row * len;
+    half8_t h[VPT];
+    uint32_t at[VPT];
+#pragma unroll
+    for (int j = 0; j < VPT; j++) {
+        const uint32_t e0 = (j * TEAM + t) * 8;
+        at[j] = e0 + 8 <= len ? e0 : len - 8;
+        const half8_any* src = reinterpret_cast<const half8_any*>(in + base + at[j]);
+        if constexpr (READ_ONCE) h[j] = __builtin_nontemporal_load(src);
+        else h[j] = *src;
+    }
+    half8_t m8 = h[0];
+#pragma unroll
+    for (int j = 1; j < VPT; j++) m8 = __builtin_elementwise_max(m8, h[j]);
+    const half4_t m4 = __builtin_elementwise_max(__builtin_shufflevector(m8, m8, 0, 1, 2, 3), __builtin_shufflevector(m8, m8, 4, 5, 6, 7));
+    half2_t m2 = __builtin_elementwise_max(__builtin_shufflevector(m4, m4, 0, 1), __builtin_shufflevector(m4, m4, 2, 3));
+    m2 = __builtin_elementwise_max(m2, dpp_h2<0xB1>(m2));
+    m2 = __builtin_elementwise_max(m2, dpp_h2<0x4E>(m2));
+    if (TEAM >= 8) m2 = __builtin_elementwise_max(m2, dpp_h2<0x141>(m2));
+    if (TEAM >= 16) m2 = __builtin_elementwise_max(m2, dpp_h2<0x140>(m2));
+    if (TEAM >= 32) m2 = __builtin_elementwise_max(m2, __builtin_bit_cast(half2_t, __builtin_amdgcn_ds_swizzle(__builtin_bit_cast(int, m2), 0x401F)));
+    if (TEAM == 64)
+        m2 = __builtin_elementwise_max(__builtin_bit_cast(half2_t, __builtin_amdgcn_readlane(__builtin_bit_cast(int, m2), 0)),
+                                       __builtin_bit_cast(half2_t, __builtin_amdgcn_readlane(__builtin_bit_cast(int, m2), 32)));
+    const float nmb = -fmaxf((float)m2[0], (float)m2[1]) * kLog2e;
+    float e[VPT][8];
+    float s = 0.f;
+#pragma unroll
+    for (int j = 0; j < VPT; j++) {
+        const uint32_t e0 = (j * TEAM + t) * 8, again = e0 >= len ? 8 : e0 - at[j];  // values that belong to the word before
+#pragma unroll
+        for (uint32_t k = 0; k < 8; k++) {
+            e[j][k] = __builtin_amdgcn_exp2f(__builtin_fmaf((float)h[j][k], kLog2e, nmb));
+            s += k >= again ? e[j][k] : 0.f;
+        }
+    }
+    s += dpp<0xB1>(s);
+    s += dpp<0x4E>(s);
+    if (TEAM >= 8) s += dpp<0x141>(s);
+    if (TEAM >= 16) s += dpp<0x140>(s);
+    if (TEAM >= 32) s += __builtin_bit_cast(float, __builtin_amdgcn_ds_swizzle(__builtin_bit_cast(int, s), 0x401F));
+    if (TEAM == 64)
+        s = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, s), 0)) +
+            __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, s), 32));
+    const float r = __builtin_amdgcn_rcpf(s), inv = __builtin_fmaf(__builtin_fmaf(-s, r, 1.0f), r, r);
+#pragma unroll
+    for (int j = 0; j < VPT; j++) {
+        if ((j * TEAM + t) * 8 >= len) continue;
+        half8_t o;
+#pragma unroll
+        for (int k = 0; k < 8; k++) o[k] = (half_t)(e[j][k] * inv);
+        half8_any* const to = reinterpret_cast<half8_any*>(out + base + at[j]);
+        if constexpr (READ_ONCE) __builtin_nontemporal_store(o, to);
+        else *to = o;
+    }
+}
+
 // ---------------------------------------------------------------- rows_block
 __device__ __forceinline__ float block_allreduce_max(float v, float* smem) {
     v = wave_allreduce(v, MaxOp{});
@@ -544,10 +613,10 @@ __global__ __launch_bounds__(256) void softmax_tiny_rows_f16(const half_t* __res
     __builtin_nontemporal_store(o, reinterpret_cast<u32x4*>(out) + v);
 }
 
-// Many short fp16 rows that follow one another in memory (rows of 32 ... 1024 values, any length: 197 as well as
-// 64): a workgroup takes a run of whole rows of about 4096 values, moves it between global memory and LDS in aligned
-// 128-bit words whatever the row length (values of neighbouring rows that share its first and last word are read
-// too, never written), and every half-wavefront handles one row at a time with the row's values in registers.
+// Many fp16 rows of fewer than eight values that follow one another in memory: a workgroup takes a run of whole rows of about
+// 4096 values, moves it between global memory and LDS in aligned 128-bit words whatever the row length (values of
+// neighbouring rows that share its first and last word are read too, never written), and every half-wavefront handles one
+// row at a time, a value a lane.
 constexpr int kShortChunk = 4096;
 // All-reduce over the 32 lanes of half a wavefront: four DPP steps and one 16-lane swap, which all stay inside the half.
 template <class Op>
@@ -564,7 +633,6 @@ __device__ __forceinline__ float half_wave_max(float v) {
 __device__ __forceinline__ float half_wave_sum(float v) {
     return half_wave_allreduce(v, [](float a, float b) { return a + b; });
 }
-template <int K>  // values per lane: a row has at most 32 K
 __global__ __launch_bounds__(256) void softmax_short_rows_f16(const half_t* __restrict__ in, half_t* __restrict__ out, int64_t rows,
                                                               int len, int per_wg) {
     __shared__ __attribute__((aligned(16))) half_t buf[kShortChunk + 16];
@@ -586,28 +654,11 @@ __global__ __launch_bounds__(256) void softmax_short_rows_f16(const half_t* __re
     const int lane = threadIdx.x & 31, team = threadIdx.x >> 5;
     for (int r = team; r < nr; r += 8) {  // uniform per half-wavefront
         half_t* x = buf + (int)(e0 - a0) + r * len;
-        float v[K];
-        float m = -INFINITY;
-#pragma unroll
-        for (int k = 0; k < K; k++) {
-            const int i = lane + 32 * k;
-            v[k] = i < len ? (float)x[i] : -INFINITY;
-            m = fmaxf(m, v[k]);
-        }
-        m = half_wave_max(m);
-        const float nmb = -m * kLog2e;
-        float sum = 0.f;
-#pragma unroll
-        for (int k = 0; k < K; k++) {
-            v[k] = __builtin_amdgcn_exp2f(__builtin_fmaf(v[k], kLog2e, nmb));  // exp2(-inf) = 0 for the slots past the row
-            sum += v[k];
-        }
-        const float inv = 1.0f / half_wave_sum(sum);
-#pragma unroll
-        for (int k = 0; k < K; k++) {
-            const int i = lane + 32 * k;
-            if (i < len) x[i] = (half_t)(v[k] * inv);
-        }
+        const float v = lane < len ? (float)x[lane] : -INFINITY;
+        const float nmb = -half_wave_max(v) * kLog2e;
+        const float e = __builtin_amdgcn_exp2f(__builtin_fmaf(v, kLog2e, nmb));  // exp2(-inf) = 0 for the lanes past the row
+        const float inv = 1.0f / half_wave_sum(e);
+        if (lane < len) x[lane] = (half_t)(e * inv);
     }
     __syncthreads();
     for (int w = threadIdx.x; w < words; w += 256) {
@@ -897,7 +948,6 @@ int softmax_typed(const SoftmaxPlan& p, const T* in, T* out, hipStream_t s) {
             aligned = aligned && map.in_stride[d] % 8 == 0 && map.out_stride[d] % 8 == 0;
             same_mis = same_mis && (map.in_stride[d] - map.out_stride[d]) % 8 == 0;
         }
-        // short rows, one after another in memory: runs of rows through LDS, half a wavefront per row
         const bool packed = map.nd == 0 || (map.nd == 1 && map.in_stride[0] == len && map.out_stride[0] == len);
         const bool base16 = ((reinterpret_cast<uintptr_t>(in) | reinterpret_cast<uintptr_t>(out)) & 15) == 0;
         if (packed && base16 && (len == 8 || len == 16 || len == 32 || len == 64 || len == 128 || len == 256) && rows * (len / 8) < (1ll << 39)) {
@@ -914,9 +964,58 @@ int softmax_typed(const SoftmaxPlan& p, const T* in, T* out, hipStream_t s) {
             VPX_HIP_CHECK(hipGetLastError());
             return VPX_RESULT_SUCCESS;
         }
-        if (packed && rows >= 64 && (len < 256 || (len % 8 != 0 && len <= 384)) && base16) {  // one wavefront per row idles lanes below 256 values
+        // rows of any other length up to 2048 values one after another: registers, unless softmax_rows_f16 has whole words of them from 256 on (us in a
+        // HIP graph, there / here: [500 x 512] 2.9 / 2.8, [5000 x 1024] 5.0 / 5.8; where a row is no whole words [500 x 535] 4.1 / 2.9, [5000 x 923] 6.4 / 5.7,
+        // [500 x 1890] 4.4 / 3.4) or the tensor is large and its rows long ([20574 x 1143] 19.8 / 18.3, [16848 x 1404] 17.8 / 18.0, [15864 x 1983] 22.9 / 23.2)
+        const bool once = rows * len >= (16ll << 20);  // 32 MB of input and more: read-once loads
+        if (packed && len >= 8 && len <= 2048 && (!aligned || len < 256) && !(same_mis && once && len > 1280)) {
+            int cus = 0;
+            const int rc = device_compute_units(&cus);
+            if (rc) return rc;
+            // A word a lane where rows are few (the shortest chain); from twelve wavefronts of those a compute unit on half the lanes and two or three
+            // words, which share the sums' crossings and, with three, leave fewer lanes idle -- but for tensors beyond the caches, which want whole
+            // lines at a time.  us, a word a lane / so: [16000 x 97] 3.6 / 3.4, [200000 x 97] 16.4 / 20.8 (left), [16000 x 197] 4.9 / 4.7, [200000 x 149] 27.8 /
+            // 25.1, [16000 x 285] 7.2 / 6.0, [60000 x 285] in two words 18.7 / 15.1, in three 17.1, [16000 x 535] in two words of 64 lanes 9.8, three of 32 8.5.
+            int team = len <= 32 ? 4 : len <= 64 ? 8 : len <= 128 ? 16 : len <= 256 ? 32 : 64, words = (int)((len + 511) / 512);
+            if (rows * team >= 12 * 64 * (int64_t)cus) {
+                if (team == 16 && !once) team = 8, words = 2;
+                else if (team == 32) team = 16, words = 2;
+                else if (len > 256 && len <= 384 && !once) team = 16, words = 3;
+                else if (len > 256 && len <= 512) team = 32, words = 2;
+                else if (len > 512 && len <= 768) team = 32, words = 3;
+            }
+            const int64_t most = (1ll << 31) / team;  // rows of a launch, which holds fewer than 2^32 lanes
+            for (int64_t r0 = 0; r0 < rows; r0 += most) {
+                const uint32_t n = (uint32_t)(rows - r0 < most ? rows - r0 : most), per = 256 / team;
+                const dim3 grid((n + per - 1) / per);
+                const half_t* from = hin + r0 * len;
+                half_t* to = hout + r0 * len;
+                const auto form = [&](auto team_c, auto words_c) {
+                    constexpr int LANES = decltype(team_c)::value, WORDS = decltype(words_c)::value;
+                    if (once) hipLaunchKernelGGL((softmax_packed_rows<LANES, WORDS, true>), grid, dim3(256), 0, s, from, to, n, (uint32_t)len);
+                    else hipLaunchKernelGGL((softmax_packed_rows<LANES, WORDS, false>), grid, dim3(256), 0, s, from, to, n, (uint32_t)len);
+                };
+                constexpr std::integral_constant<int, 1> one{};
+                constexpr std::integral_constant<int, 2> two{};
+                constexpr std::integral_constant<int, 3> three{};
+                constexpr std::integral_constant<int, 4> four{};
+                constexpr std::integral_constant<int, 8> t8{};
+                constexpr std::integral_constant<int, 16> t16{};
+                constexpr std::integral_constant<int, 32> t32{};
+                constexpr std::integral_constant<int, 64> t64{};
+                if (team == 4) form(four, one);
+                else if (team == 8) words == 1 ? form(t8, one) : form(t8, two);
+                else if (team == 16) words == 1 ? form(t16, one) : words == 2 ? form(t16, two) : form(t16, three);
+                else if (team == 32) words == 1 ? form(t32, one) : words == 2 ? form(t32, two) : form(t32, three);
+                else words == 1 ? form(t64, one) : words == 2 ? form(t64, two) : words == 3 ? form(t64, three) : form(t64, four);
+                VPX_HIP_CHECK(hipGetLastError());
+            }
+            return VPX_RESULT_SUCCESS;
+        }
+        // rows of fewer than eight values, one after another: runs of rows through LDS, half a wavefront per row
+        if (packed && rows >= 64 && len < 8 && base16) {
             // rows per workgroup: about 4096 values, fewer (whole passes of the eight half-wavefronts) while there are not two
-            // workgroups for every compute unit ([9,12,17,17]: 240 rows each in 8 workgroups took 8.9 us, a chain of 30 rows)
+            // workgroups for every compute unit
             int cus = 0;
             const int rc = device_compute_units(&cus);
             if (rc) return rc;
@@ -924,19 +1023,12 @@ int softmax_typed(const SoftmaxPlan& p, const T* in, T* out, hipStream_t s) {
             const int64_t spread = (rows / (2 * cus) + 7) / 8 * 8;
             if (per_wg > spread) per_wg = spread < 8 ? 8 : (int)spread;
             const dim3 grid((unsigned)((rows + per_wg - 1) / per_wg));
-#define VPX_SHORT(K) hipLaunchKernelGGL(softmax_short_rows_f16<K>, grid, dim3(256), 0, s, hin, hout, rows, (int)len, per_wg)
-            if (len <= 32) VPX_SHORT(1);
-            else if (len <= 64) VPX_SHORT(2);
-            else if (len <= 128) VPX_SHORT(4);
-            else if (len <= 256) VPX_SHORT(8);
-            else VPX_SHORT(12);
-#undef VPX_SHORT
+            hipLaunchKernelGGL(softmax_short_rows_f16, grid, dim3(256), 0, s, hin, hout, rows, (int)len, per_wg);
             VPX_HIP_CHECK(hipGetLastError());
             return VPX_RESULT_SUCCESS;
         }
         if (aligned || same_mis) {
             const int l = (int)len;
-            const bool once = rows * len >= (16ll << 20);  // 32 MB of input and more: read-once loads (aligned rows)
             const int span = aligned ? l : l + 7;  // aligned vectors a misaligned row can touch
             const dim3 block(256);
             const dim3 gw((unsigned)((rows + 3) / 4)), gb((unsigned)rows);
