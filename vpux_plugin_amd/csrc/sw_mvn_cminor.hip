@@ -6,10 +6,13 @@
 // registers -- 512 lanes of up to 50 words of 128 bits, 400 KB of the 512 KB a compute unit has -- between the sums and the
 // normalisation, and the workgroups that share a channel exchange their partial sums inside the launch.
 //
-// Deal.  R positions are a row of `words` 128-bit words, R the least count that makes it whole words whatever the channel
-// count (1 for a multiple of 8, else 2, 4 or 8).  A lane owns one word of the row and walks rows, so each of its eight
-// values belongs to one channel throughout and its sums are eight registers; all accesses are whole words.  A workgroup
-// takes whole rows, or, with R = 1, `ob` adjacent words of each (channel octets; eight of them are a 128-byte line).
+// Deal.  A lane owns one word of a row and walks rows, so each of its eight values belongs to one channel throughout and its
+// sums are eight registers.  Octets: a row is a position, a workgroup takes `ob` adjacent octets of its channels (eight of them are
+// 128 bytes); of a channel count that is no multiple of eight the last octet begins inside the one before, both hold those channels
+// and store them alike.  Rows: R positions are a row of `words` whole 128-bit words, R the least count that makes it so (1 for a multiple of
+// 8 channels, else 2, 4 or 8), and a workgroup takes whole rows, whose sums fold through LDS; they serve fewer than eight channels, odd channel
+// counts in place, and where they cost less.  (Octets of odd channel counts against rows or the three launches, us: [1,15,10,349] 4.0 / 11.6,
+// [7,10,14,359] 4.2 / 11.5, [3,141,122,426] 21 / 138, [2,211,167,511] 36 / 238; 250 drawn tensors of them take 0.58 of the time, 500 of whole octets 0.92.)
 #include "vpx_common.h"
 
 namespace vpx {
@@ -34,6 +37,7 @@ constexpr int kMostRecords = 2048;    // partial sums a workgroup reads from the
 struct Geom {
     uint32_t C, S, per_n;             // channels, positions and values of an image
     uint32_t R, words, rows;          // positions and words of a row, rows of an image (the last one may be cut short)
+    uint32_t pitch;                   // values from row to row
     uint32_t ob, ob_log, nb;          // words a workgroup takes of each row, and how many such blocks make the row
     uint32_t parts, rows_per_part;    // workgroups that share a block's rows
     uint32_t units;                   // images x parts
@@ -62,8 +66,8 @@ __device__ __forceinline__ half_t round_f16(float v) {
 
 // Tags.  The workgroups that share a block of channels of an image are a group with launch counts and a run of records of
 // its own, so that a record only ever carries tags of its own group's counts; a launch's tag is the count + 1, and it is the
-// device that counts, as a replayed graph needs.  Every workgroup has counts of its own (a run of the group's kMostParts, all
-// of which a launch moves on, however many workgroups it has): nobody else writes them during a launch, so a workgroup finds
+// device that counts, as a replayed graph needs.  Every workgroup has counts of its own (the group's kMostParts are dealt out in
+// turn, and a launch moves all of them on, however many workgroups it has): nobody else writes them during a launch, so a workgroup finds
 // the launch's tag however late it starts, and no record of an earlier launch carries it.  No read-modify-write is involved:
 // 192 arrivals at one counter took 1.5 us.
 // The wait is bounded: a workgroup whose partners do not show up in time (they are not resident: the device is shared)
@@ -73,7 +77,7 @@ __device__ __forceinline__ half_t round_f16(float v) {
 // part at most once.  (Each computing all parts for itself took 6.5 ms for [1,448,448,256] beside a launch that held 224 of 256
 // compute units; now 1.4.)
 //
-// How the sums meet.  With whole words per position (OCTETS) ob is a power of two: lanes that own the same word are ob apart
+// How the sums meet.  With OCTETS ob is a power of two: lanes that own the same word are ob apart
 // in a wavefront and add up by rotations and swaps, and so do a channel's partial sums of other workgroups; eight wavefronts
 // meet in LDS.  (A fold through LDS alone, group after group of lanes, took 4 us of a small tensor's 9.)  Rows of several
 // positions, whose channels lie anywhere in the words, fold through LDS.
@@ -106,11 +110,11 @@ __device__ __forceinline__ float swap_add(float a, float b) {
 }
 
 //
-// Results are written past the caches (a plain store of [16,112,112,256] costs 8 of its 49 us) except in runs of 16 or 32
-// bytes (SHORT), which the neighbouring blocks' runs complete to lines there: a kernel of its own, because one branch with
-// either store is compiled to plain ones.
+// Results are written past the caches (a plain store of [16,112,112,256] costs 8 of its 49 us), except (kShort) in runs of 16 or 32 bytes and in runs
+// that end within lines, which the neighbouring workgroups' runs complete to lines there: of 700 drawn tensors, those with such runs that hold 12 M
+// values or more take 0.60 ... 0.88 of the time of stores past the caches.  A kernel of its own, because one branch with either store is compiled
+// to plain ones.
 enum Form { kRows, kOctets, kShort };
-constexpr int kMostShortWords = 16;
 template <int V, Form FORM>
 __global__ __launch_bounds__(kT) void mvn_cminor_resident(const half_t* __restrict__ in, half_t* __restrict__ out, Geom g, unsigned* sync,
                                                           int normalize_variance, float eps, unsigned long long spin_ticks) {
@@ -129,43 +133,42 @@ __global__ __launch_bounds__(kT) void mvn_cminor_resident(const half_t* __restri
     const int t = (int)threadIdx.x;
     const half_t* img = in + (int64_t)n * g.per_n;
     half_t* oimg = out + (int64_t)n * g.per_n;
+    asm volatile("" ::"s"(out), "s"(sync), "s"(g.S), "s"(g.C), "s"(g.per_n), "s"(g.rows), "s"(normalize_variance), "s"(eps));  // (one trip to the arguments)
     const uint32_t w0 = b * g.ob, nw = g.words - w0 < g.ob ? g.words - w0 : g.ob;
     // OCTETS: a last block of fewer words leaves lanes idle
     const uint32_t slots = OCTETS ? kT >> g.ob_log : kT / nw, slot = OCTETS ? (uint32_t)t >> g.ob_log : (uint32_t)t / nw;
     const uint32_t wl = OCTETS ? (uint32_t)t & (g.ob - 1) : (uint32_t)t - slot * nw;
     const bool active = OCTETS ? wl < nw : slot < slots;
-    const uint32_t w = OCTETS && !active ? w0 : w0 + wl;
+    // first value of a word in its row; OCTETS: a last word that is not whole takes the last eight channels, which the word before has in part
+    const auto word_at = [&](uint32_t word) { return OCTETS && word * 8 + 8 > g.C ? g.C - 8 : word * 8; };
+    const uint32_t at = word_at(OCTETS && !active ? w0 : w0 + wl);
     const uint32_t cols = OCTETS ? g.ob * 8 : nw * 8, nch = OCTETS ? cols : g.C, ch0 = w0 * 8;  // (R > 1: ch0 is 0)
     const uint32_t G = kT / nch, gi = (uint32_t)t / nch, c = (uint32_t)t - gi * nch;
     // of the channel whose statistics this lane finishes
-    const float own_shift = (float)img[(uint32_t)t < nch && ch0 + t < g.C ? ch0 + t : 0];
+    const half_t own_first = img[OCTETS ? ((uint32_t)t < nch && w0 + t / 8 < g.words ? word_at(w0 + t / 8) + t % 8 : 0) : (uint32_t)t < nch && ch0 + t < g.C ? ch0 + t : 0];
     const uint32_t rem = OCTETS ? 0 : g.per_n % 8;  // values of the image's last, partial word
     const uint32_t group = OCTETS ? n * g.nb + b : kMostGroups + n;
-    // this workgroup's launch counts
+    // this workgroup's launch counts: every parts-th of the group's, from its own place on
     unsigned* counts = sync + (size_t)group * (kMostParts * kCountStride);
-    const uint32_t first_count = part * kMostParts / g.parts, end_count = (part + 1) * kMostParts / g.parts;
     Tagged* records = reinterpret_cast<Tagged*>(sync + (size_t)(kMostGroups + kMostRowGroups) * (kMostParts * kCountStride)) +
                       (OCTETS ? (size_t)group * kMostRecords : (size_t)kMostGroups * kMostRecords + (size_t)n * kMostRowRecords);
-    unsigned tag = 0;
-    if (g.parts > 1 && t == 0) tag = __hip_atomic_load(counts + first_count * kCountStride, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) + 1u;
-
     // sums are of x - x[first position of the channel]: no cancellation where a channel's mean is far from zero
     halfx8 first;
     if (OCTETS) {
-        first = __builtin_bit_cast(halfx8, *reinterpret_cast<const u32x4_any*>(img + w * 8));
+        first = __builtin_bit_cast(halfx8, *reinterpret_cast<const u32x4_any*>(img + at));
     } else {
 #pragma unroll
-        for (int k = 0; k < 8; k++) first[k] = img[(w * 8 + k) % g.C];
+        for (int k = 0; k < 8; k++) first[k] = img[(at + k) % g.C];
     }
     u32x4 q[V];
     uint32_t have = 0;  // words of this lane
     // The sums of part p over channel t, for the lanes below nch; its words stay in q.
-    const auto part_sums = [&](uint32_t p) -> float2 {
+    const auto part_sums = [&](uint32_t p, auto behind_first) __attribute__((always_inline)) -> float2 {
         const uint32_t r0 = p * g.rows_per_part, r1 = r0 + g.rows_per_part < g.rows ? r0 + g.rows_per_part : g.rows;
         const uint32_t r = r0 + slot;
         have = active && r < r1 ? (r1 - r + slots - 1) / slots : 0;
-        uint32_t f = (r * g.words + w) * 8;
-        const uint32_t step = slots * g.words * 8;
+        uint32_t f = r * g.pitch + at;
+        const uint32_t step = slots * g.pitch;
         // the last row's words past the image, and the partial one, are not among a lane's words
         if (have && (uint64_t)f + (uint64_t)(have - 1) * step + 8 > g.per_n) have--;
         // No branch around a load (lanes without a word read the image's first one), and kAhead of them under way while
@@ -178,6 +181,7 @@ __global__ __launch_bounds__(kT) void mvn_cminor_resident(const half_t* __restri
         };
 #pragma unroll
         for (int j = 0; j < (V < kAhead ? V : kAhead); j++) load(j);
+        behind_first();
         float sum[8], sq[8], shift[8];
 #pragma unroll
         for (int k = 0; k < 8; k++) {
@@ -273,11 +277,19 @@ __global__ __launch_bounds__(kT) void mvn_cminor_resident(const half_t* __restri
         return a;
     };
 
-    float2 total = part_sums(part);
+    // The launch's tag, asked for by one lane behind its first words (in front of them, worked with at once, it was a trip to memory before the first
+    // load) and dealt out behind the sums: workgroups that publish later for it, but all of whose wavefronts start to poll together, are ahead of
+    // those where seven poll while the first sums up (all lanes asking, no barrier: [8,69,106,64] 8.9 us, so 8.4).
+    unsigned counted = 0;
+    const auto ask_tag = [&]() __attribute__((always_inline)) {
+        if (g.parts > 1 && t == 0) counted = __hip_atomic_load(counts + part * kCountStride, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    };
+    float2 total = part_sums(part, ask_tag);
     if (g.parts > 1) {
-        if (t == 0) s_tag = tag == 0u ? 1u : tag;
+        asm volatile("" : "+v"(counted));  // (what is done with it stays here)
+        if (t == 0) s_tag = counted + 1u == 0u ? 1u : counted + 1u;
         __syncthreads();
-        tag = s_tag;
+        const unsigned tag = s_tag;
         const uint32_t count = g.parts * nch;
         const auto publish = [&](uint32_t p, float2 v) {
             if ((uint32_t)t < nch) {
@@ -287,8 +299,8 @@ __global__ __launch_bounds__(kT) void mvn_cminor_resident(const half_t* __restri
         };
         publish(part, total);
         // (here and not at the end: their way to memory then ends under the wait, 1.2 of 43 us at [16,112,112,256])
-        if (first_count + t < end_count)
-            __hip_atomic_store(counts + (first_count + t) * kCountStride, tag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        if (part + t * g.parts < kMostParts)
+            __hip_atomic_store(counts + (part + t * g.parts) * kCountStride, tag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         const unsigned long long began = wall_clock64();
         const auto poll = [&](uint32_t i, unsigned long long& rs, unsigned long long& rq) {
             rs = __hip_atomic_load(&records[i].sum, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -352,13 +364,13 @@ __global__ __launch_bounds__(kT) void mvn_cminor_resident(const half_t* __restri
                 __syncthreads();
                 const uint32_t pick = s_pick, p = (from + pick) % g.parts;
                 if (pick == g.parts) break;
-                publish(p, part_sums(p));
+                publish(p, part_sums(p, [] {}));
                 __threadfence();
                 if (t == 0) helped[p] = 1;
                 __syncthreads();
             }
             collect(false);
-            part_sums(part);  // its own words again
+            part_sums(part, [] {});  // its own words again
             __syncthreads();
         }
         if (OCTETS) {
@@ -397,7 +409,7 @@ __global__ __launch_bounds__(kT) void mvn_cminor_resident(const half_t* __restri
     }
     if ((uint32_t)t < nch) {
         const float count = (float)g.S, m = total.x / count, var = fmaxf(total.y / count - m * m, 0.f);
-        s_mean[t] = own_shift + m;
+        s_mean[t] = (float)own_first + m;
         s_inv[t] = normalize_variance ? 1.0f / __builtin_sqrtf(var + eps) : 1.0f;
     }
     __syncthreads();
@@ -409,8 +421,8 @@ __global__ __launch_bounds__(kT) void mvn_cminor_resident(const half_t* __restri
         mean[k] = s_mean[ch];
         inv[k] = s_inv[ch];
     }
-    uint32_t f = ((part * g.rows_per_part + slot) * g.words + w) * 8;
-    const uint32_t step = slots * g.words * 8;
+    uint32_t f = (part * g.rows_per_part + slot) * g.pitch + at;
+    const uint32_t step = slots * g.pitch;
 #pragma unroll
     for (int j = 0; j < V; j++) {
         asm volatile("" : "+v"(q[j]), "+v"(f));  // (values converted for the sums are not kept: twice the registers)
@@ -436,6 +448,26 @@ uint32_t ceil_div(uint64_t a, uint64_t b) {
 
 }  // namespace
 
+// Microseconds of a form: the launch, a word of a lane, the way of the fullest die's share of the tensor (of eight: a unit's workgroups are on one) at the
+// rate of a copy (runs of 16 ... 64 bytes cross the caches several times), more of both where that die is dealt more workgroups than it has compute units
+// (1.3 ... 1.8 times where a lane holds more than 16 words), a partial sum that is exchanged, a channel of the fold through LDS.  Fitted to 1095 drawn
+// tensors under each form that serves them (8500 times, median error 4 %, one tenth beyond 8 to 20): the least of these takes 1.2 % more than the best
+// form of each; without the crowding, 4.6 %.
+struct FormTime {
+    float launch, word, copy, crowded, exchange, channel;
+};
+// by whether workgroups exchange sums, octets a workgroup takes of each position (1, 2, 4, 8), whether C is no multiple of 8, one of 8, or one of
+// the workgroup's run (every run of a position is then as far from a line as the first one)
+constexpr FormTime kOctetTime[2][4][3] = {{{{3.27f, 0.425f, 1.80f, 0, 0, 0}, {3.27f, 0.274f, 1.73f, 0, 0, 0}, {3.27f, 0.274f, 1.73f, 0, 0, 0}},
+                                           {{3.29f, 0.423f, 0.90f, 0.48f, 0, 0}, {3.32f, 0.295f, 1.03f, 0, 0, 0}, {3.26f, 0.265f, 0.86f, 0.13f, 0, 0}},
+                                           {{3.40f, 0.318f, 0.66f, 0, 0, 0}, {3.23f, 0.273f, 0.60f, 0, 0, 0}, {3.27f, 0.249f, 0.48f, 0, 0, 0}},
+                                           {{3.30f, 0.312f, 0.47f, 0, 0, 0}, {3.20f, 0.276f, 0.49f, 0, 0, 0}, {3.34f, 0.265f, 0.14f, 0, 0, 0}}},
+                                          {{{2.56f, 1.143f, 1.09f, 0.75f, 0, 0}, {3.72f, 0.652f, 1.27f, 0.47f, 0, 0}, {3.72f, 0.652f, 1.27f, 0.47f, 0, 0}},
+                                           {{3.98f, 0.598f, 0.94f, 2.15f, 0.50e-3f, 0}, {4.12f, 0.562f, 0.79f, 2.31f, 0, 0}, {4.45f, 0.376f, 0.82f, 0.78f, 0.59e-3f, 0}},
+                                           {{4.49f, 0.389f, 0.78f, 1.71f, 0.72e-3f, 0}, {4.60f, 0.285f, 0.75f, 1.23f, 0.84e-3f, 0}, {4.28f, 0.393f, 0.52f, 1.14f, 0.63e-3f, 0}},
+                                           {{4.72f, 0.284f, 0.78f, 4.89f, 0.78e-3f, 0}, {4.73f, 0.228f, 0.75f, 4.53f, 0.76e-3f, 0}, {4.81f, 0.211f, 0.60f, 1.30f, 0.59e-3f, 0}}}};
+constexpr FormTime kRowTime[2] = {{4.98f, 0.257f, 0.46f, 0, 2.30e-3f, 0}, {8.27f, 0.146f, 0.66f, 0, 0.26e-3f, 2.94e-3f}};
+
 // Takes the launch when the tensor fits the registers of one workgroup per compute unit; *done is set when it has.
 int launch_mvn_cminor_resident(const void* in, void* out, int64_t N, int64_t S, int64_t C, int nv, float eps, hipStream_t s, bool* done) {
     *done = false;
@@ -449,43 +481,52 @@ int launch_mvn_cminor_resident(const void* in, void* out, int64_t N, int64_t S, 
     float best_cost = 0.f;
     bool best_rows = false;
     const uint32_t R = C % 8 == 0 ? 1 : C % 4 == 0 ? 2 : C % 2 == 0 ? 4 : 8, words = (uint32_t)(R * C / 8), rows = ceil_div(S, R);
+    const uint32_t octets = ceil_div(C, 8);
+    const float copied = 4.0f / 5.9e6f * (float)N * (float)S * (float)C;
+    const uint32_t cus_of_die = (uint32_t)cus >= 8 ? (uint32_t)cus / 8 : 1;
     const auto consider = [&](bool whole, uint32_t ob, uint32_t ob_log, uint32_t nb, uint32_t parts) {
-        const uint32_t slots = kT / ob, per_part = ceil_div(rows, parts), v = ceil_div(per_part, slots);
-        if (v > (!whole && ob < 4 ? kMostShortWords : kMostWords)) return;
-        parts = ceil_div(rows, per_part);
-        // Microseconds, fitted to some twenty shapes under each form: a word per lane takes a compute unit 0.28 us in and
-        // out, the whole chip 0.8; the exchange costs 3.3 us, more where many channels are read of many partners; runs of 32
-        // or 16 bytes of each line cost more than whole ones, and so do runs that start inside one ([5,130,205,176] 42 us in
-        // runs of 128 bytes, 30 in whole rows).
-        const float groups = (float)((uint32_t)N * nb * parts), full = groups / (float)cus;
-        const float run = whole ? 1.0f : ob == 1 ? 2.5f : ob == 2 ? 1.5f : C % (ob * 8) == 0 ? 1.0f : 2.0f;
-        const float cost = (float)v * (full > 0.35f ? 0.8f * full : 0.28f) * run + (parts > 1 ? 3.3f + (whole ? 0.0005f * (float)(parts * (uint32_t)C) : 0.0f) : 0.0f) + (whole ? 1.0f : 0.0f);
+        const uint32_t of = whole ? rows : (uint32_t)S, slots = kT / ob, per_part = ceil_div(of, parts), v = ceil_div(per_part, slots);
+        if (v > kMostWords) return;
+        parts = ceil_div(of, per_part);
+        const FormTime& f = whole ? kRowTime[parts > 1] : kOctetTime[parts > 1][ob_log][C % 8 != 0 ? 0 : C % (8 * ob) != 0 ? 1 : 2];
+        const uint32_t units = (uint32_t)N * parts, of_die = ceil_div(units, 8), dealt = of_die * nb;
+        const float crowd = dealt > cus_of_die ? (float)dealt / (float)cus_of_die : 1.0f, share = copied * 8.0f * (float)of_die / (float)units;
+        const float cost = f.launch + f.word * (float)v * crowd + (f.copy + f.crowded * (crowd - 1.0f)) * share +
+                           f.exchange * (float)(parts * (whole ? (uint32_t)C : ob * 8)) + (whole ? f.channel * (float)C : 0.0f);
         if (best_v != 0 && cost >= best_cost) return;
-        best = Geom{(uint32_t)C, (uint32_t)S, (uint32_t)(S * C), R, words, rows, ob, ob_log, nb, parts, per_part, (uint32_t)N * parts};
+        best = Geom{(uint32_t)C, (uint32_t)S, (uint32_t)(S * C), whole ? R : 1, whole ? words : octets, of, whole ? words * 8 : (uint32_t)C, ob, ob_log, nb, parts, per_part,
+                    (uint32_t)N * parts};
         best_v = v;
         best_cost = cost;
         best_rows = whole;
     };
     // Workgroups that share channels: as many as are resident together, with two words per lane or more, and no more
     // partial sums than there are records.
-    const auto most_parts = [&](uint32_t ob, uint32_t blocks, uint32_t records) {
+    const auto most_parts = [&](uint32_t of, uint32_t ob, uint32_t blocks, uint32_t records) {
         uint32_t parts = (uint32_t)cus / blocks;
         if (parts > kMostParts) parts = kMostParts;
-        if (parts > rows / (2 * (kT / ob))) parts = rows / (2 * (kT / ob));
+        if (parts > of / (2 * (kT / ob))) parts = of / (2 * (kT / ob));
         return parts < records ? parts : records;
     };
-    if (R == 1)
+    // Octets of channels, where a channel count that is no multiple of eight has a last one that begins inside the one before: in place, the workgroup
+    // of either could find results of the other's.
+    if (C >= 8 && (C % 8 == 0 || in != out))
         for (int k = 3; k >= 0; k--) {
-            const uint32_t ob = 1u << k, nb = ceil_div(words, ob);
-            if (ob > 1 && ob / 2 >= words) continue;
+            const uint32_t ob = 1u << k, nb = ceil_div(octets, ob);
+            if (ob > 1 && ob / 2 >= octets) continue;
             consider(false, ob, (uint32_t)k, nb, 1);
-            const uint32_t parts = most_parts(ob, (uint32_t)N * nb, kMostRecords / (ob * 8));
-            if (parts > 1 && N * nb <= kMostGroups) consider(false, ob, (uint32_t)k, nb, parts);
+            const uint32_t parts = most_parts((uint32_t)S, ob, (uint32_t)N * nb, kMostRecords / (ob * 8));
+            if (parts > 1 && N * nb <= kMostGroups) {
+                consider(false, ob, (uint32_t)k, nb, parts);
+                // (as many as leave no die with more workgroups than compute units: the others would wait for those that are dealt a second time)
+                const uint32_t even = 8 * (cus_of_die / nb) / (uint32_t)N;
+                if (even > 1 && even < parts) consider(false, ob, (uint32_t)k, nb, even);
+            }
         }
     if (words <= kT && C <= kT) {
         consider(true, words, 0, 1, 1);
         // (all that are resident read each other's partial sums of every channel: half and a quarter of them less)
-        const uint32_t parts = most_parts(words, (uint32_t)N, kMostRowRecords / (uint32_t)C);
+        const uint32_t parts = most_parts(rows, words, (uint32_t)N, kMostRowRecords / (uint32_t)C);
         for (uint32_t div = 1; div <= 4 && parts / div > 1 && N <= kMostRowGroups; div *= 2) consider(true, words, 0, 1, parts / div);
     }
     if (best_v == 0) return VPX_RESULT_SUCCESS;
@@ -505,17 +546,14 @@ int launch_mvn_cminor_resident(const void* in, void* out, int64_t N, int64_t S, 
     const dim3 grid((unsigned)blocks);
 #define VPX_CMINOR_AS(V, FORM) \
     hipLaunchKernelGGL((mvn_cminor_resident<V, FORM>), grid, dim3(kT), 0, s, (const half_t*)in, (half_t*)out, best, (unsigned*)sync, nv, eps, spin)
-#define VPX_CMINOR(V)                         \
-    do {                                      \
-        if (best_rows) VPX_CMINOR_AS(V, kRows); \
-        else VPX_CMINOR_AS(V, kOctets);       \
+#define VPX_CMINOR(V)                           \
+    do {                                        \
+        if (best_rows) VPX_CMINOR_AS(V, kRows);   \
+        else if (plain) VPX_CMINOR_AS(V, kShort); \
+        else VPX_CMINOR_AS(V, kOctets);         \
     } while (0)
-    if (!best_rows && best.ob < 4) {
-        if (best_v <= 2) VPX_CMINOR_AS(2, kShort);
-        else if (best_v <= 4) VPX_CMINOR_AS(4, kShort);
-        else if (best_v <= 8) VPX_CMINOR_AS(8, kShort);
-        else VPX_CMINOR_AS(kMostShortWords, kShort);
-    } else if (best_v <= 2) VPX_CMINOR(2);
+    const bool plain = best.ob < 4 || C % (8 * best.ob) != 0;
+    if (best_v <= 2) VPX_CMINOR(2);
     else if (best_v <= 4) VPX_CMINOR(4);
     else if (best_v <= 8) VPX_CMINOR(8);
     else if (best_v <= 16) VPX_CMINOR(16);
