@@ -4,6 +4,7 @@
 #include <cstring>
 #include <map>
 #include <mutex>
+#include <new>
 #include <utility>
 #include <vector>
 
@@ -13,18 +14,25 @@ namespace vpx {
 
 int launch_nce(const vpx_nce_task_t& t, hipStream_t s, const char** kernel_name);
 
-std::string& last_error() {
-    static thread_local std::string text;
-    return text;
+namespace {
+thread_local char t_error[1024] = "";
+}  // namespace
+
+const char* last_error() {
+    return t_error;
+}
+
+void clear_error() {
+    t_error[0] = 0;
 }
 
 int fail(int code, const char* fmt, ...) {
-    char buf[1024];
+    char buf[sizeof(t_error)];  // (an argument may be the last text)
     va_list ap;
     va_start(ap, fmt);
     vsnprintf(buf, sizeof(buf), fmt, ap);
     va_end(ap);
-    last_error() = buf;
+    memcpy(t_error, buf, sizeof(buf));
     return code;
 }
 
@@ -214,7 +222,10 @@ constexpr int kMaxMemRefs = VPX_MAX_KERNEL_INPUTS + VPX_MAX_KERNEL_OUTPUTS;
 
 // The operands of one launch, on the caller's stack: a launch allocates nothing on the heap.
 struct Args {
-    MemRef mem[kMaxMemRefs];
+    union {
+        MemRef mem[kMaxMemRefs];  // parse_blob makes the first n_mem of them (all together are 4.6 KB to clear)
+    };
+    Args() {}
     int n_mem = 0;
     const uint8_t* attrs = nullptr;
     size_t attrs_size = 0;
@@ -244,7 +255,7 @@ int parse_blob(const char* entry, int n_in, int n_out, const void* params, size_
     for (int i = 0; i < n_mem; i++) {
         vpx_memref_data_t md;
         memcpy(&md, p + (size_t)i * sizeof(md), sizeof(md));
-        MemRef& m = a.mem[i];
+        MemRef& m = *new (&a.mem[i]) MemRef;
         VPX_REQUIRE(md.numDims >= 1 && md.numDims <= VPX_MAX_ND_DIMS, VPX_RESULT_ERROR_INVALID_ARGUMENT,
                     "%s: memref %d has %u dimensions (1..%d allowed)", entry, i, md.numDims, VPX_MAX_ND_DIMS);
         m.nd = (int)md.numDims;
@@ -292,6 +303,7 @@ int parse_blob(const char* entry, int n_in, int n_out, const void* params, size_
         MemRef& m = a.mem[i];
         const bool is_in = i < n_in;
         size_t& cursor = is_in ? di : dout;
+        const int shift = __builtin_ctz((unsigned)m.elem_bits);  // (8, 16, 32 or 64)
         for (int d = 0; d < m.nd; d++) {
             int32_t dim;
             int64_t stride_bits;
@@ -303,11 +315,11 @@ int parse_blob(const char* entry, int n_in, int n_out, const void* params, size_
                 memcpy(&stride_bits, (is_in ? in_strides : out_strides) + (cursor + d) * 8, 8);
             }
             VPX_REQUIRE(dim >= 0, VPX_RESULT_ERROR_INVALID_ARGUMENT, "%s: memref %d dimension %d is negative (%d)", entry, i, d, dim);
-            VPX_REQUIRE(stride_bits >= 0 && stride_bits % m.elem_bits == 0, VPX_RESULT_ERROR_INVALID_ARGUMENT,
+            VPX_REQUIRE(stride_bits >= 0 && (stride_bits & (m.elem_bits - 1)) == 0, VPX_RESULT_ERROR_INVALID_ARGUMENT,
                         "%s: memref %d stride %lld bits is not a multiple of the %d-bit element", entry, i,
                         (long long)stride_bits, m.elem_bits);
             m.dims[d] = dim;
-            m.strides[d] = stride_bits / m.elem_bits;
+            m.strides[d] = stride_bits >> shift;
         }
         cursor += m.nd;
         m.compact = is_compact(m);
@@ -336,16 +348,16 @@ float half_bits_to_float(uint16_t h) {
 
 // quantize / dequantize attributes: int64 n, then n scales and n zero points, both as packed
 // floating-point values of the non-quantized operand's type (sw_kernel.cpp:97-163).
-int read_quant_params(const char* entry, const Args& a, uint32_t float_type, std::vector<double>& scales,
-                      std::vector<int64_t>& zps) {
-    int64_t n = 0;
-    VPX_REQUIRE(read_attr(a, 0, &n), VPX_RESULT_ERROR_INVALID_ARGUMENT, "%s: params blob has no quantization parameters", entry);
-    VPX_REQUIRE(n >= 1 && n <= (1 << 24), VPX_RESULT_ERROR_INVALID_ARGUMENT, "%s: quantization parameter count is %lld", entry,
-                (long long)n);
+int read_quant_count(const char* entry, const Args& a, int64_t* n) {
+    VPX_REQUIRE(read_attr(a, 0, n), VPX_RESULT_ERROR_INVALID_ARGUMENT, "%s: params blob has no quantization parameters", entry);
+    VPX_REQUIRE(*n >= 1 && *n <= (1 << 24), VPX_RESULT_ERROR_INVALID_ARGUMENT, "%s: quantization parameter count is %lld", entry,
+                (long long)*n);
+    return VPX_RESULT_SUCCESS;
+}
+
+int read_quant_params(const char* entry, const Args& a, uint32_t float_type, int64_t n, double* scales, int64_t* zps) {
     const int per_word = float_type == VPX_NN_FP16 ? 4 : 2;
     const size_t words = (size_t)((n + per_word - 1) / per_word);
-    scales.resize((size_t)n);
-    zps.resize((size_t)n);
     for (int64_t i = 0; i < n; i++) {
         uint64_t sw = 0, zw = 0;
         const size_t word = (size_t)(i / per_word), slot = (size_t)(i % per_word);
@@ -360,10 +372,29 @@ int read_quant_params(const char* entry, const Args& a, uint32_t float_type, std
             memcpy(&sf, &sb, 4);
             memcpy(&zf, &zb, 4);
         }
-        scales[(size_t)i] = (double)sf;
-        zps[(size_t)i] = (int64_t)std::llround(zf);
+        scales[i] = (double)sf;
+        zps[i] = (int64_t)std::llround(zf);
     }
     return VPX_RESULT_SUCCESS;
+}
+
+// The parameters of a launch, then one(scale, zero point) or each(scales, zero points, n).
+template <class One, class Each>
+int with_quant_params(const char* entry, const Args& a, uint32_t float_type, const One& one, const Each& each) {
+    int64_t n = 0;
+    if (const int rc = read_quant_count(entry, a, &n)) return rc;
+    if (n == 1) {
+        double scale = 0.0;
+        int64_t zp = 0;
+        const int rc = read_quant_params(entry, a, float_type, 1, &scale, &zp);
+        return rc ? rc : one(scale, zp);
+    }
+    thread_local std::vector<double> scales;  // (their storage is kept from launch to launch)
+    thread_local std::vector<int64_t> zps;
+    scales.resize((size_t)n);
+    zps.resize((size_t)n);
+    const int rc = read_quant_params(entry, a, float_type, n, scales.data(), zps.data());
+    return rc ? rc : each(scales.data(), zps.data(), n);
 }
 
 // Restatement of the compiler's softmax parameter packing for callers that pass the first form
@@ -479,7 +510,7 @@ struct Entry {
 
 enum { K_CONVERT, K_ELTWISE, K_FQ, K_QUANT, K_DEQUANT, K_MVN, K_SOFTMAX, K_ACT, K_MVN_SUM, K_MVN_MEAN_VAR, K_MVN_NORM, K_MVN6, K_DYN_DEQUANT, K_DYN_QUANT };
 
-const Entry kEntries[] = {
+constexpr Entry kEntries[] = {
         {"convert", 1, 1, K_CONVERT, 0},
         {"eltwise_add", 2, 1, K_ELTWISE, ELT_ADD},
         {"eltwise_sub", 2, 1, K_ELTWISE, ELT_SUB},
@@ -527,17 +558,32 @@ const Entry kEntries[] = {
 };
 constexpr uint32_t kNumEntries = sizeof(kEntries) / sizeof(kEntries[0]);
 
-const Entry* find_entry(const char* name) {
-    // callers pass the same string again and again: the last pointer's entry is checked first (one comparison)
-    thread_local const char* last_name = nullptr;
-    thread_local const Entry* last_entry = nullptr;
-    if (name == last_name && last_entry != nullptr && strcmp(last_entry->name, name) == 0) return last_entry;
-    for (uint32_t i = 0; i < kNumEntries; i++)
-        if (strcmp(kEntries[i].name, name) == 0) {
-            last_name = name;
-            last_entry = &kEntries[i];
-            return last_entry;
+// Entries by a hash of their name: the kernels of a network come in turn, and a search through the list is up to forty comparisons.
+struct EntryTable {
+    static constexpr uint32_t kSlots = 256;
+    uint8_t at[kSlots] = {};  // 1 + the entry's place in the list
+
+    static constexpr uint32_t hash(const char* name) {
+        uint32_t h = 2166136261u;
+        for (; *name; name++) h = (h ^ (uint8_t)*name) * 16777619u;
+        return (h ^ h >> 16) % kSlots;
+    }
+    constexpr EntryTable() {
+        for (uint32_t i = 0; i < kNumEntries; i++) {
+            uint32_t slot = hash(kEntries[i].name);
+            while (at[slot]) slot = (slot + 1) % kSlots;
+            at[slot] = (uint8_t)(i + 1);
         }
+    }
+};
+static_assert(kNumEntries < EntryTable::kSlots);
+constexpr EntryTable kEntryTable;
+
+const Entry* find_entry(const char* name) {
+    for (uint32_t slot = EntryTable::hash(name); kEntryTable.at[slot]; slot = (slot + 1) % EntryTable::kSlots) {
+        const Entry& e = kEntries[kEntryTable.at[slot] - 1];
+        if (strcmp(e.name, name) == 0) return &e;
+    }
     return nullptr;
 }
 
@@ -551,7 +597,7 @@ using namespace vpx;
 extern "C" {
 
 const char* vpx_get_last_error(void) {
-    return last_error().c_str();
+    return last_error();
 }
 
 uint32_t vpx_get_version(void) {
@@ -604,22 +650,14 @@ static int sw_kernel_launch(const char* entry, const void* params, size_t params
         VPX_REQUIRE(read_attr(a, 0, &levels), VPX_RESULT_ERROR_INVALID_ARGUMENT, "fake_quantize: params blob has no levels attribute");
         return launch_fake_quantize(a.mem[0], &a.mem[1], a.mem[5], levels, s);
     }
-    case K_QUANT: {
-        thread_local std::vector<double> scales;  // (their storage is kept from launch to launch)
-        thread_local std::vector<int64_t> zps;
-        rc = read_quant_params(entry, a, a.mem[0].dtype, scales, zps);
-        if (rc) return rc;
-        if (scales.size() == 1) return launch_quantize(a.mem[0], a.mem[1], scales[0], zps[0], s);
-        return launch_quantize_per_axis(a.mem[0], a.mem[1], scales.data(), zps.data(), (int64_t)scales.size(), s);
-    }
-    case K_DEQUANT: {
-        thread_local std::vector<double> scales;  // (their storage is kept from launch to launch)
-        thread_local std::vector<int64_t> zps;
-        rc = read_quant_params(entry, a, a.mem[1].dtype, scales, zps);
-        if (rc) return rc;
-        if (scales.size() == 1) return launch_dequantize(a.mem[0], a.mem[1], scales[0], zps[0], s);
-        return launch_dequantize_per_axis(a.mem[0], a.mem[1], scales.data(), zps.data(), (int64_t)scales.size(), s);
-    }
+    case K_QUANT:
+        return with_quant_params(
+                entry, a, a.mem[0].dtype, [&](double scale, int64_t zp) { return launch_quantize(a.mem[0], a.mem[1], scale, zp, s); },
+                [&](const double* scales, const int64_t* zps, int64_t n) { return launch_quantize_per_axis(a.mem[0], a.mem[1], scales, zps, n, s); });
+    case K_DEQUANT:
+        return with_quant_params(
+                entry, a, a.mem[1].dtype, [&](double scale, int64_t zp) { return launch_dequantize(a.mem[0], a.mem[1], scale, zp, s); },
+                [&](const double* scales, const int64_t* zps, int64_t n) { return launch_dequantize_per_axis(a.mem[0], a.mem[1], scales, zps, n, s); });
     case K_MVN: {
         int64_t across = 0, normvar = 0;
         float eps = 0.f;
@@ -689,13 +727,13 @@ static int sw_kernel_launch(const char* entry, const void* params, size_t params
 
 int vpx_sw_kernel_launch(const char* entry, const void* params, size_t params_size, const vpx_memref_addr_t* addrs,
                          uint32_t num_addrs, void* stream) {
-    last_error().clear();
+    clear_error();
     return sw_kernel_launch(entry, params, size_t(params_size), addrs, num_addrs, stream);
 }
 
 int vpx_sw_kernel_launch_noalloc(const char* entry, const void* params, size_t params_size, const vpx_memref_addr_t* addrs,
                                  uint32_t num_addrs, void* stream) {
-    last_error().clear();
+    clear_error();
     // set-up, once per device: the device address of the fixed scratch array
     void* fixed = nullptr;
     const int rc = static_scratch_address(&fixed);
@@ -708,7 +746,7 @@ int vpx_sw_kernel_launch_noalloc(const char* entry, const void* params, size_t p
 }
 
 int vpx_nce_task(const vpx_nce_task_t* t, void* stream) {
-    last_error().clear();
+    clear_error();
     VPX_REQUIRE(t != nullptr, VPX_RESULT_ERROR_INVALID_NULL_HANDLE, "NCE task descriptor is null");
     VPX_REQUIRE(t->task_type == VPX_NCE_CONV || t->task_type == VPX_NCE_ELTWISE, VPX_RESULT_ERROR_UNSUPPORTED_FEATURE,
                 "NCE task type %d is not implemented (CONV and ELTWISE only)", t->task_type);
@@ -763,27 +801,27 @@ int vpx_nce_task(const vpx_nce_task_t* t, void* stream) {
 }
 
 int vpx_workspace_reserve(void* stream, size_t bytes) {
-    last_error().clear();
+    clear_error();
     return workspace_reserve(static_cast<hipStream_t>(stream), bytes);
 }
 
 int vpx_workspace_release(void* stream) {
-    last_error().clear();
+    clear_error();
     return workspace_release(static_cast<hipStream_t>(stream));
 }
 
 int vpx_set_tuning(const char* knob, const char* value) {
-    last_error().clear();
+    clear_error();
     return set_tuning(knob, value);
 }
 
 int vpx_calib_mfma_i8(const void* operands, void* sink, int iters, int fragment_reads, int64_t* ops, void* stream) {
-    last_error().clear();
+    clear_error();
     return calib_mfma_i8(operands, sink, iters, fragment_reads, ops, static_cast<hipStream_t>(stream));
 }
 
 int vpx_calib_coissue(int valu_kind, int wide_mfma, int mode, int iters, void* sink, void* stream) {
-    last_error().clear();
+    clear_error();
     return calib_coissue(valu_kind, wide_mfma, mode, iters, sink, static_cast<hipStream_t>(stream));
 }
 

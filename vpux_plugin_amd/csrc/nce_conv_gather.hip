@@ -329,14 +329,12 @@ __global__ __launch_bounds__(256) void nce_conv_mfma16(const int8_t* __restrict_
 
 int launch_fold(const int8_t* w, const int32_t* wt, ChanPrep* prep, int64_t OC, int64_t K, int corr, const Ppe& ppe, int shift_sub,
                 hipStream_t s) {
-    hipLaunchKernelGGL(nce_fold_kernel, dim3((unsigned)((OC + 3) / 4)), dim3(256), 0, s, w, wt, prep, OC, K, corr, ppe, shift_sub);
-    VPX_HIP_CHECK(hipGetLastError());
+    VPX_LAUNCH(nce_fold_kernel, dim3((unsigned)((OC + 3) / 4)), dim3(256), 0, s, w, wt, prep, OC, K, corr, ppe, shift_sub);
     return VPX_RESULT_SUCCESS;
 }
 
 int launch_colsum(const int8_t* w, int32_t* colsum, int64_t OC, int64_t K, hipStream_t s) {
-    hipLaunchKernelGGL(nce_colsum_kernel, dim3((unsigned)((OC + 3) / 4)), dim3(256), 0, s, w, colsum, OC, K);
-    VPX_HIP_CHECK(hipGetLastError());
+    VPX_LAUNCH(nce_colsum_kernel, dim3((unsigned)((OC + 3) / 4)), dim3(256), 0, s, w, colsum, OC, K);
     return VPX_RESULT_SUCCESS;
 }
 
@@ -357,7 +355,7 @@ int launch_conv_mfma(const int8_t* in, const int8_t* w, const ChanPrep* prep, ui
         auto kern = nce_conv_mfma<BM, BN, U8, SGN>;                                                                  \
         rc = set_dyn_lds(kern, lds);                                                                                 \
         if (rc) return rc;                                                                                           \
-        hipLaunchKernelGGL(kern, grid, dim3(256), lds, s, in, w, prep, out, g, pad_byte, swz, tc, icc, pf);          \
+        VPX_LAUNCH(kern, grid, dim3(256), lds, s, in, w, prep, out, g, pad_byte, swz, tc, icc, pf);                  \
     } while (0)
     const bool out_f16 = out_kind == OUT_F16, out_signed = out_kind == OUT_I8;
     if (out_f16 && in_u8) VPX_CONV(true, OUT_F16);
@@ -367,7 +365,6 @@ int launch_conv_mfma(const int8_t* in, const int8_t* w, const ChanPrep* prep, ui
     else if (out_signed) VPX_CONV(false, OUT_I8);
     else VPX_CONV(false, OUT_U8);
 #undef VPX_CONV
-    VPX_HIP_CHECK(hipGetLastError());
     return VPX_RESULT_SUCCESS;
 }
 
@@ -378,14 +375,13 @@ int launch_conv_mfma16(const int8_t* in, const int8_t* w, const ChanPrep* prep, 
     const dim3 grid((unsigned)((Mtot + 255) / 256), (unsigned)((g.OC + 63) / 64));
     const bool out_f16 = out_kind == OUT_F16;
 #define VPX_CONV16(U8, OUT)                                                                                           \
-    hipLaunchKernelGGL((nce_conv_mfma16<U8, OUT>), grid, dim3(256), lds, s, in, w, prep, out, g, pad_byte, pf)
+    VPX_LAUNCH((nce_conv_mfma16<U8, OUT>), grid, dim3(256), lds, s, in, w, prep, out, g, pad_byte, pf)
     // (the PPE's clamp window is already inside the storage range, so signed and unsigned bytes share a kernel)
     if (in_u8 && out_f16) VPX_CONV16(true, OUT_F16);
     else if (in_u8) VPX_CONV16(true, OUT_U8);
     else if (out_f16) VPX_CONV16(false, OUT_F16);
     else VPX_CONV16(false, OUT_U8);
 #undef VPX_CONV16
-    VPX_HIP_CHECK(hipGetLastError());
     return VPX_RESULT_SUCCESS;
 }
 
@@ -397,7 +393,7 @@ int launch_conv_naive(const uint8_t* in, const uint8_t* w, const int32_t* wt, ui
     const dim3 grid((unsigned)((total + 255) / 256));
     const bool out_f16 = out_kind == OUT_F16, out_signed = out_kind == OUT_I8;
 #define VPX_NAIVE(IS, WS, OS)                                                                                        \
-    hipLaunchKernelGGL((nce_conv_naive<IS, WS, OS>), grid, dim3(256), 0, s, in, w, wt, out, g, zp_in, zp_w, ppe, total)
+    VPX_LAUNCH((nce_conv_naive<IS, WS, OS>), grid, dim3(256), 0, s, in, w, wt, out, g, zp_in, zp_w, ppe, total)
     const int sel = (in_u8 ? 0 : 4) | (w_u8 ? 0 : 2) | (out_signed ? 1 : 0);
     if (out_f16) {
         switch (sel >> 1) {
@@ -417,7 +413,6 @@ int launch_conv_naive(const uint8_t* in, const uint8_t* w, const int32_t* wt, ui
     default: VPX_NAIVE(true, true, OUT_I8); break;
     }
 #undef VPX_NAIVE
-    VPX_HIP_CHECK(hipGetLastError());
     return VPX_RESULT_SUCCESS;
 }
 

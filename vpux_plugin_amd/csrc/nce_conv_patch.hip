@@ -832,14 +832,13 @@ int launch_conv_regw(const PatchLaunch& a, hipStream_t s) {
         auto kern = nce_conv_regw<U8, SAME, 3, 3>;                                                                    \
         rc = set_dyn_lds(kern, a.lds);                                                                                \
         if (rc) return rc;                                                                                            \
-        hipLaunchKernelGGL(kern, a.grid, dim3(512), a.lds, s, a.in, a.w, a.wt, a.out, a.g, a.pg, a.pad_byte, a.ppe);  \
+        VPX_LAUNCH(kern, a.grid, dim3(512), a.lds, s, a.in, a.w, a.wt, a.out, a.g, a.pg, a.pad_byte, a.ppe);          \
     } while (0)
     if (a.in_u8 && a.same_f) VPX_REGW(true, true);
     else if (a.in_u8) VPX_REGW(true, false);
     else if (a.same_f) VPX_REGW(false, true);
     else VPX_REGW(false, false);
 #undef VPX_REGW
-    VPX_HIP_CHECK(hipGetLastError());
     return VPX_RESULT_SUCCESS;
 }
 
@@ -853,7 +852,7 @@ int launch_conv_tile(const PatchLaunch& a, int per_wave, int ics, int waves, hip
         auto kern = nce_conv_tile<U8, TMW, SAME, ICS, NW>;                                                            \
         rc = set_dyn_lds(kern, a.lds);                                                                                \
         if (rc) return rc;                                                                                            \
-        hipLaunchKernelGGL(kern, a.grid, dim3(64 * NW), a.lds, s, a.in, a.w, a.wt, a.out, a.g, a.pg, a.pad_byte, a.ppe); \
+        VPX_LAUNCH(kern, a.grid, dim3(64 * NW), a.lds, s, a.in, a.w, a.wt, a.out, a.g, a.pg, a.pad_byte, a.ppe);         \
     } while (0)
 #define VPX_TILE(U8, TMW, SAME, ICS)                                                                                  \
     do {                                                                                                              \
@@ -879,7 +878,6 @@ int launch_conv_tile(const PatchLaunch& a, int per_wave, int ics, int waves, hip
 #undef VPX_TILE_I
 #undef VPX_TILE
 #undef VPX_TILE_W
-    VPX_HIP_CHECK(hipGetLastError());
     return VPX_RESULT_SUCCESS;
 }
 
@@ -892,8 +890,8 @@ int launch_conv_stream(const PatchLaunch& a, int ksplit_waves, int per_wave, hip
         auto kern = nce_conv_stream<U8, TMW, SAME, NW, KS>;                                                           \
         rc = set_dyn_lds(kern, a.lds);                                                                                \
         if (rc) return rc;                                                                                            \
-        hipLaunchKernelGGL(kern, a.grid, dim3(64 * NW), a.lds, s, a.in, a.w, a.wt, a.colsum, a.out, a.g, a.pg, a.sg,   \
-                           a.pad_byte, a.ppe);                                                                        \
+        VPX_LAUNCH(kern, a.grid, dim3(64 * NW), a.lds, s, a.in, a.w, a.wt, a.colsum, a.out, a.g, a.pg, a.sg,           \
+                   a.pad_byte, a.ppe);                                                                                \
     } while (0)
 #define VPX_STREAM(TMW, NW, KS)                                                                                       \
     do {                                                                                                              \
@@ -913,7 +911,6 @@ int launch_conv_stream(const PatchLaunch& a, int ksplit_waves, int per_wave, hip
     else VPX_STREAM(4, 8, 0);
 #undef VPX_STREAM
 #undef VPX_STREAM_W
-    VPX_HIP_CHECK(hipGetLastError());
     return VPX_RESULT_SUCCESS;
 }
 

@@ -383,12 +383,12 @@ int launch_conv_rows16(const RowsLaunch& a, hipStream_t s) {
             auto kern = nce_conv_rows16<U8, TMV, TNV, MULTIV, true>;                                                  \
             rc = set_dyn_lds(kern, a.lds);                                                                            \
             if (rc) return rc;                                                                                        \
-            hipLaunchKernelGGL(kern, a.grid, dim3(512), a.lds, s, a.in, a.w, a.wt, a.out, a.g, a.rg, a.pad_byte, a.ppe); \
+            VPX_LAUNCH(kern, a.grid, dim3(512), a.lds, s, a.in, a.w, a.wt, a.out, a.g, a.rg, a.pad_byte, a.ppe);         \
         } else {                                                                                                      \
             auto kern = nce_conv_rows16<U8, TMV, TNV, MULTIV, false>;                                                 \
             rc = set_dyn_lds(kern, a.lds);                                                                            \
             if (rc) return rc;                                                                                        \
-            hipLaunchKernelGGL(kern, a.grid, dim3(512), a.lds, s, a.in, a.w, a.wt, a.out, a.g, a.rg, a.pad_byte, a.ppe); \
+            VPX_LAUNCH(kern, a.grid, dim3(512), a.lds, s, a.in, a.w, a.wt, a.out, a.g, a.rg, a.pad_byte, a.ppe);         \
         }                                                                                                             \
     } while (0)
 #define VPX_ROWS(U8, TNV)                                                                                             \
@@ -409,7 +409,6 @@ int launch_conv_rows16(const RowsLaunch& a, hipStream_t s) {
     else VPX_ROWS(false, 2);
 #undef VPX_ROWS
 #undef VPX_ROWS_T
-    VPX_HIP_CHECK(hipGetLastError());
     return VPX_RESULT_SUCCESS;
 }
 

@@ -350,12 +350,11 @@ int launch_conv_strips(const StripLaunch& a, hipStream_t s) {
     const auto launch = [&](auto kernel) -> int {
         const int rc = set_dyn_lds(kernel, a.lds);
         if (rc) return rc;
-        hipLaunchKernelGGL(kernel, a.grid, dim3(64 * kStripWaves), a.lds, s, a.in, a.w, a.wt, a.out, a.sg, a.ppe);
+        VPX_LAUNCH(kernel, a.grid, dim3(64 * kStripWaves), a.lds, s, a.in, a.w, a.wt, a.out, a.sg, a.ppe);
         return VPX_RESULT_SUCCESS;
     };
     const int rc = a.in_u8 ? launch(nce_conv_strips<true>) : launch(nce_conv_strips<false>);
     if (rc) return rc;
-    VPX_HIP_CHECK(hipGetLastError());
     return VPX_RESULT_SUCCESS;
 }
 

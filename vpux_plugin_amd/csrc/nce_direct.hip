@@ -347,33 +347,53 @@ __global__ __launch_bounds__(SPLIT ? 64 * kMaxWaves : 256) void nce_direct(const
 // that would be shortest with 0.17 us for a step of a walk and 0.025 for a wave's value at the meeting: of 327 layers that takes 0.8 % over
 // the best of all combinations, 17 more than 5 % (by the time itself 1.4 %, 37: [600 x 256] . [256 x 64] without a split 3.5 us, with
 // one 2.9; 7x7 x 16 -> 64 of one image of [139,257] 6.5 and 5.9).
+// (Every layer asks, so the arithmetic is whole numbers of 32 bits and divisions by constants as far as it goes.)
 DirectShape direct_shape(int64_t P, int64_t OC, int64_t K, int64_t in_bytes, int cus) {
-    static constexpr struct { int tm, tn, waves; } kShapes[] = {{1, 1, 1}, {1, 1, 4}, {1, 1, 8}, {2, 1, 1}, {2, 1, 4}, {2, 1, 8}, {2, 2, 1}, {2, 2, 4}, {2, 2, 8}, {2, 4, 1}, {4, 4, 1}};
-    const int64_t steps = (K / 16 + 3) / 4;
+    const uint32_t steps = (uint32_t)((K / 16 + 3) / 4);
     const double mbytes = 1e-6 * ((double)P * (double)OC + (double)OC * (double)K + (double)in_bytes), mout = 1e-6 * (double)P * (double)OC;
+    struct Walk {
+        uint32_t share, S;  // steps of a wave, waves that have any
+    };
+    const auto walk = [&](uint32_t most) {
+        const uint32_t waves = most < steps ? most : steps, share = (steps + waves - 1) / waves;
+        return Walk{share, (steps + share - 1) / share};
+    };
+    const Walk by1{steps, 1}, by4 = walk(4), by8 = walk(8);
     DirectShape best{0, 0, 0, 0.0};
     double least = 0.0;
-    for (const auto& c : kShapes) {
-        const int64_t noc = (OC + 16 * c.tm - 1) / (16 * c.tm), npos = (P + 16 * c.tn - 1) / (16 * c.tn), tiles = noc * npos;
-        const int64_t waves = c.waves < steps ? c.waves : steps, share = (steps + waves - 1) / waves, S = (steps + share - 1) / share;
+    const auto consider = [&](auto tm_c, auto tn_c, auto waves_c) {
+        constexpr int tm = decltype(tm_c)::value, tn = decltype(tn_c)::value, most = decltype(waves_c)::value;
+        constexpr uint32_t depth = direct_depth(tm, tn);
+        const int64_t noc = (OC + 16 * tm - 1) / (16 * tm), npos = (P + 16 * tn - 1) / (16 * tn), tiles = noc * npos;
+        const Walk& w = most == 1 ? by1 : (most == 4 ? by4 : by8);
+        const uint32_t share = w.share, S = w.S;
         const bool split = S > 1;
         const int64_t wgs = split ? tiles : noc * ((npos + 3) / 4);
-        if (wgs >= (1ll << 31)) continue;
-        const int64_t depth = direct_depth(c.tm, c.tn);
-        const double cu_tiles = (double)((wgs + cus - 1) / cus * (split ? 1 : 4));  // on the fullest compute unit
-        const double simd_waves = std::ceil(cu_tiles * (double)S / 4.0), values = cu_tiles * c.tm * c.tn;
-        const double rounds = std::ceil(simd_waves / (c.tm * c.tn <= 4 ? 4.0 : 2.0));
-        const double us = 2.2 + (split ? 0.484 : 0.0) + 0.491 * (rounds - 1.0) + 0.0066 * (double)tiles / cus * (double)steps * (c.tm + c.tn) +
-                          0.07 * (double)((share + depth - 1) / depth) + 0.126 * (double)share + 0.0174 * simd_waves * (double)share * c.tm * (c.tn + 1) +
-                          values * (split ? 0.0122 + 0.0295 * (double)S : 0.0259) + kDirectPerMByte * mbytes + mout * (c.tm == 1 ? 0.913 : (c.tm == 2 ? 0.18 : 0.0));
+        if (wgs >= (1ll << 31)) return;
+        const uint64_t fullest = (uint64_t)(((uint32_t)wgs + (uint32_t)cus - 1) / (uint32_t)cus) * (split ? 1 : 4);  // tiles of the fullest compute unit
+        const uint64_t of_simd = (fullest * S + 3) / 4;
+        const double cu_tiles = (double)fullest, simd_waves = (double)of_simd, values = cu_tiles * tm * tn;
+        const double rounds = (double)(tm * tn <= 4 ? (of_simd + 3) / 4 : (of_simd + 1) / 2);
+        const double us = 2.2 + (split ? 0.484 : 0.0) + 0.491 * (rounds - 1.0) + 0.0066 * (double)tiles / cus * (double)steps * (tm + tn) +
+                          0.07 * (double)((share + depth - 1) / depth) + 0.126 * (double)share + 0.0174 * simd_waves * (double)share * tm * (tn + 1) +
+                          values * (split ? 0.0122 + 0.0295 * (double)S : 0.0259) + kDirectPerMByte * mbytes + mout * (tm == 1 ? 0.913 : (tm == 2 ? 0.18 : 0.0));
         const double rank = us + 0.044 * (double)share - (split ? 0.0045 * values * (double)S : 0.0);
         const double shortest = best.tm == 0 || us < best.us ? us : best.us;
         if (best.tm == 0 || rank < least) {
             least = rank;
-            best = DirectShape{c.tm, c.tn, c.waves, shortest};
+            best = DirectShape{tm, tn, most, shortest};
         }
         best.us = shortest;
-    }
+    };
+    const std::integral_constant<int, 1> one;
+    const std::integral_constant<int, 2> two;
+    const std::integral_constant<int, 4> four;
+    const std::integral_constant<int, 8> eight;
+    consider(one, one, one), consider(one, one, four), consider(one, one, eight);
+    consider(two, one, one), consider(two, one, four), consider(two, one, eight);
+    consider(two, two, one), consider(two, two, four), consider(two, two, eight);
+    consider(two, four, one);
+    consider(four, four, one);
     return best;
 }
 
@@ -388,7 +408,7 @@ int launch_direct(const DirectLaunch& a, hipStream_t s) {
     const auto launch = [&](auto kernel) -> int {
         const int rc = set_dyn_lds(kernel, lds);
         if (rc) return rc;
-        hipLaunchKernelGGL(kernel, grid, block, lds, s, a.in, a.w, a.wt, a.out, a.g, a.ppe, a.d, pad, flip);
+        VPX_LAUNCH(kernel, grid, block, lds, s, a.in, a.w, a.wt, a.out, a.g, a.ppe, a.d, pad, flip);
         return VPX_RESULT_SUCCESS;
     };
     const auto by_taps = [&](auto tm_c, auto tn_c) -> int {
@@ -412,7 +432,6 @@ int launch_direct(const DirectLaunch& a, hipStream_t s) {
     default: return fail(VPX_RESULT_ERROR_UNKNOWN, "nce_direct has no tile of %d x %d", a.tm, a.tn);
     }
     if (rc) return rc;
-    VPX_HIP_CHECK(hipGetLastError());
     return VPX_RESULT_SUCCESS;
 }
 

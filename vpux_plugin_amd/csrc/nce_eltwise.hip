@@ -219,8 +219,8 @@ int launch_nce_eltwise(const vpx_nce_task_t& t, const Ppe& ppe, hipStream_t s, c
         const int64_t blocks = (chunks + 255) / 256;
         VPX_REQUIRE(blocks < (1ll << 31), VPX_RESULT_ERROR_UNSUPPORTED_FEATURE, "NCE eltwise: tensor of %lld elements is too large", (long long)n);
 #define VPX_ELTV(AS, BS, SF, F16)                                                                                      \
-    hipLaunchKernelGGL((nce_eltwise_views_kernel<AS, BS, SF, F16>), dim3((unsigned)blocks), dim3(256), 0, s,          \
-                       (const uint8_t*)t.input, (const uint8_t*)t.weights, (uint8_t*)t.output, chunks, ev, e)
+    VPX_LAUNCH((nce_eltwise_views_kernel<AS, BS, SF, F16>), dim3((unsigned)blocks), dim3(256), 0, s,                  \
+               (const uint8_t*)t.input, (const uint8_t*)t.weights, (uint8_t*)t.output, chunks, ev, e)
 #define VPX_ELTV_S(AS, BS)                                                                                             \
     do {                                                                                                               \
         if (out_f16) VPX_ELTV(AS, BS, false, true);                                                                    \
@@ -233,7 +233,6 @@ int launch_nce_eltwise(const vpx_nce_task_t& t, const Ppe& ppe, hipStream_t s, c
         else VPX_ELTV_S(false, false);
 #undef VPX_ELTV_S
 #undef VPX_ELTV
-        VPX_HIP_CHECK(hipGetLastError());
         *kernel_name = "nce_eltwise_views_kernel";
         return VPX_RESULT_SUCCESS;
     }
@@ -244,18 +243,17 @@ int launch_nce_eltwise(const vpx_nce_task_t& t, const Ppe& ppe, hipStream_t s, c
     VPX_REQUIRE(blocks64 < (1ll << 31), VPX_RESULT_ERROR_UNSUPPORTED_FEATURE, "NCE eltwise: tensor of %lld elements is too large", (long long)n);
     const dim3 grid((unsigned)blocks64), block(256);
 #define VPX_ELT(AS, BS, SF)                                                                                            \
-    hipLaunchKernelGGL((nce_eltwise_kernel<AS, BS, SF>), grid, block, 0, s, (const uint8_t*)t.input,                   \
-                       (const uint8_t*)t.weights, (uint8_t*)t.output, n_vec, n, e)
+    VPX_LAUNCH((nce_eltwise_kernel<AS, BS, SF>), grid, block, 0, s, (const uint8_t*)t.input,                           \
+               (const uint8_t*)t.weights, (uint8_t*)t.output, n_vec, n, e)
 #define VPX_ELT16(AS, BS)                                                                                              \
-    hipLaunchKernelGGL((nce_eltwise_kernel<AS, BS, false, true>), grid, block, 0, s, (const uint8_t*)t.input,          \
-                       (const uint8_t*)t.weights, (uint8_t*)t.output, n_vec, n, e)
+    VPX_LAUNCH((nce_eltwise_kernel<AS, BS, false, true>), grid, block, 0, s, (const uint8_t*)t.input,                  \
+               (const uint8_t*)t.weights, (uint8_t*)t.output, n_vec, n, e)
     if (out_f16) {
         if (a_signed && b_signed) VPX_ELT16(true, true);
         else if (a_signed) VPX_ELT16(true, false);
         else if (b_signed) VPX_ELT16(false, true);
         else VPX_ELT16(false, false);
 #undef VPX_ELT16
-        VPX_HIP_CHECK(hipGetLastError());
         return VPX_RESULT_SUCCESS;
     }
     const int sel = (a_signed ? 4 : 0) | (b_signed ? 2 : 0) | (same_f ? 1 : 0);
@@ -270,7 +268,6 @@ int launch_nce_eltwise(const vpx_nce_task_t& t, const Ppe& ppe, hipStream_t s, c
     default: VPX_ELT(true, true, true); break;
     }
 #undef VPX_ELT
-    VPX_HIP_CHECK(hipGetLastError());
     return VPX_RESULT_SUCCESS;
 }
 

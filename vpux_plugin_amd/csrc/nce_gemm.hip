@@ -793,8 +793,8 @@ int launch_gemm_mfma(const GemmLaunch& a, hipStream_t s) {
         const size_t lds = GemmLds<__VA_ARGS__>::bytes(a.K);                                                         \
         rc = set_dyn_lds(kern, lds);                                                                                 \
         if (rc) return rc;                                                                                           \
-        hipLaunchKernelGGL(kern, grid, dim3(64 * nw), lds, s, a.A, a.B, a.wt, colsum, a.out, a.M, a.N, a.K, tiles_m,  \
-                           tiles_n, quotient_magic(4 * (unsigned)tiles_n), a.ppe, a.rows, a.dst, a.conv);                                                   \
+        VPX_LAUNCH(kern, grid, dim3(64 * nw), lds, s, a.A, a.B, a.wt, colsum, a.out, a.M, a.N, a.K, tiles_m,          \
+                   tiles_n, quotient_magic(4 * (unsigned)tiles_n), a.ppe, a.rows, a.dst, a.conv);                                                           \
     } while (0)
     // the tiles of 64 and 128, any kind of output
 #define VPX_GEMM_SMALL(U8, SGN)                                                                                      \
@@ -836,7 +836,6 @@ int launch_gemm_mfma(const GemmLaunch& a, hipStream_t s) {
 #undef VPX_GEMM_SMALL
 #undef VPX_GEMM_CONV
 #undef VPX_GEMM_K
-    VPX_HIP_CHECK(hipGetLastError());
     return VPX_RESULT_SUCCESS;
 }
 

@@ -356,11 +356,14 @@ int launch_gemm_regb(const GemmLaunch& a, const RegbShape& r, int workgroups, hi
     const int nch = 16 * r.nt * r.cbw;
     const int past_cache = nch % 64 == 0 && ((a.dst.sw & 127) == 0 || a.dst.sw == nch) && a.M * a.N <= (16ll << 20) ? 1 : 0;
     if (supers < 1 || workgroups % supers != 0 || a.K % 16 != 0) return VPX_RESULT_ERROR_UNKNOWN;
-    const auto launch = [&](auto kernel) {
-        hipLaunchKernelGGL(kernel, dim3((unsigned)workgroups), dim3(64 * kRegbWaves), 0, s, a.A, a.B, a.wt, a.out, a.M, (int)a.N, (int)(a.K / 16),
-                           a.rows.lda, a.dst.sw, a.ppe, supers, sign_flip, past_cache);
+    const auto launch = [&](auto kernel) -> int {
+        VPX_LAUNCH(kernel, dim3((unsigned)workgroups), dim3(64 * kRegbWaves), 0, s, a.A, a.B, a.wt, a.out, a.M, (int)a.N, (int)(a.K / 16),
+                   a.rows.lda, a.dst.sw, a.ppe, supers, sign_flip, past_cache);
+        return VPX_RESULT_SUCCESS;
     };
-    bool known = true;
+    const auto unknown = [&] {
+        return fail(VPX_RESULT_ERROR_UNKNOWN, "nce_gemm_regb has no form for K = %lld in blocks of %d x %d channels", (long long)a.K, r.cbw, 16 * r.nt);
+    };
     const auto by_groups = [&](auto same_c, auto ks_c, auto cbw_c, auto nt_c) {
         constexpr bool SAME = decltype(same_c)::value;
         constexpr int KS = decltype(ks_c)::value, CBW = decltype(cbw_c)::value, NT = decltype(nt_c)::value;
@@ -371,7 +374,7 @@ int launch_gemm_regb(const GemmLaunch& a, const RegbShape& r, int workgroups, hi
         if constexpr (CBW == 1) {
             if (r.gw == 4) return launch(nce_gemm_regb<SAME, KS, 1, 4, NT>);
         }
-        known = false;
+        return unknown();
     };
     const auto by_blocks = [&](auto same_c, auto ks_c) {
         constexpr int KS = decltype(ks_c)::value;
@@ -386,20 +389,16 @@ int launch_gemm_regb(const GemmLaunch& a, const RegbShape& r, int workgroups, hi
         if constexpr (KS == 1) {
             if (r.nt == 4 && r.cbw == 4) return by_groups(same_c, ks_c, four, four);
         }
-        known = false;
+        return unknown();
     };
     const auto by_length = [&](auto same_c) {
         if (ks == 1) return by_blocks(same_c, std::integral_constant<int, 1>{});
         if (ks == 2) return by_blocks(same_c, std::integral_constant<int, 2>{});
         if (ks == 3) return by_blocks(same_c, std::integral_constant<int, 3>{});
         if (ks == 4) return by_blocks(same_c, std::integral_constant<int, 4>{});
-        known = false;
+        return unknown();
     };
-    if (same_f) by_length(std::true_type{});
-    else by_length(std::false_type{});
-    if (!known) return fail(VPX_RESULT_ERROR_UNKNOWN, "nce_gemm_regb has no form for K = %lld in blocks of %d x %d channels", (long long)a.K, r.cbw, 16 * r.nt);
-    VPX_HIP_CHECK(hipGetLastError());
-    return VPX_RESULT_SUCCESS;
+    return same_f ? by_length(std::true_type{}) : by_length(std::false_type{});
 }
 
 }  // namespace nce

@@ -3,6 +3,7 @@
 // All of them are HBM-bound maps.  The fast path views compact operands as flat arrays and moves
 // 128 bits per lane per access, several independent accesses in flight per lane; a strided /
 // broadcasting path covers sub-views and NUMPY broadcast one element per lane.
+#include <limits>
 #include <type_traits>
 #include <vector>
 
@@ -221,10 +222,9 @@ int launch_stream(const F& f, int64_t n, hipStream_t s) {
     VPX_REQUIRE(blocks < (1ll << 31), VPX_RESULT_ERROR_UNSUPPORTED_FEATURE, "tensor of %lld elements is too large",
                 (long long)n);
     const dim3 grid((unsigned)blocks);
-    if (tier == 2) hipLaunchKernelGGL((stream_kernel<F, kBlock, kUnroll>), grid, dim3(kBlock), 0, s, f, n_vec, n);
-    else if (tier == 1) hipLaunchKernelGGL((stream_kernel<F, kBlock, 1>), grid, dim3(kBlock), 0, s, f, n_vec, n);
-    else hipLaunchKernelGGL((stream_kernel<F, 64, 1>), grid, dim3(64), 0, s, f, n_vec, n);
-    VPX_HIP_CHECK(hipGetLastError());
+    if (tier == 2) VPX_LAUNCH((stream_kernel<F, kBlock, kUnroll>), grid, dim3(kBlock), 0, s, f, n_vec, n);
+    else if (tier == 1) VPX_LAUNCH((stream_kernel<F, kBlock, 1>), grid, dim3(kBlock), 0, s, f, n_vec, n);
+    else VPX_LAUNCH((stream_kernel<F, 64, 1>), grid, dim3(64), 0, s, f, n_vec, n);
     return VPX_RESULT_SUCCESS;
 }
 
@@ -635,8 +635,9 @@ __device__ __forceinline__ int quantize_simple(float x, const FqConst& c) {
     const float r = __builtin_rintf(m);
     return (int)r + (int)c.olo + (m - r == 0.5f ? 1 : 0);
 }
-// Whether level / lm1 * (qmax - qmin) + qmin gives back level + qmin for every level, in float arithmetic (host).
-static bool levels_are_identity(float qmin, float qmax, float lm1) {
+// Whether level / lm1 * (qmax - qmin) + qmin gives back level + qmin for every level, in float arithmetic (known when this is compiled: the ranges
+// are those of the types).
+constexpr bool levels_are_identity(float qmin, float qmax, float lm1) {
     bool same = lm1 >= 1.0f && lm1 <= 65535.0f;
     for (int level = 0; same && level <= (int)lm1; level++) same = (float)level / lm1 * (qmax - qmin) + qmin == (float)(level + (int)qmin);
     return same;
@@ -1015,8 +1016,7 @@ bool make_vnd(const MemRef* const (&ops)[NOPS], VndIndex& ix, uint32_t& total_ve
 template <typename T, int NOPS, class Fn, bool TWO, int BCAST>
 int launch_vrow_as(const dim3& grid, const T* p0, const T* p1, const T* p2, const T* p3, const T* p4, T* pout, const Fn& fn,
                    const VndIndex& vx, uint32_t rows, hipStream_t s) {
-    hipLaunchKernelGGL((vrow_kernel<T, NOPS, Fn, TWO, BCAST>), grid, dim3(kBlock), 0, s, p0, p1, p2, p3, p4, pout, fn, vx, rows);
-    VPX_HIP_CHECK(hipGetLastError());
+    VPX_LAUNCH((vrow_kernel<T, NOPS, Fn, TWO, BCAST>), grid, dim3(kBlock), 0, s, p0, p1, p2, p3, p4, pout, fn, vx, rows);
     return VPX_RESULT_SUCCESS;
 }
 
@@ -1058,9 +1058,8 @@ int launch_vnd(const T* p0, const T* p1, const T* p2, const T* p3, const T* p4, 
         const int rc = launch_vrow<T, NOPS, Fn, true>(mask, grid, p0, p1, p2, p3, p4, pout, fn, vx, vx.dims[0], s);
         if (rc >= 0) return rc;
     }
-    hipLaunchKernelGGL((vnd_kernel<T, NOPS, Fn>), dim3((total_vec + kBlock - 1) / kBlock), dim3(kBlock), 0, s, p0, p1, p2, p3, p4,
-                       pout, fn, vx, total_vec);
-    VPX_HIP_CHECK(hipGetLastError());
+    VPX_LAUNCH((vnd_kernel<T, NOPS, Fn>), dim3((total_vec + kBlock - 1) / kBlock), dim3(kBlock), 0, s, p0, p1, p2, p3, p4,
+               pout, fn, vx, total_vec);
     return VPX_RESULT_SUCCESS;
 }
 
@@ -1124,9 +1123,8 @@ static int convert_impl(const MemRef& in, const MemRef& out, Fn fn, hipStream_t 
     rc = grid_1d(n, &blocks);
     if (rc) return rc;
     if (n == 0) return VPX_RESULT_SUCCESS;
-    hipLaunchKernelGGL((nd_unary_kernel<TI, TO, Fn>), dim3(blocks), dim3(kBlock), 0, s, (const TI*)in.data,
-                       (TO*)out.data, fn, ix, n);
-    VPX_HIP_CHECK(hipGetLastError());
+    VPX_LAUNCH((nd_unary_kernel<TI, TO, Fn>), dim3(blocks), dim3(kBlock), 0, s, (const TI*)in.data,
+               (TO*)out.data, fn, ix, n);
     return VPX_RESULT_SUCCESS;
 }
 
@@ -1208,9 +1206,8 @@ static int eltwise_impl(const MemRef& a, const MemRef& b, const MemRef& out, hip
     rc = grid_1d(n, &blocks);
     if (rc) return rc;
     if (n == 0) return VPX_RESULT_SUCCESS;
-    hipLaunchKernelGGL((nd_binary_kernel<T, Fn>), dim3(blocks), dim3(kBlock), 0, s, (const T*)a.data, (const T*)b.data,
-                       (T*)out.data, Fn{}, ix, n);
-    VPX_HIP_CHECK(hipGetLastError());
+    VPX_LAUNCH((nd_binary_kernel<T, Fn>), dim3(blocks), dim3(kBlock), 0, s, (const T*)a.data, (const T*)b.data,
+               (T*)out.data, Fn{}, ix, n);
     return VPX_RESULT_SUCCESS;
 }
 
@@ -1350,10 +1347,9 @@ int launch_fake_quantize(const MemRef& in, const MemRef lims[4], const MemRef& o
             per_channel |= 1u << k;
         }
         if (ok) {
-            hipLaunchKernelGGL(fq_inner8_kernel, dim3(inner_deal_blocks((uint32_t)(ch / 8), rows, kFqInnerRows)), dim3(kBlock), 0, s, (const half_t*)in.data,
-                               (half_t*)out.data, (const half_t*)lims[0].data, (const half_t*)lims[1].data, (const half_t*)lims[2].data,
-                               (const half_t*)lims[3].data, per_channel, (uint32_t)(ch / 8), rows, lm1, 1.0f / lm1);
-            VPX_HIP_CHECK(hipGetLastError());
+            VPX_LAUNCH(fq_inner8_kernel, dim3(inner_deal_blocks((uint32_t)(ch / 8), rows, kFqInnerRows)), dim3(kBlock), 0, s, (const half_t*)in.data,
+                       (half_t*)out.data, (const half_t*)lims[0].data, (const half_t*)lims[1].data, (const half_t*)lims[2].data,
+                       (const half_t*)lims[3].data, per_channel, (uint32_t)(ch / 8), rows, lm1, 1.0f / lm1);
             return VPX_RESULT_SUCCESS;
         }
     }
@@ -1414,17 +1410,16 @@ int launch_fake_quantize(const MemRef& in, const MemRef lims[4], const MemRef& o
     rc = grid_1d(n, &blocks);
     if (rc) return rc;
     if (n == 0) return VPX_RESULT_SUCCESS;
-    hipLaunchKernelGGL(nd_fq_kernel, dim3(blocks), dim3(kBlock), 0, s, (const half_t*)in.data, (half_t*)out.data,
-                       (const half_t*)lims[0].data, (const half_t*)lims[1].data, (const half_t*)lims[2].data,
-                       (const half_t*)lims[3].data, io, lim, lm1, n);
-    VPX_HIP_CHECK(hipGetLastError());
+    VPX_LAUNCH(nd_fq_kernel, dim3(blocks), dim3(kBlock), 0, s, (const half_t*)in.data, (half_t*)out.data,
+               (const half_t*)lims[0].data, (const half_t*)lims[1].data, (const half_t*)lims[2].data,
+               (const half_t*)lims[3].data, io, lim, lm1, n);
     return VPX_RESULT_SUCCESS;
 }
 
 // ---------------------------------------------------------------- quantize / dequantize
 template <typename TI, typename TQ>
-static int quantize_impl(const MemRef& in, const MemRef& out, double scale, int64_t zp, int64_t qmin, int64_t qmax,
-                         hipStream_t s) {
+static int quantize_impl(const MemRef& in, const MemRef& out, double scale, int64_t zp, hipStream_t s) {
+    constexpr int64_t qmin = std::numeric_limits<TQ>::min(), qmax = std::numeric_limits<TQ>::max();
     // Limits of the FakeQuantize the reference quantizer is built from (quantize.cpp:91-96); the same float
     // operations as the device's own preparation of a FakeQuantize (FqMap::prep).
     FqConst c;
@@ -1437,17 +1432,18 @@ static int quantize_impl(const MemRef& in, const MemRef& out, double scale, int6
     c.r_irange = 1.0f / c.irange;
     c.r_lm1 = 1.0f / c.lm1;
     c.orange = c.ohi - c.olo;
-    if (c.irange > 0.0f && levels_are_identity(c.olo, c.ohi, c.lm1)) return convert_impl<TI, TQ>(in, out, QuantFn<TI, TQ, true>{c}, s);
+    constexpr bool simple = levels_are_identity((float)qmin, (float)qmax, (float)(qmax - qmin + 1) - 1.0f);
+    if (c.irange > 0.0f && simple) return convert_impl<TI, TQ>(in, out, QuantFn<TI, TQ, true>{c}, s);
     return convert_impl<TI, TQ>(in, out, QuantFn<TI, TQ, false>{c}, s);
 }
 
 int launch_quantize(const MemRef& in, const MemRef& out, double scale, int64_t zp, hipStream_t s) {
     VPX_REQUIRE(same_shape(in, out), VPX_RESULT_ERROR_INVALID_ARGUMENT, "quantize: input and output shapes differ");
     VPX_REQUIRE(scale > 0.0, VPX_RESULT_ERROR_INVALID_ARGUMENT, "quantize: scale must be positive, got %g", scale);
-    if (in.dtype == VPX_NN_FP16 && out.dtype == VPX_NN_U8) return quantize_impl<half_t, uint8_t>(in, out, scale, zp, 0, 255, s);
-    if (in.dtype == VPX_NN_FP16 && out.dtype == VPX_NN_I8) return quantize_impl<half_t, int8_t>(in, out, scale, zp, -128, 127, s);
-    if (in.dtype == VPX_NN_FP32 && out.dtype == VPX_NN_U8) return quantize_impl<float, uint8_t>(in, out, scale, zp, 0, 255, s);
-    if (in.dtype == VPX_NN_FP32 && out.dtype == VPX_NN_I8) return quantize_impl<float, int8_t>(in, out, scale, zp, -128, 127, s);
+    if (in.dtype == VPX_NN_FP16 && out.dtype == VPX_NN_U8) return quantize_impl<half_t, uint8_t>(in, out, scale, zp, s);
+    if (in.dtype == VPX_NN_FP16 && out.dtype == VPX_NN_I8) return quantize_impl<half_t, int8_t>(in, out, scale, zp, s);
+    if (in.dtype == VPX_NN_FP32 && out.dtype == VPX_NN_U8) return quantize_impl<float, uint8_t>(in, out, scale, zp, s);
+    if (in.dtype == VPX_NN_FP32 && out.dtype == VPX_NN_I8) return quantize_impl<float, int8_t>(in, out, scale, zp, s);
     return fail(VPX_RESULT_ERROR_UNSUPPORTED_FEATURE, "quantize: %s -> %s is not implemented", dtype_name(in.dtype),
                 dtype_name(out.dtype));
 }
@@ -1488,19 +1484,16 @@ int launch_dynamic_quantize(const MemRef& in, const MemRef& out, const MemRef& s
     void* ws = nullptr;
     int rc = get_workspace(s, sizeof(MinMax) * (size_t)blocks, &ws);
     if (rc) return rc;
-    hipLaunchKernelGGL(dynq_range_kernel, dim3((unsigned)blocks), dim3(kBlock), 0, s, (const float*)in.data, n, (MinMax*)ws);
-    VPX_HIP_CHECK(hipGetLastError());
-    hipLaunchKernelGGL(dynq_params_kernel, dim3(1), dim3(kBlock), 0, s, (const MinMax*)ws, (int)blocks, (float*)scale.data,
-                       (uint8_t*)zp.data);
-    VPX_HIP_CHECK(hipGetLastError());
+    VPX_LAUNCH(dynq_range_kernel, dim3((unsigned)blocks), dim3(kBlock), 0, s, (const float*)in.data, n, (MinMax*)ws);
+    VPX_LAUNCH(dynq_params_kernel, dim3(1), dim3(kBlock), 0, s, (const MinMax*)ws, (int)blocks, (float*)scale.data,
+               (uint8_t*)zp.data);
     if (n == 0) return VPX_RESULT_SUCCESS;
     DynQuantMap f{(const float*)in.data, (uint8_t*)out.data, (const float*)scale.data, (const uint8_t*)zp.data};
     if (aligned16(in.data) && (reinterpret_cast<uintptr_t>(out.data) & 3) == 0) return launch_stream(f, n, s);
     unsigned g;
     rc = grid_1d(n, &g);
     if (rc) return rc;
-    hipLaunchKernelGGL(dynq_scalar_kernel, dim3(g), dim3(kBlock), 0, s, f, n);
-    VPX_HIP_CHECK(hipGetLastError());
+    VPX_LAUNCH(dynq_scalar_kernel, dim3(g), dim3(kBlock), 0, s, f, n);
     return VPX_RESULT_SUCCESS;
 }
 
@@ -1573,29 +1566,27 @@ static int dyn_dequant_impl(const MemRef& in, const MemRef& scale, const MemRef*
             const dim3 grid(((unsigned)ix.dims[0] + kBlock - 1) / kBlock, rows < kRowsPerGridY ? rows : kRowsPerGridY,
                             (rows + kRowsPerGridY - 1) / kRowsPerGridY);
             if (per_row)
-                hipLaunchKernelGGL((dyn_dequant_kernel<TQ, TS, TO, VEC, false, true>), grid, dim3(kBlock), 0, s, (const TQ*)in.data,
-                                   (const TS*)scale.data, pz, zp_signed, (TO*)out.data, ix, n);
+                VPX_LAUNCH((dyn_dequant_kernel<TQ, TS, TO, VEC, false, true>), grid, dim3(kBlock), 0, s, (const TQ*)in.data,
+                           (const TS*)scale.data, pz, zp_signed, (TO*)out.data, ix, n);
             else
-                hipLaunchKernelGGL((dyn_dequant_kernel<TQ, TS, TO, VEC, true, true>), grid, dim3(kBlock), 0, s, (const TQ*)in.data,
-                                   (const TS*)scale.data, pz, zp_signed, (TO*)out.data, ix, n);
-            VPX_HIP_CHECK(hipGetLastError());
+                VPX_LAUNCH((dyn_dequant_kernel<TQ, TS, TO, VEC, true, true>), grid, dim3(kBlock), 0, s, (const TQ*)in.data,
+                           (const TS*)scale.data, pz, zp_signed, (TO*)out.data, ix, n);
             return VPX_RESULT_SUCCESS;
         }
         rc = grid_1d(n, &blocks);
         if (rc) return rc;
         if (per_row)
-            hipLaunchKernelGGL((dyn_dequant_kernel<TQ, TS, TO, VEC, false>), dim3(blocks), dim3(kBlock), 0, s, (const TQ*)in.data,
-                               (const TS*)scale.data, pz, zp_signed, (TO*)out.data, ix, n);
+            VPX_LAUNCH((dyn_dequant_kernel<TQ, TS, TO, VEC, false>), dim3(blocks), dim3(kBlock), 0, s, (const TQ*)in.data,
+                       (const TS*)scale.data, pz, zp_signed, (TO*)out.data, ix, n);
         else
-            hipLaunchKernelGGL((dyn_dequant_kernel<TQ, TS, TO, VEC, true>), dim3(blocks), dim3(kBlock), 0, s, (const TQ*)in.data,
-                               (const TS*)scale.data, pz, zp_signed, (TO*)out.data, ix, n);
+            VPX_LAUNCH((dyn_dequant_kernel<TQ, TS, TO, VEC, true>), dim3(blocks), dim3(kBlock), 0, s, (const TQ*)in.data,
+                       (const TS*)scale.data, pz, zp_signed, (TO*)out.data, ix, n);
     } else {
         rc = grid_1d(n, &blocks);
         if (rc) return rc;
-        hipLaunchKernelGGL((dyn_dequant_kernel<TQ, TS, TO, 1>), dim3(blocks), dim3(kBlock), 0, s, (const TQ*)in.data,
-                           (const TS*)scale.data, pz, zp_signed, (TO*)out.data, ix, n);
+        VPX_LAUNCH((dyn_dequant_kernel<TQ, TS, TO, 1>), dim3(blocks), dim3(kBlock), 0, s, (const TQ*)in.data,
+                   (const TS*)scale.data, pz, zp_signed, (TO*)out.data, ix, n);
     }
-    VPX_HIP_CHECK(hipGetLastError());
     return VPX_RESULT_SUCCESS;
 }
 
@@ -1870,8 +1861,7 @@ int axis_setup(const char* what, const MemRef& ref, const MemRef& other, int64_t
             ch.b[k] = b[c0 + k];
         }
         for (int k = cnt; k < 256; k++) ch.a[k] = ch.b[k] = 0.f;
-        hipLaunchKernelGGL(fill_axis_table, dim3(1), dim3(256), 0, s, *table + c0, (float*)(*table + n) + c0, n, ch, cnt);
-        VPX_HIP_CHECK(hipGetLastError());
+        VPX_LAUNCH(fill_axis_table, dim3(1), dim3(256), 0, s, *table + c0, (float*)(*table + n) + c0, n, ch, cnt);
     }
     if (keep) {
         std::lock_guard<std::mutex> lock(g_axis_mutex);
@@ -1999,32 +1989,31 @@ int quantize_axis_impl(const MemRef& in, const MemRef& out, const double* scales
     const bool simple = levels_are_identity(fmin_, fmax_, lm1);
     if (al && g.inner % V == 0) {
         if (simple)
-            hipLaunchKernelGGL((quantize_axis_vec_kernel<TI, TQ, true>), vgrid, dim3(kBlock), 0, s, (const TI*)in.data, (TQ*)out.data, table,
-                               g, total / V, fmin_, fmax_, lm1);
+            VPX_LAUNCH((quantize_axis_vec_kernel<TI, TQ, true>), vgrid, dim3(kBlock), 0, s, (const TI*)in.data, (TQ*)out.data, table,
+                       g, total / V, fmin_, fmax_, lm1);
         else
-            hipLaunchKernelGGL((quantize_axis_vec_kernel<TI, TQ, false>), vgrid, dim3(kBlock), 0, s, (const TI*)in.data, (TQ*)out.data, table,
-                               g, total / V, fmin_, fmax_, lm1);
+            VPX_LAUNCH((quantize_axis_vec_kernel<TI, TQ, false>), vgrid, dim3(kBlock), 0, s, (const TI*)in.data, (TQ*)out.data, table,
+                       g, total / V, fmin_, fmax_, lm1);
     }
     else if (g.inner == 1) {
         const uint32_t rows = total / g.count;
         if (g.count % 8 == 0 && (reinterpret_cast<uintptr_t>(in.data) % (8 * sizeof(TI))) == 0 && (reinterpret_cast<uintptr_t>(out.data) & 7) == 0) {
             const dim3 igrid(inner_deal_blocks(g.count / 8, rows, kAxisRows));
             if (simple)
-                hipLaunchKernelGGL((quantize_axis_inner8_kernel<TI, TQ, true>), igrid, dim3(kBlock), 0, s, (const TI*)in.data, (TQ*)out.data,
-                                   table, g.count, rows, fmin_, fmax_, lm1);
+                VPX_LAUNCH((quantize_axis_inner8_kernel<TI, TQ, true>), igrid, dim3(kBlock), 0, s, (const TI*)in.data, (TQ*)out.data,
+                           table, g.count, rows, fmin_, fmax_, lm1);
             else
-                hipLaunchKernelGGL((quantize_axis_inner8_kernel<TI, TQ, false>), igrid, dim3(kBlock), 0, s, (const TI*)in.data, (TQ*)out.data,
-                                   table, g.count, rows, fmin_, fmax_, lm1);
+                VPX_LAUNCH((quantize_axis_inner8_kernel<TI, TQ, false>), igrid, dim3(kBlock), 0, s, (const TI*)in.data, (TQ*)out.data,
+                           table, g.count, rows, fmin_, fmax_, lm1);
         } else {
             const dim3 igrid(((g.count + kBlock - 1) / kBlock) * ((rows + kAxisRows - 1) / kAxisRows));
-            hipLaunchKernelGGL((quantize_axis_inner_kernel<TI, TQ>), igrid, dim3(kBlock), 0, s, (const TI*)in.data, (TQ*)out.data, table,
-                               g.count, rows, fmin_, fmax_, lm1);
+            VPX_LAUNCH((quantize_axis_inner_kernel<TI, TQ>), igrid, dim3(kBlock), 0, s, (const TI*)in.data, (TQ*)out.data, table,
+                       g.count, rows, fmin_, fmax_, lm1);
         }
     }
     else
-        hipLaunchKernelGGL((quantize_axis_kernel<TI, TQ>), dim3((total + kBlock - 1) / kBlock), dim3(kBlock), 0, s, (const TI*)in.data,
-                           (TQ*)out.data, table, g, total, fmin_, fmax_, lm1);
-    VPX_HIP_CHECK(hipGetLastError());
+        VPX_LAUNCH((quantize_axis_kernel<TI, TQ>), dim3((total + kBlock - 1) / kBlock), dim3(kBlock), 0, s, (const TI*)in.data,
+                   (TQ*)out.data, table, g, total, fmin_, fmax_, lm1);
     return VPX_RESULT_SUCCESS;
 }
 
@@ -2045,24 +2034,23 @@ int dequantize_axis_impl(const MemRef& in, const MemRef& out, const double* scal
     const bool al = (reinterpret_cast<uintptr_t>(in.data) % V) == 0 && (reinterpret_cast<uintptr_t>(out.data) & 15) == 0;
     const dim3 vgrid((total / V + kBlock - 1) / kBlock);
     if (al && g.inner % V == 0)
-        hipLaunchKernelGGL((dequantize_axis_vec_kernel<TQ, TO>), vgrid, dim3(kBlock), 0, s, (const TQ*)in.data, (TO*)out.data,
-                           table, g, total / V);
+        VPX_LAUNCH((dequantize_axis_vec_kernel<TQ, TO>), vgrid, dim3(kBlock), 0, s, (const TQ*)in.data, (TO*)out.data,
+                   table, g, total / V);
     else if (g.inner == 1) {
         const uint32_t rows = total / g.count;
         if (g.count % 8 == 0 && (reinterpret_cast<uintptr_t>(in.data) & 7) == 0 && (reinterpret_cast<uintptr_t>(out.data) % (8 * sizeof(TO))) == 0) {
             const dim3 igrid(inner_deal_blocks(g.count / 8, rows, kAxisRows));
-            hipLaunchKernelGGL((dequantize_axis_inner8_kernel<TQ, TO>), igrid, dim3(kBlock), 0, s, (const TQ*)in.data, (TO*)out.data, table,
-                               g.count, rows);
+            VPX_LAUNCH((dequantize_axis_inner8_kernel<TQ, TO>), igrid, dim3(kBlock), 0, s, (const TQ*)in.data, (TO*)out.data, table,
+                       g.count, rows);
         } else {
             const dim3 igrid(((g.count + kBlock - 1) / kBlock) * ((rows + kAxisRows - 1) / kAxisRows));
-            hipLaunchKernelGGL((dequantize_axis_inner_kernel<TQ, TO>), igrid, dim3(kBlock), 0, s, (const TQ*)in.data, (TO*)out.data, table,
-                               g.count, rows);
+            VPX_LAUNCH((dequantize_axis_inner_kernel<TQ, TO>), igrid, dim3(kBlock), 0, s, (const TQ*)in.data, (TO*)out.data, table,
+                       g.count, rows);
         }
     }
     else
-        hipLaunchKernelGGL((dequantize_axis_kernel<TQ, TO>), dim3((total + kBlock - 1) / kBlock), dim3(kBlock), 0, s, (const TQ*)in.data,
-                           (TO*)out.data, table, g, total);
-    VPX_HIP_CHECK(hipGetLastError());
+        VPX_LAUNCH((dequantize_axis_kernel<TQ, TO>), dim3((total + kBlock - 1) / kBlock), dim3(kBlock), 0, s, (const TQ*)in.data,
+                   (TO*)out.data, table, g, total);
     return VPX_RESULT_SUCCESS;
 }
 

@@ -407,8 +407,7 @@ static int launch_lds_groups(const half_t* in, half_t* out, int64_t groups, int6
     // more than 64 KiB of dynamic LDS is an opt-in per device and function; asking again costs little
     VPX_HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(mvn_lds_group_kernel), hipFuncAttributeMaxDynamicSharedMemorySize,
                                       kLdsGroupMax * (int)sizeof(half_t)));
-    hipLaunchKernelGGL(mvn_lds_group_kernel, dim3((unsigned)groups), dim3(1024), lds, s, in, out, len, nv, eps_mode, eps);
-    VPX_HIP_CHECK(hipGetLastError());
+    VPX_LAUNCH(mvn_lds_group_kernel, dim3((unsigned)groups), dim3(1024), lds, s, in, out, len, nv, eps_mode, eps);
     return VPX_RESULT_SUCCESS;
 }
 
@@ -459,7 +458,7 @@ static bool tiny_groups_ok(const half_t* in, const half_t* out, int64_t groups, 
 static int launch_tiny_groups(const half_t* in, half_t* out, int64_t groups, int64_t len, int nv, int eps_mode, float eps, hipStream_t s) {
     const int64_t n_vec = groups * (len / 8);
     const dim3 grid((unsigned)((n_vec + kThreads - 1) / kThreads));
-#define VPX_TINY(T) hipLaunchKernelGGL(mvn_tiny_groups_kernel<T>, grid, dim3(kThreads), 0, s, in, out, n_vec, nv, eps_mode, eps)
+#define VPX_TINY(T) VPX_LAUNCH(mvn_tiny_groups_kernel<T>, grid, dim3(kThreads), 0, s, in, out, n_vec, nv, eps_mode, eps)
     if (len == 8) VPX_TINY(1);
     else if (len == 16) VPX_TINY(2);
     else if (len == 32) VPX_TINY(4);
@@ -467,7 +466,6 @@ static int launch_tiny_groups(const half_t* in, half_t* out, int64_t groups, int
     else if (len == 128) VPX_TINY(16);
     else VPX_TINY(32);
 #undef VPX_TINY
-    VPX_HIP_CHECK(hipGetLastError());
     return VPX_RESULT_SUCCESS;
 }
 
@@ -490,13 +488,12 @@ static bool small_groups_ok(const half_t* in, const half_t* out, int64_t groups,
 static int launch_small_groups(const half_t* in, half_t* out, int64_t groups, int64_t len, int nv, int eps_mode, float eps, hipStream_t s) {
     const int per_wg = small_groups_run(groups, len);
     const unsigned blocks = (unsigned)((groups + per_wg - 1) / per_wg);
-#define VPX_SMALL(K) hipLaunchKernelGGL(mvn_small_groups_kernel<K>, dim3(blocks), dim3(kThreads), 0, s, in, out, groups, (int)len, per_wg, nv, eps_mode, eps)
+#define VPX_SMALL(K) VPX_LAUNCH(mvn_small_groups_kernel<K>, dim3(blocks), dim3(kThreads), 0, s, in, out, groups, (int)len, per_wg, nv, eps_mode, eps)
     if (len <= 64) VPX_SMALL(2);
     else if (len <= 128) VPX_SMALL(4);
     else if (len <= 256) VPX_SMALL(8);
     else VPX_SMALL(16);
 #undef VPX_SMALL
-    VPX_HIP_CHECK(hipGetLastError());
     return VPX_RESULT_SUCCESS;
 }
 
@@ -822,8 +819,8 @@ int launch_fused_groups(const half_t* in, half_t* out, int64_t groups, int64_t g
     const unsigned long long spin = mode == 2 ? 0ull : 50000ull;  // 0.5 ms of the 100 MHz counter
     const dim3 grid((unsigned)wpg, (unsigned)groups);
 #define VPX_FUSED(V, T)                                                                                                        \
-    hipLaunchKernelGGL((mvn_fused_kernel<V, T>), grid, dim3(T), 0, s, in, out, (uint32_t)group_size, (int)wpg, (uint32_t)slice, \
-                       (unsigned*)sync, nv, eps, spin)
+    VPX_LAUNCH((mvn_fused_kernel<V, T>), grid, dim3(T), 0, s, in, out, (uint32_t)group_size, (int)wpg, (uint32_t)slice,         \
+               (unsigned*)sync, nv, eps, spin)
     // up to eight words per lane four wavefronts do (eight measured 0.3 us slower there)
     if (lane_words <= kThreads) VPX_FUSED(1, 256);
     else if (lane_words <= 2 * kThreads) VPX_FUSED(2, 256);
@@ -836,7 +833,6 @@ int launch_fused_groups(const half_t* in, half_t* out, int64_t groups, int64_t g
     else if (lane_words <= 40 * 512) VPX_FUSED(40, 512);
     else VPX_FUSED(kFusedMaxVec, 512);
 #undef VPX_FUSED
-    VPX_HIP_CHECK(hipGetLastError());
     *done = true;
     return VPX_RESULT_SUCCESS;
 }
@@ -854,9 +850,8 @@ int launch_groups(const half_t* in, half_t* out, int64_t groups, int64_t group_s
         if (rc || done) return rc;
     }
     if (chunks == 1) {
-        hipLaunchKernelGGL((mvn_chunk_kernel<0, ALIGNED>), dim3(blocks), dim3(kThreads), 0, s, in, out, group_size, 1,
-                           (Record*)nullptr, (const Record*)nullptr, nv, eps);
-        VPX_HIP_CHECK(hipGetLastError());
+        VPX_LAUNCH((mvn_chunk_kernel<0, ALIGNED>), dim3(blocks), dim3(kThreads), 0, s, in, out, group_size, 1,
+                   (Record*)nullptr, (const Record*)nullptr, nv, eps);
         return VPX_RESULT_SUCCESS;
     }
     void* ws = nullptr;
@@ -866,18 +861,15 @@ int launch_groups(const half_t* in, half_t* out, int64_t groups, int64_t group_s
     Record* partial = (Record*)ws;
     Record* merged = partial + blocks;
 
-    hipLaunchKernelGGL((mvn_chunk_kernel<1, ALIGNED>), dim3(blocks), dim3(kThreads), 0, s, in, out, group_size, chunks,
-                       partial, (const Record*)nullptr, nv, eps);
-    VPX_HIP_CHECK(hipGetLastError());
+    VPX_LAUNCH((mvn_chunk_kernel<1, ALIGNED>), dim3(blocks), dim3(kThreads), 0, s, in, out, group_size, chunks,
+               partial, (const Record*)nullptr, nv, eps);
     const Record* use_merged = nullptr;
     if (chunks > kMergeInKernel) {
-        hipLaunchKernelGGL(mvn_merge_kernel, dim3((unsigned)groups), dim3(kThreads), 0, s, partial, merged, chunks);
-        VPX_HIP_CHECK(hipGetLastError());
+        VPX_LAUNCH(mvn_merge_kernel, dim3((unsigned)groups), dim3(kThreads), 0, s, partial, merged, chunks);
         use_merged = merged;
     }
-    hipLaunchKernelGGL((mvn_chunk_kernel<2, ALIGNED>), dim3(blocks), dim3(kThreads), 0, s, in, out, group_size, chunks,
-                       partial, use_merged, nv, eps);
-    VPX_HIP_CHECK(hipGetLastError());
+    VPX_LAUNCH((mvn_chunk_kernel<2, ALIGNED>), dim3(blocks), dim3(kThreads), 0, s, in, out, group_size, chunks,
+               partial, use_merged, nv, eps);
     return VPX_RESULT_SUCCESS;
 }
 
@@ -1045,13 +1037,12 @@ static int launch_sum_cminor(const half_t* in, int64_t N, int64_t S, int64_t C, 
     if (C % 8 == 0 && C >= 8 && C <= 2048 && (reinterpret_cast<uintptr_t>(in) & 15) == 0) {
         const int slots = kThreads / (int)(C / 8);
         const size_t lds = sizeof(float2) * (size_t)slots * (size_t)C;  // at most 16 KiB
-        hipLaunchKernelGGL(mvn_sum_cminor8_kernel<SHIFT>, dim3((unsigned)(N * subparts)), dim3(kThreads), lds, s, in, S, C, (int)subparts,
-                           cpad, partial);
+        VPX_LAUNCH(mvn_sum_cminor8_kernel<SHIFT>, dim3((unsigned)(N * subparts)), dim3(kThreads), lds, s, in, S, C, (int)subparts,
+                   cpad, partial);
     } else {
-        hipLaunchKernelGGL(mvn_sum_cminor_kernel<SHIFT>, dim3((unsigned)(N * subparts * (cpad / 64))), dim3(kThreads), 0, s, in, S, C,
-                           (int)subparts, cpad, partial);
+        VPX_LAUNCH(mvn_sum_cminor_kernel<SHIFT>, dim3((unsigned)(N * subparts * (cpad / 64))), dim3(kThreads), 0, s, in, S, C,
+                   (int)subparts, cpad, partial);
     }
-    VPX_HIP_CHECK(hipGetLastError());
     return VPX_RESULT_SUCCESS;
 }
 
@@ -1562,11 +1553,11 @@ int launch_rows_of(const half_t* pi, half_t* po, const half_t* ps, const half_t*
         constexpr int T = team_threads(TEAM), PER = RPT * (T / TEAM);                                                        \
         const dim3 grid((unsigned)((g.rows + PER - 1) / PER));                                                               \
         if (words)                                                                                                           \
-            hipLaunchKernelGGL((mvn6_rows_kernel<GEOM, TEAM, VPT, RPT, true>), grid, dim3(T), 0, s, pi, po, ps, pb, g, nv,         \
-                               eps_mode, eps);                                                                               \
+            VPX_LAUNCH((mvn6_rows_kernel<GEOM, TEAM, VPT, RPT, true>), grid, dim3(T), 0, s, pi, po, ps, pb, g, nv,                 \
+                       eps_mode, eps);                                                                                       \
         else                                                                                                                 \
-            hipLaunchKernelGGL((mvn6_rows_kernel<GEOM, TEAM, VPT, RPT, false>), grid, dim3(T), 0, s, pi, po, ps, pb, g, nv,        \
-                               eps_mode, eps);                                                                               \
+            VPX_LAUNCH((mvn6_rows_kernel<GEOM, TEAM, VPT, RPT, false>), grid, dim3(T), 0, s, pi, po, ps, pb, g, nv,                \
+                       eps_mode, eps);                                                                                       \
     } while (0)
 #define VPX_MVN6_ROWS(TEAM, VPT) VPX_MVN6_ROWS_R(TEAM, VPT, 1)
 #define VPX_MVN6_SHORT(TEAM, VPT)                         \
@@ -1611,7 +1602,6 @@ int launch_rows_of(const half_t* pi, half_t* po, const half_t* ps, const half_t*
 #undef VPX_MVN6_ROWS
 #undef VPX_MVN6_ROWS_R
 #undef VPX_MVN6_SHORT
-    VPX_HIP_CHECK(hipGetLastError());
     return VPX_RESULT_SUCCESS;
 }
 
@@ -1665,18 +1655,16 @@ int launch_channel_minor(const half_t* in, half_t* out, int64_t N, int64_t S, in
     float* stats = (float*)((char*)ws + partial_bytes);
     rc = launch_sum_cminor<true>(in, N, S, C, subparts, cpad, partial, s);
     if (rc) return rc;
-    hipLaunchKernelGGL(mvn_cminor_stats_kernel, dim3((unsigned)((N * C + kThreads - 1) / kThreads)), dim3(kThreads), 0, s, in,
-                       (const float2*)partial, stats, N * C, S, C, cpad, (int)subparts, nv, eps);
-    VPX_HIP_CHECK(hipGetLastError());
+    VPX_LAUNCH(mvn_cminor_stats_kernel, dim3((unsigned)((N * C + kThreads - 1) / kThreads)), dim3(kThreads), 0, s, in,
+               (const float2*)partial, stats, N * C, S, C, cpad, (int)subparts, nv, eps);
     const bool vec = C % 8 == 0 && ((reinterpret_cast<uintptr_t>(in) | reinterpret_cast<uintptr_t>(out)) & 15) == 0 &&
                      (reinterpret_cast<uintptr_t>(stats) & 31) == 0;
     if (vec)
-        hipLaunchKernelGGL((mvn_norm_cminor_kernel<float, true>), dim3((unsigned)(N * pieces)), dim3(kThreads), 0, s, in, out,
-                           (const float*)stats, per_n, C, (int)pieces, 2);
+        VPX_LAUNCH((mvn_norm_cminor_kernel<float, true>), dim3((unsigned)(N * pieces)), dim3(kThreads), 0, s, in, out,
+                   (const float*)stats, per_n, C, (int)pieces, 2);
     else
-        hipLaunchKernelGGL((mvn_norm_cminor_kernel<float, false>), dim3((unsigned)(N * pieces)), dim3(kThreads), 0, s, in, out,
-                           (const float*)stats, per_n, C, (int)pieces, 2);
-    VPX_HIP_CHECK(hipGetLastError());
+        VPX_LAUNCH((mvn_norm_cminor_kernel<float, false>), dim3((unsigned)(N * pieces)), dim3(kThreads), 0, s, in, out,
+                   (const float*)stats, per_n, C, (int)pieces, 2);
     return VPX_RESULT_SUCCESS;
 }
 
@@ -1770,9 +1758,8 @@ int launch_mvn_sum(const MemRef& in, const MemRef& out, bool across_channels, bo
         if (rc) return rc;
         rc = launch_sum_cminor<false>(pi, sh.N, sh.S, sh.C, subparts, cpad, (float2*)ws, s);
         if (rc) return rc;
-        hipLaunchKernelGGL(mvn_sum_cminor_finish_kernel, dim3((unsigned)((total + kThreads - 1) / kThreads)), dim3(kThreads), 0,
-                           s, (const float2*)ws, total, sh.C, cpad, (int)subparts, (int)isplit, o);
-        VPX_HIP_CHECK(hipGetLastError());
+        VPX_LAUNCH(mvn_sum_cminor_finish_kernel, dim3((unsigned)((total + kThreads - 1) / kThreads)), dim3(kThreads), 0,
+                   s, (const float2*)ws, total, sh.C, cpad, (int)subparts, (int)isplit, o);
         return VPX_RESULT_SUCCESS;
     }
 
@@ -1791,16 +1778,14 @@ int launch_mvn_sum(const MemRef& in, const MemRef& out, bool across_channels, bo
     const bool aligned = group_size % 8 == 0 && (reinterpret_cast<uintptr_t>(pi) & 15) == 0;
     const dim3 grid((unsigned)(groups * chunks));
     if (aligned)
-        hipLaunchKernelGGL((mvn_sum_chunk_kernel<true>), grid, dim3(kThreads), 0, s, pi, group_size, chunks, (float2*)ws, o,
-                           direct ? 1 : 0);
+        VPX_LAUNCH((mvn_sum_chunk_kernel<true>), grid, dim3(kThreads), 0, s, pi, group_size, chunks, (float2*)ws, o,
+                   direct ? 1 : 0);
     else
-        hipLaunchKernelGGL((mvn_sum_chunk_kernel<false>), grid, dim3(kThreads), 0, s, pi, group_size, chunks, (float2*)ws, o,
-                           direct ? 1 : 0);
-    VPX_HIP_CHECK(hipGetLastError());
+        VPX_LAUNCH((mvn_sum_chunk_kernel<false>), grid, dim3(kThreads), 0, s, pi, group_size, chunks, (float2*)ws, o,
+                   direct ? 1 : 0);
     if (!direct) {
-        hipLaunchKernelGGL(mvn_sum_finish_kernel, dim3((unsigned)(groups * o.parts)), dim3(kThreads), 0, s, (const float2*)ws,
-                           chunks, o);
-        VPX_HIP_CHECK(hipGetLastError());
+        VPX_LAUNCH(mvn_sum_finish_kernel, dim3((unsigned)(groups * o.parts)), dim3(kThreads), 0, s, (const float2*)ws,
+                   chunks, o);
     }
     return VPX_RESULT_SUCCESS;
 }
@@ -1834,12 +1819,11 @@ int launch_mvn_mean_var(const MemRef& sum, const MemRef& out, const int64_t orig
     const double count = (double)orig_shape[2] * (double)orig_shape[3] * (double)(across_channels ? C : group_c);
     const dim3 grid((unsigned)((N * out_c + kThreads - 1) / kThreads));
     if (out.dtype == VPX_NN_FP16)
-        hipLaunchKernelGGL((mvn_mean_var_kernel<half_t>), grid, dim3(kThreads), 0, s, (const float*)sum.data, (half_t*)out.data, N,
-                           id[1], (int)id[2], (int)id[3], out_c, out_w, across_channels ? 1 : 0, group_c, count, eps);
+        VPX_LAUNCH((mvn_mean_var_kernel<half_t>), grid, dim3(kThreads), 0, s, (const float*)sum.data, (half_t*)out.data, N,
+                   id[1], (int)id[2], (int)id[3], out_c, out_w, across_channels ? 1 : 0, group_c, count, eps);
     else
-        hipLaunchKernelGGL((mvn_mean_var_kernel<float>), grid, dim3(kThreads), 0, s, (const float*)sum.data, (float*)out.data, N,
-                           id[1], (int)id[2], (int)id[3], out_c, out_w, across_channels ? 1 : 0, group_c, count, eps);
-    VPX_HIP_CHECK(hipGetLastError());
+        VPX_LAUNCH((mvn_mean_var_kernel<float>), grid, dim3(kThreads), 0, s, (const float*)sum.data, (float*)out.data, N,
+                   id[1], (int)id[2], (int)id[3], out_c, out_w, across_channels ? 1 : 0, group_c, count, eps);
     return VPX_RESULT_SUCCESS;
 }
 
@@ -1858,12 +1842,11 @@ static int mvn_norm_impl(const MemRef& in, const MemRef& mv, const MemRef& out, 
         const bool vec = sh.C % 8 == 0 && ((reinterpret_cast<uintptr_t>(pi) | reinterpret_cast<uintptr_t>(po)) & 15) == 0 &&
                          (reinterpret_cast<uintptr_t>(pm) & 31) == 0;
         if (vec)
-            hipLaunchKernelGGL((mvn_norm_cminor_kernel<TS, true>), dim3((unsigned)(sh.N * pieces)), dim3(kThreads), 0, s, pi, po, pm,
-                               per_n, sh.C, (int)pieces, out_w);
+            VPX_LAUNCH((mvn_norm_cminor_kernel<TS, true>), dim3((unsigned)(sh.N * pieces)), dim3(kThreads), 0, s, pi, po, pm,
+                       per_n, sh.C, (int)pieces, out_w);
         else
-            hipLaunchKernelGGL((mvn_norm_cminor_kernel<TS, false>), dim3((unsigned)(sh.N * pieces)), dim3(kThreads), 0, s, pi, po, pm,
-                               per_n, sh.C, (int)pieces, out_w);
-        VPX_HIP_CHECK(hipGetLastError());
+            VPX_LAUNCH((mvn_norm_cminor_kernel<TS, false>), dim3((unsigned)(sh.N * pieces)), dim3(kThreads), 0, s, pi, po, pm,
+                       per_n, sh.C, (int)pieces, out_w);
         return VPX_RESULT_SUCCESS;
     }
     const int64_t rows = across_channels ? sh.N : sh.N * sh.C;
@@ -1875,12 +1858,11 @@ static int mvn_norm_impl(const MemRef& in, const MemRef& mv, const MemRef& out, 
     const int64_t out_c = across_channels ? 1 : sh.C;
     const dim3 grid((unsigned)(rows * pieces));
     if (aligned)
-        hipLaunchKernelGGL((mvn_norm_runs_kernel<TS, true>), grid, dim3(kThreads), 0, s, pi, po, pm, run, (int)pieces, rows_per_n,
-                           out_c, out_w);
+        VPX_LAUNCH((mvn_norm_runs_kernel<TS, true>), grid, dim3(kThreads), 0, s, pi, po, pm, run, (int)pieces, rows_per_n,
+                   out_c, out_w);
     else
-        hipLaunchKernelGGL((mvn_norm_runs_kernel<TS, false>), grid, dim3(kThreads), 0, s, pi, po, pm, run, (int)pieces, rows_per_n,
-                           out_c, out_w);
-    VPX_HIP_CHECK(hipGetLastError());
+        VPX_LAUNCH((mvn_norm_runs_kernel<TS, false>), grid, dim3(kThreads), 0, s, pi, po, pm, run, (int)pieces, rows_per_n,
+                   out_c, out_w);
     return VPX_RESULT_SUCCESS;
 }
 
@@ -2050,15 +2032,14 @@ int launch_mvn6(const MemRef& in, const MemRef* scale, const MemRef* bias, const
         const int64_t outer = g.rows / g.kdim[0];
         const auto blocks = [&](int p) { return outer * ((g.kdim[0] + p - 1) / p); };
         if (blocks(64) >= 512)
-            hipLaunchKernelGGL(mvn6_inner_kernel<64>, dim3((unsigned)blocks(64)), dim3(kThreads), 0, s, pi, po, ps, pb, g, nv, eps_mode, eps);
+            VPX_LAUNCH(mvn6_inner_kernel<64>, dim3((unsigned)blocks(64)), dim3(kThreads), 0, s, pi, po, ps, pb, g, nv, eps_mode, eps);
         else if (blocks(32) >= 512)
-            hipLaunchKernelGGL(mvn6_inner_kernel<32>, dim3((unsigned)blocks(32)), dim3(kThreads), 0, s, pi, po, ps, pb, g, nv, eps_mode, eps);
+            VPX_LAUNCH(mvn6_inner_kernel<32>, dim3((unsigned)blocks(32)), dim3(kThreads), 0, s, pi, po, ps, pb, g, nv, eps_mode, eps);
         else
-            hipLaunchKernelGGL(mvn6_inner_kernel<16>, dim3((unsigned)blocks(16)), dim3(kThreads), 0, s, pi, po, ps, pb, g, nv, eps_mode, eps);
+            VPX_LAUNCH(mvn6_inner_kernel<16>, dim3((unsigned)blocks(16)), dim3(kThreads), 0, s, pi, po, ps, pb, g, nv, eps_mode, eps);
     } else {
-        hipLaunchKernelGGL(mvn6_generic_kernel, dim3((unsigned)g.rows), dim3(kThreads), 0, s, pi, po, ps, pb, g, nv, eps_mode, eps);
+        VPX_LAUNCH(mvn6_generic_kernel, dim3((unsigned)g.rows), dim3(kThreads), 0, s, pi, po, ps, pb, g, nv, eps_mode, eps);
     }
-    VPX_HIP_CHECK(hipGetLastError());
     return VPX_RESULT_SUCCESS;
 }
 

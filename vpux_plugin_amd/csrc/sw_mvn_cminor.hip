@@ -545,7 +545,7 @@ int launch_mvn_cminor_resident(const void* in, void* out, int64_t N, int64_t S, 
     const unsigned long long spin = mode == 2 ? 0ull : 50000ull;  // 0.5 ms of the 100 MHz counter
     const dim3 grid((unsigned)blocks);
 #define VPX_CMINOR_AS(V, FORM) \
-    hipLaunchKernelGGL((mvn_cminor_resident<V, FORM>), grid, dim3(kT), 0, s, (const half_t*)in, (half_t*)out, best, (unsigned*)sync, nv, eps, spin)
+    VPX_LAUNCH((mvn_cminor_resident<V, FORM>), grid, dim3(kT), 0, s, (const half_t*)in, (half_t*)out, best, (unsigned*)sync, nv, eps, spin)
 #define VPX_CMINOR(V)                           \
     do {                                        \
         if (best_rows) VPX_CMINOR_AS(V, kRows);   \
@@ -563,7 +563,6 @@ int launch_mvn_cminor_resident(const void* in, void* out, int64_t N, int64_t S, 
     else VPX_CMINOR(kMostWords);
 #undef VPX_CMINOR
 #undef VPX_CMINOR_AS
-    VPX_HIP_CHECK(hipGetLastError());
     *done = true;
     return VPX_RESULT_SUCCESS;
 }

@@ -885,10 +885,11 @@ __global__ __launch_bounds__(1024) void softmax_cols(const T* __restrict__ in, T
 }
 
 template <typename T, int NV, int ROWS>
-void launch_rows_wave(const T* in, T* out, const RowMap& map, int64_t rows, int len, int valid, hipStream_t s) {
+int launch_rows_wave(const T* in, T* out, const RowMap& map, int64_t rows, int len, int valid, hipStream_t s) {
     const int64_t waves = (rows + ROWS - 1) / ROWS;
     const unsigned blocks = (unsigned)((waves + 3) / 4);
-    hipLaunchKernelGGL((softmax_rows_wave<T, NV, ROWS>), dim3(blocks), dim3(256), 0, s, in, out, map, rows, len, valid);
+    VPX_LAUNCH((softmax_rows_wave<T, NV, ROWS>), dim3(blocks), dim3(256), 0, s, in, out, map, rows, len, valid);
+    return VPX_RESULT_SUCCESS;
 }
 
 // What the two kernels for an outer axis take, us: fitted to 1530 tensors of 2^16 ... 2^24 values in runs of 2 ... 127, axes of
@@ -953,7 +954,7 @@ int softmax_typed(const SoftmaxPlan& p, const T* in, T* out, hipStream_t s) {
         if (packed && base16 && (len == 8 || len == 16 || len == 32 || len == 64 || len == 128 || len == 256) && rows * (len / 8) < (1ll << 39)) {
             const int64_t n_vec = rows * (len / 8);
             const dim3 grid((unsigned)((n_vec + 255) / 256));
-#define VPX_TINY(T) hipLaunchKernelGGL(softmax_tiny_rows_f16<T>, grid, dim3(256), 0, s, hin, hout, n_vec)
+#define VPX_TINY(T) VPX_LAUNCH(softmax_tiny_rows_f16<T>, grid, dim3(256), 0, s, hin, hout, n_vec)
             if (len == 8) VPX_TINY(1);
             else if (len == 16) VPX_TINY(2);
             else if (len == 32) VPX_TINY(4);
@@ -961,7 +962,6 @@ int softmax_typed(const SoftmaxPlan& p, const T* in, T* out, hipStream_t s) {
             else if (len == 128) VPX_TINY(16);
             else VPX_TINY(32);
 #undef VPX_TINY
-            VPX_HIP_CHECK(hipGetLastError());
             return VPX_RESULT_SUCCESS;
         }
         // rows of any other length up to 2048 values one after another: registers, unless softmax_rows_f16 has whole words of them from 256 on (us in a
@@ -990,10 +990,11 @@ int softmax_typed(const SoftmaxPlan& p, const T* in, T* out, hipStream_t s) {
                 const dim3 grid((n + per - 1) / per);
                 const half_t* from = hin + r0 * len;
                 half_t* to = hout + r0 * len;
-                const auto form = [&](auto team_c, auto words_c) {
+                const auto form = [&](auto team_c, auto words_c) -> int {
                     constexpr int LANES = decltype(team_c)::value, WORDS = decltype(words_c)::value;
-                    if (once) hipLaunchKernelGGL((softmax_packed_rows<LANES, WORDS, true>), grid, dim3(256), 0, s, from, to, n, (uint32_t)len);
-                    else hipLaunchKernelGGL((softmax_packed_rows<LANES, WORDS, false>), grid, dim3(256), 0, s, from, to, n, (uint32_t)len);
+                    if (once) VPX_LAUNCH((softmax_packed_rows<LANES, WORDS, true>), grid, dim3(256), 0, s, from, to, n, (uint32_t)len);
+                    else VPX_LAUNCH((softmax_packed_rows<LANES, WORDS, false>), grid, dim3(256), 0, s, from, to, n, (uint32_t)len);
+                    return VPX_RESULT_SUCCESS;
                 };
                 constexpr std::integral_constant<int, 1> one{};
                 constexpr std::integral_constant<int, 2> two{};
@@ -1003,12 +1004,12 @@ int softmax_typed(const SoftmaxPlan& p, const T* in, T* out, hipStream_t s) {
                 constexpr std::integral_constant<int, 16> t16{};
                 constexpr std::integral_constant<int, 32> t32{};
                 constexpr std::integral_constant<int, 64> t64{};
-                if (team == 4) form(four, one);
-                else if (team == 8) words == 1 ? form(t8, one) : form(t8, two);
-                else if (team == 16) words == 1 ? form(t16, one) : words == 2 ? form(t16, two) : form(t16, three);
-                else if (team == 32) words == 1 ? form(t32, one) : words == 2 ? form(t32, two) : form(t32, three);
-                else words == 1 ? form(t64, one) : words == 2 ? form(t64, two) : words == 3 ? form(t64, three) : form(t64, four);
-                VPX_HIP_CHECK(hipGetLastError());
+                const int rc = team == 4    ? form(four, one)
+                               : team == 8  ? (words == 1 ? form(t8, one) : form(t8, two))
+                               : team == 16 ? (words == 1 ? form(t16, one) : words == 2 ? form(t16, two) : form(t16, three))
+                               : team == 32 ? (words == 1 ? form(t32, one) : words == 2 ? form(t32, two) : form(t32, three))
+                                            : (words == 1 ? form(t64, one) : words == 2 ? form(t64, two) : words == 3 ? form(t64, three) : form(t64, four));
+                if (rc) return rc;
             }
             return VPX_RESULT_SUCCESS;
         }
@@ -1023,8 +1024,7 @@ int softmax_typed(const SoftmaxPlan& p, const T* in, T* out, hipStream_t s) {
             const int64_t spread = (rows / (2 * cus) + 7) / 8 * 8;
             if (per_wg > spread) per_wg = spread < 8 ? 8 : (int)spread;
             const dim3 grid((unsigned)((rows + per_wg - 1) / per_wg));
-            hipLaunchKernelGGL(softmax_short_rows_f16, grid, dim3(256), 0, s, hin, hout, rows, (int)len, per_wg);
-            VPX_HIP_CHECK(hipGetLastError());
+            VPX_LAUNCH(softmax_short_rows_f16, grid, dim3(256), 0, s, hin, hout, rows, (int)len, per_wg);
             return VPX_RESULT_SUCCESS;
         }
         if (aligned || same_mis) {
@@ -1034,9 +1034,9 @@ int softmax_typed(const SoftmaxPlan& p, const T* in, T* out, hipStream_t s) {
             const dim3 gw((unsigned)((rows + 3) / 4)), gb((unsigned)rows);
 #define VPX_SM(NV, ROWS, LANES, GRID)                                                                                 \
     do {                                                                                                              \
-        if (aligned && once) hipLaunchKernelGGL((softmax_rows_f16<NV, ROWS, LANES, false, true>), GRID, block, 0, s, hin, hout, map, rows, l); \
-        else if (aligned) hipLaunchKernelGGL((softmax_rows_f16<NV, ROWS, LANES, false, false>), GRID, block, 0, s, hin, hout, map, rows, l); \
-        else hipLaunchKernelGGL((softmax_rows_f16<NV, ROWS, LANES, true, false>), GRID, block, 0, s, hin, hout, map, rows, l);         \
+        if (aligned && once) VPX_LAUNCH((softmax_rows_f16<NV, ROWS, LANES, false, true>), GRID, block, 0, s, hin, hout, map, rows, l);         \
+        else if (aligned) VPX_LAUNCH((softmax_rows_f16<NV, ROWS, LANES, false, false>), GRID, block, 0, s, hin, hout, map, rows, l);         \
+        else VPX_LAUNCH((softmax_rows_f16<NV, ROWS, LANES, true, false>), GRID, block, 0, s, hin, hout, map, rows, l);                 \
     } while (0)
             // short rows, many of them: two rows per wave keep more bytes in flight (measured best)
             if (span <= 512 && rows >= 16384) VPX_SM(1, 2, 64, dim3((unsigned)((rows + 7) / 8)));
@@ -1049,7 +1049,6 @@ int softmax_typed(const SoftmaxPlan& p, const T* in, T* out, hipStream_t s) {
             else if (span <= 16384) VPX_SM(8, 1, 256, gb);
             else VPX_SM(16, 1, 256, gb);
 #undef VPX_SM
-            VPX_HIP_CHECK(hipGetLastError());
             return VPX_RESULT_SUCCESS;
         }
     }
@@ -1062,12 +1061,10 @@ int softmax_typed(const SoftmaxPlan& p, const T* in, T* out, hipStream_t s) {
             const int l = (int)len, v = (int)valid;
             const int64_t per = 64 * N;
             // general form (fp32, padded axis)
-            if (len <= per) launch_rows_wave<T, 1, 1>(in, out, map, rows, l, v, s);
-            else if (len <= 2 * per) launch_rows_wave<T, 2, 1>(in, out, map, rows, l, v, s);
-            else if (len <= 4 * per) launch_rows_wave<T, 4, 1>(in, out, map, rows, l, v, s);
-            else launch_rows_wave<T, 8, 1>(in, out, map, rows, l, v, s);
-            VPX_HIP_CHECK(hipGetLastError());
-            return VPX_RESULT_SUCCESS;
+            if (len <= per) return launch_rows_wave<T, 1, 1>(in, out, map, rows, l, v, s);
+            if (len <= 2 * per) return launch_rows_wave<T, 2, 1>(in, out, map, rows, l, v, s);
+            if (len <= 4 * per) return launch_rows_wave<T, 4, 1>(in, out, map, rows, l, v, s);
+            return launch_rows_wave<T, 8, 1>(in, out, map, rows, l, v, s);
         }
     }
     if (inner && std::is_same<T, half_t>::value && valid == len && len % 8 == 0 && len <= kLdsRowMax && rows >= 64 &&
@@ -1077,21 +1074,18 @@ int softmax_typed(const SoftmaxPlan& p, const T* in, T* out, hipStream_t s) {
         if (al) {
             VPX_HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(softmax_lds_rows_f16), hipFuncAttributeMaxDynamicSharedMemorySize,
                                               kLdsRowMax * 2));
-            hipLaunchKernelGGL(softmax_lds_rows_f16, dim3((unsigned)rows), dim3(1024), (size_t)len * 2, s, reinterpret_cast<const half_t*>(in),
-                               reinterpret_cast<half_t*>(out), map, (int)len);
-            VPX_HIP_CHECK(hipGetLastError());
+            VPX_LAUNCH(softmax_lds_rows_f16, dim3((unsigned)rows), dim3(1024), (size_t)len * 2, s, reinterpret_cast<const half_t*>(in),
+                       reinterpret_cast<half_t*>(out), map, (int)len);
             return VPX_RESULT_SUCCESS;
         }
     }
     if (ax == 0 && p.in_stride[0] == 1 && p.out_stride[0] == 1 && len >= 2048) {
-        hipLaunchKernelGGL(softmax_long_rows<T>, dim3((unsigned)rows), dim3(1024), 0, s, in, out, map, len, valid);
-        VPX_HIP_CHECK(hipGetLastError());
+        VPX_LAUNCH(softmax_long_rows<T>, dim3((unsigned)rows), dim3(1024), 0, s, in, out, map, len, valid);
         return VPX_RESULT_SUCCESS;
     }
     if (ax == 0) {
-        hipLaunchKernelGGL(softmax_rows_block<T>, dim3((unsigned)rows), dim3(256), 0, s, in, out, map, len, valid,
-                           p.in_stride[0], p.out_stride[0]);
-        VPX_HIP_CHECK(hipGetLastError());
+        VPX_LAUNCH(softmax_rows_block<T>, dim3((unsigned)rows), dim3(256), 0, s, in, out, map, len, valid,
+                   p.in_stride[0], p.out_stride[0]);
         return VPX_RESULT_SUCCESS;
     }
     // fp16, outer axis, contiguous inner dimension: register-resident slabs
@@ -1173,7 +1167,7 @@ int softmax_typed(const SoftmaxPlan& p, const T* in, T* out, hipStream_t s) {
                 const int by_die = lines ? 0 : 1;
                 const dim3 grid((unsigned)(kw == 1 ? (tiles + 3) / 4 : tiles)), block(kw == 1 ? 256 : 64 * kw);
 #define VPX_SLAB_NT(VEC, KW, SMAX, CL, NT) \
-    hipLaunchKernelGGL((softmax_slab_f16<VEC, KW, SMAX, CL, NT>), grid, block, 0, s, hin, hout, om, tiles, tpo, L, I, in_as, out_as, by_die)
+    VPX_LAUNCH((softmax_slab_f16<VEC, KW, SMAX, CL, NT>), grid, block, 0, s, hin, hout, om, tiles, tpo, L, I, in_as, out_as, by_die)
 #define VPX_SLAB(VEC, KW, SMAX)                                      \
     do {                                                             \
         if (small) VPX_SLAB_NT(VEC, KW, SMAX, 64, false);            \
@@ -1205,7 +1199,6 @@ int softmax_typed(const SoftmaxPlan& p, const T* in, T* out, hipStream_t s) {
 #undef VPX_SLAB_NT
 #undef VPX_SLAB_HALF
 #undef VPX_SLAB
-                VPX_HIP_CHECK(hipGetLastError());
                 return VPX_RESULT_SUCCESS;
             }
         }
@@ -1247,22 +1240,20 @@ int softmax_typed(const SoftmaxPlan& p, const T* in, T* out, hipStream_t s) {
             const int64_t tpo = (inner + 64 * vec - 1) / (64 * vec);
             if (outer * tpo < (1ll << 22)) {  // 2^32 lanes in a launch
                 const dim3 grid((unsigned)(outer * tpo));
-#define VPX_COLS(V) hipLaunchKernelGGL((softmax_cols<T, V>), grid, dim3(1024), 0, s, in, out, om, (int)tpo, len, valid, inner, in_as, out_as)
+#define VPX_COLS(V) VPX_LAUNCH((softmax_cols<T, V>), grid, dim3(1024), 0, s, in, out, om, (int)tpo, len, valid, inner, in_as, out_as)
                 if (vec == 8) {
                     if constexpr (sizeof(T) == 2) VPX_COLS(8);
                 } else if (vec == 4) VPX_COLS(4);
                 else if (vec == 2) VPX_COLS(2);
                 else VPX_COLS(1);
 #undef VPX_COLS
-                VPX_HIP_CHECK(hipGetLastError());
                 return VPX_RESULT_SUCCESS;
             }
         }
     }
     const unsigned blocks = (unsigned)((rows + 255) / 256);
-    hipLaunchKernelGGL(softmax_lines<T>, dim3(blocks), dim3(256), 0, s, in, out, map, rows, len, valid, p.in_stride[ax],
-                       p.out_stride[ax]);
-    VPX_HIP_CHECK(hipGetLastError());
+    VPX_LAUNCH(softmax_lines<T>, dim3(blocks), dim3(256), 0, s, in, out, map, rows, len, valid, p.in_stride[ax],
+               p.out_stride[ax]);
     return VPX_RESULT_SUCCESS;
 }
 
@@ -1334,13 +1325,12 @@ int launch_softmax_dynamic(const MemRef& in, const MemRef& out, int axis, int pa
     DynDims dd{in.live_dims, in.live_strides, out.live_strides, in.nd, axis, pad, in.elem_bits, {}};
     for (int d = 0; d < in.nd; d++) dd.bound[d] = (int32_t)in.dims[d];
     if (in.dtype == VPX_NN_FP16) {
-        hipLaunchKernelGGL(softmax_dynamic_kernel<half_t>, dim3((unsigned)rows), dim3(256), 0, s, (const half_t*)in.data, (half_t*)out.data, dd);
+        VPX_LAUNCH(softmax_dynamic_kernel<half_t>, dim3((unsigned)rows), dim3(256), 0, s, (const half_t*)in.data, (half_t*)out.data, dd);
     } else if (in.dtype == VPX_NN_FP32) {
-        hipLaunchKernelGGL(softmax_dynamic_kernel<float>, dim3((unsigned)rows), dim3(256), 0, s, (const float*)in.data, (float*)out.data, dd);
+        VPX_LAUNCH(softmax_dynamic_kernel<float>, dim3((unsigned)rows), dim3(256), 0, s, (const float*)in.data, (float*)out.data, dd);
     } else {
         return fail(VPX_RESULT_ERROR_UNSUPPORTED_FEATURE, "softmax: element type %s is not implemented", dtype_name(in.dtype));
     }
-    VPX_HIP_CHECK(hipGetLastError());
     return VPX_RESULT_SUCCESS;
 }
 

@@ -12,7 +12,6 @@
 
 namespace vpx {
 int fail(int code, const char* fmt, ...) __attribute__((format(printf, 2, 3)));
-std::string& last_error();
 }  // namespace vpx
 
 namespace vpx {
@@ -307,32 +306,34 @@ int vpx_generate_softmax_attr(uint32_t rank, const int64_t* dims, const int64_t*
         return fail(VPX_RESULT_ERROR_INVALID_ARGUMENT, "softmax parameters: axis %lld outside rank %u", (long long)axis, rank);
     struct Level {
         int64_t size, in_step, out_step;
-        bool reduced;  // the softmax axis
     };
+    // (a launch derives this: nothing of it is on the heap)
+    Level kept[VPX_MAX_ND_DIMS], levels[VPX_MAX_ND_DIMS + 3];
+    size_t n_kept = 0, n_levels = 0, axis_at = 0;
     // 1. levels of size one say nothing, except the axis itself
-    std::vector<Level> kept;
-    for (uint32_t d = 0; d < rank; d++)
-        if (dims[d] != 1 || (int64_t)d == axis) kept.push_back(Level{dims[d], in_strides[d], out_strides[d], (int64_t)d == axis});
+    for (uint32_t d = 0; d < rank; d++) {
+        if ((int64_t)d == axis) axis_at = n_kept;
+        if (dims[d] != 1 || (int64_t)d == axis) kept[n_kept++] = Level{dims[d], in_strides[d], out_strides[d]};
+    }
     // 2. above the axis, neighbours that both operands walk without a gap become one level
-    size_t axis_at = 0;
-    while (!kept[axis_at].reduced) axis_at++;
-    std::vector<Level> levels(kept.begin(), kept.begin() + (std::ptrdiff_t)axis_at + 1);
-    for (size_t d = axis_at + 1; d < kept.size(); d++) {
+    for (; n_levels <= axis_at; n_levels++) levels[n_levels] = kept[n_levels];
+    for (size_t d = axis_at + 1; d < n_kept; d++) {
         const Level& below = kept[d - 1];
         const bool gapless = kept[d].in_step == below.in_step * below.size && kept[d].out_step == below.out_step * below.size;
         if (d >= axis_at + 2 && gapless)
-            levels.back().size *= kept[d].size;
+            levels[n_levels - 1].size *= kept[d].size;
         else
-            levels.push_back(kept[d]);
+            levels[n_levels++] = kept[d];
     }
     // 3. an innermost axis that is not unit-stride is served as an outer axis over an inner level of one element
     if (axis_at == 0 && (levels[0].in_step > 1 || levels[0].out_step > 1)) {
-        levels.insert(levels.begin(), Level{1, levels[0].in_step, levels[0].out_step, false});
+        for (size_t d = n_levels++; d > 0; d--) levels[d] = levels[d - 1];
+        levels[0].size = 1;
         axis_at = 1;
     }
     // 4. the kernel wants at least three levels: unit levels stacked on the outermost one
-    const Level top = levels.back();
-    while (levels.size() < 3) levels.push_back(Level{1, top.in_step * top.size, top.out_step * top.size, false});
+    const Level top = levels[n_levels - 1];
+    while (n_levels < 3) levels[n_levels++] = Level{1, top.in_step * top.size, top.out_step * top.size};
 
     int64_t mode = VPX_SOFTMAX_OUTER;
     if (axis_at == 0) {
@@ -343,10 +344,10 @@ int vpx_generate_softmax_attr(uint32_t rank, const int64_t* dims, const int64_t*
     const auto two_i32 = [](int64_t lo, int64_t hi) { return ((uint64_t)(uint32_t)hi << 32) | (uint64_t)(uint32_t)lo; };
     uint32_t n = 0;
     words[n++] = two_i32((int64_t)axis_at, pad_size);
-    words[n++] = two_i32(mode, (int64_t)levels.size());
-    for (const Level& l : levels) {
-        words[n++] = two_i32(l.size, l.size);
-        words[n++] = two_i32(l.in_step, l.out_step);
+    words[n++] = two_i32(mode, (int64_t)n_levels);
+    for (size_t d = 0; d < n_levels; d++) {
+        words[n++] = two_i32(levels[d].size, levels[d].size);
+        words[n++] = two_i32(levels[d].in_step, levels[d].out_step);
     }
     *n_words = n;
     return VPX_RESULT_SUCCESS;

@@ -3,7 +3,7 @@
 // What bounds a call on a small tensor is the host: the kernel of a FakeQuantize over [1,64,56,56] takes 3 us, a bare
 // hipLaunchKernel 2.4 us.  Describing the operands through ctypes and numpy objects took 12 ... 23 us more per call
 // (torch.cuda.current_stream() alone 2.9 us); here the tensors' sizes, strides and addresses are read from their C++
-// objects, the params blob or the task is laid out on the stack / in a kept buffer, and the same entry points of
+// objects, the params blob or the task is laid out on the stack, and the same entry points of
 // include/vpx_runtime.h that any other host would call are called.  Nothing is remembered between calls.
 #include <torch/csrc/autograd/python_variable.h>
 #include <c10/hip/HIPStream.h>
@@ -28,7 +28,7 @@ struct Raised {};
 }
 
 const at::Tensor& tensor(PyObject* o) {
-    if (!THPVariable_Check(o)) {
+    if (Py_TYPE(o) != reinterpret_cast<PyTypeObject*>(THPVariableClass) && !THPVariable_Check(o)) {
         PyErr_Format(PyExc_TypeError, "expected a torch tensor, got %s", Py_TYPE(o)->tp_name);
         throw Raised{};
     }
@@ -115,70 +115,67 @@ uint64_t order_code(PyObject* order, int64_t rank) {
     return code;
 }
 
-// The params blob of one launch: MemRefData records, attributes, then input dims | input strides | output dims | output
-// strides (the layout vpx_create_kernel_params writes).  The buffer is the thread's own and keeps its storage.
-struct Blob {
-    std::vector<uint8_t>& bytes;
-    std::vector<vpx_memref_addr_t>& addrs;
-
-    static Blob fresh() {
-        static thread_local std::vector<uint8_t> bytes;
-        static thread_local std::vector<vpx_memref_addr_t> addrs;
-        bytes.clear();
-        addrs.clear();
-        return Blob{bytes, addrs};
-    }
-    void put(const void* p, size_t n) {
-        const size_t at = bytes.size();
-        bytes.resize(at + n);
-        if (n) std::memcpy(bytes.data() + at, p, n);
-    }
-    void memref(const at::Tensor& t, uint64_t order) {
-        vpx_memref_data_t m{};
-        m.isStatic = 1;
-        m.numDims = (uint32_t)t.dim();
-        m.dataType = type_code(t);
-        m.dimsOrder = order;
-        m.location = VPX_LOC_DDR;
-        put(&m, sizeof(m));
-        addrs.push_back(vpx_memref_addr_t{t.data_ptr(), nullptr, nullptr});
-    }
-    void tail(const at::Tensor* const* t, int n) {
-        for (int i = 0; i < n; i++)
-            for (int64_t d = t[i]->dim(); d-- > 0;) {
-                const int32_t v = (int32_t)t[i]->size(d);
-                put(&v, sizeof(v));
-            }
-        for (int i = 0; i < n; i++) {
-            const int64_t bits = (int64_t)t[i]->element_size() * 8;
-            for (int64_t d = t[i]->dim(); d-- > 0;) {
-                const int64_t v = t[i]->stride(d) * bits;
-                put(&v, sizeof(v));
-            }
-        }
-    }
-};
-
 constexpr int kMostTensors = 16, kMostAxes = 32;
 
-// order: one layout for all tensors, or a tuple with one each.
+// The dims, then the strides in bits, of some operands of a blob, innermost first.
+uint8_t* put_shapes(uint8_t* p, const at::Tensor* const* t, int n) {
+    for (int i = 0; i < n; i++) {
+        const auto sizes = t[i]->sizes();
+        for (size_t d = sizes.size(); d-- > 0; p += 4) {
+            const int32_t v = (int32_t)sizes[d];
+            std::memcpy(p, &v, 4);
+        }
+    }
+    for (int i = 0; i < n; i++) {
+        const auto strides = t[i]->strides();
+        const int64_t bits = (int64_t)t[i]->element_size() * 8;
+        for (size_t d = strides.size(); d-- > 0; p += 8) {
+            const int64_t v = strides[d] * bits;
+            std::memcpy(p, &v, 8);
+        }
+    }
+    return p;
+}
+
+// One launch: the params blob is MemRefData records, attributes, then input dims | input strides | output dims | output
+// strides (the layout vpx_create_kernel_params writes).  order: one layout for all tensors, or a tuple with one each.
 PyObject* launch_tensors(const char* entry, int n_in, int n, PyObject* const* objects, PyObject* order, const void* attrs, size_t attrs_size,
                          PyObject* stream, bool noalloc) {
     if (n > kMostTensors || n_in < 0 || n_in > n) raise(PyExc_ValueError, "a number of operands that no launch has");
-    if (PyTuple_Check(order) && PyTuple_GET_SIZE(order) != n) raise(PyExc_ValueError, "one layout per operand, or one for all");
+    const bool each = PyTuple_Check(order);
+    if (each && PyTuple_GET_SIZE(order) != n) raise(PyExc_ValueError, "one layout per operand, or one for all");
     const at::Tensor* t[kMostTensors];
-    Blob b = Blob::fresh();
+    vpx_memref_data_t records[kMostTensors];
+    vpx_memref_addr_t addrs[kMostTensors];
+    size_t levels = 0;
     for (int i = 0; i < n; i++) {
         t[i] = &tensor(objects[i]);
-        b.memref(*t[i], order_code(PyTuple_Check(order) ? PyTuple_GET_ITEM(order, i) : order, t[i]->dim()));
+        const int64_t rank = t[i]->dim();
+        vpx_memref_data_t& m = records[i];
+        m = vpx_memref_data_t{};
+        m.isStatic = 1;
+        m.numDims = (uint32_t)rank;
+        m.dataType = type_code(*t[i]);
+        m.dimsOrder = order_code(each ? PyTuple_GET_ITEM(order, i) : order, rank);
+        m.location = VPX_LOC_DDR;
+        addrs[i] = vpx_memref_addr_t{t[i]->data_ptr(), nullptr, nullptr};
+        levels += (size_t)rank;
     }
-    b.put(attrs, attrs_size);
-    b.tail(t, n_in);
-    b.tail(t + n_in, n - n_in);
+    uint8_t here[2048];  // (six operands of eight dimensions take 800 bytes)
+    std::vector<uint8_t> more;
+    const size_t size = (size_t)n * sizeof(vpx_memref_data_t) + attrs_size + levels * (sizeof(int32_t) + sizeof(int64_t));
+    if (size > sizeof(here)) more.resize(size);
+    uint8_t* const blob = more.empty() ? here : more.data();
+    uint8_t* p = blob;
+    std::memcpy(p, records, (size_t)n * sizeof(vpx_memref_data_t));
+    p += (size_t)n * sizeof(vpx_memref_data_t);
+    if (attrs_size) std::memcpy(p, attrs, attrs_size);
+    p = put_shapes(p + attrs_size, t, n_in);
+    put_shapes(p, t + n_in, n - n_in);
     void* s = stream_handle(stream);
     int rc;
     Py_BEGIN_ALLOW_THREADS
-    rc = (noalloc ? vpx_sw_kernel_launch_noalloc : vpx_sw_kernel_launch)(entry, b.bytes.data(), b.bytes.size(), b.addrs.data(), (uint32_t)n, s);
+    rc = (noalloc ? vpx_sw_kernel_launch_noalloc : vpx_sw_kernel_launch)(entry, blob, size, addrs, (uint32_t)n, s);
     Py_END_ALLOW_THREADS
     return PyLong_FromLong(rc);
 }
