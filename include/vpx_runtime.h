@@ -239,7 +239,7 @@ VPX_API int vpx_nce_task(const vpx_nce_task_t* task, void* stream);
  * the form that stages nothing, which by itself serves layers that are over before a tile is staged; 1,1 / 2,1 / 2,2 with one to
  * eight waves, 2,4 / 4,4 with one, others are refused),
  * "VPX_GEMM_PINGPONG" (on: the two waves of a SIMD take turns at the MFMAs of the large matmul tile; measured slower, off by default),
- * "VPX_CONV_KERNEL" (regw | tile | stream | gemm), "VPX_CONV_ROWS" (n), "VPX_CONV_COLS" (n), "VPX_CONV_WAVES" (4 | 8), "VPX_STREAM_KSPLIT" (off: the streamed-weights
+ * "VPX_CONV_KERNEL" (regw | tile | stream | gemm | regb), "VPX_CONV_ROWS" (n), "VPX_CONV_COLS" (n), "VPX_CONV_WAVES" (4 | 8), "VPX_STREAM_KSPLIT" (off: the streamed-weights
  * convolution kernel gives every wave a 32 x 32 tile also on small planes, instead of splitting K over the waves of a group),
  * "VPX_MVN_FUSED" (off: long MVN groups take
  * the two-launch kernels and channel-minor tensors the three-launch ones; nowait: the one-launch kernels' workgroups do not

@@ -9,7 +9,7 @@ LIB = os.path.join(HERE, "libvpx_amd.so")
 BINDING = os.path.join(HERE, "_binding.so")
 
 HIP_SOURCES = ["csrc/abi.hip", "csrc/sw_elementwise.hip", "csrc/sw_softmax.hip", "csrc/sw_mvn.hip", "csrc/sw_mvn_cminor.hip", "csrc/nce.hip", "csrc/nce_gemm.hip", "csrc/nce_gemm_regb.hip",
-               "csrc/nce_direct.hip", "csrc/nce_conv_patch.hip", "csrc/nce_conv_rows.hip", "csrc/nce_conv_strips.hip", "csrc/nce_conv_gather.hip", "csrc/nce_eltwise.hip", "csrc/calib.hip"]
+               "csrc/nce_direct.hip", "csrc/nce_conv_patch.hip", "csrc/nce_conv_rows.hip", "csrc/nce_conv_strips.hip", "csrc/nce_conv_regb.hip", "csrc/nce_conv_gather.hip", "csrc/nce_eltwise.hip", "csrc/calib.hip"]
 HOST_SOURCES = ["host/compiler_utils.cpp"]
 
 # -ffp-contract=off: fp32 expressions must round as written (FakeQuantize / Quantize parity).

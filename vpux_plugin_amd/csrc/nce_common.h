@@ -792,6 +792,39 @@ struct StripLaunch {
 };
 int launch_conv_strips(const StripLaunch& a, hipStream_t s);
 
+// nce_conv_regb.hip: K of at most 13 * 64 bytes, 16 * nt output channels, as far as conv_regb_steps says; byte output, offsets inside the operands
+// fit 31 bits.
+struct RegbConvGeom {
+    int P, nblk;         // output positions, blocks of 16 of them
+    int chunks;          // K / 16
+    int OC, H, W, isn, ish, isw, osn, osh, osw;
+    int SY, SX, PT, PL;
+    int OH, ow, ohow;
+    int oy_lo, oy_n, ox_lo, ox_n;  // output rows and columns whose windows lie inside the image: the first, and how many
+    unsigned ow_magic, ohow_magic;
+    int pad32;           // the padding byte, four times
+    FastDiv cpp, kx;     // 16-byte chunks per tap, taps per kernel row
+};
+struct RegbConvLaunch {
+    const int8_t* in;
+    const int8_t* w;
+    const int32_t* wt;
+    uint8_t* out;
+    RegbConvGeom g;
+    GemmPpe ppe;
+    bool in_u8;
+    int nt, cus;
+};
+int launch_conv_regb(const RegbConvLaunch& a, hipStream_t s);
+// K steps of 64 of the form that serves K bytes and OC output channels; 0: none
+constexpr int conv_regb_steps(int64_t K, int64_t OC) {
+    const int ks = K <= 192 ? 3 : (K <= 320 ? 5 : (K <= 448 ? 7 : (K <= 832 ? 13 : 0)));
+    if (OC == 16) return ks;
+    if (OC == 32) return ks <= 7 ? ks : 0;
+    if (OC == 48) return ks == 5 || ks == 7 ? 7 : 0;
+    return OC == 64 && ks == 3 ? 3 : 0;
+}
+
 // nce_conv_gather.hip
 int launch_fold(const int8_t* w, const int32_t* wt, ChanPrep* prep, int64_t OC, int64_t K, int corr, const Ppe& ppe, int shift_sub,
                 hipStream_t s);
