@@ -539,6 +539,9 @@ __device__ __forceinline__ unsigned long long tagged(float v, unsigned tag) {
 
 // A slice in registers: V words of 128 bits for each of T lanes, plus the group's last few values, one per lane, where the
 // group is no whole number of words (groups of any length at any address).
+// Slices of more words than kFusedAhead a lane are summed while they arrive, so many under way at a time: all at once, up to 400 KB a compute unit,
+// they reach the memory in an order that costs a third of its rate.
+constexpr int kFusedAhead = 12;
 template <int V>
 struct Slice {
     u32x4 q[V];
@@ -546,21 +549,28 @@ struct Slice {
     float last;  // its value of the partial word
     bool has_last;
     float wave_count, count;  // values of the wavefront, of the slice
+    const half_t* from;       // of the word to load next: the group's values, and its place among them
+    uint32_t at;
 };
 
+template <int V, int T>
+__device__ __forceinline__ void load_word(Slice<V>& sl, int j) {
+    sl.q[j] = *reinterpret_cast<const u32x4_any*>(sl.from + (j < sl.have ? sl.at : 0));
+    sl.at += T * 8;
+    asm volatile("" : "+v"(sl.at));  // one running offset, not V of them
+}
 template <int V, int T>
 __device__ __forceinline__ void load_slice(const half_t* __restrict__ g, uint32_t base, uint32_t end, uint32_t group_size, Slice<V>& sl) {
     const uint32_t words = (end - base) / 8;  // (only the group's last slice is not whole words)
     sl.have = threadIdx.x < words ? (int)((words - threadIdx.x + T - 1) / T) : 0;
-    uint32_t f = base + threadIdx.x * 8;
+    sl.from = g;
+    sl.at = base + threadIdx.x * 8;
 #pragma unroll
-    for (int j = 0; j < V; j++) {
-        sl.q[j] = *reinterpret_cast<const u32x4_any*>(g + (j < sl.have ? f : 0));
-        f += T * 8;
-        asm volatile("" : "+v"(f));  // one running offset, not V of them
+    for (int j = 0; j < (V <= kFusedAhead ? V : kFusedAhead); j++) load_word<V, T>(sl, j);
+    if (V <= kFusedAhead) {
+#pragma unroll
+        for (int j = 0; j < V; j++) sl.q[j] = j < sl.have ? sl.q[j] : u32x4{0, 0, 0, 0};
     }
-#pragma unroll
-    for (int j = 0; j < V; j++) sl.q[j] = j < sl.have ? sl.q[j] : u32x4{0, 0, 0, 0};
     const uint32_t rest = base + words * 8 + threadIdx.x;
     sl.has_last = rest < end && threadIdx.x < 8;
     sl.last = sl.has_last ? (float)g[rest] : 0.f;
@@ -581,34 +591,79 @@ __device__ __forceinline__ void widen_word(u32x4& q, float (&f)[8]) {
 
 // Moments of the slice held by the workgroup: per wavefront by lane shuffles (mean first, then centred squares), the
 // wavefronts' results merged in a fixed order by every lane.
+// Long slices (V > kFusedAhead): one pass while the words arrive, over values less the mean of the wavefront's first kFirst words.  Those are
+// a share f = kFirst / V of the values themselves, so their mean lies within sqrt((1 - f) / f) standard deviations of the whole's, and the
+// subtraction of the squared mean magnifies the rounding of the squares 1 / f = 13 times at the very most, 1.2 for values of one
+// distribution.  (us across channels, all words at once and two passes behind the last one /
+// this: [1,368,182,224] 19.0 / 16.4, [2,181,194,308] 24.7 / 21.6, [2,452,175,218] 35.3 / 30.3, [5,146,180,352] 52.2 / 41.1.)
 template <int V, int T>
 __device__ __forceinline__ Moments slice_moments(Slice<V>& sl, Moments* red) {
     constexpr bool KEEP = V <= 8;
-    float sum = sl.last;
-#pragma unroll
-    for (int j = 0; j < V; j++) {
-        float f[8];
-        widen_word<KEEP>(sl.q[j], f);
-#pragma unroll
-        for (int k = 0; k < 8; k++) sum += f[k];
-        if (!KEEP) asm volatile("" : "+v"(sum));
-    }
+    constexpr int kFirst = 4;
     const float n = sl.wave_count, inv_n = 1.f / n;  // (of loads that are still on their way)
-    const float mean = n > 0.f ? over(wave_sum_soon(sum), n, inv_n) : 0.f;
-    float q = sl.has_last ? (sl.last - mean) * (sl.last - mean) : 0.f;
+    float mean, q;
+    if constexpr (V > kFusedAhead) {
+        float shift = 0.f;
+        int firsts = sl.have < kFirst ? sl.have : kFirst;
 #pragma unroll
-    for (int j = 0; j < V; j++) {
-        float f[8], qj = 0.f;
-        widen_word<KEEP>(sl.q[j], f);
+        for (int j = 0; j < kFirst; j++) {
+            float f[8], sum = 0.f;
+            widen_word<false>(sl.q[j], f);
 #pragma unroll
-        for (int k = 0; k < 8; k++) {
-            const float d = f[k] - mean;
-            qj += d * d;
+            for (int k = 0; k < 8; k++) sum += f[k];
+            shift += j < sl.have ? sum : 0.f;
         }
-        q += j < sl.have ? qj : 0.f;
-        if (!KEEP) asm volatile("" : "+v"(q));
+        const float of = wave_sum_soon((float)(8 * firsts));
+        shift = wave_sum_soon(shift);
+        shift = of > 0.f ? shift / of : 0.f;
+        float sum = sl.has_last ? sl.last - shift : 0.f;
+        q = sum * sum;
+#pragma unroll
+        for (int j = 0; j < V; j++) {
+            // word after word: the values of V words at once are more than the registers hold
+            asm volatile("" : "+v"(sl.q[j]), "+v"(sum), "+v"(q));
+            if (j + kFusedAhead < V) load_word<V, T>(sl, j + kFusedAhead);
+            float f[8], sj = 0.f, qj = 0.f;
+            widen_word<false>(sl.q[j], f);
+#pragma unroll
+            for (int k = 0; k < 8; k++) {
+                const float d = f[k] - shift;
+                sj += d;
+                qj = __builtin_fmaf(d, d, qj);
+            }
+            sum += j < sl.have ? sj : 0.f;
+            q += j < sl.have ? qj : 0.f;
+        }
+        sum = wave_sum_soon(sum);
+        const float off = n > 0.f ? over(sum, n, inv_n) : 0.f;
+        mean = shift + off;
+        q = fmaxf(wave_sum_soon(q) - sum * off, 0.f);
+    } else {
+        float sum = sl.last;
+#pragma unroll
+        for (int j = 0; j < V; j++) {
+            float f[8];
+            widen_word<KEEP>(sl.q[j], f);
+#pragma unroll
+            for (int k = 0; k < 8; k++) sum += f[k];
+            if (!KEEP) asm volatile("" : "+v"(sum));
+        }
+        mean = n > 0.f ? over(wave_sum_soon(sum), n, inv_n) : 0.f;
+        q = sl.has_last ? (sl.last - mean) * (sl.last - mean) : 0.f;
+#pragma unroll
+        for (int j = 0; j < V; j++) {
+            float f[8], qj = 0.f;
+            widen_word<KEEP>(sl.q[j], f);
+#pragma unroll
+            for (int k = 0; k < 8; k++) {
+                const float d = f[k] - mean;
+                qj += d * d;
+            }
+            q += j < sl.have ? qj : 0.f;
+            if (!KEEP) asm volatile("" : "+v"(q));
+        }
+        q = wave_sum_soon(q);
     }
-    q = wave_sum_soon(q);
     __syncthreads();  // the previous use of `red` is over
     if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = Moments{n, mean, q};
     __syncthreads();
@@ -763,6 +818,7 @@ __global__ __launch_bounds__(T) void mvn_fused_kernel(const half_t* __restrict__
             }
             if (threadIdx.x < 64) collect(false);
             load_slice<V, T>(gin, base, end, group_size, sl);  // its own again
+            if (V > kFusedAhead) slice_moments<V, T>(sl, red);
             __syncthreads();
         }
         total = shared_total;
