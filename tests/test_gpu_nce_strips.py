@@ -68,3 +68,14 @@ def test_narrow_planes(rt, dev, W):
         assert rt.nce_last_kernel() == kernel
         outs.append(out)
     assert torch.equal(*outs)
+
+
+@pytest.mark.parametrize("in_u8", [True, False])
+@pytest.mark.parametrize("layer", [dict(N=3, H=37, W=70, IC=16, OC=64, KY=7, KX=7, strides=(2, 2), pads=(3, 3, 3, 3)),
+                                   dict(N=2, H=70, W=45, IC=32, OC=112, KY=3, KX=3, pads=(1, 1, 1, 1))])
+@pytest.mark.parametrize("out_kind", ["dense", "window_chan"])
+def test_whole_channels(rt, orc, dev, layer, in_u8, out_kind):
+    """patches of up to 14 rows, whole chunks of channels, output rows on words: tiles that end past the image, in a tensor and in a window of one"""
+    rng = np.random.default_rng(seed("strips whole", layer["OC"], in_u8, out_kind))
+    for mode in ("NOOP", "LPRELU"):
+        assert run_views(rt, orc, dev, rng, layer, "dense", out_kind, in_u8=in_u8, out_signed=not in_u8, mode=mode, tuning=(("VPX_CONV_STRIPS", 16),)) == "nce_conv_strips"

@@ -601,7 +601,7 @@ struct StripGeom {
     int ish, isw, osh, osw;
     int H, W, OH, OW, OC;
     int SY, SX, PT, PL;
-    int R, cw_log;         // output rows per tile; its columns: 16 or 32
+    int R, cw_log;         // output rows per tile; its columns: 8, 16 or 32
     int PH, RB;            // patch rows: (R - 1) * SY + KY; bytes per patch row in LDS: m planes of `plane` chunks
     int row_chunks;        // 16-byte chunks per patch row, 128 at most
     int m, plane;          // chunks between neighbouring output positions; chunks per plane
@@ -609,6 +609,7 @@ struct StripGeom {
     int PW;                // input columns under a tile
     int nchunks, S, WS;    // K / 16; MFMA steps; bytes per weight row in LDS
     int every, more;       // tiles a wave walks; waves that walk one more
+    unsigned out_bits;     // as ConvGeom's
     int pad32;             // the padding byte, four times
     FastDiv tiles_x, tiles_y, cpp, kc, fm, rin;  // as in RowsGeom
 };

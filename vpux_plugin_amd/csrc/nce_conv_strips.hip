@@ -21,7 +21,10 @@ namespace vpx {
 namespace nce {
 namespace {
 
-template <bool IN_U8>
+typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+constexpr int kStripRows = 14;  // rows that travel ahead, in registers
+
+template <bool IN_U8, bool REST>
 __global__ __launch_bounds__(64 * kStripWaves) void nce_conv_strips(const int8_t* __restrict__ in, const int8_t* __restrict__ w,
                                                                      const int32_t* __restrict__ wt, uint8_t* __restrict__ out, StripGeom g, GemmPpe ppe) {
     constexpr int TM = 2, TN = 2, BN = 32 * TN, NT = 64 * kStripWaves;  // blocks of 32 positions and of 32 channels per tile
@@ -48,7 +51,7 @@ __global__ __launch_bounds__(64 * kStripWaves) void nce_conv_strips(const int8_t
 
     // ---- a tile's input rows -> this wave's patch, a row per instruction (two where a row has more than 64 chunks); padding
     // and the sign flip applied here.  What a lane holds of a row does not depend on the tile: worked out once.
-    constexpr int GROUPS = 2, ROWS = 14;  // rows that travel ahead, in registers
+    constexpr int GROUPS = REST ? 2 : 1, ROWS = kStripRows;
     const int flip = IN_U8 ? (int)0x80808080 : 0, pad = g.pad32 ^ flip;
     int lsrc[GROUPS], ldst[GROUPS], lcol[GROUPS];
 #pragma unroll
@@ -69,10 +72,14 @@ __global__ __launch_bounds__(64 * kStripWaves) void nce_conv_strips(const int8_t
         return TilePos{img, ty * g.R, (tc - img * (int)g.tiles_x.d) << g.cw_log};
     };
     i32x4 ahead[ROWS];
-    // (a row's first byte is wave-uniform, the lane's offset the same for all rows; rows outside the image read the border row)
-    const auto load_row = [&](const int8_t* img, int y, int col) __attribute__((always_inline)) {
-        const int8_t* const row = img + (int64_t)(y < 0 ? 0 : (y < g.H ? y : g.H - 1)) * g.ish;
-        return *reinterpret_cast<const i32x4*>(row + (unsigned)col);
+    // (A row's place in its image is wave-uniform, the lane's offset the same for all rows: a scalar and a vector offset of a buffer that is the
+    // image.  As one address per lane the compiler multiplies 64 bits wide for every row.  Rows outside the image read the border row.)
+    const auto image = [&](int img) __attribute__((always_inline)) {
+        return __builtin_amdgcn_make_buffer_rsrc(const_cast<int8_t*>(in) + (int64_t)img * g.isn, (short)0, -1, 0x00020000);
+    };
+    const auto load_row = [&](const __amdgpu_buffer_rsrc_t& img, int y, int col) __attribute__((always_inline)) {
+        const int row = (y < 0 ? 0 : (y < g.H ? y : g.H - 1)) * g.ish;
+        return __builtin_bit_cast(i32x4, __builtin_amdgcn_raw_buffer_load_b128(img, col, row, 0));
     };
     // byte offset of group u's chunk in a row, from the row's first pixel; a column outside the image reads the pixel at the border
     const auto column = [&](int ix0, auto u_c) __attribute__((always_inline)) {
@@ -84,13 +91,13 @@ __global__ __launch_bounds__(64 * kStripWaves) void nce_conv_strips(const int8_t
     constexpr std::integral_constant<int, 1> g1{};
     const auto load_patch = [&](const TilePos& tp) __attribute__((always_inline)) {
         const int iy0 = tp.oy0 * g.SY - g.PT, col = column(tp.ox0 * g.SX - g.PL, g0);
-        const int8_t* const img = in + (int64_t)tp.img * g.isn;
+        const auto img = image(tp.img);
 #pragma unroll
         for (int r = 0; r < ROWS; r++) ahead[r] = load_row(img, iy0 + (r < g.PH ? r : 0), col);
     };
     const auto store_patch = [&](const TilePos& tp) __attribute__((always_inline)) {
         const int iy0 = tp.oy0 * g.SY - g.PT, ix0 = tp.ox0 * g.SX - g.PL;
-        const int8_t* const img = in + (int64_t)tp.img * g.isn;
+        const auto img = image(tp.img);
         const auto put_rows = [&](auto border_c) __attribute__((always_inline)) {
             constexpr bool BORDER = decltype(border_c)::value;
             const bool ok0 = (unsigned)(ix0 + lcol[0]) < (unsigned)g.W;
@@ -128,8 +135,8 @@ __global__ __launch_bounds__(64 * kStripWaves) void nce_conv_strips(const int8_t
                 }
             }
         };
-        if (g.PH > ROWS) rest(ROWS, g0);
-        if (g.row_chunks > 64) rest(0, g1);
+        if (REST && g.PH > ROWS) rest(ROWS, g0);
+        if (REST && g.row_chunks > 64) rest(0, g1);
     };
 
     int wt2 = 0, wt3 = 0;  // this thread's channel of the weight table, asked for before anything else
@@ -290,6 +297,9 @@ __global__ __launch_bounds__(64 * kStripWaves) void nce_conv_strips(const int8_t
             }
         }
         uint8_t* const dst0 = out + (int64_t)tp.img * g.osn + (oy * g.osh + ox * g.osw + q16);
+        // Without REST: the image as a buffer that drops what lies past its end, so that no branch makes the number of stores under way unknown (the
+        // wait for the next tile's rows would be one for these stores too).
+        const auto dst_image = __builtin_amdgcn_make_buffer_rsrc(out + (int64_t)tp.img * g.osn, (short)0, (g.OH - 1) * g.osh + (g.OW - 1) * g.osw + OC, 0x00020000);
         const auto finish = [&](auto kind_c) __attribute__((always_inline)) {
             constexpr int KIND = decltype(kind_c)::value;
 #pragma unroll
@@ -324,8 +334,14 @@ __global__ __launch_bounds__(64 * kStripWaves) void nce_conv_strips(const int8_t
                 const int qc = q16 + 32 * j;
 #pragma unroll
                 for (int i = 0; i < TM; i++) {
-                    if (oy + i * rows_per_block >= g.OH || ox >= g.OW || qc >= OC) continue;
                     o[i] ^= (int)pk.flip;
+                    const bool there = (oy + i * rows_per_block < g.OH) & (ox < g.OW) & (qc < OC);
+                    if (!REST) {
+                        const unsigned at = (unsigned)((oy + i * rows_per_block) * g.osh + ox * g.osw + qc);
+                        __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, o[i]), dst_image, there ? (int)at : (int)0x80000000, 0, 0);
+                        continue;
+                    }
+                    if (!there) continue;
                     uint8_t* const dst = dst0 + (i * rows_per_block * g.osh + 32 * j);
                     if (qc + 16 <= OC) *reinterpret_cast<i32x4_any*>(dst) = o[i];
                     else
@@ -353,7 +369,15 @@ int launch_conv_strips(const StripLaunch& a, hipStream_t s) {
         VPX_LAUNCH(kernel, a.grid, dim3(64 * kStripWaves), a.lds, s, a.in, a.w, a.wt, a.out, a.sg, a.ppe);
         return VPX_RESULT_SUCCESS;
     };
-    const int rc = a.in_u8 ? launch(nce_conv_strips<true>) : launch(nce_conv_strips<false>);
+    // What few layers have is a kernel of its own (REST): patches of more than 14 rows or 64 chunks a row, last chunks of fewer than 16 channels, rows
+    // of the output that do not start on words, images of 2^31 elements and more.  In one kernel with the rest it made every tile begin with a wait for
+    // the last one's stores.  us, one kernel / two, and row addresses of 64 bits a lane / two offsets: [32,224,224,16] -> 64 7x7 stride 2 30.9 / 29.8,
+    // [8,243,563,16] -> 64 3x3 stride 2 16.7 / 15.6, [8,521,314,16] -> 64 5x5 stride 2 22.0 / 21.1, [30,160,37,16] -> 64 3x3 13.5 / 12.7.
+    const StripGeom& g = a.sg;
+    const int64_t extent = (int64_t)(g.OH - 1) * g.osh + (int64_t)(g.OW - 1) * g.osw + g.OC;
+    const bool rest = g.PH > kStripRows || g.row_chunks > 64 || g.OC % 16 != 0 || (g.out_bits & 3) != 0 || extent >= (1ll << 31);
+    const int rc = a.in_u8 ? (rest ? launch(nce_conv_strips<true, true>) : launch(nce_conv_strips<true, false>))
+                           : (rest ? launch(nce_conv_strips<false, true>) : launch(nce_conv_strips<false, false>));
     if (rc) return rc;
     return VPX_RESULT_SUCCESS;
 }
