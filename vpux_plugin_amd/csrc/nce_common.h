@@ -663,14 +663,6 @@ struct View {
 };
 int operand_view(const int64_t st[4], int64_t N, int64_t H, int64_t W, int64_t C, const char* what, View* v);
 
-// n / d for any n and d of 32 bits: magic = floor((2^32 - 1) / d) lies at most one below 2^32 / d (one where d is a power of two), so n * magic
-// falls short of 2^32 * n / d by at most n < 2^32, and its high half is the quotient or one less.
-inline unsigned quotient_magic(unsigned d) { return 0xffffffffu / d; }
-__device__ __forceinline__ unsigned quotient(unsigned n, unsigned d, unsigned magic) {
-    const unsigned q = __umulhi(n, magic);
-    return q + (n - q * d >= d ? 1u : 0u);
-}
-
 // A convolution as a matmul: row m is output position (image, oy, ox), byte k of it byte k % (16 cpt) of tap k / (16 cpt).
 struct GemmConv {
     int H, W, isn, ish, isw;  // of the input, strides in bytes
@@ -718,6 +710,7 @@ struct DirectGeom {
     int S, share;  // waves of a workgroup, K steps of 64 each
     int H, W, ow, ohow;
     int flat_in;   // 1x1: position m is the pixel m * isw
+    unsigned noc_magic, ohow_magic, ow_magic;  // quotient_magic of those
     FastDiv cpp, kx;  // 16-byte chunks per pixel, taps per kernel row
 };
 struct DirectLaunch {

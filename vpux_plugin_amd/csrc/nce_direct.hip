@@ -52,12 +52,17 @@ __global__ __launch_bounds__(SPLIT ? 64 * kMaxWaves : 256) void nce_direct(const
     extern __shared__ __attribute__((aligned(16))) i32x4 s_part[];  // SPLIT: [wave][tile][lane]
     __shared__ ChanPrep s_prep[CH];
     __shared__ int s_general;
+    // (a value of every line of the launch's arguments: one trip to memory for all, see vpx_common.h)
+    asm volatile("" ::"s"(in), "s"(w), "s"(wt), "s"(out), "s"(g.SX), "s"(g.ish), "s"(ppe.corr), "s"(d.noc), "s"(d.ow), "s"(flip));
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int n16 = lane & 15, c4 = lane >> 4;
     const int noc = d.noc;
-    const int oct = (int)(blockIdx.x % (unsigned)noc);
-    const int post = (int)(blockIdx.x / (unsigned)noc) * (SPLIT ? 1 : 4) + (SPLIT ? 0 : wave);
+    // (Everything up to the first load is a chain: divisions are products with what the host has worked out, a dozen dependent instructions less each.
+    // us in a HIP graph, divided / this: [4,14,14,96] -> 96 3x3 3.49 / 3.31, [1,14,14,256] -> 256 4.76 / 4.56, [1,112,112,16] -> 16 7x7 3.03 / 2.89.)
+    const unsigned pos = quotient(blockIdx.x, (unsigned)noc, d.noc_magic);
+    const int oct = (int)(blockIdx.x - pos * (unsigned)noc);
+    const int post = (int)pos * (SPLIT ? 1 : 4) + (SPLIT ? 0 : wave);
     const int oc0 = oct * CH, P = d.P, OC = (int)g.OC;
     const int chunks = d.chunks;
     const int steps = (chunks + 3) >> 2;
@@ -86,8 +91,8 @@ __global__ __launch_bounds__(SPLIT ? 64 * kMaxWaves : 256) void nce_direct(const
         int m = (post * TN + j) * 16 + n16;
         m = m < P ? m : P - 1;
         if (CONV || !d.flat_in) {
-            const unsigned img = (unsigned)m / (unsigned)d.ohow, rem = (unsigned)m - img * (unsigned)d.ohow, oy = rem / (unsigned)d.ow,
-                           ox = rem - oy * (unsigned)d.ow;
+            const unsigned img = quotient((unsigned)m, (unsigned)d.ohow, d.ohow_magic), rem = (unsigned)m - img * (unsigned)d.ohow,
+                           oy = quotient(rem, (unsigned)d.ow, d.ow_magic), ox = rem - oy * (unsigned)d.ow;
             iy0[j] = (int)oy * g.SY - g.PT;
             ix0[j] = (int)ox * g.SX - g.PL;
             pofs[j] = (int)img * (int)g.isn + iy0[j] * (int)g.ish + ix0[j] * (int)g.isw;
@@ -232,8 +237,8 @@ __global__ __launch_bounds__(SPLIT ? 64 * kMaxWaves : 256) void nce_direct(const
     // element offset of output position m
     const auto position = [&](int m) -> int64_t {
         if (g.out_flat == 2) return (int64_t)m * g.osw;
-        const unsigned img = (unsigned)m / (unsigned)d.ohow, rem = (unsigned)m - img * (unsigned)d.ohow, oy = rem / (unsigned)d.ow,
-                       ox = rem - oy * (unsigned)d.ow;
+        const unsigned img = quotient((unsigned)m, (unsigned)d.ohow, d.ohow_magic), rem = (unsigned)m - img * (unsigned)d.ohow,
+                       oy = quotient(rem, (unsigned)d.ow, d.ow_magic), ox = rem - oy * (unsigned)d.ow;
         return (int64_t)img * g.osn + (int64_t)oy * g.osh + (int64_t)ox * g.osw;
     };
     // 4 * TM channels from ch on of one position

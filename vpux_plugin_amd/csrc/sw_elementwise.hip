@@ -932,6 +932,12 @@ __global__ __launch_bounds__(kBlock) void vrow_kernel(const T* __restrict__ p0, 
                                                       const T* __restrict__ p3, const T* __restrict__ p4, T* __restrict__ pout,
                                                       Fn fn, VndIndex ix, uint32_t rows) {
     constexpr int VEC = 16 / sizeof(T);
+    // (a value of every line of the launch's arguments: one trip to memory for all, see vpx_common.h)
+    if constexpr (NOPS == 3)
+        asm volatile("" ::"s"(p0), "s"(p1), "s"(pout), "s"(ix.vec_per_row), "s"(ix.stride[0][0]), "s"(ix.stride[1][0]), "s"(ix.stride[2][0]), "s"(ix.inner_stride[0]), "s"(rows));
+    else
+        asm volatile("" ::"s"(p0), "s"(p1), "s"(p4), "s"(pout), "s"(ix.vec_per_row), "s"(ix.stride[0][0]), "s"(ix.stride[1][0]), "s"(ix.stride[2][0]), "s"(ix.stride[3][0]),
+                     "s"(ix.stride[4][0]), "s"(ix.stride[5][0]), "s"(ix.inner_stride[0]), "s"(rows));
     const uint32_t iv = blockIdx.x * kBlock + threadIdx.x;
     const uint32_t row = TWO ? blockIdx.y : blockIdx.y + blockIdx.z * kRowsPerGridY;
     if (iv >= ix.vec_per_row || row >= rows) return;

@@ -31,6 +31,13 @@ int fail(int code, const char* fmt, ...) __attribute__((format(printf, 2, 3)));
         if (!(cond)) return ::vpx::fail(code, __VA_ARGS__); \
     } while (0)
 
+// ---- a kernel's arguments -------------------------------------------------------------------
+// They lie in memory, and a wave reads a line of 64 bytes when it comes to the first value in it.  Kernels whose first load waits for values of several
+// lines, come to one after another, name a value of each in an empty asm at their start, in front of which all of them are asked for together (us in a
+// HIP graph, without / with it: softmax of 4 x 512 x 512 2.40 / 2.28, add with one value a channel [2,64,56,56] 2.18 / 2.08, [2,160,160,16] -> 32 3x3
+// on nce_direct 3.20 / 3.05; where the set-up does not wait for them it is none of these or, registers held from the start, a loss: [16,7,7,512] -> 512
+// 3x3 on nce_conv_stream 12.5 / 13.1).
+
 // ---- launches --------------------------------------------------------------------------------
 // The arguments go straight to hipLaunchKernel, which says whether the launch was taken: the triple-chevron form keeps the launch's shape in a stack of
 // the runtime's and takes it from there again, and its result has to be asked for, three calls into the runtime of 0.04 ... 0.05 us each.
@@ -54,6 +61,15 @@ int launch(void (*kernel)(P...), const dim3& grid, const dim3& block, size_t lds
     do {                                                                                                     \
         if (const int _rc = ::vpx::launch(kernel, grid, block, lds, stream, __VA_ARGS__)) return _rc; \
     } while (0)
+
+// ---- divisions ---------------------------------------------------------------------------------
+// n / d for any n and d of 32 bits: magic = floor((2^32 - 1) / d) lies at most one below 2^32 / d (one where d is a power of two), so n * magic
+// falls short of 2^32 * n / d by at most n < 2^32, and its high half is the quotient or one less.
+inline unsigned quotient_magic(unsigned d) { return 0xffffffffu / d; }
+__device__ __forceinline__ unsigned quotient(unsigned n, unsigned d, unsigned magic) {
+    const unsigned q = __umulhi(n, magic);
+    return q + (n - q * d >= d ? 1u : 0u);
+}
 
 // ---- tensor views parsed from a params blob ---------------------------------------------------
 constexpr int kMaxDims = 8;  // deepest rank the strided kernels accept
