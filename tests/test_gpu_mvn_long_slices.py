@@ -1,4 +1,4 @@
-"""MVN across channels over slices that are summed while they arrive (more than twelve words a lane), at the sizes where a lane's words and the
+"""MVN across channels over slices that are summed while they arrive (those for 512 lanes), at the sizes where a lane's words and the
 kernel's forms end, over values whose first ones say little about the others."""
 import pytest
 
@@ -19,7 +19,8 @@ def values(torch, kind, groups, length, dev):
 
 
 @pytest.mark.parametrize("kind", ["plain", "far", "steps"])
-@pytest.mark.parametrize("groups,words", [(1, 8.01), (1, 12), (1, 12.02), (3, 16), (1, 16.03), (2, 23.99), (1, 32.01), (1, 40), (1, 40.02), (2, 51.9)])
+@pytest.mark.parametrize("groups,words", [(1, 4.01), (2, 7.98), (1, 8.01), (1, 12), (1, 12.02), (3, 16), (1, 16.03), (1, 20), (2, 23.99), (1, 24.01), (1, 28.01), (1, 32.01), (1, 35.99),
+                                          (1, 40), (1, 40.02), (2, 44.01), (1, 48), (2, 51.9)])
 def test_long_slices(rt, dev, kind, groups, words):
     import torch
     wpg = 256 // groups

@@ -539,7 +539,7 @@ __device__ __forceinline__ unsigned long long tagged(float v, unsigned tag) {
 
 // A slice in registers: V words of 128 bits for each of T lanes, plus the group's last few values, one per lane, where the
 // group is no whole number of words (groups of any length at any address).
-// Slices of more words than kFusedAhead a lane are summed while they arrive, so many under way at a time: all at once, up to 400 KB a compute unit,
+// Slices for 512 lanes are summed while they arrive, kFusedAhead words a lane under way at a time: all at once, up to 400 KB a compute unit,
 // they reach the memory in an order that costs a third of its rate.
 constexpr int kFusedAhead = 12;
 template <int V>
@@ -567,7 +567,7 @@ __device__ __forceinline__ void load_slice(const half_t* __restrict__ g, uint32_
     sl.at = base + threadIdx.x * 8;
 #pragma unroll
     for (int j = 0; j < (V <= kFusedAhead ? V : kFusedAhead); j++) load_word<V, T>(sl, j);
-    if (V <= kFusedAhead) {
+    if (T < 512) {
 #pragma unroll
         for (int j = 0; j < V; j++) sl.q[j] = j < sl.have ? sl.q[j] : u32x4{0, 0, 0, 0};
     }
@@ -591,18 +591,18 @@ __device__ __forceinline__ void widen_word(u32x4& q, float (&f)[8]) {
 
 // Moments of the slice held by the workgroup: per wavefront by lane shuffles (mean first, then centred squares), the
 // wavefronts' results merged in a fixed order by every lane.
-// Long slices (V > kFusedAhead): one pass while the words arrive, over values less the mean of the wavefront's first kFirst words.  Those are
+// Long slices (T == 512): one pass while the words arrive, over values less the mean of the wavefront's first kFirst words.  Those are
 // a share f = kFirst / V of the values themselves, so their mean lies within sqrt((1 - f) / f) standard deviations of the whole's, and the
 // subtraction of the squared mean magnifies the rounding of the squares 1 / f = 13 times at the very most, 1.2 for values of one
-// distribution.  (us across channels, all words at once and two passes behind the last one /
-// this: [1,368,182,224] 19.0 / 16.4, [2,181,194,308] 24.7 / 21.6, [2,452,175,218] 35.3 / 30.3, [5,146,180,352] 52.2 / 41.1.)
+// distribution.  us across channels, all words at once and two passes behind the last one / this: [3,128,124,88] 8.5 / 8.0, [2,202,224,80] 10.5 /
+// 9.7, [1,368,182,224] 19.0 / 16.4, [2,181,194,308] 24.7 / 21.6, [2,452,175,218] 35.3 / 30.3, [5,146,180,352] 52.2 / 41.1.  With 256 lanes, whose words
+// arrive together, the second pass is shorter than what this adds in front of it: [1,176,113,145] 7.0 / 7.6.
 template <int V, int T>
 __device__ __forceinline__ Moments slice_moments(Slice<V>& sl, Moments* red) {
-    constexpr bool KEEP = V <= 8;
-    constexpr int kFirst = 4;
+    constexpr int kFirst = V > 8 ? 4 : 1;
     const float n = sl.wave_count, inv_n = 1.f / n;  // (of loads that are still on their way)
     float mean, q;
-    if constexpr (V > kFusedAhead) {
+    if constexpr (T == 512) {
         float shift = 0.f;
         int firsts = sl.have < kFirst ? sl.have : kFirst;
 #pragma unroll
@@ -643,24 +643,22 @@ __device__ __forceinline__ Moments slice_moments(Slice<V>& sl, Moments* red) {
 #pragma unroll
         for (int j = 0; j < V; j++) {
             float f[8];
-            widen_word<KEEP>(sl.q[j], f);
+            widen_word<true>(sl.q[j], f);
 #pragma unroll
             for (int k = 0; k < 8; k++) sum += f[k];
-            if (!KEEP) asm volatile("" : "+v"(sum));
         }
         mean = n > 0.f ? over(wave_sum_soon(sum), n, inv_n) : 0.f;
         q = sl.has_last ? (sl.last - mean) * (sl.last - mean) : 0.f;
 #pragma unroll
         for (int j = 0; j < V; j++) {
             float f[8], qj = 0.f;
-            widen_word<KEEP>(sl.q[j], f);
+            widen_word<true>(sl.q[j], f);
 #pragma unroll
             for (int k = 0; k < 8; k++) {
                 const float d = f[k] - mean;
                 qj += d * d;
             }
             q += j < sl.have ? qj : 0.f;
-            if (!KEEP) asm volatile("" : "+v"(q));
         }
         q = wave_sum_soon(q);
     }
@@ -818,7 +816,7 @@ __global__ __launch_bounds__(T) void mvn_fused_kernel(const half_t* __restrict__
             }
             if (threadIdx.x < 64) collect(false);
             load_slice<V, T>(gin, base, end, group_size, sl);  // its own again
-            if (V > kFusedAhead) slice_moments<V, T>(sl, red);
+            if (V > kFusedAhead) slice_moments<V, T>(sl, red);  // (which asks for the rest)
             __syncthreads();
         }
         total = shared_total;
@@ -883,10 +881,16 @@ int launch_fused_groups(const half_t* in, half_t* out, int64_t groups, int64_t g
     else if (lane_words <= 4 * kThreads) VPX_FUSED(4, 256);
     else if (lane_words <= 8 * kThreads) VPX_FUSED(8, 256);
     else if (lane_words <= 8 * 512) VPX_FUSED(8, 512);
+    else if (lane_words <= 12 * 512) VPX_FUSED(12, 512);
     else if (lane_words <= 16 * 512) VPX_FUSED(16, 512);
+    else if (lane_words <= 20 * 512) VPX_FUSED(20, 512);
     else if (lane_words <= 24 * 512) VPX_FUSED(24, 512);
+    else if (lane_words <= 28 * 512) VPX_FUSED(28, 512);
     else if (lane_words <= 32 * 512) VPX_FUSED(32, 512);
+    else if (lane_words <= 36 * 512) VPX_FUSED(36, 512);
     else if (lane_words <= 40 * 512) VPX_FUSED(40, 512);
+    else if (lane_words <= 44 * 512) VPX_FUSED(44, 512);
+    else if (lane_words <= 48 * 512) VPX_FUSED(48, 512);
     else VPX_FUSED(kFusedMaxVec, 512);
 #undef VPX_FUSED
     *done = true;
