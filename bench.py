@@ -693,7 +693,7 @@ NOTES = {
     "c1_fake_quantize": "0.8 MB per launch: launch-bound, not bandwidth-bound. An empty kernel of the same grid takes 2.6 us, the "
                         "kernel 2.5-3 us (graph_device_ms_per_step); the eager figure of record is the host's launch rate over "
                         "418 separate parameter blobs. A single launch of this size cannot reach 0.70 of the HBM peak (that would be 0.14 us).",
-    "c3_mvn": "16 MB in one launch of 8.2 us, of which about 2.6 us are the launch floor; 0.70 of the HBM peak would be 3.0 us end to end.",
+    "c3_mvn": "16 MB in one launch of 7.6 to 7.9 us, of which about 2.6 us are the launch floor; 0.70 of the HBM peak would be 3.0 us end to end.",
     "c4_conv": "7.4 GOP: about 1.5 us of MFMA time and 1.5 us of HBM time. Measured by early returns: an empty kernel of this grid "
                "1.6 us, the tile's loads back after 4.0 us, operands staged after 6.1 us, MFMAs + requantisation + stores 3.5 us "
                "(on this part vector-ALU work does not run under MFMAs of the same SIMD, so the PPE's 5.5 instructions per value add to the MFMA time).",
