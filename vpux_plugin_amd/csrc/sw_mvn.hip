@@ -2,9 +2,9 @@
 // square root) or x - mean; group = (C,H,W) of one batch element when across_channels, else (H,W)
 // of one channel (VPU.MVN, src/vpux_compiler/tblgen/vpux/compiler/dialect/VPU/ops.td:3600-3652).
 //
-// Statistics are fp32: mean and centred sum of squares in two passes over values that stay on chip.  Where a group is more
-// than one workgroup's, each publishes {count, mean, M2} of its part and the parts are merged with the pairwise update of
-// Chan et al. in a fixed order, so results do not depend on scheduling.  This is the
+// Statistics are fp32: mean and centred sum of squares in two passes over values that stay on chip, or in one about a first mean where that is
+// as exact (slice_moments).  Where a group is more than one workgroup's, each publishes the moments {count, mean, M2} of its part and the parts
+// meet in a fixed order -- pairwise with the update of Chan et al., or all at once about their common mean -- so results do not depend on scheduling.  This is the
 // decomposition the compiler itself uses when a group does not fit local memory
 // (MVN1Sum -> MVN1MeanVar -> MVN1Normalize,
 // src/vpux_compiler/src/NPU37XX/dialect/VPU/transforms/passes/decompose_mvn.cpp:82-129), with
@@ -589,13 +589,16 @@ __device__ __forceinline__ void widen_word(u32x4& q, float (&f)[8]) {
     for (int k = 0; k < 8; k++) f[k] = (float)h[k];
 }
 
-// Moments of the slice held by the workgroup: per wavefront by lane shuffles (mean first, then centred squares), the
-// wavefronts' results merged in a fixed order by every lane.
-// Long slices (T == 512): one pass while the words arrive, over values less the mean of the wavefront's first kFirst words.  Those are
-// a share f = kFirst / V of the values themselves, so their mean lies within sqrt((1 - f) / f) standard deviations of the whole's, and the
-// subtraction of the squared mean magnifies the rounding of the squares 1 / f = 13 times at the very most, 1.2 for values of one
-// distribution.  us across channels, all words at once and two passes behind the last one / this: [3,128,124,88] 8.5 / 8.0, [2,202,224,80] 10.5 /
-// 9.7, [1,368,182,224] 19.0 / 16.4, [2,181,194,308] 24.7 / 21.6, [2,452,175,218] 35.3 / 30.3, [5,146,180,352] 52.2 / 41.1.  With 256 lanes, whose words
+// Moments of the slice held by the workgroup: per wavefront by lane shuffles, the wavefronts' results met by every lane.
+// Long slices (T == 512): one pass while the words arrive, over values less the mean of the wavefront's first kFirst words.  That is rounded to
+// half precision, so that a difference is exact and the sum of differences as good as one of the values, whose grid they are on.  Where the first
+// words say little about the others the squares about their mean are up to V / kFirst = 13 times those about the mean, and so is what
+// rounding does to them: from an eighth of them on the wavefront sums the squares again, about the mean, from its registers.  Relative errors of the
+// variance against 64 bits (worst of 16 tensors of eight slices, the kernel's arithmetic on a host), two passes / this: values of one distribution 1.8e-7 /
+// 1.0e-7, the mean 40 deviations away 1.5e-7 / 1.2e-7, constant first words at another level 2.0e-6 / 1.8e-6 (8.0e-6 without the second sum).  us
+// across channels, all words at once and two passes behind the last one / this, where the second sum is not taken / where every wavefront takes it:
+// [3,128,124,88] 9.2 / 7.7 / 8.3, [2,202,224,80] 9.9 / 8.5 / 9.3, [1,368,182,224] 16.0 / 14.8 / 15.9, [2,181,194,308] 23.5 / 21.3 / 23.2,
+// [2,452,175,218] 34.1 / 29.0 / 31.9, [5,146,180,352] 50.6 / 39.7 / 44.3.  With 256 lanes, whose words
 // arrive together, the second pass is shorter than what this adds in front of it: [1,176,113,145] 7.0 / 7.6.
 template <int V, int T>
 __device__ __forceinline__ Moments slice_moments(Slice<V>& sl, Moments* red) {
@@ -615,7 +618,7 @@ __device__ __forceinline__ Moments slice_moments(Slice<V>& sl, Moments* red) {
         }
         const float of = wave_sum_soon((float)(8 * firsts));
         shift = wave_sum_soon(shift);
-        shift = of > 0.f ? shift / of : 0.f;
+        shift = of > 0.f ? (float)(half_t)(shift / of) : 0.f;
         float sum = sl.has_last ? sl.last - shift : 0.f;
         q = sum * sum;
 #pragma unroll
@@ -637,7 +640,25 @@ __device__ __forceinline__ Moments slice_moments(Slice<V>& sl, Moments* red) {
         sum = wave_sum_soon(sum);
         const float off = n > 0.f ? over(sum, n, inv_n) : 0.f;
         mean = shift + off;
-        q = fmaxf(wave_sum_soon(q) - sum * off, 0.f);
+        q = wave_sum_soon(q);
+        if (sum * off > 0.125f * q) {  // (the same for the wavefront)
+            q = sl.has_last ? (sl.last - mean) * (sl.last - mean) : 0.f;
+#pragma unroll
+            for (int j = 0; j < V; j++) {
+                asm volatile("" : "+v"(sl.q[j]), "+v"(q));
+                float f[8], qj = 0.f;
+                widen_word<false>(sl.q[j], f);
+#pragma unroll
+                for (int k = 0; k < 8; k++) {
+                    const float d = f[k] - mean;
+                    qj = __builtin_fmaf(d, d, qj);
+                }
+                q += j < sl.have ? qj : 0.f;
+            }
+            q = wave_sum_soon(q);
+        } else {
+            q -= sum * off;
+        }
     } else {
         float sum = sl.last;
 #pragma unroll
@@ -665,21 +686,23 @@ __device__ __forceinline__ Moments slice_moments(Slice<V>& sl, Moments* red) {
     __syncthreads();  // the previous use of `red` is over
     if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = Moments{n, mean, q};
     __syncthreads();
-    // all at once, about the first one's mean: a tree of pairwise merges is three reciprocals in a row
+    // all at once (a tree of pairwise merges is three reciprocals in a row), about the mean as found from the distances to the first one's, which what
+    // is left of those about it then corrects: the first one may lie far from the others
     Moments w[T / 64];
 #pragma unroll
     for (int k = 0; k < T / 64; k++) w[k] = red[k];
     const float count = sl.count, inv_count = 1.f / count;
-    float shift = 0.f, m2 = 0.f;
+    float shift = 0.f, rest = 0.f, m2 = 0.f;
 #pragma unroll
     for (int k = 0; k < T / 64; k++) shift += w[k].n * (w[k].mean - w[0].mean);
-    shift = over(shift, count, inv_count);
+    mean = w[0].mean + over(shift, count, inv_count);
 #pragma unroll
     for (int k = 0; k < T / 64; k++) {
-        const float d = (w[k].mean - w[0].mean) - shift;
+        const float d = w[k].mean - mean;
+        rest += w[k].n * d;
         m2 += w[k].m2 + w[k].n * d * d;
     }
-    return Moments{count, w[0].mean + shift, m2};
+    return Moments{count, mean + over(rest, count, inv_count), m2};
 }
 
 template <int V, int T>
@@ -748,21 +771,23 @@ __global__ __launch_bounds__(T) void mvn_fused_kernel(const half_t* __restrict__
                 if (ok || !waits || wall_clock64() - t0 >= spin_ticks) break;  // (pausing between polls measured slower)
             }
             if (ok || !waits) {
-                // all at once, about the first slice's mean, in a fixed order (a butterfly of pairwise merges: six reciprocals in a row)
-                const float first = lane_bcast(__builtin_bit_cast(float, (unsigned)rm[0]), 0);
-                float shift = 0.f, m2 = 0.f;
+                // all at once, as the wavefronts' in slice_moments (a butterfly of pairwise merges: six reciprocals in a row)
+                const auto value = [&](int k) { return __builtin_bit_cast(float, (unsigned)rm[k]); };
+                const float first = lane_bcast(value(0), 0);
+                float shift = 0.f, rest = 0.f, m2 = 0.f;
                 const auto count = [&](int i) { return i >= wpg ? 0.f : i + 1 < wpg ? (float)slice : (float)(group_size - (uint32_t)i * slice); };
-                const auto off = [&](int k) { return k * 64 + lane < wpg ? __builtin_bit_cast(float, (unsigned)rm[k]) - first : 0.f; };
 #pragma unroll
-                for (int k = 0; k < kMergeInKernel / 64; k++) shift += count(k * 64 + lane) * off(k);
-                shift = over(wave_sum_soon(shift), group_count, inv_count);
+                for (int k = 0; k < kMergeInKernel / 64; k++) shift += k * 64 + lane < wpg ? count(k * 64 + lane) * (value(k) - first) : 0.f;
+                const float mean = first + over(wave_sum_soon(shift), group_count, inv_count);
 #pragma unroll
                 for (int k = 0; k < kMergeInKernel / 64; k++) {
-                    const float d = off(k) - shift;
+                    const float d = k * 64 + lane < wpg ? value(k) - mean : 0.f;
+                    rest += count(k * 64 + lane) * d;
                     m2 += k * 64 + lane < wpg ? __builtin_bit_cast(float, (unsigned)rq[k]) + count(k * 64 + lane) * d * d : 0.f;
                 }
                 m2 = wave_sum_soon(m2);
-                if (lane == 0) shared_total = Moments{group_count, first + shift, m2};
+                rest = wave_sum_soon(rest);
+                if (lane == 0) shared_total = Moments{group_count, mean + over(rest, group_count, inv_count), m2};
             }
             return ok;
         };
