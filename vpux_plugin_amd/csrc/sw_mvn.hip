@@ -474,7 +474,7 @@ static int launch_tiny_groups(const half_t* in, half_t* out, int64_t groups, int
 // [16384 x 21] 12.9 / 4.4, [65536 x 110] 12.1 / 9.6, [65536 x 361] 22.8 / 19.7, [131072 x 49] 16.5 / 12.6.
 static int small_groups_run(int64_t groups, int64_t len) {
     const int64_t fits = kSmallChunk / len, most = len <= 64 ? (groups < 16384 ? 8 : 32) : len > 128 ? 8 : groups < (1 << 18) ? 16 : fits;
-    return (int)(fits < most ? fits : most);
+    return (int)(fits < most || groups / most >= (1 << 24) - 1 ? fits : most);  // (a launch holds fewer than 2^32 lanes)
 }
 // Whether the short-group form applies, and its launch.  It serves what the registers of mvn6_rows_kernel do not, groups of fewer than eight
 // values, and many groups of up to 512 that are no whole number of words: a row of those leaves most of a team's lanes idle or ends in a word that
@@ -1690,6 +1690,20 @@ int launch_rows_of(const half_t* pi, half_t* po, const half_t* ps, const half_t*
     return VPX_RESULT_SUCCESS;
 }
 
+// A launch holds fewer than 2^32 lanes, a row of many takes 32, 64 or 256 of them: several launches from 2^31 on (2^26 rows of 24 values, 2^25 of 520).
+int launch_flat_rows(const half_t* pi, half_t* po, const half_t* ps, const half_t* pb, const FlatGeom& g, bool shared_rows, bool words, int nv, int eps_mode,
+                     float eps, hipStream_t s) {
+    const int64_t most = (1ll << 31) / (g.row_len <= 256 ? 32 : g.row_len <= 3072 ? 64 : 256);
+    for (int64_t r0 = 0; r0 < g.rows; r0 += most) {
+        FlatGeom part = g;
+        part.rows = g.rows - r0 < most ? g.rows - r0 : most;
+        const int rc = launch_rows_of(pi + r0 * g.in, po + r0 * g.out, ps ? ps + r0 * g.sc : nullptr, pb ? pb + r0 * g.bi : nullptr, part, shared_rows, words, nv,
+                                      eps_mode, eps, s);
+        if (rc) return rc;
+    }
+    return VPX_RESULT_SUCCESS;
+}
+
 // rows of a tensor with any kept dimensions
 int launch_rows(const half_t* pi, half_t* po, const half_t* ps, const half_t* pb, const Mvn6Geom& g, bool words, int nv, int eps_mode,
                 float eps, hipStream_t s) {
@@ -1710,13 +1724,13 @@ int launch_rows(const half_t* pi, half_t* po, const half_t* ps, const half_t* pb
     const bool kept = g.nk > 0;
     const FlatGeom f{kept ? g.k_in[0] : 0, kept ? g.k_out[0] : 0, kept && ps ? g.k_sc[0] : 0, kept && pb ? g.k_bi[0] : 0, g.rows, g.row_len,
                      g.sc_along_row, g.bi_along_row};
-    return launch_rows_of(pi, po, ps, pb, f, shared_rows, words, nv, eps_mode, eps, s);
+    return launch_flat_rows(pi, po, ps, pb, f, shared_rows, words, nv, eps_mode, eps, s);
 }
 
 // mvn1 over groups that follow one another in memory, as rows
 int launch_group_rows(const half_t* in, half_t* out, int64_t groups, int64_t len, int nv, float eps, hipStream_t s) {
     const bool words = len % 8 == 0 && ((reinterpret_cast<uintptr_t>(in) | reinterpret_cast<uintptr_t>(out)) & 15) == 0;
-    return launch_rows_of(in, out, nullptr, nullptr, FlatGeom{len, len, 0, 0, groups, (uint32_t)len, 0, 0}, false, words, nv, 0, eps, s);
+    return launch_flat_rows(in, out, nullptr, nullptr, FlatGeom{len, len, 0, 0, groups, (uint32_t)len, 0, 0}, false, words, nv, 0, eps, s);
 }
 
 // mvn1 with per-channel statistics on a channel-minor layout: shifted partial sums over spatial ranges,

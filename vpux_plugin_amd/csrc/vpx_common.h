@@ -41,9 +41,12 @@ int fail(int code, const char* fmt, ...) __attribute__((format(printf, 2, 3)));
 // ---- launches --------------------------------------------------------------------------------
 // The arguments go straight to hipLaunchKernel, which says whether the launch was taken: the triple-chevron form keeps the launch's shape in a stack of
 // the runtime's and takes it from there again, and its result has to be asked for, three calls into the runtime of 0.04 ... 0.05 us each.
+// A launch holds fewer than 2^32 lanes; what is beyond them would be dropped without an error.
 template <class... P, class... A>
 int launch(void (*kernel)(P...), const dim3& grid, const dim3& block, size_t lds, hipStream_t s, const A&... args) {
     static_assert(sizeof...(P) == sizeof...(A), "a launch gives every argument of its kernel");
+    if ((uint64_t)grid.x * block.x >= (1ull << 32))
+        return fail(VPX_RESULT_ERROR_UNSUPPORTED_FEATURE, "%u workgroups of %u lanes exceed the launch limit", grid.x, block.x);
     const std::tuple<P...> held(static_cast<P>(args)...);  // (of the kernel's own types: the runtime copies bytes)
     return std::apply(
             [&](const P&... p) -> int {
