@@ -452,7 +452,9 @@ uint32_t ceil_div(uint64_t a, uint64_t b) {
 // rate of a copy (runs of 16 ... 64 bytes cross the caches several times), more of both where that die is dealt more workgroups than it has compute units
 // (1.3 ... 1.8 times where a lane holds more than 16 words), a partial sum that is exchanged, a channel of the fold through LDS.  Fitted to 1095 drawn
 // tensors under each form that serves them (8500 times, median error 4 %, one tenth beyond 8 to 20): the least of these takes 1.2 % more than the best
-// form of each; without the crowding, 4.6 %.
+// form of each; without the crowding, 4.6 %.  The kernels that run take 0.87 of that alone with up to 16 words a lane, 0.94 with an exchange and 1.04 in rows (medians of 4500
+// tensors).  Of 6400 drawn ones 60 are more than 3 % slower than under the rule that knew no runs of 16 or 32 bytes with more than 16 words, 1.2 us at
+// most but for [8,54,54,544], 12.4 / 15.4; unscaled it would be twice as many.
 struct FormTime {
     float launch, word, copy, crowded, exchange, channel;
 };
@@ -484,6 +486,10 @@ int launch_mvn_cminor_resident(const void* in, void* out, int64_t N, int64_t S, 
     const uint32_t octets = ceil_div(C, 8);
     const float copied = 4.0f / 5.9e6f * (float)N * (float)S * (float)C;
     const uint32_t cus_of_die = (uint32_t)cus >= 8 ? (uint32_t)cus / 8 : 1;
+    // What the three launches of the general form take, which read the tensor twice and whose sums of few large images are long chains: this is 0.77 ... 1.08 of it for
+    // nine tenths of 212 of whole octets and 3 M values or more.
+    const float many = 0.6e-3f * (float)S, few = 80.0f / (float)N;
+    const float launches_us = 8.0f + (C % 8 == 0 ? 0.95e-6f : 5.4e-6f) * (float)N * (float)S * (float)C + (many < few ? many : few);
     const auto consider = [&](bool whole, uint32_t ob, uint32_t ob_log, uint32_t nb, uint32_t parts) {
         const uint32_t of = whole ? rows : (uint32_t)S, slots = kT / ob, per_part = ceil_div(of, parts), v = ceil_div(per_part, slots);
         if (v > kMostWords) return;
@@ -491,8 +497,12 @@ int launch_mvn_cminor_resident(const void* in, void* out, int64_t N, int64_t S, 
         const FormTime& f = whole ? kRowTime[parts > 1] : kOctetTime[parts > 1][ob_log][C % 8 != 0 ? 0 : C % (8 * ob) != 0 ? 1 : 2];
         const uint32_t units = (uint32_t)N * parts, of_die = ceil_div(units, 8), dealt = of_die * nb;
         const float crowd = dealt > cus_of_die ? (float)dealt / (float)cus_of_die : 1.0f, share = copied * 8.0f * (float)of_die / (float)units;
-        const float cost = f.launch + f.word * (float)v * crowd + (f.copy + f.crowded * (crowd - 1.0f)) * share +
-                           f.exchange * (float)(parts * (whole ? (uint32_t)C : ob * 8)) + (whole ? f.channel * (float)C : 0.0f);
+        const float cost = (f.launch + f.word * (float)v * crowd + (f.copy + f.crowded * (crowd - 1.0f)) * share +
+                            f.exchange * (float)(parts * (whole ? (uint32_t)C : ob * 8)) + (whole ? f.channel * (float)C : 0.0f)) *
+                           (whole ? 1.04f : parts > 1 ? 0.94f : v <= 16 ? 0.87f : 1.0f);
+        // Runs of 16 or 32 bytes and many words a lane are few workgroups, each with the whole image of its channels, dealt a second time: [4,155,155,560] 157
+        // us, in three launches 72, [9,137,138,312] 126 / 67, [6,118,136,480] 79 / 59; but [3,110,111,600] 18 / 47.
+        if (ob < 4 && v > 16 && cost >= launches_us) return;
         if (best_v != 0 && cost >= best_cost) return;
         best = Geom{(uint32_t)C, (uint32_t)S, (uint32_t)(S * C), whole ? R : 1, whole ? words : octets, of, whole ? words * 8 : (uint32_t)C, ob, ob_log, nb, parts, per_part,
                     (uint32_t)N * parts};
