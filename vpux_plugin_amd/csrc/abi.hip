@@ -133,8 +133,9 @@ int get_workspace(hipStream_t stream, size_t bytes, void** out) {
 // Launch counts and tagged records that start as zeros; a launch leaves its groups' counts moved on by one and its records
 // behind, which carry a tag that no later launch uses, so launches on one stream can share them without a clearing pass.
 // One area of kSyncBytes (8.7 MiB) per (device, stream handle), allocated and cleared on first need (the one-launch MVN
-// kernels, vpx_workspace_reserve); nothing else is ever written there.
-int get_sync_area(hipStream_t stream, void** out) {
+// kernels, vpx_workspace_reserve); nothing else is ever written there.  `absent`: for a caller with another way, set in place of an error
+// where the stream is capturing and has none.
+int get_sync_area(hipStream_t stream, void** out, bool* absent) {
     if (t_noalloc) {
         void* base = nullptr;
         const int rc = static_scratch_address(&base);
@@ -147,6 +148,10 @@ int get_sync_area(hipStream_t stream, void** out) {
     std::lock_guard<std::mutex> lock(g_ws_mutex);
     Scratch& sc = g_ws[std::make_pair(dev, stream)];
     if (!sc.sync) {
+        if (absent != nullptr && stream_is_capturing(stream)) {
+            *absent = true;
+            return VPX_RESULT_SUCCESS;
+        }
         VPX_REQUIRE(!stream_is_capturing(stream), VPX_RESULT_ERROR_UNSUPPORTED_FEATURE,
                     "the stream is capturing and has no area for launch counts and records yet: call vpx_workspace_reserve before the capture, "
                     "or use vpx_sw_kernel_launch_noalloc");

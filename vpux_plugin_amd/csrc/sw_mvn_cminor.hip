@@ -490,7 +490,7 @@ int launch_mvn_cminor_resident(const void* in, void* out, int64_t N, int64_t S, 
     // nine tenths of 212 of whole octets and 3 M values or more.
     const float many = 0.6e-3f * (float)S, few = 80.0f / (float)N;
     const float launches_us = 8.0f + (C % 8 == 0 ? 0.95e-6f : 5.4e-6f) * (float)N * (float)S * (float)C + (many < few ? many : few);
-    const auto consider = [&](bool whole, uint32_t ob, uint32_t ob_log, uint32_t nb, uint32_t parts) {
+    const auto consider = [&](bool whole, uint32_t ob, uint32_t ob_log, uint32_t nb, uint32_t parts, bool ahead) {
         const uint32_t of = whole ? rows : (uint32_t)S, slots = kT / ob, per_part = ceil_div(of, parts), v = ceil_div(per_part, slots);
         if (v > kMostWords) return;
         parts = ceil_div(of, per_part);
@@ -502,7 +502,7 @@ int launch_mvn_cminor_resident(const void* in, void* out, int64_t N, int64_t S, 
                            (whole ? 1.04f : parts > 1 ? 0.94f : v <= 16 ? 0.87f : 1.0f);
         // Runs of 16 or 32 bytes and many words a lane are few workgroups, each with the whole image of its channels, dealt a second time: [4,155,155,560] 157
         // us, in three launches 72, [9,137,138,312] 126 / 67, [6,118,136,480] 79 / 59; but [3,110,111,600] 18 / 47.
-        if (ob < 4 && v > 16 && cost >= launches_us) return;
+        if ((ahead || (ob < 4 && v > 16)) && cost >= launches_us) return;
         if (best_v != 0 && cost >= best_cost) return;
         best = Geom{(uint32_t)C, (uint32_t)S, (uint32_t)(S * C), whole ? R : 1, whole ? words : octets, of, whole ? words * 8 : (uint32_t)C, ob, ob_log, nb, parts, per_part,
                     (uint32_t)N * parts};
@@ -518,40 +518,47 @@ int launch_mvn_cminor_resident(const void* in, void* out, int64_t N, int64_t S, 
         if (parts > of / (2 * (kT / ob))) parts = of / (2 * (kT / ob));
         return parts < records ? parts : records;
     };
-    // Octets of channels, where a channel count that is no multiple of eight has a last one that begins inside the one before: in place, the workgroup
-    // of either could find results of the other's.
-    if (C >= 8 && (C % 8 == 0 || in != out))
-        for (int k = 3; k >= 0; k--) {
-            const uint32_t ob = 1u << k, nb = ceil_div(octets, ob);
-            if (ob > 1 && ob / 2 >= octets) continue;
-            consider(false, ob, (uint32_t)k, nb, 1);
-            const uint32_t parts = most_parts((uint32_t)S, ob, (uint32_t)N * nb, kMostRecords / (ob * 8));
-            if (parts > 1 && N * nb <= kMostGroups) {
-                consider(false, ob, (uint32_t)k, nb, parts);
-                // (as many as leave no die with more workgroups than compute units: the others would wait for those that are dealt a second time)
-                const uint32_t even = 8 * (cus_of_die / nb) / (uint32_t)N;
-                if (even > 1 && even < parts) consider(false, ob, (uint32_t)k, nb, even);
+    // exchange: forms whose workgroups exchange sums too; ahead: only what takes less than the three launches
+    const auto pick = [&](bool exchange, bool ahead) {
+        best_v = 0;
+        // Octets of channels, where a channel count that is no multiple of eight has a last one that begins inside the one before: in place, the workgroup
+        // of either could find results of the other's.
+        if (C >= 8 && (C % 8 == 0 || in != out))
+            for (int k = 3; k >= 0; k--) {
+                const uint32_t ob = 1u << k, nb = ceil_div(octets, ob);
+                if (ob > 1 && ob / 2 >= octets) continue;
+                consider(false, ob, (uint32_t)k, nb, 1, ahead);
+                const uint32_t parts = most_parts((uint32_t)S, ob, (uint32_t)N * nb, kMostRecords / (ob * 8));
+                if (exchange && parts > 1 && N * nb <= kMostGroups) {
+                    consider(false, ob, (uint32_t)k, nb, parts, ahead);
+                    // (as many as leave no die with more workgroups than compute units: the others would wait for those that are dealt a second time)
+                    const uint32_t even = 8 * (cus_of_die / nb) / (uint32_t)N;
+                    if (even > 1 && even < parts) consider(false, ob, (uint32_t)k, nb, even, ahead);
+                }
             }
+        if (words <= kT && C <= kT) {
+            consider(true, words, 0, 1, 1, ahead);
+            // (all that are resident read each other's partial sums of every channel: half and a quarter of them less)
+            const uint32_t parts = most_parts(rows, words, (uint32_t)N, kMostRowRecords / (uint32_t)C);
+            for (uint32_t div = 1; exchange && div <= 4 && parts / div > 1 && N <= kMostRowGroups; div *= 2) consider(true, words, 0, 1, parts / div, ahead);
         }
-    if (words <= kT && C <= kT) {
-        consider(true, words, 0, 1, 1);
-        // (all that are resident read each other's partial sums of every channel: half and a quarter of them less)
-        const uint32_t parts = most_parts(rows, words, (uint32_t)N, kMostRowRecords / (uint32_t)C);
-        for (uint32_t div = 1; div <= 4 && parts / div > 1 && N <= kMostRowGroups; div *= 2) consider(true, words, 0, 1, parts / div);
+    };
+    pick(true, false);
+    // In place, a workgroup that computes a partner's partial sums could find results there: those launches take a workgroup alone with its channels, which
+    // reads everything before it writes, or the kernels that finish all reads first.
+    if (best_v != 0 && best.parts > 1 && in == out) pick(false, true);
+    void* sync = nullptr;
+    if (best_v != 0 && best.parts > 1) {
+        bool absent = false;
+        rc = get_sync_area(s, &sync, &absent);
+        if (rc) return rc;
+        sync = (char*)sync + kSyncCminor;
+        if (absent) pick(false, false);  // (a capture on a stream without one)
     }
     if (best_v == 0) return VPX_RESULT_SUCCESS;
-    // In place, a workgroup that computes a partner's partial sums could find results there: those launches take the
-    // kernels that finish all reads first.  (A workgroup alone with its channels reads everything before it writes.)
-    if (best.parts > 1 && in == out) return VPX_RESULT_SUCCESS;
     // A launch holds fewer than 2^32 lanes; small images of many channels ask for more from N * nb = 2^23 on.
     const uint64_t blocks = ((uint64_t)best.units + 7) / 8 * best.nb * 8;
     if (blocks * kT >= (1ull << 32)) return VPX_RESULT_SUCCESS;
-    void* sync = nullptr;
-    if (best.parts > 1) {
-        rc = get_sync_area(s, &sync);
-        if (rc) return rc;
-        sync = (char*)sync + kSyncCminor;
-    }
     const unsigned long long spin = mode == 2 ? 0ull : 50000ull;  // 0.5 ms of the 100 MHz counter
     const dim3 grid((unsigned)blocks);
 #define VPX_CMINOR_AS(V, FORM) \

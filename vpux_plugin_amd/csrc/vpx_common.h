@@ -134,7 +134,7 @@ int get_workspace(hipStream_t stream, size_t bytes, void** out);
 constexpr size_t kSyncCminor = 128 * 1024;  // the channel-minor MVN's part: 128 groups of 2048 records of 16 bytes and 16 of
                                             // 16384, 256 launch counts of 16 bytes for each group
 constexpr size_t kSyncBytes = kSyncCminor + (128 + 16) * (256 * 16) + 128 * (2048 * 16) + 16 * (16384 * 16);
-int get_sync_area(hipStream_t stream, void** out);
+int get_sync_area(hipStream_t stream, void** out, bool* absent = nullptr);
 // Compute units of the current device (cached per device).
 int device_compute_units(int* out);
 // True while the calling thread is inside the entry point that may not allocate: get_workspace() then hands out the
