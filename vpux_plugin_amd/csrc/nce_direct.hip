@@ -227,6 +227,13 @@ __global__ __launch_bounds__(SPLIT ? 64 * kMaxWaves : 256) void nce_direct(const
             use(f[p]);
         }
     }
+    // The first reader of an MFMA's result has to come eight issue slots behind it.  Behind the branches of the walk the compiler keeps them only on the paths
+    // that it takes to be possible -- this condition is the one in use(); on the others there were four with one tile of one block --, so
+    // they are kept here: everything read below goes through the second of these, which come in order.
+    if constexpr (TM * TN == 1) {
+        asm volatile("" : "+v"(acc[0][0]), "+v"(sums[0]));
+        asm volatile("s_nop 7" : "+v"(acc[0][0]), "+v"(sums[0]));
+    }
     if (corrects) {
 #pragma unroll
         for (int i = 0; i < TM; i++)
