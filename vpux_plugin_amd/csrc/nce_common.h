@@ -810,7 +810,7 @@ struct RegbConvLaunch {
     int nt, cus;
 };
 int launch_conv_regb(const RegbConvLaunch& a, hipStream_t s);
-// K steps of 64 of the form that serves K bytes and OC output channels; 0: none
+// K steps of 64 of the form that serves K bytes, of any number of channels and taps, and OC output channels; 0: none
 constexpr int conv_regb_steps(int64_t K, int64_t OC) {
     const int ks = K <= 192 ? 3 : (K <= 320 ? 5 : (K <= 448 ? 7 : (K <= 832 ? 13 : 0)));
     if (OC == 16) return ks;

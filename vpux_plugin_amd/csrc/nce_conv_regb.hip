@@ -1,5 +1,6 @@
-// nce_conv_regb: convolutions of few input channels (16, 32, 48) onto few output channels (16 to 64) at many positions -- the first layers
-// of image networks -- as nce_gemm_regb.hip's product, with the taps of a position in the place of a row of the matrix.
+// nce_conv_regb: convolutions of a short K onto few output channels (16 to 64) at many positions -- the first layers of image networks, 16, 32 or 48 channels
+// under square taps, and wider inputs under few taps (80 under 3x3, 368 under 1x2) -- as nce_gemm_regb.hip's product, with the taps of a position in
+// the place of a row of the matrix.
 //
 // A wave keeps the weights of all its 16 * NT output channels in registers (NT x KS fragments of `v_mfma_i32_16x16x64_i8`, first operand, so that a
 // lane's accumulators are neighbouring bytes of the output) and walks blocks of 16 output positions: KS 16-byte loads a lane straight from global
@@ -12,7 +13,9 @@
 // lanes of a quad read neighbouring words where positions are 32 bytes apart: 4 % slower, it is not the cache's banks.
 // us in a HIP graph, nce_conv_rows16 or nce_conv_strips / here: [14,338,585,16] -> 16 3x3 stride 2 24.5 / 12.0, [8,521,314,16] -> 32 13.8 / 9.5,
 // [32,224,224,16] -> 32 14.4 / 10.9, [6,349,320,48] -> 32 19.3 / 10.0, [5,593,523,16] -> 16 7x7 stride 2 23.4 / 19.2, [18,88,88,48] -> 48 3x3
-// 13.3 / 11.1, [9,367,486,16] -> 64 3x3 stride 2 19.9 / 17.9; nce_direct / here: [3,376,640,16] -> 16 3x3 stride 2 8.0 / 6.0.
+// 13.3 / 11.1, [9,367,486,16] -> 64 3x3 stride 2 19.9 / 17.9; nce_direct / here: [3,376,640,16] -> 16 3x3 stride 2 8.0 / 6.0.  Wider inputs, nce_conv_rows16
+// or nce_direct / here: [14,109,164,80] -> 16 2x2 12.7 / 8.1, [13,168,87,240] -> 16 3x1 stride 2 25.0 / 7.9, [26,268,159,80] -> 48 2x2 stride 2 34.2 / 20.2, [30,74,79,96]
+// -> 16 2x1 8.1 / 6.1; 150 drawn layers of 80 to 368 channels take 0.82 of the time, one is more than 3 % slower ([2,233,391,144] -> 16 1x2 stride 2 4.6 / 4.8).
 #include <algorithm>
 
 #include "nce_common.h"
