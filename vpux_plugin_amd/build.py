@@ -14,9 +14,8 @@ HOST_SOURCES = ["host/compiler_utils.cpp"]
 
 # -ffp-contract=off: fp32 expressions must round as written (FakeQuantize / Quantize parity).
 # packed-fp32 VALU forms are switched off for every HIP translation unit.
-# TLS descriptors: a thread's own variables of a library that is loaded late cost a call through __tls_get_addr each time (0.02 ... 0.08 us) otherwise.
 HIP_FLAGS = ["--offload-arch=gfx950", "-O3", "-std=c++17", "-fPIC", "-ffp-contract=off", "-fvisibility=hidden",
-             "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops", "-Xarch_host", "-mtls-dialect=gnu2", "-Wall", "-Wno-unused-function"]
+             "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops", "-Wall", "-Wno-unused-function"]
 
 
 def build(verbose=True, jobs=8):
@@ -75,7 +74,9 @@ def build_binding(verbose=True):
         sys.stderr.write("%s is not built: %s not found (the C library and its hosts do not need it)\n" % (os.path.basename(BINDING), ", ".join(absent)))
         return False
     rocm = os.environ.get("ROCM_PATH", "/opt/rocm")
-    cmd = [os.environ.get("CXX", "g++"), "-O2", "-std=c++17", "-fPIC", "-shared", "-fvisibility=hidden", "-mtls-dialect=gnu2", "-Wall", "-D__HIP_PLATFORM_AMD__", "-DUSE_ROCM",
+    # -DNDEBUG: torch's headers bring a counter of pybind11's with them otherwise, thread-local storage that no call comes to.  While a thread has not come
+    # to the storage of the library that was loaded last, the C library (2.35) takes the long way for every lookup of every library in it: 0.1 ... 0.3 us a call.
+    cmd = [os.environ.get("CXX", "g++"), "-O2", "-DNDEBUG", "-std=c++17", "-fPIC", "-shared", "-fvisibility=hidden", "-Wall", "-D__HIP_PLATFORM_AMD__", "-DUSE_ROCM",
            "-D_GLIBCXX_USE_CXX11_ABI=%d" % torch._C._GLIBCXX_USE_CXX11_ABI, "-I", os.path.join(ROOT, "include")]
     for d in (os.path.join(top, "include"), os.path.join(rocm, "include"), python):
         cmd += ["-isystem", d]
