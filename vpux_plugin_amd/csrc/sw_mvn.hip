@@ -1632,7 +1632,9 @@ int launch_rows_of(const half_t* pi, half_t* po, const half_t* ps, const half_t*
     const bool half768 = shared_rows && row_len == 768;  // 32 lanes x 3 words, none idle: pays with scale / bias
     const int team = row_len <= 256 || half768 ? 32 : 64;
     const int64_t team_rows = g.rows / (kThreads / team);
-    const int rpt = !shared_rows ? 1 : team_rows >= 4 * 4096 ? 4 : team_rows >= 2 * 4096 ? 2 : 1;
+    // (two rows of three words a lane and more only where they are whole words: with the values that words share the registers run out, and a row at a time is ahead;
+    // us, two / one: [40382 x 1233] 42.6 / 35.8, [62548 x 1322] 75.3 / 58.8, [39878 x 1606] 55.0 / 43.8, [58293 x 2031] 109.4 / 108.3)
+    const int rpt = !shared_rows ? 1 : team_rows >= 4 * 4096 ? 4 : team_rows >= 2 * 4096 && (words || (row_len <= 1024 && !half768)) ? 2 : 1;
 #define VPX_MVN6_ROWS_R(TEAM, VPT, RPT)                                                                                      \
     do {                                                                                                                     \
         constexpr int T = team_threads(TEAM), PER = RPT * (T / TEAM);                                                        \
@@ -1640,7 +1642,7 @@ int launch_rows_of(const half_t* pi, half_t* po, const half_t* ps, const half_t*
         if (words)                                                                                                           \
             VPX_LAUNCH((mvn6_rows_kernel<GEOM, TEAM, VPT, RPT, true>), grid, dim3(T), 0, s, pi, po, ps, pb, g, nv,                 \
                        eps_mode, eps);                                                                                       \
-        else                                                                                                                 \
+        else if constexpr (RPT != 2 || VPT <= 2)                                                                             \
             VPX_LAUNCH((mvn6_rows_kernel<GEOM, TEAM, VPT, RPT, false>), grid, dim3(T), 0, s, pi, po, ps, pb, g, nv,                \
                        eps_mode, eps);                                                                                       \
     } while (0)
