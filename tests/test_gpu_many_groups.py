@@ -1,10 +1,10 @@
-"""Tensors of so many short groups or rows that one workgroup for every few of them would be more lanes than a launch holds, 2^32.  About 13 GB of device memory."""
+"""Tensors of so many short groups or rows that one workgroup for every few of them would be more lanes than a launch holds, 2^32.  About 30 GB of device memory."""
 import pytest
 
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("groups,len_", [((1 << 29) + 3, 2), ((1 << 29) + 40, 7), ((1 << 27) + 11, 24)])
+@pytest.mark.parametrize("groups,len_", [((1 << 29) + 3, 2), ((1 << 29) + 40, 7), ((1 << 27) + 11, 24), ((1 << 26) + 11, 104)])
 def test_groups(rt, dev, groups, len_):
     import torch
     x = torch.empty((groups, len_), dtype=torch.float16, device=dev).normal_(0, 2, generator=torch.Generator(device="cuda").manual_seed(len_))

@@ -471,18 +471,21 @@ static int launch_tiny_groups(const half_t* in, half_t* out, int64_t groups, int
 
 // Groups a workgroup takes: what its eight half-wavefronts walk one after another.  As many as fill kSmallChunk, 37 of 110 values, left a small
 // tensor to a few workgroups with a long walk each and a large one waiting for it too (us, that many / these): [512 x 7] 24.6 / 3.3,
-// [16384 x 21] 12.9 / 4.4, [65536 x 110] 12.1 / 9.6, [65536 x 361] 22.8 / 19.7, [131072 x 49] 16.5 / 12.6.
+// [16384 x 21] 12.9 / 4.4, [65536 x 110] 12.1 / 9.6, [65536 x 361] 22.8 / 19.7, [131072 x 49] 16.5 / 12.6.  Sixteen in place of eight where groups of up to 256
+// values are many: eight / these [308452 x 130] 41.2 / 36.3, [237176 x 217] 37.1 / 32.8, [176306 x 166] 25.7 / 23.6.
 static int small_groups_run(int64_t groups, int64_t len) {
-    const int64_t fits = kSmallChunk / len, most = len <= 64 ? (groups < 16384 ? 8 : 32) : len > 128 ? 8 : groups < (1 << 18) ? 16 : fits;
+    const int64_t fits = kSmallChunk / len, most = len <= 64 ? (groups < 16384 ? 8 : 32) : len > 128 ? (len <= 256 && groups >= (1 << 17) ? 16 : 8) : groups < (1 << 18) ? 16 : fits;
     return (int)(fits < most || groups / most >= (1 << 24) - 1 ? fits : most);  // (a launch holds fewer than 2^32 lanes)
 }
 // Whether the short-group form applies, and its launch.  It serves what the registers of mvn6_rows_kernel do not, groups of fewer than eight
 // values, and many groups of up to 512 that are no whole number of words: a row of those leaves most of a team's lanes idle or ends in a word that
 // two lanes take.  us in a HIP graph, that kernel / this one: [448 x 110] 3.2 / 3.3, [1024 x 390] 3.3 / 4.2, [8192 x 361] 5.85 / 5.83,
 // [65536 x 110] 12.3 / 9.6, [131072 x 390] 25.6 / 20.6 a half of them, [131072 x 49] 20.0 / 12.6; but [16384 x 675] 11.6 / 13.7, [16384 x 784] 10.1 / 14.2.
+// Of whole words it serves up to twelve, which leave two thirds of that kernel's lanes idle, where they are so many that memory does not hide it:
+// [315392 x 24] 25.7 / 20.0, [1056847 x 24] 83.8 / 60.1, [494619 x 56] 41.2 / 32.4, [648482 x 72] 53.9 / 48.5, [403511 x 96] 35.7 / 33.5; even at 2^18.
 static bool small_groups_ok(const half_t* in, const half_t* out, int64_t groups, int64_t len) {
     const int64_t run = len >= 1 ? small_groups_run(groups, len) : 1;
-    return len >= 1 && groups >= 64 && (len < 8 || (groups > 8192 && len <= 512 && len % 8 != 0)) &&
+    return len >= 1 && groups >= 64 && (len < 8 || (groups > 8192 && len <= 512 && len % 8 != 0) || (groups >= (1 << 18) && len <= 96)) &&
            ((reinterpret_cast<uintptr_t>(in) | reinterpret_cast<uintptr_t>(out)) & 15) == 0 && (groups + run - 1) / run < (1ll << 31);
 }
 static int launch_small_groups(const half_t* in, half_t* out, int64_t groups, int64_t len, int nv, int eps_mode, float eps, hipStream_t s) {
