@@ -997,7 +997,11 @@ int softmax_typed(const SoftmaxPlan& p, const T* in, T* out, hipStream_t s) {
                 half_t* to = hout + r0 * len;
                 const auto form = [&](auto team_c, auto words_c) -> int {
                     constexpr int LANES = decltype(team_c)::value, WORDS = decltype(words_c)::value;
-                    if (once) VPX_LAUNCH((softmax_packed_rows<LANES, WORDS, true>), grid, dim3(256), 0, s, from, to, n, (uint32_t)len);
+                    // (Rows of 129 to 256 values in two words a lane end within lines in every fourth word of a wave's store, which go better through the caches,
+                    // us, past them / through them, buffers that change from call to call: [180443 x 249] 35.6 / 33.7, [249737 x 180] 34.7 / 32.6; that stay:
+                    // 33.9 / 27.5, 34.4 / 27.1.  Of other rows those that stay gain as much, those that change lose 3 ... 8 %.)
+                    constexpr bool kLines = LANES == 16 && WORDS == 2;
+                    if (once && !kLines) VPX_LAUNCH((softmax_packed_rows<LANES, WORDS, !kLines>), grid, dim3(256), 0, s, from, to, n, (uint32_t)len);
                     else VPX_LAUNCH((softmax_packed_rows<LANES, WORDS, false>), grid, dim3(256), 0, s, from, to, n, (uint32_t)len);
                     return VPX_RESULT_SUCCESS;
                 };
