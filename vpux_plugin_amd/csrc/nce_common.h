@@ -791,7 +791,7 @@ int launch_conv_strips(const StripLaunch& a, hipStream_t s);
 struct RegbConvGeom {
     int P, nblk;         // output positions, blocks of 16 of them
     int chunks;          // K / 16
-    int OC, H, W, isn, ish, isw, osn, osh, osw;
+    int H, W, isn, ish, isw, osn, osh, osw;
     int SY, SX, PT, PL;
     int OH, ow, ohow;
     int oy_lo, oy_n, ox_lo, ox_n;  // output rows and columns whose windows lie inside the image: the first, and how many

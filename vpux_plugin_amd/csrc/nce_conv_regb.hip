@@ -34,7 +34,6 @@ __global__ __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_eu(EU)
     const int tid = threadIdx.x, lane = tid & 63;
     const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int n16 = lane & 15, c4 = lane >> 4;
-    const int n0 = (int)blockIdx.y * TCH, N = g.OC;
     // Every die has a run of blocks of its own, which its waves walk side by side: the rows that neighbouring blocks share are in its cache.
     const int nwg = (int)gridDim.x, dies = (nwg & 7) == 0 ? 8 : 1;
     const int die = (int)blockIdx.x & (dies - 1), step = nwg / dies * kWaves;
@@ -55,14 +54,14 @@ __global__ __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_eu(EU)
     i32x4 wb[NT][KS];
 #pragma unroll
     for (int j = 0; j < NT; j++) {
-        const int ch = n0 + (n16 >> 2) * (4 * NT) + j * 4 + (n16 & 3);
+        const int ch = (n16 >> 2) * (4 * NT) + j * 4 + (n16 & 3);
 #pragma unroll
         for (int ks = 0; ks < KS; ks++) {
             const int c = ks * 4 + c4;
             wb[j][ks] = *reinterpret_cast<const i32x4*>(wts + ((int64_t)ch * g.chunks + (c < g.chunks ? c : 0)) * 16);
         }
     }
-    const int2 words = *reinterpret_cast<const int2*>(wt + (int64_t)(n0 + (tid < TCH ? tid : 0)) * 4 + 2);
+    const int2 words = *reinterpret_cast<const int2*>(wt + (tid < TCH ? tid : 0) * 4 + 2);
 #pragma unroll
     for (int j = 0; j < NT; j++)
 #pragma unroll
@@ -126,7 +125,7 @@ __global__ __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_eu(EU)
         oy = (int)quotient(rem, (unsigned)g.ow, g.ow_magic);
         ox = (int)rem - oy * g.ow;
         src = img * (unsigned)g.isn + (unsigned)((oy * g.SY - g.PT) * g.ish + (ox * g.SX - g.PL) * g.isw);
-        dst = img * (unsigned)g.osn + (unsigned)(oy * g.osh + ox * g.osw + n0 + c4 * (4 * NT));
+        dst = img * (unsigned)g.osn + (unsigned)(oy * g.osh + ox * g.osw + c4 * (4 * NT));
     }
     const unsigned by = (unsigned)step * 16, by_img = by / (unsigned)g.ohow, by_rem = by - by_img * (unsigned)g.ohow, by_oy = by_rem / (unsigned)g.ow,
                    by_ox = by_rem - by_oy * (unsigned)g.ow;
@@ -268,7 +267,7 @@ int launch_conv_regb(const RegbConvLaunch& a, hipStream_t s) {
     const auto launch = [&](auto kernel, int per_cu) -> int {
         // as many as are resident at once, or one for every four blocks; whole dies
         const int64_t wgs = std::min<int64_t>((int64_t)a.cus * per_cu, ((int64_t)a.g.nblk + 8 * kWaves - 1) / (8 * kWaves) * 8);
-        VPX_LAUNCH(kernel, dim3((unsigned)wgs, (unsigned)(a.g.OC / (16 * a.nt))), dim3(64 * kWaves), 0, s, a.in, a.w, a.wt, a.out, a.g, a.ppe, sign_flip);
+        VPX_LAUNCH(kernel, dim3((unsigned)wgs), dim3(64 * kWaves), 0, s, a.in, a.w, a.wt, a.out, a.g, a.ppe, sign_flip);
         return VPX_RESULT_SUCCESS;
     };
     const auto by_taps = [&](auto same_c, auto nt_c) -> int {

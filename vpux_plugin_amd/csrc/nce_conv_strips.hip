@@ -135,8 +135,10 @@ __global__ __launch_bounds__(64 * kStripWaves) void nce_conv_strips(const int8_t
                 }
             }
         };
-        if (REST && g.PH > ROWS) rest(ROWS, g0);
-        if (REST && g.row_chunks > 64) rest(0, g1);
+        if constexpr (REST) {
+            if (g.PH > ROWS) rest(ROWS, g0);
+            if (g.row_chunks > 64) rest(0, g1);
+        }
     };
 
     int wt2 = 0, wt3 = 0;  // this thread's channel of the weight table, asked for before anything else
