@@ -33,3 +33,25 @@ def test_outputs_are_the_nearest(rt, dev, words, first, others):
     half_unit = torch.exp2(torch.floor(torch.log2(z.abs())) - 11)
     more = ((y[:, -LANES:].double() - z).abs() - half_unit) / z.abs()
     assert float(more[z.abs() >= 0.5].max()) <= (words / 2 + 17) * 2.0 ** -25 + 8 * 2.0 ** -24
+
+
+@pytest.mark.parametrize("words", [1, 8, 24, 52])
+def test_the_mean_where_the_first_slice_lies_far_off(rt, dev, words):
+    """Values next to the mean show how far off it is."""
+    import torch
+    g = torch.Generator(device="cuda").manual_seed(words)
+    x = torch.randn((256, words * LANES), device=dev, generator=g) * 0.02
+    x[0] += 8.0
+    x = x.half()
+    y = torch.empty_like(x)
+    rt.mvn(x.view(1, 1, 256, -1), y.view(1, 1, 256, -1), True, True, 1e-9, "NCHW")
+    mean = float(x.double().sum()) / x.numel()
+    deviation = (float((x.double() - mean).square().sum()) / x.numel() + 1e-9) ** 0.5
+    z = (x.double() - mean) / deviation
+    near = z.abs() < 2.0 ** -9
+    # half a unit of fp16, and the mean: rounded to 2^-24 of itself in three steps (slices, their meeting, the last sum), and slices' means of 2^-24 of a
+    # slice's largest in 256 of them, of which the errors of 16 add up
+    half_unit = torch.exp2(torch.floor(torch.log2(z.abs())).clamp(min=-14) - 11)
+    more = (y.double() - z).abs() - half_unit
+    assert int(near.sum()) > 1000
+    assert float(more[near].max()) <= (3 * abs(mean) + 0.1 * 16 / 256) * 2.0 ** -24 / deviation + 2.0 ** -33

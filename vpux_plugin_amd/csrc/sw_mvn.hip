@@ -689,16 +689,15 @@ __device__ __forceinline__ Moments slice_moments(Slice<V>& sl, Moments* red) {
     __syncthreads();  // the previous use of `red` is over
     if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = Moments{n, mean, q};
     __syncthreads();
-    // all at once (a tree of pairwise merges is three reciprocals in a row), about the mean as found from the distances to the first one's, which what
-    // is left of those about it then corrects: the first one may lie far from the others
+    // all at once (a tree of pairwise merges is three reciprocals in a row), about their mean, which the distances to it then correct by what was rounded off
     Moments w[T / 64];
 #pragma unroll
     for (int k = 0; k < T / 64; k++) w[k] = red[k];
     const float count = sl.count, inv_count = 1.f / count;
-    float shift = 0.f, rest = 0.f, m2 = 0.f;
+    float all = 0.f, rest = 0.f, m2 = 0.f;
 #pragma unroll
-    for (int k = 0; k < T / 64; k++) shift += w[k].n * (w[k].mean - w[0].mean);
-    mean = w[0].mean + over(shift, count, inv_count);
+    for (int k = 0; k < T / 64; k++) all += w[k].n * w[k].mean;
+    mean = over(all, count, inv_count);
 #pragma unroll
     for (int k = 0; k < T / 64; k++) {
         const float d = w[k].mean - mean;
@@ -774,23 +773,35 @@ __global__ __launch_bounds__(T) void mvn_fused_kernel(const half_t* __restrict__
                 if (ok || !waits || wall_clock64() - t0 >= spin_ticks) break;  // (pausing between polls measured slower)
             }
             if (ok || !waits) {
-                // all at once, as the wavefronts' in slice_moments (a butterfly of pairwise merges: six reciprocals in a row)
+                // All at once, about the first slice's mean, in a fixed order (a butterfly of pairwise merges: six reciprocals in a row).  Where that lies
+                // further than a deviation from the whole's, about the latter, which the distances to it correct by what was rounded off (for
+                // every launch: 0.1 us).
                 const auto value = [&](int k) { return __builtin_bit_cast(float, (unsigned)rm[k]); };
                 const float first = lane_bcast(value(0), 0);
-                float shift = 0.f, rest = 0.f, m2 = 0.f;
+                float shift = 0.f, m2 = 0.f;
                 const auto count = [&](int i) { return i >= wpg ? 0.f : i + 1 < wpg ? (float)slice : (float)(group_size - (uint32_t)i * slice); };
+                const auto off = [&](int k, float from) { return k * 64 + lane < wpg ? value(k) - from : 0.f; };
+                const auto squares = [&](int k, float d) { return k * 64 + lane < wpg ? __builtin_bit_cast(float, (unsigned)rq[k]) + count(k * 64 + lane) * d * d : 0.f; };
 #pragma unroll
-                for (int k = 0; k < kMergeInKernel / 64; k++) shift += k * 64 + lane < wpg ? count(k * 64 + lane) * (value(k) - first) : 0.f;
-                const float mean = first + over(wave_sum_soon(shift), group_count, inv_count);
+                for (int k = 0; k < kMergeInKernel / 64; k++) shift += count(k * 64 + lane) * off(k, first);
+                shift = over(wave_sum_soon(shift), group_count, inv_count);
 #pragma unroll
-                for (int k = 0; k < kMergeInKernel / 64; k++) {
-                    const float d = k * 64 + lane < wpg ? value(k) - mean : 0.f;
-                    rest += count(k * 64 + lane) * d;
-                    m2 += k * 64 + lane < wpg ? __builtin_bit_cast(float, (unsigned)rq[k]) + count(k * 64 + lane) * d * d : 0.f;
-                }
+                for (int k = 0; k < kMergeInKernel / 64; k++) m2 += squares(k, off(k, first) - shift);
                 m2 = wave_sum_soon(m2);
-                rest = wave_sum_soon(rest);
-                if (lane == 0) shared_total = Moments{group_count, mean + over(rest, group_count, inv_count), m2};
+                float mean = first + shift;
+                if (shift * shift * group_count > m2) {  // (the same for the wavefront)
+                    float rest = 0.f;
+                    m2 = 0.f;
+#pragma unroll
+                    for (int k = 0; k < kMergeInKernel / 64; k++) {
+                        const float d = off(k, mean);
+                        rest += count(k * 64 + lane) * d;
+                        m2 += squares(k, d);
+                    }
+                    m2 = wave_sum_soon(m2);
+                    mean += over(wave_sum_soon(rest), group_count, inv_count);
+                }
+                if (lane == 0) shared_total = Moments{group_count, mean, m2};
             }
             return ok;
         };
