@@ -35,10 +35,10 @@ METRIC = "int8 conv/matmul TOPS (% MFMA peak); SW-kernel GB/s (% HBM peak)"
 # WRITE_SIZE counters of an earlier run of the same workload, scaled by a plain copy of known size
 # (profiles/<workload>__*.md hold those runs and their commands); the JSON line labels them as such.
 MEASURED_TRAFFIC = {
-    "c1_fake_quantize": 888450, "c2_softmax": 134261983, "c3_mvn": 17093583, "c4_conv": 14913796,
+    "c1_fake_quantize": 888450, "c2_softmax": 134261983, "c3_mvn": 17111040, "c4_conv": 14913796,
     "c5_matmul": 339794672, "c5_dequantize": 135262411, "c5_eltwise_add": 270552950, "c5_nce_eltwise": 135260008,
     "calib_copy": 134217728, "calib_int_mm": 534882288, "x_mvn6_layernorm": 268564672, "x_activation_hswish": 180471319,
-    "x_mvn1_three_steps": 25341653, "x_stem_conv": 54509346, "x_small_plane_conv": 20886567, "x_large_conv": 54601720,
+    "x_mvn1_three_steps": 25341653, "x_stem_conv": 54125568, "x_small_plane_conv": 20886567, "x_large_conv": 54601720,
     "x_wide_conv": 58733750, "x_pointwise_conv": 32401682, "x_softmax_outer_axis": 402620437, "x_mvn_nhwc_per_channel": 212576856,
 }
 

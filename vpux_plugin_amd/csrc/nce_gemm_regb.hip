@@ -191,6 +191,8 @@ __global__ __launch_bounds__(64 * kRegbWaves) __attribute__((amdgpu_waves_per_eu
         for (int ks = 0; ks < KS; ks++)
 #pragma unroll
             for (int j = 0; j < NT; j++) acc[j] = __builtin_amdgcn_mfma_i32_16x16x64_i8(wb[cbl][j][ks], f[ks], acc[j], 0, 0, 0);
+        // (a condition between MFMAs and the first reader of their results, which has to come eight issue slots behind: a unit has two MFMAs at the least, the
+        // second of which the matrix unit takes when it is through with the first, and the compiler keeps the slots of the last on both sides of the branch)
         if (rt) {
 #pragma unroll
             for (int j = 0; j < NT; j++) acc[j] += rowterm;
