@@ -352,7 +352,7 @@ int launch_gemm_regb(const GemmLaunch& a, const RegbShape& r, int workgroups, hi
     // the cache / past it, us, alone: [25088 x 64] . [64 x 256] 6.0 / 5.2, [100352 x 64] . [64 x 128] 9.2 / 7.4, [25088 x 128] . [128
     // x 512] 12.3 / 10.5; with the eltwise that reads the result 11.4 / 10.9, 18.7 / 17.6, 21.7 / 21.2.  A larger one is found in the
     // Infinity Cache by the next call, which gains what the store lost: [100352 x 64] . [64 x 256] 13.7 / 10.7 alone, but in a
-    // residual block (three convolutions and the eltwise) 46.0 / 46.7; [401408 x 64] . [64 x 256] 39.3 / 36.3, with the eltwise 84 / 87.
+    // residual block (three convolutions and the eltwise) 41.2 / 42.5; [401408 x 64] . [64 x 256] 39.3 / 36.3, with the eltwise 84 / 87.
     // Rows that begin inside a line share it with their neighbours and are left to the cache to put together ([100352 x 64] .
     // [64 x 192] 11.8 / 11.8, with the eltwise 23.6 / 24.3).
     const int nch = 16 * r.nt * r.cbw;
